@@ -125,29 +125,39 @@ def row_offsets(flags: torch.Tensor, S: int) -> torch.Tensor:
     return out
 
 
-def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Tensor, n_kv: int, scratch=None) -> Page:
-    """Encode x (bf16 [H, S, D], on the GPU) with the given bases.  Two launches: every tile is encoded with its escapes in a worst-case
-    slot, then the slots are packed head by head into one stream (the steps of encoder.py:111-123)."""
+def rows_in_place(x: torch.Tensor, head_dim: int, row_dim: int) -> tuple[torch.Tensor, int, int]:
+    """(x, head stride, row stride) for the encoder, which reads [., ., 128] elements through any strides as long as a row is 16-byte
+    aligned and contiguous; other layouts are copied first."""
+    hs, rs = x.stride(head_dim) if x.shape[head_dim] > 1 else 0, x.stride(row_dim) if x.shape[row_dim] > 1 else D
+    if x.stride(2) == 1 and rs >= D and rs % 8 == 0 and hs % 8 == 0 and x.data_ptr() % 16 == 0: return x, hs, rs
+    x = x.clone(memory_format=torch.contiguous_format)
+    strides = (x.shape[1] * D, D)
+    return x, strides[head_dim], strides[row_dim]
+
+
+def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Tensor, n_kv: int) -> Page:
+    """Encode x (bf16 [H, S, D], on the GPU) with the given bases.  Three launches: every tile is encoded with its escapes in a worst-case
+    slot; the sizes of the slots are scanned per head; then, with the stream sized by the host (the totals arrive in host memory that
+    the scan writes to), the slots are packed head by head and the row offsets written (the steps of encoder.py:111-123)."""
     H, S, _ = x.shape
     dev = x.device
-    x = x.contiguous()
+    x, hs, rs = rows_in_place(x, 0, 1)
     S_pad = (S + T - 1) // T * T
-    ntiles = S_pad // T
-    sm = torch.empty(H, S_pad * D, dtype=torch.uint8, device=dev)
-    cd = torch.empty(H, S_pad * CB, dtype=torch.uint8, device=dev)
-    flags = torch.empty(H, S_pad, dtype=torch.int32, device=dev)
-    slots = scratch(H * ntiles * TILE_MAX_ESC, dev) if scratch else torch.empty(H * ntiles * TILE_MAX_ESC, dtype=torch.uint8, device=dev)
-    tile_bytes = torch.empty(H, ntiles, dtype=torch.int32, device=dev)
-    k = 0 if kind == "k" else 1
-    _lib.call("gaac_encode_tiles", k, _lib.ptr(x), S * D, D, H, S, S_pad, _lib.ptr(base3), _lib.ptr(base4), n_kv, None,
-              _lib.ptr(sm), _lib.ptr(cd), _lib.ptr(flags), _lib.ptr(slots), _lib.ptr(tile_bytes), _lib.stream())
-    head_bytes = tile_bytes.sum(1)
-    head_start = torch.cat([torch.zeros(1, dtype=torch.int64, device=dev), torch.cumsum(head_bytes, 0)]).to(torch.int32).contiguous()
-    ovf = torch.zeros(int(head_start[-1]) + 8, dtype=torch.uint8, device=dev)
-    tile_off = torch.empty_like(tile_bytes)
-    _lib.call("gaac_compact", _lib.ptr(slots), _lib.ptr(tile_bytes), _lib.ptr(tile_off), _lib.ptr(head_start), _lib.ptr(ovf),
-              H, ntiles, _lib.stream())
-    return Page(sm, cd, flags, row_offsets(flags, S), ovf, head_start, tile_off, base3, base4, H, S, n_kv, kind)
+    nt = H * (S_pad // T)
+    new = lambda *shape, dtype=torch.uint8: torch.empty(shape, dtype=dtype, device=dev)
+    sm, cd, slots = new(H, S_pad * D), new(H, S_pad * CB), new(nt * TILE_MAX_ESC)
+    flags, ovf_off, tile_off = new(H, S_pad, dtype=torch.int32), new(H, S, dtype=torch.int32), new(H, S_pad // T, dtype=torch.int32)
+    head_start, sizes = new(H + 1, dtype=torch.int32), new(nt + H, dtype=torch.int32)      # sizes: per tile, then per head
+    totals = torch.empty(H, dtype=torch.int32, pin_memory=True)
+    p, st = _lib.ptr, _lib.stream()
+    tile_bytes, head_bytes = p(sizes), p(sizes) + 4 * nt
+    _lib.call("gaac_encode_tiles", 0 if kind == "k" else 1, p(x), hs, rs, H, S, S_pad, p(base3), p(base4), n_kv, None,
+              p(sm), p(cd), p(flags), p(slots), tile_bytes, st)
+    _lib.call("gaac_tile_scan", tile_bytes, H, S_pad // T, p(tile_off), head_bytes, totals.data_ptr(), st)
+    torch.cuda.current_stream(dev).synchronize()
+    ovf = new(sum(totals.tolist()) + 8)
+    _lib.call("gaac_page_pack", p(slots), tile_bytes, p(tile_off), head_bytes, p(flags), H, S, S_pad, p(head_start), p(ovf), p(ovf_off), st)
+    return Page(sm, cd, flags, ovf_off, ovf, head_start, tile_off, base3, base4, H, S, n_kv, kind)
 
 
 class Codec:

@@ -79,77 +79,162 @@ __global__ void __launch_bounds__(256) k_bases_from_hist(const long long* __rest
 }
 
 // ---------------------------------------------------------------------------------------------------- page encoder
-// A block of four waves takes 16 consecutive tiles of one head, wave w the tiles w, w+4, w+8, w+12 of them (one-wave blocks, one per
-// tile, would be limited by the rate at which workgroups can be launched).  The rows of a wave's next tile are fetched into
-// registers while it encodes the current one.
-constexpr int CODEC_WAVES = 4, CODEC_TPW = 4, CODEC_TPB = CODEC_WAVES * CODEC_TPW;
-template <int KIND>
-__global__ void __launch_bounds__(64 * CODEC_WAVES) k_encode_tiles(const u16* __restrict__ x, int S, long x_head_stride, long x_row_stride, int S_pad,
-                                                                   const uint8_t* __restrict__ base3, const uint8_t* __restrict__ base4,
-                                                                   int n_kv, const int* __restrict__ bidx, uint8_t* __restrict__ sm,
-                                                                   uint8_t* __restrict__ cd, int* __restrict__ flags,
-                                                                   uint8_t* __restrict__ esc_slots, int* __restrict__ tile_bytes, int ntiles) {
-  __shared__ EncodeLds Ls[CODEC_WAVES];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = blockIdx.y;
-  EncodeLds& L = Ls[wave];
-  const int brow = bidx ? bidx[h] : h % n_kv;
-  int tile = blockIdx.x * CODEC_TPB + wave;
-  if (tile >= ntiles) return;
-  const u16* xh = x + (long)h * x_head_stride;
+// A block of four waves takes 4 * TPW consecutive tiles of one head, wave w the tiles w, w+4, ... of them (one-wave blocks, one per tile,
+// would be limited by the rate at which workgroups can be launched).  The rows of a wave's next tile are fetched into registers while it
+// encodes the current one.  K and V of a prompt share a launch (blockIdx.z): one start-up and one drain for both.
+constexpr int CODEC_WAVES = 4;
+struct EncodeKind {      // one of K, V
+  const u16* x; long head_stride, row_stride;
+  const uint8_t* b3; const uint8_t* b4;
+  uint8_t* sm; uint8_t* cd; int* flags;            // head 0 of the call; token stride S_pad
+  uint8_t* slots; int* tile_bytes;                 // [H][ntiles] worst-case escape slots and the bytes used in each
+};
+struct EncodeArgs { EncodeKind k, v; int kind0, S, S_pad, ntiles, brow0, NB; const int* bidx; };      // blockIdx.z = 0 is kind0
+template <int KIND, int TPW>
+__device__ __forceinline__ void encode_tiles_body(const EncodeArgs& A, const EncodeKind& J, EncodeLds& L, int h, int tile, int lane) {
+  const int S = A.S, ntiles = A.ntiles;
+  const int brow = A.bidx ? A.bidx[h] : (A.brow0 + h) % A.NB;
+  const u16* xh = J.x + (long)h * J.head_stride;
   RowRegs R, Rn;
-  load_rows(R, xh + (long)tile * T * x_row_stride, x_row_stride, min(T, S - tile * T), lane);
-  stage_bases(L, base3 + (long)brow * D, base4 + (long)brow * D, lane);
+  load_rows(R, xh + (long)tile * T * J.row_stride, J.row_stride, min(T, S - tile * T), lane);
+  stage_bases(L, J.b3 + (long)brow * D, J.b4 + (long)brow * D, lane);
   wave_lds_sync();
   BaseRegs Bs;                // the base words of the lane's units: the same for every tile of the head
   load_base_regs<KIND>(L, lane & 15, lane >> 4, Bs);
-  for (int i = 0; i < CODEC_TPW && tile < ntiles; ++i, tile += CODEC_WAVES) {
+  for (int i = 0; i < TPW && tile < ntiles; ++i, tile += CODEC_WAVES) {
     const int nvalid = min(T, S - tile * T), next = tile + CODEC_WAVES;
     store_rows(L, R, lane);
-    if (i + 1 < CODEC_TPW && next < ntiles) load_rows(Rn, xh + (long)next * T * x_row_stride, x_row_stride, min(T, S - next * T), lane);
+    if (i + 1 < TPW && next < ntiles) load_rows(Rn, xh + (long)next * T * J.row_stride, J.row_stride, min(T, S - next * T), lane);
     wave_lds_sync();
-    const long row0 = (long)h * S_pad + (long)tile * T;
-    const int total = encode_staged_tile<KIND>(L, Bs, nvalid, lane, sm + row0 * D, cd + row0 * CB, flags + row0,
-                                               esc_slots + ((long)h * ntiles + tile) * TILE_MAX_ESC);
-    if (lane == 0) tile_bytes[(long)h * ntiles + tile] = total;
+    const long row0 = (long)h * A.S_pad + (long)tile * T;
+    const int total = encode_staged_tile<KIND>(L, Bs, nvalid, lane, J.sm + row0 * D, J.cd + row0 * CB, J.flags + row0,
+                                               J.slots + ((long)h * ntiles + tile) * TILE_MAX_ESC);
+    if (lane == 0) J.tile_bytes[(long)h * ntiles + tile] = total;
     wave_lds_sync();          // the staged rows and tag words are free again
     R = Rn;
   }
 }
+template <int TPW>
+__global__ void __launch_bounds__(64 * CODEC_WAVES) k_encode_tiles(const EncodeArgs A) {
+  __shared__ EncodeLds Ls[CODEC_WAVES];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, tile = blockIdx.x * (CODEC_WAVES * TPW) + wave;
+  if (tile >= A.ntiles) return;
+  if (A.kind0 + (int)blockIdx.z == KIND_K) encode_tiles_body<KIND_K, TPW>(A, A.k, Ls[wave], blockIdx.y, tile, lane);
+  else encode_tiles_body<KIND_V, TPW>(A, A.v, Ls[wave], blockIdx.y, tile, lane);
+}
+static void launch_encode(const EncodeArgs& A, int H, int kinds, hipStream_t stream) {
+  // Four tiles in a row per wave hide a tile's row loads behind the previous tile and share the base words; below 8192 tiles (eight
+  // waves per SIMD with one tile each) that leaves SIMDs idle, and one tile per wave is faster:
+  // 7.9 against 10.4 us at 2048 tiles, 17.8 against 15.8 us at 8192, 56 against 52 us at 32768
+  if ((long)A.ntiles * H * kinds >= 8192)
+    hipLaunchKernelGGL(k_encode_tiles<4>, dim3((A.ntiles + 4 * CODEC_WAVES - 1) / (4 * CODEC_WAVES), H, kinds), dim3(64 * CODEC_WAVES), 0, stream, A);
+  else
+    hipLaunchKernelGGL(k_encode_tiles<1>, dim3((A.ntiles + CODEC_WAVES - 1) / CODEC_WAVES, H, kinds), dim3(64 * CODEC_WAVES), 0, stream, A);
+}
 
-// Packs the per-tile escape slots into the head's stream and writes the tile offsets (exclusive sum of the tile sizes of the head).
-// A block takes 64 consecutive tiles: it sums the sizes of all earlier tiles of the head itself (a few thousand integers at most),
-// scans its own 64 and copies, one wave per tile: most tiles hold a few dozen escape bytes.
-constexpr int COMPACT_TPB = 64;
-__global__ void __launch_bounds__(256) k_compact(const uint8_t* __restrict__ esc_slots, const int* __restrict__ tile_bytes,
-                                                 int* __restrict__ tile_off, const int* __restrict__ head_start,
-                                                 uint8_t* __restrict__ ovf, int ntiles) {
-  __shared__ int part[4];
-  __shared__ int offs[COMPACT_TPB];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = blockIdx.y, t0 = blockIdx.x * COMPACT_TPB;
-  const int* tb = tile_bytes + (long)h * ntiles;
-  int before = 0;
-  for (int i = tid; i < t0; i += 256) before += tb[i];
+// Exclusive prefix sums of one head's tile sizes into off, and their total; called by all threads of a block, of which each SCAN_NT
+// scan one list (tid: the thread's index among these; sh: one int per wave of the list).
+constexpr int SCAN_NT = 512, SCAN_PER = 8;
+__device__ __forceinline__ int scan_tile_bytes(const int* __restrict__ tb, int* __restrict__ off, int ntiles, int tid, int* sh) {
+  const int wave = tid >> 6, lane = tid & 63;
+  int carry = 0;
+  for (int base = 0; base < ntiles; base += SCAN_NT * SCAN_PER) {
+    const int t0 = base + tid * SCAN_PER;
+    int n[SCAN_PER], mine = 0;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
-  if (lane == 0) part[wave] = before;
-  __syncthreads();
-  if (wave == 0) {
-    const int n = t0 + lane < ntiles ? tb[t0 + lane] : 0;
-    int incl = n;
+    for (int k = 0; k < SCAN_PER; ++k) n[k] = tb[min(t0 + k, ntiles - 1)];
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; ++k) { n[k] = t0 + k < ntiles ? n[k] : 0; mine += n[k]; }
+    int incl = mine;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
-    const int off = part[0] + part[1] + part[2] + part[3] + incl - n;
-    offs[lane] = off;
-    if (t0 + lane < ntiles) tile_off[(long)h * ntiles + t0 + lane] = off;
+    if (lane == 63) sh[wave] = incl;
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < SCAN_NT / 64; ++w) { const int v = sh[w]; all += v; before += w < wave ? v : 0; }
+    int o = carry + before + incl - mine;
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; ++k) { if (t0 + k < ntiles) off[t0 + k] = o; o += n[k]; }
+    carry += all;
+    __syncthreads();
   }
-  __syncthreads();
-  const int hs = head_start[h];
-  for (int k = wave; k < COMPACT_TPB && t0 + k < ntiles; k += 4) {
-    const long i = (long)h * ntiles + t0 + k;
-    const int n = tb[t0 + k];
-    const uint8_t* src = esc_slots + i * TILE_MAX_ESC;
-    uint8_t* dst = ovf + hs + offs[k];
-    for (int j = lane; j < n; j += 64) dst[j] = src[j];
+  return carry;
+}
+// Tile offsets and escape totals of the heads, one block per head.  host_bytes (or null): the totals once more in host memory that the
+// device can write, for the caller that sizes the stream: it spares a copy and its latency.
+__global__ void __launch_bounds__(SCAN_NT) k_tile_scan(const int* __restrict__ tile_bytes, int* __restrict__ tile_off, int ntiles,
+                                                       int* __restrict__ head_bytes, int* __restrict__ host_bytes) {
+  __shared__ int sh[SCAN_NT / 64];
+  const long h = blockIdx.x;
+  const int total = scan_tile_bytes(tile_bytes + h * ntiles, tile_off + h * ntiles, ntiles, threadIdx.x, sh);
+  if (threadIdx.x == 0) {
+    if (head_bytes) head_bytes[h] = total;
+    if (host_bytes) host_bytes[h] = total;
+  }
+}
+
+// Packs the per-tile escape slots into the heads' streams.  A block takes 64 consecutive tiles of a head, a wave 16 of them: the sizes and
+// offsets of its tiles in one load each, then the first 64 bytes of all 16 slots in flight together (a tile has about 30 escape bytes;
+// what is beyond 64 follows in a loop).  A wave that copied its tiles one after the other, each a chain of size -> bytes -> store, took
+// 20.7 us for the 8 x 4096 tiles of a 64K-token page; this one takes 6.6 us and writes the row offsets as well (9.2 us of their own before).
+// HEADS: the streams lie back to back and the block derives its head's start from the totals of the heads before it (a Page; it also
+// writes head_start, the row offsets and the stream's padding); else head_start is given and a head whose window is too small is left out.
+constexpr int PACK_TPB = 64;
+struct PackKind { const uint8_t* slots; const int* tile_bytes; const int* tile_off; long off_stride; const int* head_start; uint8_t* ovf; };
+struct PackArgs {
+  PackKind j[2]; int ntiles;
+  const int* head_bytes;                 // [kinds * H] totals (null without HEADS: every window is large enough)
+  int window;                            // bytes that a head's stream must fit in (without HEADS)
+  const int* flags; int S, S_pad; int* head_start_out; int* ovf_off;      // HEADS
+};
+template <bool HEADS>
+__global__ void __launch_bounds__(256) k_pack(const PackArgs A) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = blockIdx.y, H = gridDim.y;
+  const PackKind& J = A.j[blockIdx.z];
+  const int t0 = blockIdx.x * PACK_TPB + 16 * wave, n_own = min(16, A.ntiles - t0);      // (may be <= 0)
+  const int tl = min(t0 + (lane & 15), A.ntiles - 1);
+  const int nb = J.tile_bytes[(long)h * A.ntiles + tl], of = J.tile_off[(long)h * J.off_stride + tl];
+  const uint8_t* src = J.slots + (long)h * A.ntiles * TILE_MAX_ESC;
+  u32 v[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, A.ntiles - 1) * TILE_MAX_ESC + lane];
+  long start = 0;
+  if (HEADS) {
+    __shared__ int part[4];
+    int before = 0;
+    for (int i = tid; i < h; i += 256) before += A.head_bytes[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    if (lane == 0) part[wave] = before;
+    __syncthreads();
+    start = part[0] + part[1] + part[2] + part[3];
+    if (blockIdx.x == 0 && tid == 0) {
+      A.head_start_out[h] = (int)start;
+      if (h == H - 1) A.head_start_out[H] = (int)start + A.head_bytes[h];
+    }
+    if (blockIdx.x == 0 && h == H - 1 && tid < 8) J.ovf[start + A.head_bytes[h] + tid] = 0;      // readers fetch eight bytes at a time
+  } else {
+    if (A.head_bytes && A.head_bytes[(long)blockIdx.z * H + h] > A.window) return;
+    start = J.head_start[h];
+  }
+  uint8_t* dst = J.ovf + start;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int n = __builtin_amdgcn_readlane(nb, k), o = __builtin_amdgcn_readlane(of, k);
+    if (k >= n_own) break;
+    if (lane < n) dst[o + lane] = (uint8_t)v[k];
+    for (int i = 64 + lane; i < n; i += 64) dst[o + i] = src[(long)(t0 + k) * TILE_MAX_ESC + i];
+  }
+  if (HEADS) {      // row offsets: tile offset + the escape bytes of the tile's earlier tag words
+    const int* fl = A.flags + (long)h * A.S_pad;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int i = t0 * T + 64 * k + lane;
+      const u32 rb = (u32)esc_bytes((u32)fl[min(i, A.S_pad - 1)]), incl = row_scan16(rb);
+      const int to = __shfl(of, 4 * k + (lane >> 4), 64);
+      if (i < A.S && n_own > 0) A.ovf_off[(long)h * A.S + i] = to + (int)(incl - rb);
+    }
   }
 }
 
@@ -201,8 +286,8 @@ __global__ void __launch_bounds__(256) k_row_offsets(const int* __restrict__ fla
 }
 
 // ---------------------------------------------------------------------------------------------------- page decoder
-// One wave per tile: short-lived waves at full occupancy overlap the dependent loads of a tile (tag words -> escape bytes) with the
-// arithmetic and the stores of others (four tiles in a row per wave were a third slower).
+// One wave per tile, four to a block: short-lived waves at full occupancy overlap the dependent loads of a tile (tag words -> escape
+// bytes) with the arithmetic and the stores of others (four tiles in a row per wave were a third slower).
 template <int KIND>
 __global__ void __launch_bounds__(64) k_decode_tiles(const uint8_t* __restrict__ sm, const uint8_t* __restrict__ cd, const int* __restrict__ flags,
                                                      const int* __restrict__ tile_off, const uint8_t* __restrict__ ovf,
@@ -257,17 +342,39 @@ int gaac_encode_tiles(int kind, const void* x, long x_head_stride, long x_row_st
                "gaac_encode_tiles: bad sizes H=%d S=%d S_pad=%d n_kv=%d", H, S, S_pad, n_kv);
   GAAC_REQUIRE(x_row_stride >= D && x_row_stride % 8 == 0 && x_head_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0,
                "gaac_encode_tiles: rows must be 16-byte aligned (strides in elements: head %ld, row %ld)", x_head_stride, x_row_stride);
-  const int ntiles = (S + T - 1) / T;
-  dim3 grid((ntiles + CODEC_TPB - 1) / CODEC_TPB, H);
-  if (kind == 0) hipLaunchKernelGGL(k_encode_tiles<KIND_K>, grid, dim3(64 * CODEC_WAVES), 0, (hipStream_t)stream, (const u16*)x, S, x_head_stride, x_row_stride, S_pad, base3, base4, n_kv, bidx, sm, codes, flags, esc_slots, tile_bytes, ntiles);
-  else hipLaunchKernelGGL(k_encode_tiles<KIND_V>, grid, dim3(64 * CODEC_WAVES), 0, (hipStream_t)stream, (const u16*)x, S, x_head_stride, x_row_stride, S_pad, base3, base4, n_kv, bidx, sm, codes, flags, esc_slots, tile_bytes, ntiles);
+  EncodeArgs A{};
+  A.kind0 = kind; A.S = S; A.S_pad = S_pad; A.ntiles = (S + T - 1) / T; A.brow0 = 0; A.NB = n_kv; A.bidx = bidx;
+  (kind == 0 ? A.k : A.v) = EncodeKind{(const u16*)x, x_head_stride, x_row_stride, base3, base4, sm, codes, flags, esc_slots, tile_bytes};
+  launch_encode(A, H, 1, (hipStream_t)stream);
   return launch_status("gaac_encode_tiles");
+}
+
+int gaac_tile_scan(const int* tile_bytes, int H, int ntiles, int* tile_off, int* head_bytes, int* host_bytes, void* stream) {
+  GAAC_REQUIRE(tile_bytes && tile_off && head_bytes && H > 0 && ntiles > 0, "gaac_tile_scan: bad arguments");
+  hipLaunchKernelGGL(k_tile_scan, dim3(H), dim3(SCAN_NT), 0, (hipStream_t)stream, tile_bytes, tile_off, ntiles, head_bytes, host_bytes);
+  return launch_status("gaac_tile_scan");
+}
+
+int gaac_page_pack(const uint8_t* esc_slots, const int* tile_bytes, const int* tile_off, const int* head_bytes, const int* flags, int H, int S, int S_pad,
+                   int* head_start, uint8_t* ovf, int* ovf_off, void* stream) {
+  GAAC_REQUIRE(esc_slots && tile_bytes && tile_off && head_bytes && flags && head_start && ovf && ovf_off, "gaac_page_pack: null pointer");
+  GAAC_REQUIRE(H > 0 && S > 0 && S_pad >= (S + T - 1) / T * T && S_pad % T == 0, "gaac_page_pack: bad sizes H=%d S=%d S_pad=%d", H, S, S_pad);
+  PackArgs A{};
+  A.ntiles = (S + T - 1) / T;
+  A.j[0] = PackKind{esc_slots, tile_bytes, tile_off, A.ntiles, nullptr, ovf};
+  A.head_bytes = head_bytes; A.flags = flags; A.S = S; A.S_pad = S_pad; A.head_start_out = head_start; A.ovf_off = ovf_off;
+  hipLaunchKernelGGL(k_pack<true>, dim3((A.ntiles + PACK_TPB - 1) / PACK_TPB, H), dim3(256), 0, (hipStream_t)stream, A);
+  return launch_status("gaac_page_pack");
 }
 
 int gaac_compact(const uint8_t* esc_slots, const int* tile_bytes, int* tile_off, const int* head_start, uint8_t* ovf,
                  int H, int ntiles, void* stream) {
   GAAC_REQUIRE(esc_slots && tile_bytes && tile_off && head_start && ovf && H > 0 && ntiles > 0, "gaac_compact: bad arguments");
-  hipLaunchKernelGGL(k_compact, dim3((ntiles + COMPACT_TPB - 1) / COMPACT_TPB, H), dim3(256), 0, (hipStream_t)stream, esc_slots, tile_bytes, tile_off, head_start, ovf, ntiles);
+  hipLaunchKernelGGL(k_tile_scan, dim3(H), dim3(SCAN_NT), 0, (hipStream_t)stream, tile_bytes, tile_off, ntiles, (int*)nullptr, (int*)nullptr);
+  PackArgs A{};
+  A.ntiles = ntiles;
+  A.j[0] = PackKind{esc_slots, tile_bytes, tile_off, ntiles, head_start, ovf};
+  hipLaunchKernelGGL(k_pack<false>, dim3((ntiles + PACK_TPB - 1) / PACK_TPB, H), dim3(256), 0, (hipStream_t)stream, A);
   return launch_status("gaac_compact");
 }
 

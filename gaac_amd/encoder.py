@@ -6,7 +6,7 @@ each head's escape stream."""
 from __future__ import annotations
 import torch
 from . import _lib
-from .codec import Codec, Page, D, T, CB, TILE_MAX_ESC, perm, storage_index, row_offsets
+from .codec import Codec, Page, TILE_MAX_ESC, T, rows_in_place, encode_page, perm, storage_index
 
 SLOT = TILE_MAX_ESC
 
@@ -41,11 +41,10 @@ class TileEncoder:
         """Encode x [H, S_in, D] (any head / token strides, e.g. a transposed view of a token-major prompt; tiles 0..ceil(S/16)-1) into sm/cd/flags with token stride S_pad; escape bytes stay in the
         scratch slots.  Returns tile_bytes int32 [H, ntiles]; finish with compact()."""
         H = x.shape[0]; ntiles = (S + T - 1) // T; dev = x.device
-        if x.stride(2) != 1 or x.stride(0) % 8 or x.stride(1) % 8 or x.data_ptr() % 16:      # any head / row strides with 16-byte aligned rows
-            x = x.contiguous()
+        x, hs, rs = rows_in_place(x, 0, 1)
         slots = self._scratch(H * ntiles * SLOT, dev)
         tile_bytes = torch.empty(H, ntiles, dtype=torch.int32, device=dev)
-        _lib.call("gaac_encode_tiles", 0 if self.kind == "k" else 1, _lib.ptr(x), x.stride(0), x.stride(1), H, S, S_pad, _lib.ptr(base3), _lib.ptr(base4),
+        _lib.call("gaac_encode_tiles", 0 if self.kind == "k" else 1, _lib.ptr(x), hs, rs, H, S, S_pad, _lib.ptr(base3), _lib.ptr(base4),
                   n_kv, _lib.ptr(bidx), _lib.ptr(sm), _lib.ptr(cd), _lib.ptr(flags), _lib.ptr(slots), _lib.ptr(tile_bytes), _lib.stream())
         return tile_bytes
 
@@ -59,14 +58,4 @@ class TileEncoder:
 
     def encode(self, codec: Codec, x: torch.Tensor) -> Page:
         """x: [H, S, D] bf16 -> Page."""
-        H, S, _ = x.shape; dev = x.device
-        S_pad = (S + T - 1) // T * T
-        sm = torch.empty(H, S_pad * D, dtype=torch.uint8, device=dev)
-        cd = torch.empty(H, S_pad * CB, dtype=torch.uint8, device=dev)
-        flags = torch.zeros(H, S_pad, dtype=torch.int32, device=dev)
-        tile_bytes = self.encode_tiles(x, codec.base3, codec.base4, sm, cd, flags, S, S_pad, codec.n_kv)
-        head_bytes = tile_bytes.sum(1)
-        head_start = torch.cat([torch.zeros(1, dtype=torch.int64, device=dev), torch.cumsum(head_bytes, 0)]).to(torch.int32).contiguous()
-        ovf = torch.zeros(int(head_start[-1]) + 8, dtype=torch.uint8, device=dev)
-        tile_off = self.compact(tile_bytes, head_start, ovf)
-        return Page(sm, cd, flags, row_offsets(flags, S), ovf, head_start, tile_off, codec.base3, codec.base4, H, S, codec.n_kv, self.kind)
+        return encode_page(x, self.kind, codec.base3, codec.base4, codec.n_kv)
