@@ -12,38 +12,110 @@ namespace gaac {
 char* last_error_buffer() { static thread_local char buf[512] = {0}; return buf; }
 
 // ---------------------------------------------------------------------------------------------------- calibration
-// Exponent histogram per (kv head, channel).  A block owns 64 channels of the n_kv*128-wide token row and a chunk of tokens: eight
-// lanes read the 128 bytes of a row with 16-byte loads, counts go to LDS (64 x 256 x 4 B) and from there, where non-zero, to the
-// 64-bit global histogram.
-constexpr int HIST_CH = 64;
-__global__ void __launch_bounds__(256) k_exponent_hist(const u16* __restrict__ x, long n_tok, int n_kv, int chunk,
-                                                       unsigned long long* __restrict__ hist) {
-  __shared__ u32 h[HIST_CH * 256];
-  const int tid = threadIdx.x, c0 = blockIdx.x * HIST_CH;      // first of this block's channels in the n_kv*128 row
-  for (int i = tid; i < HIST_CH * 256; i += 256) h[i] = 0u;
+// Exponent histogram per (kv head, channel).  A block owns the 128 channels of one kv head of K or of V and a chunk of tokens.  Lane l of
+// every wave reads channels 2l and 2l+1 of a row (one 256-byte row per wave-wide load) and counts in a table of 256 x 64 words that the
+// block's waves share: word (bin, l) holds the counts of the two channels in its 16-bit halves (a chunk has at most 65535 tokens), so a
+// lane only ever touches bank l and the LDS adds of a wave never collide, however alike the exponents are.  A table of one word per
+// (channel, bin) with eight lanes to a row (16-byte loads) sent all rows of a wave to the same few words of a channel: 66 us for
+// the K and the V of 32768 tokens x 8 kv heads (134 MB, two launches), this one 36 us (3.7 TB/s; its loads alone take 27).
+// Non-zero counts are added to the global histogram at the end: PACKED = false: 64-bit counts hist[row][256], the layout that
+// gaac_exponent_hist hands out; PACKED = true: scratch[pair][bin][64] with the two 32-bit counts of a lane in one 64-bit word, so that a
+// wave's adds of a bin are one contiguous 512-byte access (prompts of up to 2^32 - 1 tokens).
+constexpr int HIST_WAVES = 8, HIST_MAX_CHUNK = 65535, HIST_ROWS = 16;      // HIST_ROWS: rows in flight per wave
+struct HistArgs { const u16* x[2]; long head_stride[2], row_stride[2]; long n_tok; int chunk, n_kv; unsigned long long* hist; };
+template <bool PACKED>
+__global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArgs A) {
+  __shared__ u32 h[256 * 64];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, head = blockIdx.y, kind = blockIdx.z;
+  const long t0 = (long)blockIdx.x * A.chunk, t1 = min(t0 + (long)A.chunk, A.n_tok);
+  const long rs = A.row_stride[kind];
+  const u16* xp = A.x[kind] + (long)head * A.head_stride[kind] + 2 * lane;
+  for (int i = tid; i < 256 * 64 / 4; i += 64 * HIST_WAVES) reinterpret_cast<u32x4*>(h)[i] = u32x4{0u, 0u, 0u, 0u};
   __syncthreads();
-  const long t0 = (long)blockIdx.y * chunk, t1 = min(t0 + (long)chunk, n_tok);
-  const int c8 = tid & 7, sub = tid >> 3;
-  const long row = (long)n_kv * D;
-  const u16* xp = x + c0 + 8 * c8;
-  u32* hc = h + (8 * c8) * 256;
-  for (long t = t0 + sub; t < t1; t += 4 * 32) {      // four rows in flight per thread
-    u32x4 v[4];
+  u32* hc = h + lane;
+  const auto count = [&](u32 w) {
+    atomicAdd(&hc[((w >> 7) & 0xFFu) << 6], 1u);
+    atomicAdd(&hc[((w >> 23) & 0xFFu) << 6], 0x10000u);
+  };
+  long t = t0 + wave;
+  for (; t + (HIST_ROWS - 1) * HIST_WAVES < t1; t += HIST_ROWS * HIST_WAVES) {
+    u32 w[HIST_ROWS];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = t + 32 * k < t1 ? *reinterpret_cast<const u32x4*>(xp + (t + 32 * k) * row) : u32x4{0u, 0u, 0u, 0u};
+    for (int k = 0; k < HIST_ROWS; ++k) w[k] = *reinterpret_cast<const u32*>(xp + (t + k * HIST_WAVES) * rs);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (t + 32 * k >= t1) break;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        atomicAdd(&hc[(2 * j) * 256 + ((v[k][j] >> 7) & 0xFFu)], 1u);
-        atomicAdd(&hc[(2 * j + 1) * 256 + ((v[k][j] >> 23) & 0xFFu)], 1u);
-      }
+    for (int k = 0; k < HIST_ROWS; ++k) count(w[k]);
+  }
+  for (; t < t1; t += HIST_WAVES) count(*reinterpret_cast<const u32*>(xp + t * rs));
+  __syncthreads();
+  const long pair = (long)kind * A.n_kv + head;
+  for (int i = tid; i < 256 * 64; i += 64 * HIST_WAVES) {
+    const u32 c = h[i];
+    if (c == 0u) continue;
+    if (PACKED) atomicAdd(&A.hist[pair * (256 * 64) + i], (unsigned long long)(c & 0xFFFFu) | ((unsigned long long)(c >> 16) << 32));
+    else {
+      unsigned long long* row = A.hist + (pair * D + 2 * (i & 63)) * 256 + (i >> 6);
+      if (c & 0xFFFFu) atomicAdd(row, (unsigned long long)(c & 0xFFFFu));
+      if (c >> 16) atomicAdd(row + 256, (unsigned long long)(c >> 16));
     }
   }
+}
+static void launch_hist(HistArgs& A, int kinds, bool packed, hipStream_t stream) {
+  // one block per CU, at least 256 tokens each, so that clearing and scanning the 64 KB table stays the smaller part (two blocks per CU,
+  // which the LDS has room for: 32 against 30 us for 2 x 8 heads x 32768 tokens)
+  const int pairs = kinds * A.n_kv;
+  long nchunk = min((A.n_tok + 255) / 256, (long)max(1, 256 / pairs));
+  nchunk = max(nchunk, (A.n_tok + HIST_MAX_CHUNK - 1) / HIST_MAX_CHUNK);
+  A.chunk = (int)((A.n_tok + nchunk - 1) / nchunk);
+  const dim3 grid((unsigned)((A.n_tok + A.chunk - 1) / A.chunk), A.n_kv, kinds);
+  if (packed) hipLaunchKernelGGL(k_exponent_hist<true>, grid, dim3(64 * HIST_WAVES), 0, stream, A);
+  else hipLaunchKernelGGL(k_exponent_hist<false>, grid, dim3(64 * HIST_WAVES), 0, stream, A);
+}
+
+// The bases of K and V of a prompt from the packed histogram scratch, written to base row row0 + head of the two kinds' tables.  A block
+// takes 32 channels of one (kind, head): their 256 counts in LDS, thread (channel, eighth) slides the two windows over 32 starts.
+struct PromptBasesArgs { const u64* hist; uint8_t* b3[2]; uint8_t* b4[2]; int n_kv, row0; };
+__global__ void __launch_bounds__(256) k_prompt_bases(const PromptBasesArgs A) {
+  constexpr int STRIDE = 256 + 17;      // odd: the 32 channels of a bin sit in different banks
+  __shared__ u32 cnt[32 * STRIDE];
+  __shared__ u32 best[2][8][32];
+  __shared__ int arg[2][8][32];
+  const int tid = threadIdx.x, grp = blockIdx.x, head = blockIdx.y, kind = blockIdx.z;
+  const u64* hp = A.hist + ((long)kind * A.n_kv + head) * (256 * 64) + 16 * grp;
+  u64 w[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) { const int i = tid + 256 * k; w[k] = hp[(i >> 4) * 64 + (i & 15)]; }
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int i = tid + 256 * k, bin = i >> 4, c = 2 * (i & 15);
+    cnt[c * STRIDE + bin] = (u32)w[k]; cnt[(c + 1) * STRIDE + bin] = (u32)(w[k] >> 32);
+  }
+  const int c = tid & 31, part = tid >> 5, st0 = 32 * part;
   __syncthreads();
-  for (int i = tid; i < HIST_CH * 256; i += 256)
-    if (h[i]) atomicAdd(&hist[(long)(c0 + (i >> 8)) * 256 + (i & 255)], (unsigned long long)h[i]);
+  u32 n[32 + 15];      // the counts that the thread's windows cover, read together
+#pragma unroll
+  for (int i = 0; i < 32 + 15; ++i) n[i] = cnt[c * STRIDE + min(st0 + i, 255)];
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    const int win = pass ? 16 : 8;
+    u32 sum = 0u;
+#pragma unroll
+    for (int i = 0; i < win; ++i) sum += n[i];
+    u32 b = sum; int a = st0;
+#pragma unroll
+    for (int i = 1; i < 32; ++i) {      // the lowest start of the largest sum, as k_bases_from_hist
+      sum += n[i + win - 1] - n[i - 1];
+      if (st0 + i + win <= 256 && sum > b) { b = sum; a = st0 + i; }
+    }
+    best[pass][part][c] = b; arg[pass][part][c] = a;
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const int pass = tid >> 5;
+    u32 b = best[pass][0][c]; int a = arg[pass][0][c];
+#pragma unroll
+    for (int p = 1; p < 8; ++p) if (best[pass][p][c] > b) { b = best[pass][p][c]; a = arg[pass][p][c]; }
+    (pass ? A.b4[kind] : A.b3[kind])[(long)(A.row0 + head) * D + 32 * grp + c] = (uint8_t)a;
+  }
 }
 
 // One wave per histogram row: lane l evaluates the windows that start at 4l .. 4l+3 (the reference takes the first maximum of the
@@ -309,6 +381,39 @@ __global__ void __launch_bounds__(64) k_decode_tiles(const uint8_t* __restrict__
                            min(T, S - tile * T), dst, out_row_stride);
 }
 
+// ---------------------------------------------------------------------------------------------------- prompt into the slot cache
+// Per head, K and V: tile offsets and escape totals of the encoded tiles, the last L % 16 rows into the raw tail, and the head's counters.
+// A head whose escapes do not fit its window (of K or of V) is left empty: the caller sees the totals, makes the windows larger and
+// repeats the call.  One block per head.
+struct PromptKind { const u16* x; long head_stride, row_stride; const int* tile_bytes; int* tile_off; u16* tail; int* ovf_used; };
+struct PromptScanArgs { PromptKind j[2]; int n_kv, L, ntiles, off_stride, window; int* S; int* tail_len; int* head_bytes; int* host_bytes; };
+__global__ void __launch_bounds__(2 * SCAN_NT) k_prompt_scan(const PromptScanArgs A) {
+  __shared__ int sh[2][SCAN_NT / 64];
+  __shared__ int total[2];
+  const int h = blockIdx.x, kind = threadIdx.x / SCAN_NT, tid = threadIdx.x % SCAN_NT, full = A.ntiles * T, n_tail = A.L - full;
+  const PromptKind& J = A.j[kind];
+  const int row = tid >> 4, c16 = tid & 15;
+  if (row < n_tail)
+    *reinterpret_cast<u32x4*>(J.tail + ((long)h * T + row) * D + 8 * c16) =
+        *reinterpret_cast<const u32x4*>(J.x + (long)h * J.head_stride + (long)(full + row) * J.row_stride + 8 * c16);
+  const int mine = A.ntiles > 0 ? scan_tile_bytes(J.tile_bytes + (long)h * A.ntiles, J.tile_off + (long)h * A.off_stride, A.ntiles, tid, sh[kind]) : 0;
+  if (tid == 0) {
+    total[kind] = mine;
+    A.head_bytes[kind * A.n_kv + h] = mine;
+    if (A.host_bytes) A.host_bytes[kind * A.n_kv + h] = mine;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    const bool fits = A.ntiles == 0 || max(total[0], total[1]) <= A.window;
+    J.ovf_used[h] = fits ? mine : 0;
+    if (kind == 0) { A.S[h] = fits ? full : 0; A.tail_len[h] = fits ? n_tail : 0; }
+  }
+}
+__global__ void __launch_bounds__(256) k_zero16(u32x4* __restrict__ p, long n16) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n16) p[i] = u32x4{0u, 0u, 0u, 0u};
+}
+
 }  // namespace gaac
 
 using namespace gaac;
@@ -320,10 +425,9 @@ const char* gaac_last_error(void) { return last_error_buffer(); }
 int gaac_exponent_hist(const void* x, long n_tokens, int n_kv, long long* hist, void* stream) {
   GAAC_REQUIRE(x && hist && n_kv > 0 && n_tokens >= 0, "gaac_exponent_hist: bad arguments");
   if (n_tokens == 0) return 0;
-  int nchunk = (int)min((n_tokens + 1023) / 1024, 512L);
-  int chunk = (int)((n_tokens + nchunk - 1) / nchunk);
-  hipLaunchKernelGGL(k_exponent_hist, dim3(n_kv * D / HIST_CH, nchunk), dim3(256), 0, (hipStream_t)stream,
-                     (const u16*)x, n_tokens, n_kv, chunk, (unsigned long long*)hist);
+  const long row = (long)n_kv * D;
+  HistArgs A{{(const u16*)x, nullptr}, {D, 0}, {row, 0}, n_tokens, 0, n_kv, (unsigned long long*)hist};
+  launch_hist(A, 1, false, (hipStream_t)stream);
   return launch_status("gaac_exponent_hist");
 }
 
@@ -396,6 +500,58 @@ int gaac_decode_tiles(int kind, const uint8_t* sm, const uint8_t* codes, const i
   if (kind == 0) hipLaunchKernelGGL(k_decode_tiles<KIND_K>, grid, dim3(64), 0, (hipStream_t)stream, sm, codes, flags, tile_off, ovf, head_start, base3, base4, n_kv, bidx, S, S_pad, (u16*)out, out_head_stride, out_row_stride);
   else hipLaunchKernelGGL(k_decode_tiles<KIND_V>, grid, dim3(64), 0, (hipStream_t)stream, sm, codes, flags, tile_off, ovf, head_start, base3, base4, n_kv, bidx, S, S_pad, (u16*)out, out_head_stride, out_row_stride);
   return launch_status("gaac_decode_tiles");
+}
+
+int gaac_cache_prefill(
+    const void* k, const void* v, long k_head_stride, long k_row_stride, long v_head_stride, long v_row_stride, int L, int n_kv, int head0,
+    int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
+    void* k_tail, uint8_t* k_base3, uint8_t* k_base4, uint8_t* k_sm, uint8_t* k_codes, int* k_flags, uint8_t* k_ovf, int* k_tile_off, int* k_ovf_used,
+    void* v_tail, uint8_t* v_base3, uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
+    unsigned long long* hist, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, int* host_bytes, void* stream) {
+  GAAC_REQUIRE(((k && v) || L == 0) && tail_len && S && head_start && head_bytes, "gaac_cache_prefill: null pointer");
+  GAAC_REQUIRE(k_tail && k_base3 && k_base4 && k_sm && k_codes && k_flags && k_ovf && k_tile_off && k_ovf_used, "gaac_cache_prefill: null K store pointer");
+  GAAC_REQUIRE(v_tail && v_base3 && v_base4 && v_sm && v_codes && v_flags && v_ovf && v_tile_off && v_ovf_used, "gaac_cache_prefill: null V store pointer");
+  GAAC_REQUIRE(L >= 0 && n_kv > 0 && head0 >= 0 && cap > 0 && cap % T == 0 && L <= cap && NB > 0 && ovf_cap >= 8,
+               "gaac_cache_prefill: bad sizes L=%d n_kv=%d head0=%d cap=%d ovf_cap=%d NB=%d", L, n_kv, head0, cap, ovf_cap, NB);
+  GAAC_REQUIRE(!calibrate || (hist && NB >= head0 + n_kv), "gaac_cache_prefill: calibration needs its scratch and a base row per cache head (NB=%d, heads %d..%d)", NB, head0, head0 + n_kv - 1);
+  const int ntiles = L / T;
+  GAAC_REQUIRE(ntiles == 0 || (esc_slots && tile_bytes), "gaac_cache_prefill: null scratch");
+  GAAC_REQUIRE(L == 0 || (k_row_stride >= D && k_row_stride % 8 == 0 && k_head_stride % 8 == 0 && v_row_stride >= D && v_row_stride % 8 == 0 && v_head_stride % 8 == 0 &&
+                          ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0), "gaac_cache_prefill: rows must be 16-byte aligned");
+  hipStream_t st = (hipStream_t)stream;
+  if (calibrate) {
+    const long n16 = (long)n_kv * 2 * 256 * 64 * (long)sizeof(u64) / 16;
+    hipLaunchKernelGGL(k_zero16, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, reinterpret_cast<u32x4*>(hist), n16);
+    HistArgs H{{(const u16*)k, (const u16*)v}, {k_head_stride, v_head_stride}, {k_row_stride, v_row_stride}, L, 0, n_kv, hist};
+    if (L > 0) launch_hist(H, 2, true, st);
+    const PromptBasesArgs B{reinterpret_cast<const u64*>(hist), {k_base3, v_base3}, {k_base4, v_base4}, n_kv, head0};
+    hipLaunchKernelGGL(k_prompt_bases, dim3(4, n_kv, 2), dim3(256), 0, st, B);
+  }
+  const long row0 = (long)head0 * cap, tile0 = (long)head0 * (cap / T), n_all = (long)n_kv * ntiles;
+  uint8_t* v_slots = esc_slots ? esc_slots + n_all * TILE_MAX_ESC : nullptr;
+  int* v_bytes = tile_bytes ? tile_bytes + n_all : nullptr;
+  if (ntiles > 0) {
+    EncodeArgs E{};
+    E.kind0 = KIND_K; E.S = ntiles * T; E.S_pad = cap; E.ntiles = ntiles; E.brow0 = head0; E.NB = NB; E.bidx = nullptr;
+    E.k = EncodeKind{(const u16*)k, k_head_stride, k_row_stride, k_base3, k_base4, k_sm + row0 * D, k_codes + row0 * CB, k_flags + row0, esc_slots, tile_bytes};
+    E.v = EncodeKind{(const u16*)v, v_head_stride, v_row_stride, v_base3, v_base4, v_sm + row0 * D, v_codes + row0 * CB, v_flags + row0, v_slots, v_bytes};
+    launch_encode(E, n_kv, 2, st);
+  }
+  const int window = ovf_cap - (TILE_MAX_ESC + 8);      // room for one more worst-case tile and the readers' padding stays free
+  PromptScanArgs P{};
+  P.j[0] = PromptKind{(const u16*)k, k_head_stride, k_row_stride, tile_bytes, k_tile_off + tile0, (u16*)k_tail + (long)head0 * T * D, k_ovf_used + head0};
+  P.j[1] = PromptKind{(const u16*)v, v_head_stride, v_row_stride, v_bytes, v_tile_off + tile0, (u16*)v_tail + (long)head0 * T * D, v_ovf_used + head0};
+  P.n_kv = n_kv; P.L = L; P.ntiles = ntiles; P.off_stride = cap / T; P.window = window;
+  P.S = S + head0; P.tail_len = tail_len + head0; P.head_bytes = head_bytes; P.host_bytes = host_bytes;
+  hipLaunchKernelGGL(k_prompt_scan, dim3(n_kv), dim3(2 * SCAN_NT), 0, st, P);
+  if (ntiles > 0) {
+    PackArgs A{};
+    A.ntiles = ntiles; A.head_bytes = head_bytes; A.window = window;
+    A.j[0] = PackKind{esc_slots, tile_bytes, k_tile_off + tile0, cap / T, head_start + head0, k_ovf};
+    A.j[1] = PackKind{v_slots, v_bytes, v_tile_off + tile0, cap / T, head_start + head0, v_ovf};
+    hipLaunchKernelGGL(k_pack<false>, dim3((ntiles + PACK_TPB - 1) / PACK_TPB, n_kv, 2), dim3(256), 0, st, A);
+  }
+  return launch_status("gaac_cache_prefill");
 }
 
 }  // extern "C"
