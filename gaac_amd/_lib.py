@@ -75,7 +75,9 @@ def ptr(t: torch.Tensor | None):
 
 
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device as a handle (torch.cuda.current_stream() builds a Stream object on the way: 3 us
+    against 0.1, of the 5 us that a launch takes)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def call(name: str, *args):

@@ -113,7 +113,8 @@ def shared_workspace(rows: int, nslot: int, dtype, dev) -> AttnWorkspace:
     tensor.  A workspace is never made while the stream is capturing (its memory and its zeroing would end up inside the graph):
     callers that capture pass their own, as CompressedKVCache and LayerState do."""
     dev = torch.device(dev)
-    key = (dev.type, dev.index if dev.index is not None else torch.cuda.current_device(), rows, nslot, dtype, torch.cuda.current_stream(dev).cuda_stream)
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    key = (dev.type, index, rows, nslot, dtype, torch._C._cuda_getCurrentRawStream(index))
     ws = _shared_ws.pop(key, None)
     if ws is None:
         if torch.cuda.is_current_stream_capturing():
@@ -172,9 +173,9 @@ def attention(q, kp, vp, scale=None, nsplit=None, phase="fused"):
     q: [B, n_q, D] bf16 (one query token per sequence) -> [B, n_q, D] bf16."""
     B, n_q, Dq = q.shape
     n_kv = kp.H // B
-    dev = q.device
     if nsplit is None: nsplit = choose_nsplit(B, n_kv, kp.S)
-    SL = torch.full((kp.H,), kp.S, dtype=torch.int32, device=dev)
+    # the one-kernel launch takes the length as an argument; the other phases read one per head
+    SL = None if phase == "fused" else torch.full((kp.H,), kp.S, dtype=torch.int32, device=q.device)
     out = attn_launch(kp, vp, q.reshape(B * n_q, Dq).contiguous(), None, n_q, n_kv, SL, kp.sm.shape[1] // D,
                       scale if scale is not None else Dq ** -0.5, nsplit, phase=phase, S_all=kp.S)
     return out.view(B, n_q, Dq)
