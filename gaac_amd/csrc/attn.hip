@@ -15,6 +15,7 @@
 //     two-launch alternative;
 //   * k_attn_split<true, .> reads the paged slot pool through block and mode tables (paged_kernel.py:42-241).
 //   Softmax runs in base 2 (scale * log2 e folded into the scores).
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include "gaac_tile.h"
@@ -54,6 +55,8 @@ struct AttnArgs {
   const uint8_t* pool; const u16* raw; const int* mt; const int* bt; int bt_stride; int TS;
   // paged: raw tiles queued by the preceding store (gaac_paged_store's freeq) that this launch pushes back onto the free stack (or null)
   const int* freeq; int n_free; int* stack; int* top;
+  int B;                       // batch rows
+  int plan;                    // > 0: the blocks share the rows out by length (plan_block), of which this many splits are resident at once; 0: nsplit blocks per row and kv head
 #ifdef GAAC_PHASE_TIMING
   long long* dbg;
 #endif
@@ -68,6 +71,13 @@ struct AttnArgs {
 constexpr int MAX_CHUNK = 1024;  // tiles whose slot lookups a block keeps in LDS at a time (paged mode); longer splits go on in further rounds
 constexpr int SLOT_CD = TILE_SM, SLOT_FL = TILE_SM + TILE_CD, SLOT_OV = SLOT_FL + 4 * T;      // byte offsets inside a tile slot
 
+// n / d for the block's own coordinates: the compiler's 32-bit division is a chain of quarter-rate multiplications, and a block needs five
+// quotients before it can load anything.  Below 2^21 the rounded product is exact: (n + 0.5) / d is at least 0.5 / d away from an
+// integer, the product is off by less than 2^-22 n / d.
+__device__ __forceinline__ int small_div(int n, int d) {
+  if (__builtin_expect(n >= (1 << 21), 0)) return n / d;
+  return (int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+}
 __device__ __forceinline__ float bf16_bits_to_float(u32 h) { return __uint_as_float(h << 16); }
 __device__ __forceinline__ u32 pack_bf16x2(float lo, float hi) {
   typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
@@ -109,7 +119,7 @@ __device__ __forceinline__ bool ll_stale(u64 r, u32 epoch) { return (u32)(r >> 3
 __device__ __forceinline__ float ll_value(u64 r) { return __uint_as_float((u32)r); }
 constexpr int MERGE_SPIN_LIMIT = 1 << 16;      // re-reads of a chunk before the merger gives up (each with a short sleep: ~0.1 s)
 // (no branch around the load: a load under a branch is waited for where the branch ends, together with everything issued before it)
-__device__ __forceinline__ u32 load_epoch(const AttnArgs& A, int bh) {
+__device__ __forceinline__ u32 load_epoch(const AttnArgs& A) {
   const u32* p = A.epochs ? A.epochs : reinterpret_cast<const u32*>(A.q);
   const u32 e = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return e + 1u + (e == 0xFFFFFFFFu ? 1u : 0u);      // epoch 0 is never used: zeroed records stay stale when the counter wraps
@@ -125,18 +135,18 @@ template <int NW> struct MergeScratch { float f[NW][MAX_SLOTS], l[NW][MAX_SLOTS]
 // and sums them over ALL slots, so the waves exchange nothing and no block barrier lies between the records' arrival and the
 // output: lane (g, c) = (lane / CPW, lane % CPW) reads the accumulator records of channel c of the wave for the slots g, g + SG, ...
 // (SG = 64 / CPW slot groups); the groups' sums meet through DPP.  Every wave reads the m / l records of all slots (lane = slot)
-// and derives the slots' weights itself.  Called by all threads of the block.
+// and derives the slots' weights itself.  rec: the query head's first record, nslot: its splits.  Called by all threads of the block.
 __device__ __forceinline__ void merge_failed(const AttnArgs& A, u32 bit) {
   __hip_atomic_fetch_or(A.epochs + 1, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <int NW>
-__device__ __forceinline__ void merge_half_head(const AttnArgs& A, long row, int half, u32 epoch, MergeScratch<NW>& X, int wave, int lane) {
+__device__ __forceinline__ void merge_half_head(const AttnArgs& A, long rec, int nslot, long row, int half, u32 epoch, MergeScratch<NW>& X, int wave, int lane) {
   constexpr int CPW = 64 / NW, SG = 64 / CPW;      // channels per wave (8 | 16), slot groups (8 | 4)
   constexpr int CH = 8;                             // accumulator records in flight per lane: one round for up to CH * SG splits
-  const int nslot = A.nslot, g = lane / CPW, d = 64 * half + CPW * wave + lane % CPW;
-  const u64* rm = reinterpret_cast<const u64*>(A.pm) + row * nslot;
-  const u64* rl = reinterpret_cast<const u64*>(A.pl) + row * nslot;
-  const u64* ra = reinterpret_cast<const u64*>(A.pa) + row * nslot * D + d;
+  const int g = lane / CPW, d = 64 * half + CPW * wave + lane % CPW;
+  const u64* rm = reinterpret_cast<const u64*>(A.pm) + rec;
+  const u64* rl = reinterpret_cast<const u64*>(A.pl) + rec;
+  const u64* ra = reinterpret_cast<const u64*>(A.pa) + rec * D + d;
   float* fs = X.f[wave]; float* ls = X.l[wave];
   bool ok = true;
   // all loads of the first round are issued before the first use, none under a branch (a slot past the end reads the last slot
@@ -224,35 +234,36 @@ __device__ __forceinline__ void merge_half_head(const AttnArgs& A, long row, int
 // 4 query heads: four in a row): here each wave of the merging blocks takes a half head of its own.  Launches over 1000 tokens x 8 kv
 // heads: 18.1 -> 13.2 us with two splits, 15.1 -> 11.3 with three, 12.8 -> 10.6 with four, 11.1 -> 9.0 with six.  With as many
 // splits as half heads the block-wise merge has one trip as well, and spreads its records over more waves.
-constexpr int WAVE_MERGE_SLOTS = 8;
-__device__ __forceinline__ void merge_half_head_wave(const AttnArgs& A, long row, int half, u32 epoch, int lane) {
-  const int nslot = A.nslot, d = 64 * half + lane;
-  const u64* rm = reinterpret_cast<const u64*>(A.pm) + row * nslot + min(lane, nslot - 1);
-  const u64* rl = reinterpret_cast<const u64*>(A.pl) + row * nslot + min(lane, nslot - 1);
-  const u64* ra = reinterpret_cast<const u64*>(A.pa) + row * nslot * D + d;
-  u64 v[WAVE_MERGE_SLOTS];
+constexpr int WAVE_MERGE_SLOTS = 16;
+template <int SLOTS>      // how many it reads (those past the last split again: no load under a branch)
+__device__ __forceinline__ void merge_half_head_wave(const AttnArgs& A, long rec, int nslot, long row, int half, u32 epoch, int lane) {
+  const int d = 64 * half + lane;
+  const u64* rm = reinterpret_cast<const u64*>(A.pm) + rec + min(lane, nslot - 1);
+  const u64* rl = reinterpret_cast<const u64*>(A.pl) + rec + min(lane, nslot - 1);
+  const u64* ra = reinterpret_cast<const u64*>(A.pa) + rec * D + d;
+  u64 v[SLOTS];
 #pragma unroll
-  for (int k = 0; k < WAVE_MERGE_SLOTS; ++k) v[k] = ll_load(ra + (long)min(k, nslot - 1) * D);      // (past the end: the last record again, ignored)
+  for (int k = 0; k < SLOTS; ++k) v[k] = ll_load(ra + (long)min(k, nslot - 1) * D);      // (past the end: the last record again, ignored)
   u64 mr = ll_load(rm), lr = ll_load(rl);
   bool ok = true;
   for (int spin = 0;; ++spin) {
     bool stale = ll_stale(mr, epoch) || ll_stale(lr, epoch);
 #pragma unroll
-    for (int k = 0; k < WAVE_MERGE_SLOTS; ++k) stale |= ll_stale(v[k], epoch);
+    for (int k = 0; k < SLOTS; ++k) stale |= ll_stale(v[k], epoch);
     if (__builtin_amdgcn_ballot_w64(stale) == 0) break;
     if (spin >= MERGE_SPIN_LIMIT) { ok = false; break; }
     __builtin_amdgcn_s_sleep(1);
     if (ll_stale(mr, epoch)) mr = ll_load(rm);
     if (ll_stale(lr, epoch)) lr = ll_load(rl);
 #pragma unroll
-    for (int k = 0; k < WAVE_MERGE_SLOTS; ++k) if (ll_stale(v[k], epoch)) v[k] = ll_load(ra + (long)min(k, nslot - 1) * D);
+    for (int k = 0; k < SLOTS; ++k) if (ll_stale(v[k], epoch)) v[k] = ll_load(ra + (long)min(k, nslot - 1) * D);
   }
   const float m = lane < nslot ? ll_value(mr) : -INFINITY, mx = wave_max(m);
   const float f = m != -INFINITY ? __builtin_amdgcn_exp2f(m - mx) : 0.f;      // 0 also for the lanes without a slot
   const float l = wave_sum(ll_value(lr) * f);
   float acc = 0.f;
 #pragma unroll
-  for (int k = 0; k < WAVE_MERGE_SLOTS; ++k) {
+  for (int k = 0; k < SLOTS; ++k) {
     const float fk = __uint_as_float((u32)__builtin_amdgcn_readlane((int)__float_as_uint(f), k));
     acc += fk != 0.f ? ll_value(v[k]) * fk : 0.f;      // an empty partial's accumulator may hold anything
   }
@@ -271,49 +282,35 @@ constexpr int EPOCH_WORDS = 2;      // words of the epoch buffer ahead of the ar
 __device__ __forceinline__ void mark_arrival(const AttnArgs& A, u32 epoch) {
   __hip_atomic_store(A.epochs + EPOCH_WORDS + blockIdx.x, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-template <int NWB>      // NWB: waves of the block; twelve-wave blocks (measurement build) merge with their first eight waves
-__device__ __forceinline__ void merge_heads(const AttnArgs& A, long qh0, int G, u32 epoch, int rank, int mergers, int tid, MergeScratch<(NWB > 8 ? 8 : NWB)>& X) {
-  constexpr int NW = NWB > 8 ? 8 : NWB;
-  const int wave = tid >> 6, lane = tid & 63;
-  if (NWB > NW && wave >= NW) { if (blockIdx.x == gridDim.x - 1) lds_barrier(); return; }      // (the last block meets once more below)
-  const bool last = blockIdx.x == gridDim.x - 1;
-  // The last block of the grid advances the epoch word for the next launch, once every block of this launch has marked its arrival
-  // (and so has read the word).  The marks' first read is issued here, ahead of the merge work, and looked at after it: by then the
-  // other blocks have long left their loops, so the check normally costs no trip to memory of its own.
-  constexpr int XK = 2048 / (64 * NW);      // marks per lane held in registers: the first 2048 blocks of the grid
-  const u32* marks = A.epochs + EPOCH_WORDS;
-  const int nblocks = (int)gridDim.x, xi = 64 * wave + lane;
-  u32 xm[XK];
-  if (last) {
+// The grid's last block advances the epoch word for the next launch, once every block of this launch has marked its arrival (and so has
+// read the word).  The marks' first read (the first 2048 blocks) is issued ahead of the block's merge work and looked at after it: by
+// then the other blocks have long left their loops, so the check normally costs no trip to memory of its own.
+template <int NW> struct MarkRegs { u32 m[2048 / (64 * NW)]; };
+template <int NW>
+__device__ __forceinline__ void load_marks(const AttnArgs& A, int tid, MarkRegs<NW>& R) {
 #pragma unroll
-    for (int k = 0; k < XK; ++k) xm[k] = __hip_atomic_load(marks + min(xi + 64 * NW * k, nblocks - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  // The first item stands outside the loop: at a loop header the compiler waits for every memory operation in flight, which here
-  // would be the acknowledgement of the block's own record stores (a round trip to memory) before the first record load is issued.
-  if (A.nslot <= WAVE_MERGE_SLOTS && A.nslot < 2 * G) {
-    int item = rank + mergers * wave;
-    if (item < 2 * G) { merge_half_head_wave(A, qh0 + (item >> 1), item & 1, epoch, lane); item += mergers * NW; }
-    for (; item < 2 * G; item += mergers * NW) merge_half_head_wave(A, qh0 + (item >> 1), item & 1, epoch, lane);
-  } else {
-    int item = rank;
-    if (item < 2 * G) { merge_half_head<NW>(A, qh0 + (item >> 1), item & 1, epoch, X, wave, lane); item += mergers; }
-    for (; item < 2 * G; item += mergers) merge_half_head<NW>(A, qh0 + (item >> 1), item & 1, epoch, X, wave, lane);
-  }
-  if (!last) return;
+  for (int k = 0; k < 2048 / (64 * NW); ++k)
+    R.m[k] = __hip_atomic_load(A.epochs + EPOCH_WORDS + min(tid + 64 * NW * k, (int)gridDim.x - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int NW>      // called by NW waves of the block; verdict: one word of LDS per wave
+__device__ __forceinline__ void advance_epoch(const AttnArgs& A, u32 epoch, int tid, MarkRegs<NW>& R, float* verdict, int verdict_stride) {
+  constexpr int XK = 2048 / (64 * NW);
+  const u32* marks = A.epochs + EPOCH_WORDS;
+  const int nblocks = (int)gridDim.x, wave = tid >> 6, lane = tid & 63;
   bool grid_ok = true;
   for (int spin = 0;; ++spin) {
     bool stale = false;
 #pragma unroll
-    for (int k = 0; k < XK; ++k) stale |= xm[k] != epoch;
+    for (int k = 0; k < XK; ++k) stale |= R.m[k] != epoch;
     if (__builtin_amdgcn_ballot_w64(stale) == 0) break;
     if (spin >= MERGE_SPIN_LIMIT) { grid_ok = false; break; }
     __builtin_amdgcn_s_sleep(1);
 #pragma unroll
     for (int k = 0; k < XK; ++k)
-      if (xm[k] != epoch) xm[k] = __hip_atomic_load(marks + min(xi + 64 * NW * k, nblocks - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (R.m[k] != epoch) R.m[k] = __hip_atomic_load(marks + min(tid + 64 * NW * k, nblocks - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   for (int i0 = 2048; grid_ok && i0 < nblocks; i0 += 64 * NW) {      // grids beyond 2048 blocks: the remaining marks, a round at a time
-    const int i = min(i0 + xi, nblocks - 1);
+    const int i = min(i0 + tid, nblocks - 1);
     for (int spin = 0; __builtin_amdgcn_ballot_w64(__hip_atomic_load(marks + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch) != 0; ++spin) {
       if (spin >= MERGE_SPIN_LIMIT) { grid_ok = false; break; }
       __builtin_amdgcn_s_sleep(1);
@@ -322,15 +319,41 @@ __device__ __forceinline__ void merge_heads(const AttnArgs& A, long qh0, int G, 
   // The waves' verdicts meet in LDS behind a barrier that orders LDS traffic only: a full block barrier would first wait for the
   // acknowledgement of the output rows just stored, and the epoch store would then be a second trip to memory at the launch's very end.
   grid_ok = __builtin_amdgcn_ballot_w64(!grid_ok) == 0;
-  if (lane == 0) X.l[wave][0] = grid_ok ? 1.f : 0.f;
+  if (lane == 0) verdict[wave * verdict_stride] = grid_ok ? 1.f : 0.f;
   lds_barrier();
   if (tid == 0) {
     bool all = true;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) all &= X.l[w][0] != 0.f;
+    for (int w = 0; w < NW; ++w) all &= verdict[w * verdict_stride] != 0.f;
     if (all) __hip_atomic_store(A.epochs, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else merge_failed(A, 2u);
   }
+}
+// rec0: the first record of query head 0 of the group, nslot: the splits of the head, rank < 0 or nslot 1: nothing to merge here.
+template <int NWB>      // NWB: waves of the block; twelve-wave blocks (measurement build) merge with their first eight waves
+__device__ __forceinline__ void merge_heads(const AttnArgs& A, long qh0, int G, u32 epoch, long rec0, int nslot, int rank, int mergers, int tid, MergeScratch<(NWB > 8 ? 8 : NWB)>& X) {
+  constexpr int NW = NWB > 8 ? 8 : NWB;
+  const int wave = tid >> 6, lane = tid & 63;
+  if (NWB > NW && wave >= NW) { if (blockIdx.x == gridDim.x - 1) lds_barrier(); return; }      // (the last block meets once more below)
+  const bool last = blockIdx.x == gridDim.x - 1;
+  MarkRegs<NW> xm;
+  if (last) load_marks<NW>(A, tid, xm);
+  // The first item stands outside the loop: at a loop header the compiler waits for every memory operation in flight, which here
+  // would be the acknowledgement of the block's own record stores (a round trip to memory) before the first record load is issued.
+  if (rank >= 0 && nslot > 1) {
+    if (nslot <= WAVE_MERGE_SLOTS && nslot < 2 * G) {
+      // (a wave has one item, or two at sixteen query heads and two splits)
+      for (int item = rank + mergers * wave; item < 2 * G; item += mergers * NW) {
+        if (nslot <= 8) merge_half_head_wave<8>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, lane);
+        else merge_half_head_wave<WAVE_MERGE_SLOTS>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, lane);
+      }
+    } else {
+      int item = rank;
+      if (item < 2 * G) { merge_half_head<NW>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, X, wave, lane); item += mergers; }
+      for (; item < 2 * G; item += mergers) merge_half_head<NW>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, X, wave, lane);
+    }
+  }
+  if (last) advance_epoch<NW>(A, epoch, tid, xm, &X.l[0][0], MAX_SLOTS);
 }
 
 // ---------------------------------------------------------------------------------------------------- uncompressed rows
@@ -788,6 +811,106 @@ __device__ __forceinline__ int take_tile(int* ctr, int hi, int lane) {
 }
 __device__ __forceinline__ int uniform_tile(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// ---------------------------------------------------------------------------------------------------- rows shared out by length
+// Rows of a batch differ in length, and the host does not know by how much.  With the same number of splits for every row the launch lasts
+// as long as a split of the longest row, while the blocks of short rows are mostly start and merge.  Here every block of the launch reads
+// the B lengths and derives, in the same arithmetic and so with the same result, how many splits each row gets and the rows' order, longest
+// first (blocks start in index order, so the short rows fill the end of the launch), and with them its own row, kv head and split:
+//   * one round: the launch uses no more blocks than are resident at once (two four-wave blocks or one eight-wave block per CU), rows get
+//     splits of about c tiles, c the smallest size for which sum ceil(tiles / c) fits (found to 1/120 of c).  Blocks beyond have nothing to do.
+//   * several rounds, where half a split per row, which rounding costs, is more than starting and merging blocks again: nsplit splits per
+//     row.  Their sizes then differ from row to row, which keeps the rounds from starting and ending in step: 2048 blocks of equal size
+//     took 303 us where 16 splits per row take 292 (16 sequences of 4096..65536 tokens).
+// The line: a four-wave block takes about 0.5 us per tile and a round costs some 20 us of starts and merges.  16 sequences of 1000..16000
+// tokens (rounding costs 17 tiles): 91 us in one round, 102 in four; 4096..65536 tokens (68 tiles): 325 against 292.
+// Measured with warm caches against equal split counts: paged, 8 sequences of 200..3000 tokens x 8 kv heads: 27.5 -> 21.7 us, 16 of
+// 500..6000: 71.5 -> 48, 4 of 2000..40000: 82 -> 58; slot cache, 32 rows of 300..6000: 72 -> 62, 8 of 2000..16000: 50 -> 42.
+constexpr int PLAN_ROWS = 256;           // larger batches take nsplit splits per row in batch order
+constexpr float ONE_ROUND_LOSS = 48.f;   // tiles of a four-wave block
+// Smaller splits cost more in the merge than they gain: 30 sequences of up to 3000 tokens, one kv head with 16 query heads: 31.4 us
+// with at least 4 tiles, 27.4 with 12, 30.1 with 20; eight sequences of up to 3000 tokens, 8 kv heads: 21.6, 21.8, 24.5.
+constexpr float MIN_SPLIT_TILES = 12.f;  // of a four-wave block; half as many for an eight-wave block
+struct RowPlan { int b, S, kvh, idx, ns, off, slot; };      // idx: the block's place among the ns blocks of (row, kv head); off: splits of the rows before
+constexpr int PLAN_HEADS = 4096;         // (row, kv head) pairs whose lengths a block keeps (slot cache)
+struct PlanLds { int tiles[PLAN_ROWS], slot[PLAN_ROWS], off[PLAN_ROWS], len[PLAN_HEADS]; };      // len: per row (paged) | per row and kv head
+__device__ __forceinline__ int plan_splits(int tiles, float c, float rc) {      // about ceil(tiles / c), the same wherever it is asked
+  return min(max((int)(((float)tiles + (c - 1.f)) * rc), 1), MAX_SLOTS);
+}
+template <bool PAGED, int NW>
+__device__ __forceinline__ bool plan_block(const AttnArgs& A, PlanLds& P, int tid, RowPlan& R) {
+  constexpr int NT = 64 * NW;
+  const int B = A.B, wave = tid >> 6, lane = tid & 63, sub = lane & 15;
+  // the splits go by the length of kv head 0; the block's own head is looked up from what is read here, which saves a trip to memory
+  const int per_row = PAGED ? 1 : A.n_kv;
+  for (int i = tid; i < B * per_row; i += NT) {
+    const int row = PAGED ? i : small_div(i, per_row), head = PAGED ? 0 : i - row * per_row;
+    const int s = PAGED ? 0 : (A.slot ? A.slot[row] : row);
+    int len = PAGED ? A.sl[row] : A.sl[max(s, 0) * per_row + head];
+    len = s < 0 ? 0 : max(len, 0);
+    P.len[i] = len;
+    if (head == 0) { P.tiles[row] = (len + T - 1) / T; P.slot[row] = s; P.off[row] = 0; }
+  }
+  lds_barrier();
+  float total = 0.f, longest = 0.f, shortest = -INFINITY;      // (shortest: negated)
+  for (int i = lane; i < B; i += 64) { const float t = (float)P.tiles[i]; total += t; longest = fmaxf(longest, t); shortest = fmaxf(shortest, -t); }
+  longest = wave_max(longest); shortest = -wave_max(shortest);
+  // nearly equal rows (within 1/16 of the longest) and every block resident: nsplit splits per row in batch order, and no more to work out
+  const bool equal = A.nsplit * B <= A.plan && __builtin_amdgcn_ballot_w64(longest - shortest > longest * (1.f / 16.f)) == 0;
+  total = wave_sum(total);
+  const int units = min(A.nsplit * B, A.plan);
+  // half a split per row goes to rounding: total / units * B / (2 units) tiles on every block
+  const float fu = (float)units;
+  bool one_round = !equal && A.nsplit > 1 && units >= B && (A.nsplit * B <= A.plan || total * (float)B <= ONE_ROUND_LOSS * 2.f * fu * fu);
+  float c_best = 0.f;
+  if (one_round) {
+    // sixteen sizes from the mean to three times that, then sixteen between the first that fits and the one before it; lane (j, r) =
+    // (lane & 15, lane >> 4) tries size j over the rows r, r + 4, ...
+    const float c_min = fmaxf(floorf(total * __builtin_amdgcn_rcpf(fu)) + 1.f, NW == 4 ? MIN_SPLIT_TILES : 0.5f * MIN_SPLIT_TILES), step = c_min * (2.f / 15.f);
+    float lo = c_min, width = step;
+#pragma unroll 1
+    for (int pass = 0; pass < 2 && one_round; ++pass) {
+      const float c = lo + width * (float)sub, rc = __builtin_amdgcn_rcpf(c);
+      float n = 0.f;
+#pragma unroll 1
+      for (int i = lane >> 4; i < B; i += 4) n += (float)plan_splits(P.tiles[i], c, rc);
+      n = quad_rows_sum(n);
+      const u64 fits = __builtin_amdgcn_ballot_w64(n <= (float)units) & 0xFFFFull;
+      if (fits) c_best = __uint_as_float((u32)__builtin_amdgcn_readlane((int)__float_as_uint(c), __builtin_ctzll(fits)));
+      else one_round = pass != 0;
+      lo = fmaxf(c_best - step, c_min); width = step * (1.f / 16.f);
+    }
+  }
+  const float rc_best = __builtin_amdgcn_rcpf(c_best);
+  const auto splits = [&](int tiles) { return one_round ? plan_splits(tiles, c_best, rc_best) : A.nsplit; };
+  // splits ahead of row i: each wave counts a share of the rows for all i
+  if (!equal) {
+    for (int i0 = 0; i0 < B; i0 += 64) {
+      const int i = i0 + lane, mine = P.tiles[min(i, B - 1)];
+      int ahead = 0;
+#pragma unroll 1
+      for (int k = wave; k < B; k += NW) {
+        const int tk = P.tiles[k];
+        ahead += tk > mine || (tk == mine && k < i) ? splits(tk) : 0;
+      }
+      if (i < B) atomicAdd(&P.off[i], ahead);
+    }
+    lds_barrier();
+  }
+  for (int i0 = 0; i0 < B; i0 += 64) {
+    const int i = min(i0 + lane, B - 1), ns = splits(P.tiles[i]), off = equal ? i * A.nsplit : P.off[i], w = (int)blockIdx.x - off * A.n_kv;
+    const u64 own = __builtin_amdgcn_ballot_w64(i == i0 + lane && w >= 0 && w < ns * A.n_kv);
+    if (own != 0) {
+      const int l = __builtin_ctzll(own), wl = __builtin_amdgcn_readlane(w, l);
+      R.b = i0 + l; R.ns = __builtin_amdgcn_readlane(ns, l); R.off = __builtin_amdgcn_readlane(off, l);
+      R.kvh = __builtin_amdgcn_readfirstlane(small_div(wl, R.ns)); R.idx = wl - R.kvh * R.ns;
+      R.slot = __builtin_amdgcn_readfirstlane(P.slot[R.b]);
+      R.S = __builtin_amdgcn_readfirstlane(P.len[PAGED ? R.b : R.b * A.n_kv + R.kvh]);
+      return true;
+    }
+  }
+  return false;
+}
+
 // ---------------------------------------------------------------------------------------------------- main kernel
 // NW = waves per block: 4 (two blocks per CU) or 8 (one block per CU: half as many partials to merge for the same occupancy)
 // HOST_LEN: the compressed length of every addressed head is the kernel argument S_all (not read from memory)
@@ -820,39 +943,42 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     for (int i = tid; i < A.n_free; i += NT) { const int r = A.freeq[i]; if (r >= 0) A.stack[atomicAdd(A.top, 1)] = r; }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  // Paged pool: the split index is rotated by the head index: the last split of a sequence carries the raw tile that is still filling,
-  // and with equal split counts all of them would otherwise sit on the same XCD, which then finishes long after the others.
-  const int bh = (int)blockIdx.x / A.nsplit, split = ((int)blockIdx.x + (PAGED ? bh : 0)) % A.nsplit;
-  int b = bh / A.n_kv, S_ranked = -1;
-  const int kvh = bh % A.n_kv, G = A.G;
-  if (PAGED) {
-    // Ragged batches: blocks start in index order, so the longest sequences go first and the short ones fill the end of the launch
-    // (in batch order a long sequence that happens to come last runs on with most of the GPU idle).  Batch row = the sequence whose
-    // length has rank b; every block ranks the lengths itself (thread i counts the sequences ahead of sequence i).
-    const int Bn = (int)gridDim.x / (A.nsplit * A.n_kv);
-    if (Bn > 1 && Bn <= NT) {
-      int* lens = reinterpret_cast<int*>(&M.acc[0][0][0]);      // the merge buffer is idle until the tile loop has ended
-      const int mine = tid < Bn ? max(A.sl[tid], 0) : 0;
-      if (tid < Bn) lens[tid] = mine;
-      __syncthreads();
-      if (tid < Bn) {
-        int rank = 0;
-        for (int j = 0; j < Bn; ++j) { const int lj = lens[j]; rank += (lj > mine || (lj == mine && j < tid)) ? 1 : 0; }
-        if (rank == b) { lens[NT] = tid; lens[NT + 1] = mine; }
+  const int G = A.G;
+  RowPlan R;
+  if (!HOST_LEN && A.plan) {
+    // (the merge buffer is idle until the tile loop has ended)
+    if (!plan_block<PAGED, NW>(A, *reinterpret_cast<PlanLds*>(&M.acc[0][0][0]), tid, R)) {
+      if (A.nslot > 1) {      // no unit left for this block: it only takes its part in the launch's epoch
+        const u32 epoch = load_epoch(A);
+        if (tid == 0) mark_arrival(A, epoch);
+        if (blockIdx.x == gridDim.x - 1) {
+          MarkRegs<NW> xm;
+          load_marks<NW>(A, tid, xm);
+          advance_epoch<NW>(A, epoch, tid, xm, &M.m[0][0], 1);
+        }
       }
-      __syncthreads();
-      b = __builtin_amdgcn_readfirstlane(lens[NT]); S_ranked = __builtin_amdgcn_readfirstlane(lens[NT + 1]);
+      return;
     }
+  } else {
+    const int bh = __builtin_amdgcn_readfirstlane(small_div(blockIdx.x, A.nsplit));
+    R.b = __builtin_amdgcn_readfirstlane(small_div(bh, A.n_kv)); R.kvh = bh - R.b * A.n_kv; R.idx = (int)blockIdx.x - bh * A.nsplit; R.ns = A.nsplit; R.off = R.b * A.nsplit; R.S = -1;
+    // (no slot map = row b attends over cache heads b*n_kv ..: one level of dependent loads less)
+    R.slot = PAGED ? 0 : (A.slot ? A.slot[R.b] : R.b);
+    if (!PAGED && !HOST_LEN) R.S = A.sl[max(R.slot, 0) * A.n_kv + R.kvh];
   }
+  const int b = R.b, kvh = R.kvh, ns = R.ns;
+  // Paged pool: the split index is rotated by the head's place in the grid: the last split of a sequence carries the raw tile that is still filling,
+  // and all of them would otherwise sit on the same XCD whenever the split count is a multiple of eight, which then finishes long after the others.
+  const int turn = R.idx + ((R.off * A.n_kv) >> 4) + kvh;
+  const int split = PAGED ? turn - ns * __builtin_amdgcn_readfirstlane(small_div(turn, ns)) : R.idx;
   const long qh0 = (long)b * A.n_q + (long)kvh * G;
   // Level 1: the slot of the batch row; the query rows do not depend on it
   TableRegs Tr;
   if (tid < 256) tables_load_q(Tr, tid, A.q + qh0 * D, G);
-  // (no slot map = row b attends over cache heads b*n_kv ..: one level of dependent loads less)
-  const int slot = PAGED ? 0 : (A.slot ? A.slot[b] : b), ch = PAGED ? kvh : (slot < 0 ? 0 : slot) * A.n_kv + kvh;
+  const int slot = R.slot, ch = PAGED ? kvh : (slot < 0 ? 0 : slot) * A.n_kv + kvh;
   // Level 2: everything indexed by the cache head
   int S, TLh = 0; long khs = 0, vhs = 0;
-  if (PAGED) S = S_ranked >= 0 ? S_ranked : max(A.sl[b], 0);
+  if (PAGED) S = R.S >= 0 ? R.S : max(A.sl[b], 0);
   else {
     // lengths known to the host (a Page) come as a kernel argument: the tile range, and with it the first payload loads, then depend on
     // nothing but the arguments
@@ -864,12 +990,12 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     khs = A.k.head_start[chv]; vhs = A.v.head_start[chv];
     TLh = (A.kt ? A.tl : A.k.head_start)[chv];      // no branch between the loads of this level
     if (HOST_LEN) S = A.S_all;
-    else S = A.sl[ch];
+    else S = R.S;
     if (slot < 0) S = 0;
   }
-  if (tid < 256) tables_load_bases(Tr, tid, A.k.base3, A.k.base4, A.v.base3, A.v.base4, ch % A.NB);
+  if (tid < 256) tables_load_bases(Tr, tid, A.k.base3, A.k.base4, A.v.base3, A.v.base4, ch - A.NB * __builtin_amdgcn_readfirstlane(small_div(ch, A.NB)));
 
-  const int ntiles = (S + T - 1) / T, chunk = (ntiles + A.nsplit - 1) / A.nsplit;
+  const int ntiles = (S + T - 1) / T, chunk = __builtin_amdgcn_readfirstlane(small_div(ntiles + ns - 1, ns));
   const int tlo = min(split * chunk, ntiles), thi = min(tlo + chunk, ntiles);
   const int thi_fast = PAGED ? min(thi, tlo + MAX_CHUNK) : thi;      // the pipelined loop's range: what one fill of the LDS tile table covers
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, a = lane & 15, q = lane >> 4;
@@ -920,7 +1046,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   }
   if (tid == 0) next_tile = 2 * NW;
   // this launch's epoch of the fused merge: one more load of the start-up batch, its value is needed when the block is done
-  const u32 epoch = load_epoch(A, bh);
+  const u32 epoch = load_epoch(A);
   GAAC_STAMP(6);
   if (tid < 256) tables_store(L, Tr, tid, G);
   GAAC_STAMP(7);
@@ -939,7 +1065,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   st.m_run = -INFINITY; st.mu_run = 0.f; st.l_run = 0.f;
 
   // ---- the raw tail of the cache head: wave 0 of the last split's block, before it joins the tile hand-out
-  if (!PAGED && A.kt && split == A.nsplit - 1 && wave == 0) {
+  if (!PAGED && A.kt && split == ns - 1 && wave == 0) {
     const int TL = slot < 0 ? 0 : min(__builtin_amdgcn_readfirstlane(TLh), A.tcap);
     if (TL > 0) {
       // probabilities go through this wave's own merge slot: the other waves write theirs as soon as they run out of tiles
@@ -1060,7 +1186,8 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   lds_barrier();      // only LDS data crosses (a full barrier would also wait for the acknowledgement of the arrival mark)
   GAAC_MSTAMP(6, wall_clock64());
   const bool fused = A.epochs != nullptr;
-  const int mergers = merge_ranks(G, A.nslot), rank = (int)blockIdx.x % A.nsplit - (A.nsplit - mergers);      // the head's last blocks to start
+  const int mergers = merge_ranks(G, ns), rank = R.idx - (ns - mergers);      // the head's last blocks to start
+  const long rec0 = (long)R.off * A.n_q + (long)(kvh * G) * ns;      // the group's first record
   const int d = tid & 127;
   for (int g = tid >> 7; g < G; g += NT / 128) {
     // every LDS read up front and none under a branch: nine dependent round trips otherwise
@@ -1077,11 +1204,11 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
       const float f = live ? __builtin_amdgcn_exp2f(mv[w] - Mx) : 0.f;
       Lc += lv[w] * f; Ac += (live ? av[w] : 0.f) * f;
     }
-    const long pidx = (qh0 + g) * A.nslot + split;
+    const long pidx = rec0 + (long)g * ns + split;
     if (!fused) {
       if (d == 0) { store_partial(A.pm + pidx, Mx); store_partial(A.pl + pidx, Lc); }
       store_partial(A.pa + pidx * D + d, Ac);
-    } else if (A.nslot == 1) {      // the only partial of its rows: it is the result
+    } else if (ns == 1) {      // the only partial of its rows: it is the result
       A.out[(qh0 + g) * D + d] = __builtin_bit_cast(u16, (__bf16)(Lc > 0.f ? Ac / Lc : 0.f));
     } else {
       if (d == 0) { ll_store(reinterpret_cast<u64*>(A.pm) + pidx, Mx, epoch); ll_store(reinterpret_cast<u64*>(A.pl) + pidx, Lc, epoch); }
@@ -1089,9 +1216,9 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     }
   }
   GAAC_STAMP(4);
-  if (fused && rank >= 0 && A.nslot > 1) {
+  if (fused && A.nslot > 1 && ((rank >= 0 && ns > 1) || blockIdx.x == gridDim.x - 1)) {
     lds_barrier();      // every thread is done with the block-merge buffer, which becomes the mergers' scratch
-    merge_heads<NW>(A, qh0, G, epoch, rank, mergers, tid, *reinterpret_cast<MergeScratch<(NW > 8 ? 8 : NW)>*>(&M.acc[0][0][0]));
+    merge_heads<NW>(A, qh0, G, epoch, rec0, ns, rank, mergers, tid, *reinterpret_cast<MergeScratch<(NW > 8 ? 8 : NW)>*>(&M.acc[0][0][0]));
   }
   GAAC_STAMP(5);
 }
@@ -1212,7 +1339,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_bf16_attn_split(co
   RawTile R0, R1;
   if (tA < thd) load_raw_tile(kh, vh, tA, S, a, q, R0);
   if (tid == 0) next_tile = tlo + 2 * NW;
-  const u32 epoch = load_epoch(A, bh);
+  const u32 epoch = load_epoch(A);
   // Q as the B operand: lane (head a, quad q), product j covers channels 32 j + 8 q .. + 8 (rows >= G are zero)
   for (int i = tid; i < GMAX * NG; i += NT) {
     const int h = i >> 4, c = i & 15;
@@ -1276,13 +1403,21 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_bf16_attn_split(co
   }
   if (rank >= 0 && A.nslot > 1) {
     lds_barrier();
-    merge_heads<NW>(A, qh0, G, epoch, rank, mergers, tid, *reinterpret_cast<MergeScratch<NW>*>(&L.acc[0][0][0]));
+    merge_heads<NW>(A, qh0, G, epoch, qh0 * A.nslot, A.nslot, rank, mergers, tid, *reinterpret_cast<MergeScratch<NW>*>(&L.acc[0][0][0]));
   }
 }
 
 }  // namespace gaac
 
 using namespace gaac;
+
+// How many splits of n_kv blocks plan_block may count as resident, 0: no plan.  The plan costs a block 0.8 to 1.4 us at its start (its
+// instructions come from memory on a first launch).  It cannot gain that where all blocks are resident and a split of the longest possible
+// row is no more than five tiles for each of the block's eight waves, about 7 us.
+static int plan_units(int B, int n_kv, int nsplit, long max_tiles) {
+  const long blocks = (long)B * n_kv * nsplit;
+  return B > 1 && B <= PLAN_ROWS && B * n_kv <= PLAN_HEADS && (blocks > 256 || max_tiles > 40l * nsplit) ? std::max((blocks > 256 ? 512 : 256) / n_kv, 1) : 0;
+}
 
 #ifdef GAAC_PHASE_TIMING
 static long long* g_dbg = nullptr;
@@ -1311,6 +1446,7 @@ static int attn_split_impl(
   A.n_kv = n_kv; A.n_q = n_q; A.G = n_q / n_kv; A.NB = NB;
   A.kt = (const u16*)kt; A.vt = (const u16*)vt; A.tl = TL; A.tcap = TCAP;
   A.epochs = epoch; A.out = (u16*)out;
+  A.B = B; A.plan = epoch && S_all < 0 && plan_units(B, n_kv, nsplit, S_pad / T);
   GAAC_REQUIRE(!epoch || out, "gaac_attn: the fused merge needs an output buffer");
   A.pool = nullptr; A.raw = nullptr; A.mt = nullptr; A.bt = nullptr; A.bt_stride = 0; A.TS = 0;
   A.freeq = nullptr; A.n_free = 0; A.stack = nullptr; A.top = nullptr;
@@ -1498,6 +1634,7 @@ extern "C" int gaac_paged_attn(
   A.n_kv = n_kv; A.n_q = n_q; A.G = n_q / n_kv; A.NB = NB;
   A.kt = nullptr; A.vt = nullptr; A.tl = nullptr; A.tcap = 0;
   A.epochs = epoch; A.out = (u16*)out;
+  A.B = B; A.plan = plan_units(B, n_kv, nsplit, max_tiles);
   A.pool = pool; A.raw = (const u16*)raw; A.mt = mt; A.bt = bt; A.bt_stride = bt_stride; A.TS = TS;
   A.freeq = freeq; A.n_free = freeq ? n_free : 0; A.stack = stack; A.top = top;
 #ifdef GAAC_PHASE_TIMING

@@ -60,6 +60,23 @@ def choose_nsplit(B: int, n_kv: int, S: int, target_ctas: int = 256, min_tok: in
     return min(max(1, target_ctas // (B * n_kv)), max(1, S // min_tok), cap)
 
 
+def launch_nsplit(B: int, n_kv: int, S: int, ragged: bool) -> int:
+    """Splits per (row, kv head) where the caller leaves the choice: S tokens per row, or up to S if ragged (the launch then shares its
+    blocks out by length).  Measured, 4 query heads per kv head, us:
+      * up to 256 tokens in one split (100 tokens: 6.8, against 7.3 to 8.8 with 2 to 6 splits; 300 tokens: 9.0, against 8.2 with 8);
+      * at least 32 tokens per split (1000 tokens x 8 heads: 11.3 with 3 splits, 9.0 with 6, 8.7 with 32; 3000: 11.3 with 12, 9.5 with
+        32), but no more than 64 splits of less than 256 (the merge: 8000 tokens, 1 head of 16 queries: 14.7 with 64, 24.4 with 256);
+      * one eight-wave block per CU (256 blocks: a second round of blocks costs more than it evens out), and where rows are ragged and
+        the heads alone take more than a quarter of the CUs, two four-wave blocks per CU, to have enough of them to share out
+        (32 rows of 300..6000 tokens x 8 heads: 72 us with 1 split, 62 with 2; 12 rows of up to 8000: 38 with 2, 33 with 5); two splits up
+        to 512 heads (48 rows of up to 8000 x 8 heads: 135 with 1, 107 with 2)."""
+    H = B * n_kv
+    if S <= 256: return 1
+    if ragged and B > 1 and H > 64: n = -(-512 // H) if H <= 256 else 2 if H <= 512 else 1
+    else: n = 256 // H
+    return max(1, min(n, max(S // 256, min(64, S // 32))))
+
+
 class AttnWorkspace:
     """Output + split partials of one launch shape (rows = B*n_q).  The one-kernel launch stores every partial value as a 64-bit
     record (fp32 bits | launch epoch << 32): pm, pl [rows*NSLOT], pa [rows*NSLOT*D] int64.  epoch: [0] the epoch of the last merged
@@ -173,7 +190,7 @@ def attention(q, kp, vp, scale=None, nsplit=None, phase="fused"):
     q: [B, n_q, D] bf16 (one query token per sequence) -> [B, n_q, D] bf16."""
     B, n_q, Dq = q.shape
     n_kv = kp.H // B
-    if nsplit is None: nsplit = choose_nsplit(B, n_kv, kp.S)
+    if nsplit is None: nsplit = launch_nsplit(B, n_kv, kp.S, ragged=False)
     # the one-kernel launch takes the length as an argument; the other phases read one per head
     SL = None if phase == "fused" else torch.full((kp.H,), kp.S, dtype=torch.int32, device=q.device)
     out = attn_launch(kp, vp, q.reshape(B * n_q, Dq).contiguous(), None, n_q, n_kv, SL, kp.sm.shape[1] // D,
