@@ -135,17 +135,19 @@ def rows_in_place(x: torch.Tensor, head_dim: int, row_dim: int) -> tuple[torch.T
     return x, strides[head_dim], strides[row_dim]
 
 
-def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Tensor, n_kv: int) -> Page:
+def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Tensor, n_kv: int, scratch=None) -> Page:
     """Encode x (bf16 [H, S, D], on the GPU) with the given bases.  Three launches: every tile is encoded with its escapes in a worst-case
     slot; the sizes of the slots are scanned per head; then, with the stream sized by the host (the totals arrive in host memory that
-    the scan writes to), the slots are packed head by head and the row offsets written (the steps of encoder.py:111-123)."""
+    the scan writes to), the slots are packed head by head and the row offsets written (the steps of encoder.py:111-123).
+    scratch(n, device): where the slots' n bytes come from, if not from torch's allocator."""
     H, S, _ = x.shape
     dev = x.device
     x, hs, rs = rows_in_place(x, 0, 1)
     S_pad = (S + T - 1) // T * T
     nt = H * (S_pad // T)
     new = lambda *shape, dtype=torch.uint8: torch.empty(shape, dtype=dtype, device=dev)
-    sm, cd, slots = new(H, S_pad * D), new(H, S_pad * CB), new(nt * TILE_MAX_ESC)
+    sm, cd = new(H, S_pad * D), new(H, S_pad * CB)
+    slots = scratch(nt * TILE_MAX_ESC, dev) if scratch else new(nt * TILE_MAX_ESC)
     flags, ovf_off, tile_off = new(H, S_pad, dtype=torch.int32), new(H, S, dtype=torch.int32), new(H, S_pad // T, dtype=torch.int32)
     head_start, sizes = new(H + 1, dtype=torch.int32), new(nt + H, dtype=torch.int32)      # sizes: per tile, then per head
     totals = torch.empty(H, dtype=torch.int32, pin_memory=True)
