@@ -833,6 +833,7 @@ constexpr float MIN_SPLIT_TILES = 12.f;  // of a four-wave block; half as many f
 struct RowPlan { int b, S, kvh, idx, ns, off, slot; };      // idx: the block's place among the ns blocks of (row, kv head); off: splits of the rows before
 constexpr int PLAN_HEADS = 4096;         // (row, kv head) pairs whose lengths a block keeps (slot cache)
 struct PlanLds { int tiles[PLAN_ROWS], slot[PLAN_ROWS], off[PLAN_ROWS], len[PLAN_HEADS]; };      // len: per row (paged) | per row and kv head
+static_assert(sizeof(PlanLds) <= 5 * GMAX * D * sizeof(float), "the plan's view must fit the merge buffer");
 __device__ __forceinline__ int plan_splits(int tiles, float c, float rc) {      // about ceil(tiles / c), the same wherever it is asked
   return min(max((int)(((float)tiles + (c - 1.f)) * rc), 1), MAX_SLOTS);
 }
@@ -1446,7 +1447,7 @@ static int attn_split_impl(
   A.n_kv = n_kv; A.n_q = n_q; A.G = n_q / n_kv; A.NB = NB;
   A.kt = (const u16*)kt; A.vt = (const u16*)vt; A.tl = TL; A.tcap = TCAP;
   A.epochs = epoch; A.out = (u16*)out;
-  A.B = B; A.plan = epoch && S_all < 0 && plan_units(B, n_kv, nsplit, S_pad / T);
+  A.B = B; A.plan = epoch && S_all < 0 ? plan_units(B, n_kv, nsplit, S_pad / T) : 0;
   GAAC_REQUIRE(!epoch || out, "gaac_attn: the fused merge needs an output buffer");
   A.pool = nullptr; A.raw = nullptr; A.mt = nullptr; A.bt = nullptr; A.bt_stride = 0; A.TS = 0;
   A.freeq = nullptr; A.n_free = 0; A.stack = nullptr; A.top = nullptr;
