@@ -92,6 +92,26 @@ def test_windows_grow_for_a_prompt_and_refuse_when_they_may_not():
     assert _held(fixed, 1, small, small)
 
 
+@pytest.mark.parametrize("raw_k,raw_v", [(0.0, 0.02), (0.02, 0.0), (0.02, 0.05), (0.05, 0.02), (0.0, 0.3), (0.3, 0.3)])
+def test_windows_grow_for_k_then_for_v(raw_k, raw_v):
+    """Short slots, whose default windows are smaller than the headroom, so that the first prompt makes them grow: for K's largest head,
+    and again for V's only if it needs more than that gave.  The window size that results is part of the cache's layout."""
+    dev = require_gpu()
+    from gaac_amd import CompressedKVCache
+    L = 73
+    k16, v16 = _tokens(L, 31, outliers=raw_k), _tokens(L, 32, outliers=raw_v)
+    cache = CompressedKVCache(2, N_KV, L + 7, device=dev)
+    want = cache.k.ovf_cap
+    cache.prefill(1, to_bf16(k16, dev), to_bf16(v16, dev))
+    for st in (cache.k, cache.v):
+        need = int(st.ovf_used.max()) + 1288
+        if need > want: want = max(2 * want, need + 4096 + 7) // 8 * 8
+    assert cache.k.ovf_cap == cache.v.ovf_cap == want
+    assert cache.k.ovf.numel() == cache.v.ovf.numel() == 2 * N_KV * want
+    assert cache.k.head_start.tolist() == cache.v.head_start.tolist() == [i * want for i in range(2 * N_KV + 1)]
+    assert _held(cache, 1, k16, v16)
+
+
 def test_rejected_arguments():
     dev = require_gpu()
     from gaac_amd import CompressedKVCache
