@@ -67,6 +67,46 @@ def test_no_device_no_fallback():
         Codec(2, "cpu").calibrate(torch.zeros(2, 16, 128, dtype=torch.bfloat16))
 
 
+@pytest.mark.parametrize("shape", [(2, 32, 64), (3, 1, 64), (2, 32, 127), (1, 1, 1), (2, 32, 256), (0, 4, 64), (4, 128), (1, 2, 32, 128)])
+def test_encoder_refuses_rows_of_another_size(shape):
+    """Rows that are not 128 elements are refused by every encoding call before anything is allocated for them or launched."""
+    from gaac_amd import Codec, TileEncoder
+    from gaac_amd.codec import encode_page, rows_in_place
+    x = torch.zeros(shape, dtype=torch.bfloat16)
+    base = torch.zeros(2, 128, dtype=torch.uint8)
+    codec = Codec(2, "cpu").set_bases(base, base)
+    if len(shape) == 3:
+        with pytest.raises(RuntimeError, match="rows of 128"): encode_page(x, "k", base, base, 2)
+        with pytest.raises(RuntimeError, match="rows of 128"): codec.encode(x, "v")
+        with pytest.raises(RuntimeError, match="rows of 128"): TileEncoder("k", "cpu").encode(codec, x)
+    with pytest.raises(RuntimeError, match="rows of 128"): TileEncoder("k", "cpu").encode_tiles(x, base, base, None, None, None, 16, 16, 2)
+    with pytest.raises(RuntimeError, match="rows of 128"): rows_in_place(x, 0, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.uint8])
+def test_encoder_refuses_elements_of_another_size(dtype):
+    from gaac_amd.codec import rows_in_place
+    with pytest.raises(RuntimeError, match="bf16 rows"): rows_in_place(torch.zeros(2, 32, 128, dtype=dtype), 0, 1)
+
+
+@pytest.mark.parametrize("H,S,off,hs,rs", [(2, 5, 0, 640, 128), (2, 5, 0, 128, 256), (3, 1, 0, 128, 7), (1, 4, 0, 3, 128), (2, 4, 8, 1024, 136), (2, 4, 0, 0, 128),
+                                           (2, 4, 1, 512, 128), (2, 4, 0, 512, 129), (2, 4, 0, 513, 128), (2, 4, 0, 512, 0), (2, 4, 0, 512, 64), (2, 0, 0, 0, 128)])
+def test_rows_are_read_through_strides_that_stay_inside_their_memory(H, S, off, hs, rs):
+    """Every (head, row) that the returned strides address holds the 128 elements of that row, whether the rows are used where they
+    are or from a copy; rows that the kernel reads are 16-byte aligned."""
+    from gaac_amd.codec import rows_in_place
+    mem = torch.arange(8192, dtype=torch.int16)
+    x = torch.as_strided(mem, (H, S, 128), (hs, rs, 1), off)
+    y, yh, yr = rows_in_place(x, 0, 1)
+    assert y.data_ptr() % 16 == 0 and yh % 8 == 0 and yr % 8 == 0 and yr >= 128
+    base = y.storage_offset()
+    flat = torch.as_strided(y, (y.untyped_storage().nbytes() // 2,), (1,), 0)
+    for h in range(H):
+        for t in range(S):
+            at = base + h * yh + t * yr
+            assert at + 128 <= flat.numel() and torch.equal(flat[at:at + 128], x[h, t])
+
+
 def test_product_code_does_not_import_the_oracle():
     pkg = os.path.join(ROOT, "gaac_amd")
     for dirpath, _, files in os.walk(pkg):
