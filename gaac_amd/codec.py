@@ -138,6 +138,15 @@ def rows_in_place(x: torch.Tensor, head_dim: int, row_dim: int) -> tuple[torch.T
     return x, strides[head_dim], strides[row_dim]
 
 
+def stream_bytes(totals: list[int]) -> int:
+    """Bytes of a page's escape stream from its heads' totals (gaac_tile_scan gives 2^31 - 1 for a head that has as many or more).  Offsets
+    into the stream are int32: a longer one raises, before anything is written into it."""
+    total = sum(totals)
+    if total >= 2 ** 31 - 1:
+        raise RuntimeError(f"the page's escape stream of {total} bytes or more does not fit 32-bit offsets: encode fewer tokens or heads at a time")
+    return total
+
+
 def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Tensor, n_kv: int, scratch=None) -> Page:
     """Encode x (bf16 [H, S, D], on the GPU) with the given bases.  Three launches: every tile is encoded with its escapes in a worst-case
     slot; the sizes of the slots are scanned per head; then, with the stream sized by the host (the totals arrive in host memory that
@@ -160,7 +169,7 @@ def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Te
               p(sm), p(cd), p(flags), p(slots), tile_bytes, st)
     _lib.call("gaac_tile_scan", tile_bytes, H, S_pad // T, p(tile_off), head_bytes, totals.data_ptr(), st)
     torch.cuda.current_stream(dev).synchronize()
-    ovf = new(sum(totals.tolist()) + 8)
+    ovf = new(stream_bytes(totals.tolist()) + 8)
     _lib.call("gaac_page_pack", p(slots), tile_bytes, p(tile_off), head_bytes, p(flags), H, S, S_pad, p(head_start), p(ovf), p(ovf_off), st)
     return Page(sm, cd, flags, ovf_off, ovf, head_start, tile_off, base3, base4, H, S, n_kv, kind)
 

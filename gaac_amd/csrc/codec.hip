@@ -231,7 +231,7 @@ __device__ __forceinline__ int scan_tile_bytes(const int* __restrict__ tb, int* 
     for (int w = 0; w < SCAN_NT / 64; ++w) { const int v = sh[w]; all += v; before += w < wave ? v : 0; }
 #pragma unroll
     for (int k = 0; k < SCAN_PER; ++k) if (t0 + 64 * k < ntiles) off[t0 + 64 * k] = carry + before + incl[k] - n[k];
-    carry += all;
+    carry = carry > 0x7FFFFFFF - all ? 0x7FFFFFFF : carry + all;      // (all: at most 4096 tiles of 1280 bytes)
     __syncthreads();
   }
   return carry;

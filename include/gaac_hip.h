@@ -46,9 +46,10 @@ int gaac_compact(const uint8_t* esc_slots, const int* tile_bytes, int* tile_off,
                  int H, int ntiles, void* stream);
 
 /* The same packing for a whole Page in two steps, so that the caller can size the stream in between (encoder.py:104-123):
- * gaac_tile_scan: tile_off[h, t] as above, head_bytes[h] = the head's total, and once more host_bytes[h] (or NULL), which may be host
- * memory that the device can write: it is set when the stream has reached this point.
- * gaac_page_pack: ovf [sum of head_bytes + 8] = the heads' streams back to back and eight zero bytes, head_start [H+1], and
+ * gaac_tile_scan: tile_off[h, t] as above, head_bytes[h] = the head's total (2^31 - 1 where it is that or more: the offsets are then
+ * of no use), and once more host_bytes[h] (or NULL), which may be host memory that the device can write: it is set when the stream has
+ * reached this point.
+ * gaac_page_pack (the head_bytes sum to less than 2^31 - 1): ovf [sum of head_bytes + 8] = the heads' streams back to back and eight zero bytes, head_start [H+1], and
  * ovf_off [H, S] = row_offsets(flags, S) (codec.py:221-225). */
 int gaac_tile_scan(const int* tile_bytes, int H, int ntiles, int* tile_off, int* head_bytes, int* host_bytes, void* stream);
 int gaac_page_pack(const uint8_t* esc_slots, const int* tile_bytes, const int* tile_off, const int* head_bytes, const int* flags, int H, int S, int S_pad,

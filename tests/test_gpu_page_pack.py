@@ -46,3 +46,23 @@ def test_many_tiles(kind, H, S):
     last = sum((((f >> (2 * j)) & 1) + 4 * ((f >> (2 * j + 1)) & 1)) for j in range(16))
     start = torch.cat([torch.zeros(1, dtype=torch.int64, device=dev), (rows[:, -1] + last).cumsum(0)])
     assert torch.equal(page.ovf_head_start.to(torch.int64), start) and page.ovf.numel() == int(start[-1]) + 8
+
+
+@pytest.mark.parametrize("ntiles", [4096, 3 * 4096 - 7])
+def test_scan_totals_stop_at_the_largest_int(ntiles):
+    """Totals that 32 bits cannot hold come out as 2^31 - 1, next to heads whose totals are exact up to there."""
+    dev = require_gpu()
+    from gaac_amd import _lib
+    big = (2 ** 31 - 2) // ntiles
+    per_tile = [3, big, min(big + 1 + big // 8, 2 ** 18), 2 ** 18]      # per head; a round of 4096 tiles stays below 2^31
+    sizes = torch.tensor(per_tile, dtype=torch.int32, device=dev)[:, None].expand(4, ntiles).contiguous()
+    sizes[1] = min(big, 2 ** 18)
+    off, heads, host = torch.empty_like(sizes), torch.empty(4, dtype=torch.int32, device=dev), torch.empty(4, dtype=torch.int32, pin_memory=True)
+    _lib.call("gaac_tile_scan", _lib.ptr(sizes), 4, ntiles, _lib.ptr(off), _lib.ptr(heads), host.data_ptr(), _lib.stream())
+    torch.cuda.synchronize()
+    exact = sizes.cpu().to(torch.int64)
+    want = exact.sum(1).clamp(max=2 ** 31 - 1)
+    assert heads.tolist() == host.tolist() == want.tolist()
+    assert ntiles == 4096 or (want[2:] == 2 ** 31 - 1).all()
+    for h in range(4):
+        if want[h] < 2 ** 31 - 1: assert torch.equal(off[h].cpu().to(torch.int64), exact[h].cumsum(0) - exact[h])

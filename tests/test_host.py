@@ -89,6 +89,14 @@ def test_encoder_refuses_elements_of_another_size(dtype):
     with pytest.raises(RuntimeError, match="bf16 rows"): rows_in_place(torch.zeros(2, 32, 128, dtype=dtype), 0, 1)
 
 
+def test_escape_stream_beyond_32_bits_is_refused():
+    """Totals are summed beyond 32 bits and refused before the stream is allocated; a head's total that reached the limit counts as too long."""
+    from gaac_amd.codec import stream_bytes
+    assert stream_bytes([]) == 0 and stream_bytes([5, 0, 7]) == 12 and stream_bytes([2 ** 30, 2 ** 30 - 2]) == 2 ** 31 - 2
+    for totals in ([2 ** 31 - 1], [2 ** 30, 2 ** 30 - 1], [2 ** 30] * 2, [2 ** 30] * 4, [2 ** 31 - 1] * 3):
+        with pytest.raises(RuntimeError, match="32-bit offsets"): stream_bytes(totals)
+
+
 @pytest.mark.parametrize("H,S,off,hs,rs", [(2, 5, 0, 640, 128), (2, 5, 0, 128, 256), (3, 1, 0, 128, 7), (1, 4, 0, 3, 128), (2, 4, 8, 1024, 136), (2, 4, 0, 0, 128),
                                            (2, 4, 1, 512, 128), (2, 4, 0, 512, 129), (2, 4, 0, 513, 128), (2, 4, 0, 512, 0), (2, 4, 0, 512, 64), (2, 0, 0, 0, 128)])
 def test_rows_are_read_through_strides_that_stay_inside_their_memory(H, S, off, hs, rs):
