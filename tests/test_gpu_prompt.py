@@ -112,6 +112,33 @@ def test_windows_grow_for_k_then_for_v(raw_k, raw_v):
     assert _held(cache, 1, k16, v16)
 
 
+@pytest.mark.parametrize("calibrate", [True, False])
+@pytest.mark.parametrize("L", [1, 15])
+def test_prompts_shorter_than_a_tile_are_put_in_place_without_a_wait(L, calibrate):
+    """They have no escapes to wait for: captured and replayed with new rows in the same buffers, and from other float types."""
+    dev = require_gpu()
+    from gaac_amd import CompressedKVCache
+    b = torch.full((N_KV, 128), 120, dtype=torch.uint8)
+    cache = CompressedKVCache(3, N_KV, 64, None if calibrate else dict(k3=b, k4=b, v3=b, v4=b), device=dev)
+    k16, v16 = _tokens(L, 41), _tokens(L, 42)
+    k, v = to_bf16(k16, dev), to_bf16(v16, dev)
+    cache.prefill(0, k, v)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g): cache.prefill(1, k, v)
+    for seed in (43, 44, 45):
+        a16, c16 = _tokens(L, seed), _tokens(L, seed + 10)
+        k.copy_(to_bf16(a16, dev)); v.copy_(to_bf16(c16, dev))
+        g.replay(); torch.cuda.synchronize()
+        assert _held(cache, 1, a16, c16) and _held(cache, 0, k16, v16)
+        if calibrate: assert np.array_equal(cache.k.base3[N_KV:2 * N_KV].cpu().numpy(), O.bases_from_hist(O.exponent_hist(a16, N_KV), N_KV)[0])
+    cache.prefill(2, to_bf16(k16, dev).float(), to_bf16(v16, dev).float())
+    assert _held(cache, 2, k16, v16)
+    if not calibrate:
+        cache.prefill(2, to_bf16(v16, "cpu"), to_bf16(k16, "cpu").double())
+        assert _held(cache, 2, v16, k16)
+    assert cache.S.tolist() == [0] * 3 * N_KV and cache.tail_len.tolist() == [L] * 3 * N_KV
+
+
 def test_rejected_arguments():
     dev = require_gpu()
     from gaac_amd import CompressedKVCache
