@@ -74,9 +74,11 @@ constexpr int SLOT_CD = TILE_SM, SLOT_FL = TILE_SM + TILE_CD, SLOT_OV = SLOT_FL 
 // n / d for the block's own coordinates: the compiler's 32-bit division is a chain of quarter-rate multiplications, and a block needs five
 // quotients before it can load anything.  Below 2^21 the rounded product is exact: (n + 0.5) / d is at least 0.5 / d away from an
 // integer, the product is off by less than 2^-22 n / d.
+constexpr int SMALL_DIV = 1 << 21;
+__device__ __forceinline__ int div_below_2_21(int n, int d) { return (int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d)); }
 __device__ __forceinline__ int small_div(int n, int d) {
-  if (__builtin_expect(n >= (1 << 21), 0)) return n / d;
-  return (int)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+  if (__builtin_expect(n >= SMALL_DIV, 0)) return n / d;
+  return div_below_2_21(n, d);
 }
 __device__ __forceinline__ float bf16_bits_to_float(u32 h) { return __uint_as_float(h << 16); }
 __device__ __forceinline__ u32 pack_bf16x2(float lo, float hi) {
@@ -814,102 +816,177 @@ __device__ __forceinline__ int uniform_tile(int v) { return __builtin_amdgcn_rea
 // ---------------------------------------------------------------------------------------------------- rows shared out by length
 // Rows of a batch differ in length, and the host does not know by how much.  With the same number of splits for every row the launch lasts
 // as long as a split of the longest row, while the blocks of short rows are mostly start and merge.  Here every block of the launch reads
-// the B lengths and derives, in the same arithmetic and so with the same result, how many splits each row gets and the rows' order, longest
-// first (blocks start in index order, so the short rows fill the end of the launch), and with them its own row, kv head and split:
+// the B lengths and derives, in the same arithmetic and so with the same result, how many splits each row gets, and with them its own row, kv
+// head and split:
+//   * nearly equal rows: nsplit splits per row in batch order, as without a plan, or as many as fill one round.
 //   * one round: the launch uses no more blocks than are resident at once (two four-wave blocks or one eight-wave block per CU), rows get
 //     splits of about c tiles, c the smallest size for which sum ceil(tiles / c) fits (found to 1/120 of c).  Blocks beyond have nothing to do.
 //   * several rounds, where half a split per row, which rounding costs, is more than starting and merging blocks again: nsplit splits per
-//     row.  Their sizes then differ from row to row, which keeps the rounds from starting and ending in step: 2048 blocks of equal size
-//     took 303 us where 16 splits per row take 292 (16 sequences of 4096..65536 tokens).
+//     row, longest row first (blocks start in index order, so that the short rows fill the end of the launch).  The splits' sizes differ from
+//     row to row, which keeps the rounds from starting and ending in step.
 // The line: a four-wave block takes about 0.5 us per tile and a round costs some 20 us of starts and merges.  16 sequences of 1000..16000
-// tokens (rounding costs 17 tiles): 91 us in one round, 102 in four; 4096..65536 tokens (68 tiles): 325 against 292.
-// Measured with warm caches against equal split counts: paged, 8 sequences of 200..3000 tokens x 8 kv heads: 27.5 -> 21.7 us, 16 of
-// 500..6000: 71.5 -> 48, 4 of 2000..40000: 82 -> 58; slot cache, 32 rows of 300..6000: 72 -> 62, 8 of 2000..16000: 50 -> 42.
+// tokens (rounding costs 17 tiles): 91 us in one round, 102 in four; 4096..65536 tokens (68 tiles): 325 in one round, 277 in four.
+// Measured with warm caches, 4 query heads per kv head, against equal split counts in batch order: paged, 8 sequences of 200..3000 tokens x 8
+// kv heads: 27.0 -> 20.6 us, 16 of 500..6000: 71 -> 44; slot cache, 4 rows of 2000..32000: 47.4 -> 37.4, 12 of 300..8000: 53.5 -> 32.2,
+// 32 of 300..6000: 68 -> 61.
+// What the look at the rows costs where they turn out equal (4 rows of 32000..32768): 63.7 -> 63.9.  It is in every block's start, so it
+// is kept to two trips to memory, which a block without a plan makes too, and some 300 instructions: an earlier form, which went
+// through LDS, read the lengths of all B * n_kv heads in a loop and compared each row with each, took 384 us instead of 142 for 256 rows of
+// 500 tokens x 16 kv heads and 64.5 for the 4 rows above.
 constexpr int PLAN_ROWS = 256;           // larger batches take nsplit splits per row in batch order
 constexpr float ONE_ROUND_LOSS = 48.f;   // tiles of a four-wave block
 // Smaller splits cost more in the merge than they gain: 30 sequences of up to 3000 tokens, one kv head with 16 query heads: 31.4 us
 // with at least 4 tiles, 27.4 with 12, 30.1 with 20; eight sequences of up to 3000 tokens, 8 kv heads: 21.6, 21.8, 24.5.
 constexpr float MIN_SPLIT_TILES = 12.f;  // of a four-wave block; half as many for an eight-wave block
 struct RowPlan { int b, S, kvh, idx, ns, off, slot; };      // idx: the block's place among the ns blocks of (row, kv head); off: splits of the rows before
-constexpr int PLAN_HEADS = 4096;         // (row, kv head) pairs whose lengths a block keeps (slot cache)
-struct PlanLds { int tiles[PLAN_ROWS], slot[PLAN_ROWS], off[PLAN_ROWS], len[PLAN_HEADS]; };      // len: per row (paged) | per row and kv head
-static_assert(sizeof(PlanLds) <= 5 * GMAX * D * sizeof(float), "the plan's view must fit the merge buffer");
-__device__ __forceinline__ int plan_splits(int tiles, float c, float rc) {      // about ceil(tiles / c), the same wherever it is asked
-  return min(max((int)(((float)tiles + (c - 1.f)) * rc), 1), MAX_SLOTS);
+__device__ __forceinline__ int plan_splits(int tiles, float c, float rc) {      // about ceil(tiles / c), the same wherever it is asked; no row (tiles < 0): none
+  return tiles < 0 ? 0 : min(max((int)(((float)tiles + (c - 1.f)) * rc), 1), MAX_SLOTS);
 }
-template <bool PAGED, int NW>
-__device__ __forceinline__ bool plan_block(const AttnArgs& A, PlanLds& P, int tid, RowPlan& R) {
-  constexpr int NT = 64 * NW;
-  const int B = A.B, wave = tid >> 6, lane = tid & 63, sub = lane & 15;
-  // the splits go by the length of kv head 0; the block's own head is looked up from what is read here, which saves a trip to memory
-  const int per_row = PAGED ? 1 : A.n_kv;
-  for (int i = tid; i < B * per_row; i += NT) {
-    const int row = PAGED ? i : small_div(i, per_row), head = PAGED ? 0 : i - row * per_row;
-    const int s = PAGED ? 0 : (A.slot ? A.slot[row] : row);
-    int len = PAGED ? A.sl[row] : A.sl[max(s, 0) * per_row + head];
-    len = s < 0 ? 0 : max(len, 0);
-    P.len[i] = len;
-    if (head == 0) { P.tiles[row] = (len + T - 1) / T; P.slot[row] = s; P.off[row] = 0; }
+// Every wave works the plan out by itself, without LDS or a barrier: lane l holds the rows l, l + 64, ..., one register each; counts are
+// ballots, sums DPP, a row's place among the others is found by bisection.  false: no unit left for this block.
+// K: registers of rows, B <= 64 K (a register without rows only holds lanes that are not there).
+template <bool PAGED, int NW, int K>
+__device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& R) {
+  const int B = A.B, nsplit = A.nsplit, block = (int)blockIdx.x;
+  const auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  const auto row = [&](int k) { return min(lane + 64 * k, B - 1); };
+  // The block's place if the rows turn out equal follows from its index: slot and length of that place are loaded along with the
+  // rows', so that the chain up to the block's own length has the loads of a launch without a plan.
+  const int bh = uniform(div_below_2_21(block, nsplit)), b_eq = uniform(div_below_2_21(bh, A.n_kv)), kvh_eq = bh - b_eq * A.n_kv;
+  const int* slots = A.slot ? A.slot : A.sl;      // (no load under a branch: without a slot map, B lengths or more are there to be read)
+  int slot[K], tiles[K], slot_eq = 0;
+  if (!PAGED) {
+    slot_eq = slots[b_eq];
+#pragma unroll
+    for (int k = 0; k < K; ++k) slot[k] = slots[row(k)];
+    if (!A.slot) {
+      slot_eq = b_eq;
+#pragma unroll
+      for (int k = 0; k < K; ++k) slot[k] = row(k);
+    }
   }
-  lds_barrier();
+  const auto length = [&](int b, int s, int head) { return A.sl[PAGED ? b : max(s, 0) * A.n_kv + head]; };
+  const int len_eq = length(b_eq, slot_eq, kvh_eq);
+#pragma unroll
+  for (int k = 0; k < K; ++k) tiles[k] = length(row(k), slot[k], 0);      // the splits go by the length of kv head 0
   float total = 0.f, longest = 0.f, shortest = -INFINITY;      // (shortest: negated)
-  for (int i = lane; i < B; i += 64) { const float t = (float)P.tiles[i]; total += t; longest = fmaxf(longest, t); shortest = fmaxf(shortest, -t); }
-  longest = wave_max(longest); shortest = -wave_max(shortest);
-  // nearly equal rows (within 1/16 of the longest) and every block resident: nsplit splits per row in batch order, and no more to work out
-  const bool equal = A.nsplit * B <= A.plan && __builtin_amdgcn_ballot_w64(longest - shortest > longest * (1.f / 16.f)) == 0;
-  total = wave_sum(total);
-  const int units = min(A.nsplit * B, A.plan);
-  // half a split per row goes to rounding: total / units * B / (2 units) tiles on every block
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const bool there = lane + 64 * k < B;
+    const int t = !PAGED && slot[k] < 0 ? 0 : (max(tiles[k], 0) + T - 1) / T;
+    tiles[k] = there ? t : -1;
+    total += there ? (float)t : 0.f; longest = fmaxf(longest, (float)t); shortest = fmaxf(shortest, -(float)t);      // (past the end: the last row again)
+  }
+  const int most = uniform((int)wave_max(longest)), least = uniform((int)-wave_max(shortest));
+  const bool equal = 16 * (most - least) <= most, resident = nsplit * B <= A.plan;      // equal: within 1/16 of the longest
+  const int units = min(nsplit * B, A.plan), u = uniform(div_below_2_21(block, A.n_kv));     // a unit is a split for every kv head: n_kv blocks
   const float fu = (float)units;
-  bool one_round = !equal && A.nsplit > 1 && units >= B && (A.nsplit * B <= A.plan || total * (float)B <= ONE_ROUND_LOSS * 2.f * fu * fu);
-  float c_best = 0.f;
-  if (one_round) {
-    // sixteen sizes from the mean to three times that, then sixteen between the first that fits and the one before it; lane (j, r) =
-    // (lane & 15, lane >> 4) tries size j over the rows r, r + 4, ...
-    const float c_min = fmaxf(floorf(total * __builtin_amdgcn_rcpf(fu)) + 1.f, NW == 4 ? MIN_SPLIT_TILES : 0.5f * MIN_SPLIT_TILES), step = c_min * (2.f / 15.f);
-    float lo = c_min, width = step;
-#pragma unroll 1
-    for (int pass = 0; pass < 2 && one_round; ++pass) {
-      const float c = lo + width * (float)sub, rc = __builtin_amdgcn_rcpf(c);
-      float n = 0.f;
-#pragma unroll 1
-      for (int i = lane >> 4; i < B; i += 4) n += (float)plan_splits(P.tiles[i], c, rc);
-      n = quad_rows_sum(n);
-      const u64 fits = __builtin_amdgcn_ballot_w64(n <= (float)units) & 0xFFFFull;
-      if (fits) c_best = __uint_as_float((u32)__builtin_amdgcn_readlane((int)__float_as_uint(c), __builtin_ctzll(fits)));
-      else one_round = pass != 0;
-      lo = fmaxf(c_best - step, c_min); width = step * (1.f / 16.f);
+  int ns = nsplit, b = 0, off = 0;
+  if (!equal || !resident) total = wave_sum(total);
+  if (equal) {
+    // batch order, with nsplit splits per row, or as many as make one round where that loses less than several rounds
+    if (!resident && nsplit > 1 && units >= B) {
+      const int n1 = uniform(div_below_2_21(units, B));
+      const float loss = (float)most * __builtin_amdgcn_rcpf((float)n1) - total * __builtin_amdgcn_rcpf(fu);
+      if (__builtin_amdgcn_ballot_w64(loss > ONE_ROUND_LOSS) == 0) ns = n1;
     }
-  }
-  const float rc_best = __builtin_amdgcn_rcpf(c_best);
-  const auto splits = [&](int tiles) { return one_round ? plan_splits(tiles, c_best, rc_best) : A.nsplit; };
-  // splits ahead of row i: each wave counts a share of the rows for all i
-  if (!equal) {
-    for (int i0 = 0; i0 < B; i0 += 64) {
-      const int i = i0 + lane, mine = P.tiles[min(i, B - 1)];
-      int ahead = 0;
-#pragma unroll 1
-      for (int k = wave; k < B; k += NW) {
-        const int tk = P.tiles[k];
-        ahead += tk > mine || (tk == mine && k < i) ? splits(tk) : 0;
-      }
-      if (i < B) atomicAdd(&P.off[i], ahead);
-    }
-    lds_barrier();
-  }
-  for (int i0 = 0; i0 < B; i0 += 64) {
-    const int i = min(i0 + lane, B - 1), ns = splits(P.tiles[i]), off = equal ? i * A.nsplit : P.off[i], w = (int)blockIdx.x - off * A.n_kv;
-    const u64 own = __builtin_amdgcn_ballot_w64(i == i0 + lane && w >= 0 && w < ns * A.n_kv);
-    if (own != 0) {
-      const int l = __builtin_ctzll(own), wl = __builtin_amdgcn_readlane(w, l);
-      R.b = i0 + l; R.ns = __builtin_amdgcn_readlane(ns, l); R.off = __builtin_amdgcn_readlane(off, l);
-      R.kvh = __builtin_amdgcn_readfirstlane(small_div(wl, R.ns)); R.idx = wl - R.kvh * R.ns;
-      R.slot = __builtin_amdgcn_readfirstlane(P.slot[R.b]);
-      R.S = __builtin_amdgcn_readfirstlane(P.len[PAGED ? R.b : R.b * A.n_kv + R.kvh]);
+    if (ns == nsplit) {
+      R.b = b_eq; R.kvh = kvh_eq; R.idx = block - bh * nsplit; R.ns = nsplit; R.off = b_eq * nsplit; R.slot = slot_eq; R.S = max(len_eq, 0);
       return true;
     }
+    b = uniform(div_below_2_21(u, ns)); off = b * ns;
+    if (b >= B) return false;
+  } else {
+    // half a split per row goes to rounding: total / units * B / (2 units) tiles on every block
+    bool one_round = nsplit > 1 && units >= B && (resident || __builtin_amdgcn_ballot_w64(total * (float)B > ONE_ROUND_LOSS * 2.f * fu * fu) == 0);
+    if (one_round) {
+      // sixteen sizes from the mean to three times that, then sixteen between the first that fits and the one before it; lane (j, r) =
+      // (lane & 15, lane >> 4) tries size j over the rows r, r + 4, ...
+      const float c_min = fmaxf(floorf(total * __builtin_amdgcn_rcpf(fu)) + 1.f, NW == 4 ? MIN_SPLIT_TILES : 0.5f * MIN_SPLIT_TILES), step = c_min * (2.f / 15.f);
+      float lo = c_min, width = step, c_best = 0.f;
+#pragma unroll 1
+      for (int pass = 0; pass < 2 && one_round; ++pass) {
+        const float c = lo + width * (float)(lane & 15), rc = __builtin_amdgcn_rcpf(c);
+        float n = 0.f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+#pragma unroll 1
+          for (int i = 0; i < (K > 1 ? 64 : B); i += 16)      // (lanes without a row take no splits)
+#pragma unroll
+            for (int j = 0; j < 16; j += 4) n += (float)plan_splits(__builtin_amdgcn_ds_bpermute(4 * (i + j + (lane >> 4)), tiles[k]), c, rc);
+        }
+        n = quad_rows_sum(n);
+        const u64 fits = __builtin_amdgcn_ballot_w64(n <= fu) & 0xFFFFull;
+        if (fits) c_best = __uint_as_float((u32)__builtin_amdgcn_readlane((int)__float_as_uint(c), __builtin_ctzll(fits)));
+        else one_round = pass != 0;
+        lo = fmaxf(c_best - step, c_min); width = step * (1.f / 16.f);
+      }
+      if (one_round) {      // (all blocks start together: the rows' order does not matter)
+        const float rc = __builtin_amdgcn_rcpf(c_best);
+        int first = 0;
+        b = -1;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const int n = plan_splits(tiles[k], c_best, rc), x = (int)row_scan16((u32)n);
+          const int r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31), r2 = __builtin_amdgcn_readlane(x, 47);
+          const int end = first + x + (lane >= 16 ? r0 : 0) + (lane >= 32 ? r1 : 0) + (lane >= 48 ? r2 : 0);
+          const u64 own = __builtin_amdgcn_ballot_w64(u >= end - n && u < end);
+          if (own != 0) {
+            const int l = __builtin_ctzll(own);
+            b = 64 * k + l; ns = __builtin_amdgcn_readlane(n, l); off = __builtin_amdgcn_readlane(end, l) - ns;
+            break;
+          }
+          first = __builtin_amdgcn_readlane(end, 63);
+        }
+        if (b < 0) return false;
+      }
+    }
+    if (!one_round) {      // nsplit splits per row, longest first
+      const int place = uniform(div_below_2_21(u, nsplit));
+      int below = least - 1, own = most, ahead = 0;
+#pragma unroll 1
+      while (own - below > 1) {
+        const int mid = (own + below) >> 1;
+        int n = 0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) { n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(tiles[k] > mid)); }
+        if (n <= place) { own = mid; ahead = n; } else below = mid;
+        if (n == place) break;
+      }
+      if (ahead == place) {      // the next row of up to `own` tiles
+        float t = -1.f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) { t = fmaxf(t, tiles[k] <= own ? (float)tiles[k] : -1.f); }
+        own = uniform((int)wave_max(t));
+      }
+      off = place * nsplit;
+      int rank = place - ahead;      // the block's row is the rank-th, in batch order, of those of this length
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+            const u64 m = __builtin_amdgcn_ballot_w64(tiles[k] == own);
+        const int n = __builtin_popcountll(m);
+        if (rank < n) {
+          const int before = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
+          b = 64 * k + __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles[k] == own && before == rank));
+          break;
+        }
+        rank -= n;
+      }
+    }
   }
-  return false;
+  const int w = block - off * A.n_kv;
+  R.b = b; R.ns = ns; R.off = off; R.kvh = uniform(div_below_2_21(w, ns)); R.idx = w - R.kvh * ns;
+  R.slot = 0;
+  if (!PAGED) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) if (b >> 6 == k) R.slot = __builtin_amdgcn_readlane(slot[k], b & 63);
+  }
+  R.S = max(length(b, R.slot, R.kvh), 0);      // (the line is at hand from the look at the rows)
+  return true;
+}
+template <bool PAGED, int NW>
+__device__ __forceinline__ bool plan_block(const AttnArgs& A, int lane, RowPlan& R) {
+  return __builtin_expect(A.B <= 64, 1) ? plan_rows<PAGED, NW, 1>(A, lane, R) : plan_rows<PAGED, NW, PLAN_ROWS / 64>(A, lane, R);
 }
 
 // ---------------------------------------------------------------------------------------------------- main kernel
@@ -946,9 +1023,8 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   }
   const int G = A.G;
   RowPlan R;
-  if (!HOST_LEN && A.plan) {
-    // (the merge buffer is idle until the tile loop has ended)
-    if (!plan_block<PAGED, NW>(A, *reinterpret_cast<PlanLds*>(&M.acc[0][0][0]), tid, R)) {
+  if (!HOST_LEN && __builtin_expect(A.plan != 0, 0)) {
+    if (!plan_block<PAGED, NW>(A, tid & 63, R)) {
       if (A.nslot > 1) {      // no unit left for this block: it only takes its part in the launch's epoch
         const u32 epoch = load_epoch(A);
         if (tid == 0) mark_arrival(A, epoch);
@@ -1412,12 +1488,21 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_bf16_attn_split(co
 
 using namespace gaac;
 
-// How many splits of n_kv blocks plan_block may count as resident, 0: no plan.  The plan costs a block 0.8 to 1.4 us at its start (its
-// instructions come from memory on a first launch).  It cannot gain that where all blocks are resident and a split of the longest possible
-// row is no more than five tiles for each of the block's eight waves, about 7 us.
+// How many splits of n_kv blocks plan_block may count as resident, 0: no plan.  The plan costs a block about a microsecond at its start
+// (its instructions come from memory on a first launch).  It cannot gain that
+//   * where all blocks are resident and each row is one split, or a split of the longest possible row is no more than five tiles for
+//     each of the block's eight waves, about 7 us;
+//   * where one round is out of reach whatever the lengths, so that it only orders the rows, and there are many blocks of short rows: what
+//     order can save is a split of the longest row at the end of the launch, the cost comes with every round.  One split per row, us
+//     without and with the plan: 256 rows of up to 1000 tokens x 16 kv heads (4096 blocks, 67 tiles): 150 and 168, 256 of up to 2000 x
+//     8 (2048, 129): 144 and 144, 128 of up to 4000 x 8 (1024, 254): 159 and 137.
 static int plan_units(int B, int n_kv, int nsplit, long max_tiles) {
   const long blocks = (long)B * n_kv * nsplit;
-  return B > 1 && B <= PLAN_ROWS && B * n_kv <= PLAN_HEADS && (blocks > 256 || max_tiles > 40l * nsplit) ? std::max((blocks > 256 ? 512 : 256) / n_kv, 1) : 0;
+  const int units = std::max((blocks > 256 ? 512 : 256) / n_kv, 1);
+  if (B <= 1 || B > PLAN_ROWS || blocks >= SMALL_DIV) return 0;
+  if (blocks <= 256) return nsplit > 1 && max_tiles > 40l * nsplit ? units : 0;
+  if (nsplit > 1 && units >= B) return units;
+  return 8 * max_tiles >= blocks * nsplit ? units : 0;
 }
 
 #ifdef GAAC_PHASE_TIMING

@@ -183,3 +183,27 @@ def test_engine_context_and_attention_layer_without_a_cache():
     from gaac_amd.kv_cache import CompressedKVCache
     per_slot = 4 * CompressedKVCache.bytes_per_slot(8, 4096)
     assert min(16, (3 * per_slot + 5) // per_slot) == 3
+
+
+@pytest.mark.parametrize("L,splits", [(20000, 92), (4000, 20), (1000, 63), (300, 2)])
+def test_the_row_bound_sees_a_single_split(L, splits):
+    """What the launches over ragged rows are compared with: rounding weights and output to bf16 stays far inside the bound, one split left
+    out, taken twice or read from its neighbour's tokens breaks it, next to a short row with much larger outputs."""
+    from common import assert_rows_close
+    g = torch.Generator().manual_seed(L)
+    k, v, q = (torch.randn(n, 128, generator=g, dtype=torch.float64) for n in (L, L, 4))
+    p = torch.softmax(q * 0.5 @ k.T * 128 ** -0.5, -1)
+    short = torch.randn(4, 128, generator=g, dtype=torch.float64)
+    rows = lambda out: torch.stack([short, out])
+    want = rows(p @ v)
+    assert_rows_close(rows((p.bfloat16().double() @ v / p.bfloat16().double().sum(-1, keepdim=True)).bfloat16().double()), want)
+    n = -(-L // splits)
+    for i in (0, splits // 2, (L - 1) // n):
+        w = torch.ones(L, dtype=torch.float64)
+        w[i * n:(i + 1) * n] = 0.0
+        at = slice(i * n, min((i + 1) * n, L))
+        other = (torch.arange(at.start, at.stop) + n) % L
+        for wrong in (p * w, p * (2 - w)):
+            with pytest.raises(AssertionError): assert_rows_close(rows(wrong @ v / wrong.sum(-1, keepdim=True)), want)
+        moved = v.clone(); moved[at] = v[other]
+        with pytest.raises(AssertionError): assert_rows_close(rows(p @ moved), want)
