@@ -129,12 +129,13 @@ def rows_in_place(x: torch.Tensor, head_dim: int, row_dim: int) -> tuple[torch.T
     """(x, head stride, row stride) for the encoder, which reads [., ., 128] elements through any strides as long as a row is 16-byte
     aligned and contiguous; other layouts are copied first.  Raises for rows that are not 128 elements of 16 bits: the strides would
     then reach past the tensor's memory."""
-    if x.dim() != 3 or x.shape[2] != D or x.element_size() != 2:
-        raise RuntimeError(f"the encoder expects bf16 rows of {D} elements in three dimensions, got {x.dtype} {list(x.shape)}")
-    hs, rs = x.stride(head_dim) if x.shape[head_dim] > 1 else 0, x.stride(row_dim) if x.shape[row_dim] > 1 else D
-    if x.stride(2) == 1 and rs >= D and rs % 8 == 0 and hs % 8 == 0 and x.data_ptr() % 16 == 0: return x, hs, rs
+    shape, strides = x.shape, x.stride()
+    if len(shape) != 3 or shape[2] != D or x.itemsize != 2:
+        raise RuntimeError(f"the encoder expects bf16 rows of {D} elements in three dimensions, got {x.dtype} {list(shape)}")
+    hs, rs = strides[head_dim] if shape[head_dim] > 1 else 0, strides[row_dim] if shape[row_dim] > 1 else D
+    if strides[2] == 1 and rs >= D and rs % 8 == 0 and hs % 8 == 0 and x.data_ptr() % 16 == 0: return x, hs, rs
     x = x.clone(memory_format=torch.contiguous_format)
-    strides = (x.shape[1] * D, D)
+    strides = (shape[1] * D, D)
     return x, strides[head_dim], strides[row_dim]
 
 
