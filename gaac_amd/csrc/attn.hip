@@ -884,11 +884,12 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
   int ns = nsplit, b = 0, off = 0;
   if (!equal || !resident) total = wave_sum(total);
   if (equal) {
-    // batch order, with nsplit splits per row, or as many as make one round where that loses less than several rounds
+    // batch order, with nsplit splits per row, or as many as make one round where that loses less than several rounds, or where the last
+    // of several rounds would be much emptier (24 rows of 12000 tokens x 8 kv heads, 3 splits: 576 blocks 171 us, 2 splits 152)
     if (!resident && nsplit > 1 && units >= B) {
-      const int n1 = uniform(div_below_2_21(units, B));
+      const int n1 = uniform(div_below_2_21(units, B)), rounds = uniform(div_below_2_21(nsplit * B + units - 1, units));
       const float loss = (float)most * __builtin_amdgcn_rcpf((float)n1) - total * __builtin_amdgcn_rcpf(fu);
-      if (__builtin_amdgcn_ballot_w64(loss > ONE_ROUND_LOSS) == 0) ns = n1;
+      if (10 * nsplit < 9 * rounds * n1 || __builtin_amdgcn_ballot_w64(loss > ONE_ROUND_LOSS) == 0) ns = n1;
     }
     if (ns == nsplit) {
       R.b = b_eq; R.kvh = kvh_eq; R.idx = block - bh * nsplit; R.ns = nsplit; R.off = b_eq * nsplit; R.slot = slot_eq; R.S = max(len_eq, 0);
@@ -921,22 +922,32 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
         else one_round = pass != 0;
         lo = fmaxf(c_best - step, c_min); width = step * (1.f / 16.f);
       }
-      if (one_round) {      // (all blocks start together: the rows' order does not matter)
+      if (one_round) {
+        // All blocks start together, two to a CU, the later half beside the earlier one: rows of several splits, whose blocks are all
+        // long, come first, then the others, either in batch order (all in batch order: 28 rows of 300..6000 tokens x 8 kv heads 54.6 us
+        // instead of 52.3, but 100 of 100..4000 x 4 70.5 instead of 77; longest first 52.5 and 77.7, and it takes a search).  The counts of
+        // the two kinds run in the halves of one word.
         const float rc = __builtin_amdgcn_rcpf(c_best);
-        int first = 0;
+        u32 n[K], end[K], sum = 0u;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          n[k] = (u32)plan_splits(tiles[k], c_best, rc);
+          n[k] = n[k] > 1u ? n[k] : n[k] << 16;
+          const u32 x = row_scan16(n[k]), r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31), r2 = __builtin_amdgcn_readlane(x, 47);
+          end[k] = sum + x + (lane >= 16 ? r0 : 0u) + (lane >= 32 ? r1 : 0u) + (lane >= 48 ? r2 : 0u);
+          sum = (u32)__builtin_amdgcn_readlane((int)end[k], 63);
+        }
         b = -1;
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-          const int n = plan_splits(tiles[k], c_best, rc), x = (int)row_scan16((u32)n);
-          const int r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31), r2 = __builtin_amdgcn_readlane(x, 47);
-          const int end = first + x + (lane >= 16 ? r0 : 0) + (lane >= 32 ? r1 : 0) + (lane >= 48 ? r2 : 0);
-          const u64 own = __builtin_amdgcn_ballot_w64(u >= end - n && u < end);
+          const bool several = n[k] < 65536u;
+          const int mine = several ? (int)n[k] : (int)(n[k] >> 16), to = several ? (int)(end[k] & 65535u) : (int)((end[k] >> 16) + (sum & 65535u));
+          const u64 own = __builtin_amdgcn_ballot_w64(u >= to - mine && u < to);
           if (own != 0) {
             const int l = __builtin_ctzll(own);
-            b = 64 * k + l; ns = __builtin_amdgcn_readlane(n, l); off = __builtin_amdgcn_readlane(end, l) - ns;
+            b = 64 * k + l; ns = __builtin_amdgcn_readlane(mine, l); off = __builtin_amdgcn_readlane(to, l) - ns;
             break;
           }
-          first = __builtin_amdgcn_readlane(end, 63);
         }
         if (b < 0) return false;
       }

@@ -66,13 +66,19 @@ def launch_nsplit(B: int, n_kv: int, S: int, ragged: bool) -> int:
       * up to 256 tokens in one split (100 tokens: 6.8, against 7.3 to 8.8 with 2 to 6 splits; 300 tokens: 9.0, against 8.2 with 8);
       * at least 32 tokens per split (1000 tokens x 8 heads: 11.3 with 3 splits, 9.0 with 6, 8.7 with 32; 3000: 11.3 with 12, 9.5 with
         32), but no more than 64 splits of less than 256 (the merge: 8000 tokens, 1 head of 16 queries: 14.7 with 64, 24.4 with 256);
-      * one eight-wave block per CU (256 blocks: a second round of blocks costs more than it evens out), and where rows are ragged and
-        the heads alone take more than a quarter of the CUs, two four-wave blocks per CU, to have enough of them to share out
-        (32 rows of 300..6000 tokens x 8 heads: 72 us with 1 split, 62 with 2; 12 rows of up to 8000: 38 with 2, 33 with 5); two splits up
-        to 512 heads (48 rows of up to 8000 x 8 heads: 135 with 1, 107 with 2)."""
+      * one eight-wave block per CU (256 blocks: a second round of blocks costs more than it evens out);
+      * ragged rows whose heads alone take more than a quarter of the CUs: two four-wave blocks per CU, to have enough of them to share
+        out, once the rows are long enough to pay for more starts and merges.  x 8 heads, one block per CU / two: 12 rows of 300..8000
+        tokens 37.2 / 31.5, 24 of 300..6000 67 / 45, 24 of 300..3000 37.3 / 28.3, 32 of 300..6000 68 / 59.5, 32 of 100..2000 27.9 / 26.4;
+        but 12 of 100..1000 13.7 / 15.8, 16 of 1000 14.7 / 16.8, 32 of 100..500 12.0 / 16.6.  From 170 heads to 256 this is a bet on
+        rows that differ: where long rows turn out equal, one block per (row, head) was faster (24 of 3000: 40.3 / 45.3, 32 of 3000:
+        46.2 / 49.9, 24 of 12000: 138 / 151, 28 of 4000..5000: 63 / 70);
+      * ragged, more heads than CUs: two splits, one / two: 48 rows of 300..8000 x 8 heads 132 / 109, 48 of 100..2000 39.6 / 37.5, 64 of
+        200..4000 82.5 / 79.0; but 64 of 100..2000 42.2 / 49.3, 200 of 300 x 2 heads 15.6 / 17.8.  Equal: 48 of 2000 54.6 / 55.2."""
     H = B * n_kv
     if S <= 256: return 1
-    if ragged and B > 1 and H > 64: n = -(-512 // H) if H <= 256 else 2 if H <= 512 else 1
+    if ragged and B > 1 and 64 < H <= 256 and S >= max(1500, 7 * H): n = -(-512 // H)
+    elif ragged and B > 1 and (256 < H <= 384 and S >= 1000 or 384 < H <= 512 and S >= 4000): n = 2
     else: n = 256 // H
     return max(1, min(n, max(S // 256, min(64, S // 32))))
 

@@ -29,6 +29,7 @@ CASES = [
     ([20000, 1, 16, 0, 17, 4000], 4, 5, 40, SHARED),                    # an empty row
     ([9000 + 500 * (i % 5) for i in range(16)], 16, 2, 4, NSPLIT),     # several rounds, longest first, equal lengths among them
     ([3000] * 20, 16, 2, 4, NSPLIT),                                    # equal rows, several rounds
+    ([6400] * 24, 8, 1, 3, 2),                                          # one round, instead of one and a nearly empty one
     ([1000] * 9, 8, 2, 8, 7),                                           # equal rows, one round
     ([1000] * 40, 8, 1, 4, 1),
     ([16 * (i % 7) + 40 for i in range(70)], 2, 2, 3, SHARED),         # more rows than a wave has lanes

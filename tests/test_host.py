@@ -148,6 +148,20 @@ def test_choose_nsplit_bounds():
     assert choose_nsplit(1, 1, 1 << 20) == 256         # cap
 
 
+def test_launch_nsplit_where_the_caller_leaves_the_choice():
+    from gaac_amd.kernel import launch_nsplit
+    for ragged in (False, True):
+        assert launch_nsplit(1, 8, 65536, ragged) == 32 and launch_nsplit(4, 8, 32768, ragged) == 8      # 256 blocks
+        assert launch_nsplit(1, 8, 1000, ragged) == 31 and launch_nsplit(1, 1, 8000, ragged) == 64      # 32 tokens per split, 64 splits
+        for B, n_kv in ((1, 1), (32, 8), (256, 16)): assert launch_nsplit(B, n_kv, 256, ragged) == 1
+        # short rows of many heads, and batches that fill the GPU without splits
+        for B, n_kv, S in ((200, 2, 300), (64, 8, 2000), (48, 8, 300), (32, 8, 500), (24, 8, 1000), (65, 8, 65536), (256, 16, 4000)):
+            assert launch_nsplit(B, n_kv, S, ragged) == 1, (B, n_kv, S)
+        assert launch_nsplit(12, 8, 1000, ragged) == 2
+    for B, n_kv, S, n in ((12, 8, 8000, 6), (24, 8, 6000, 3), (32, 8, 6000, 2), (48, 8, 2000, 2), (64, 8, 4000, 2)):
+        assert launch_nsplit(B, n_kv, S, True) == n and launch_nsplit(B, n_kv, S, False) == max(1, 256 // (B * n_kv))
+
+
 def test_bytes_per_slot_closed_form():
     from gaac_amd.kv_cache import CompressedKVCache
     # 8 kv heads, capacity rounded to 65552 tokens, 128 B of escape room per tile, per-sequence bases: term by term
