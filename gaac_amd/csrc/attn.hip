@@ -818,7 +818,7 @@ __device__ __forceinline__ int uniform_tile(int v) { return __builtin_amdgcn_rea
 // as long as a split of the longest row, while the blocks of short rows are mostly start and merge.  Here every block of the launch reads
 // the B lengths and derives, in the same arithmetic and so with the same result, how many splits each row gets, and with them its own row, kv
 // head and split:
-//   * nearly equal rows: nsplit splits per row in batch order, as without a plan, or as many as fill one round.
+//   * nearly equal rows (within 1/32 of the first one): nsplit splits per row in batch order, as without a plan, or as many as fill one round.
 //   * one round: the launch uses no more blocks than are resident at once (two four-wave blocks or one eight-wave block per CU), rows get
 //     splits of about c tiles, c the smallest size for which sum ceil(tiles / c) fits (found to 1/120 of c).  Blocks beyond have nothing to do.
 //   * several rounds, where half a split per row, which rounding costs, is more than starting and merging blocks again: nsplit splits per
@@ -829,7 +829,7 @@ __device__ __forceinline__ int uniform_tile(int v) { return __builtin_amdgcn_rea
 // Measured with warm caches, 4 query heads per kv head, against equal split counts in batch order: paged, 8 sequences of 200..3000 tokens x 8
 // kv heads: 27.0 -> 20.6 us, 16 of 500..6000: 71 -> 44; slot cache, 4 rows of 2000..32000: 47.4 -> 37.4, 12 of 300..8000: 53.5 -> 32.2,
 // 32 of 300..6000: 68 -> 61.
-// What the look at the rows costs where they turn out equal (4 rows of 32000..32768): 63.7 -> 63.9.  It is in every block's start, so it
+// What the look at the rows costs where they turn out equal (4 rows of 32000..32768): 63.8 -> 64.0.  It is in every block's start, so it
 // is kept to two trips to memory, which a block without a plan makes too, and some 300 instructions: an earlier form, which went
 // through LDS, read the lengths of all B * n_kv heads in a loop and compared each row with each, took 384 us instead of 142 for 256 rows of
 // 500 tokens x 16 kv heads and 64.5 for the 4 rows above.
@@ -843,7 +843,7 @@ __device__ __forceinline__ int plan_splits(int tiles, float c, float rc) {      
   return tiles < 0 ? 0 : min(max((int)(((float)tiles + (c - 1.f)) * rc), 1), MAX_SLOTS);
 }
 // Every wave works the plan out by itself, without LDS or a barrier: lane l holds the rows l, l + 64, ..., one register each; counts are
-// ballots, sums DPP, a row's place among the others is found by bisection.  false: no unit left for this block.
+// ballots, sums DPP, a row's place among many others is found by bisection.  false: no unit left for this block.
 // K: registers of rows, B <= 64 K (a register without rows only holds lanes that are not there).
 template <bool PAGED, int NW, int K>
 __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& R) {
@@ -869,32 +869,39 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
   const int len_eq = length(b_eq, slot_eq, kvh_eq);
 #pragma unroll
   for (int k = 0; k < K; ++k) tiles[k] = length(row(k), slot[k], 0);      // the splits go by the length of kv head 0
+#pragma unroll
+  for (int k = 0; k < K; ++k) tiles[k] = !PAGED && slot[k] < 0 ? 0 : (min(max(tiles[k], 0), 1 << 28) + T - 1) / T;      // (past the end: the last row again)
+  bool differs = false;
+  const int t0 = uniform(tiles[0]);
+#pragma unroll
+  for (int k = 0; k < K; ++k) differs |= 32 * abs(tiles[k] - t0) > t0;
+  const bool equal = __builtin_amdgcn_ballot_w64(differs) == 0, resident = nsplit * B <= A.plan;      // equal: within 1/32 of the first row
+  const auto stay = [&]() {      // at the place of equal rows
+    R.b = b_eq; R.kvh = kvh_eq; R.idx = block - bh * nsplit; R.ns = nsplit; R.off = b_eq * nsplit; R.slot = slot_eq; R.S = max(len_eq, 0);
+    return true;
+  };
+  if (equal && resident) return stay();
   float total = 0.f, longest = 0.f, shortest = -INFINITY;      // (shortest: negated)
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const bool there = lane + 64 * k < B;
-    const int t = !PAGED && slot[k] < 0 ? 0 : (max(tiles[k], 0) + T - 1) / T;
-    tiles[k] = there ? t : -1;
-    total += there ? (float)t : 0.f; longest = fmaxf(longest, (float)t); shortest = fmaxf(shortest, -(float)t);      // (past the end: the last row again)
+    const float t = (float)tiles[k];
+    total += there ? t : 0.f; longest = fmaxf(longest, t); shortest = fmaxf(shortest, -t);
+    tiles[k] = there ? tiles[k] : -1;
   }
-  const int most = uniform((int)wave_max(longest)), least = uniform((int)-wave_max(shortest));
-  const bool equal = 16 * (most - least) <= most, resident = nsplit * B <= A.plan;      // equal: within 1/16 of the longest
+  total = wave_sum(total);
   const int units = min(nsplit * B, A.plan), u = uniform(div_below_2_21(block, A.n_kv));     // a unit is a split for every kv head: n_kv blocks
   const float fu = (float)units;
   int ns = nsplit, b = 0, off = 0;
-  if (!equal || !resident) total = wave_sum(total);
   if (equal) {
     // batch order, with nsplit splits per row, or as many as make one round where that loses less than several rounds, or where the last
     // of several rounds would be much emptier (24 rows of 12000 tokens x 8 kv heads, 3 splits: 576 blocks 171 us, 2 splits 152)
     if (!resident && nsplit > 1 && units >= B) {
       const int n1 = uniform(div_below_2_21(units, B)), rounds = uniform(div_below_2_21(nsplit * B + units - 1, units));
-      const float loss = (float)most * __builtin_amdgcn_rcpf((float)n1) - total * __builtin_amdgcn_rcpf(fu);
+      const float loss = wave_max(longest) * __builtin_amdgcn_rcpf((float)n1) - total * __builtin_amdgcn_rcpf(fu);
       if (10 * nsplit < 9 * rounds * n1 || __builtin_amdgcn_ballot_w64(loss > ONE_ROUND_LOSS) == 0) ns = n1;
     }
-    if (ns == nsplit) {
-      R.b = b_eq; R.kvh = kvh_eq; R.idx = block - bh * nsplit; R.ns = nsplit; R.off = b_eq * nsplit; R.slot = slot_eq; R.S = max(len_eq, 0);
-      return true;
-    }
+    if (ns == nsplit) return stay();
     b = uniform(div_below_2_21(u, ns)); off = b * ns;
     if (b >= B) return false;
   } else {
@@ -954,34 +961,44 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
     }
     if (!one_round) {      // nsplit splits per row, longest first
       const int place = uniform(div_below_2_21(u, nsplit));
-      int below = least - 1, own = most, ahead = 0;
-#pragma unroll 1
-      while (own - below > 1) {
-        const int mid = (own + below) >> 1;
-        int n = 0;
-#pragma unroll
-        for (int k = 0; k < K; ++k) { n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(tiles[k] > mid)); }
-        if (n <= place) { own = mid; ahead = n; } else below = mid;
-        if (n == place) break;
-      }
-      if (ahead == place) {      // the next row of up to `own` tiles
-        float t = -1.f;
-#pragma unroll
-        for (int k = 0; k < K; ++k) { t = fmaxf(t, tiles[k] <= own ? (float)tiles[k] : -1.f); }
-        own = uniform((int)wave_max(t));
-      }
       off = place * nsplit;
-      int rank = place - ahead;      // the block's row is the rank-th, in batch order, of those of this length
+      if (K == 1) {      // each row counts the rows ahead of it (16 rows: 80 instructions, the bisection below 250)
+        const int key = tiles[0] * 64 + 63 - lane;      // (below zero: not there)
+        int ahead = 0;
+#pragma unroll 1
+        for (int i = 0; i < B; i += 8)
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-            const u64 m = __builtin_amdgcn_ballot_w64(tiles[k] == own);
-        const int n = __builtin_popcountll(m);
-        if (rank < n) {
-          const int before = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
-          b = 64 * k + __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles[k] == own && before == rank));
-          break;
+          for (int r = 0; r < 8; ++r) ahead += __builtin_amdgcn_readlane(key, i + r) > key ? 1 : 0;
+        b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(ahead == place && key >= 0));
+      } else {
+        int below = uniform((int)-wave_max(shortest)) - 1, own = uniform((int)wave_max(longest)), ahead = 0;
+#pragma unroll 1
+        while (own - below > 1) {
+          const int mid = (own + below) >> 1;
+          int n = 0;
+#pragma unroll
+          for (int k = 0; k < K; ++k) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(tiles[k] > mid));
+          if (n <= place) { own = mid; ahead = n; } else below = mid;
+          if (n == place) break;
         }
-        rank -= n;
+        if (ahead == place) {      // the next row of up to `own` tiles
+          float t = -1.f;
+#pragma unroll
+          for (int k = 0; k < K; ++k) t = fmaxf(t, tiles[k] <= own ? (float)tiles[k] : -1.f);
+          own = uniform((int)wave_max(t));
+        }
+        int rank = place - ahead;      // the block's row is the rank-th, in batch order, of those of this length
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const u64 m = __builtin_amdgcn_ballot_w64(tiles[k] == own);
+          const int n = __builtin_popcountll(m);
+          if (rank < n) {
+            const int before = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
+            b = 64 * k + __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles[k] == own && before == rank));
+            break;
+          }
+          rank -= n;
+        }
       }
     }
   }

@@ -22,7 +22,7 @@ NSPLIT, SHARED = "nsplit", "shared"
 CASES = [
     ([700, 33], 2, 4, 5, NSPLIT),                                        # few blocks, short splits: not planned
     ([12000, 700, 3000, 40], 8, 1, 8, SHARED),                          # eight-wave blocks
-    ([12000, 11900, 11500, 11950], 8, 1, 8, NSPLIT),                    # eight-wave blocks, rows within 1/16 of the longest
+    ([12000, 11900, 11800, 11950], 8, 1, 8, NSPLIT),                    # eight-wave blocks, rows within 1/32 of each other
     ([5000] + [40] * 7, 8, 1, 16, SHARED),                              # four-wave blocks, most of them left over
     ([300 + 170 * i for i in range(32)], 8, 4, 2, SHARED),             # all of them resident
     ([300 + 170 * i for i in range(32)], 8, 4, 9, SHARED),
