@@ -108,8 +108,10 @@ __device__ __forceinline__ u32 pack_bf16x2(float lo, float hi) {
 //     share from all blocks of the head and re-reads those whose epoch is not yet the launch's.  Everything a merger waits for is
 //     running, done, or one of the at most fifteen later mergers of the same head, which wait for nobody but each other's stores,
 //     and those precede every wait.  The wait is bounded all the same (MERGE_SPIN_LIMIT re-reads): a merger that gives up writes its
-//     rows as NaN and sets bit 0 of epochs[1]; the grid's last block sets bit 1 if it gives up waiting for the other blocks (it then
-//     leaves the epoch word alone).  The owner of the workspace polls epochs[1] and re-arms after a failure.
+//     rows as NaN and sets bit 0 of epochs[1].  The grid's last block may have little or nothing to do of its own (a short row; no unit left
+//     for it in a planned launch) and then waits for the whole launch: its bound (EPOCH_SPIN_LIMIT) is some seconds, far above any
+//     launch.  It sets bit 1 if it gives up (and leaves the epoch word alone).  The owner of the workspace polls epochs[1] and re-arms
+//     after a failure.
 //   * Launches that share the records and the epoch words must be ordered on one stream.  To re-arm after a failed launch, zero all.
 typedef __attribute__((ext_vector_type(4))) float f32x4v;
 __device__ __forceinline__ void store_partial(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -120,6 +122,7 @@ __device__ __forceinline__ u64 ll_load(const u64* p) { return __hip_atomic_load(
 __device__ __forceinline__ bool ll_stale(u64 r, u32 epoch) { return (u32)(r >> 32) != epoch; }
 __device__ __forceinline__ float ll_value(u64 r) { return __uint_as_float((u32)r); }
 constexpr int MERGE_SPIN_LIMIT = 1 << 16;      // re-reads of a chunk before the merger gives up (each with a short sleep: ~0.1 s)
+constexpr int EPOCH_SPIN_LIMIT = 1 << 23;      // polls of the arrival marks before the grid's last block gives up (about a microsecond each)
 // (no branch around the load: a load under a branch is waited for where the branch ends, together with everything issued before it)
 __device__ __forceinline__ u32 load_epoch(const AttnArgs& A) {
   const u32* p = A.epochs ? A.epochs : reinterpret_cast<const u32*>(A.q);
@@ -285,8 +288,8 @@ __device__ __forceinline__ void mark_arrival(const AttnArgs& A, u32 epoch) {
   __hip_atomic_store(A.epochs + EPOCH_WORDS + blockIdx.x, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // The grid's last block advances the epoch word for the next launch, once every block of this launch has marked its arrival (and so has
-// read the word).  The marks' first read (the first 2048 blocks) is issued ahead of the block's merge work and looked at after it: by
-// then the other blocks have long left their loops, so the check normally costs no trip to memory of its own.
+// read the word).  Where the block has merge work, the marks' first read (the first 2048 blocks) is issued ahead of it and looked at after it: by
+// then the other blocks of an evenly shared launch have long left their loops, so the check normally costs no trip to memory of its own.
 template <int NW> struct MarkRegs { u32 m[2048 / (64 * NW)]; };
 template <int NW>
 __device__ __forceinline__ void load_marks(const AttnArgs& A, int tid, MarkRegs<NW>& R) {
@@ -305,7 +308,7 @@ __device__ __forceinline__ void advance_epoch(const AttnArgs& A, u32 epoch, int 
 #pragma unroll
     for (int k = 0; k < XK; ++k) stale |= R.m[k] != epoch;
     if (__builtin_amdgcn_ballot_w64(stale) == 0) break;
-    if (spin >= MERGE_SPIN_LIMIT) { grid_ok = false; break; }
+    if (spin >= EPOCH_SPIN_LIMIT) { grid_ok = false; break; }
     __builtin_amdgcn_s_sleep(1);
 #pragma unroll
     for (int k = 0; k < XK; ++k)
@@ -314,7 +317,7 @@ __device__ __forceinline__ void advance_epoch(const AttnArgs& A, u32 epoch, int 
   for (int i0 = 2048; grid_ok && i0 < nblocks; i0 += 64 * NW) {      // grids beyond 2048 blocks: the remaining marks, a round at a time
     const int i = min(i0 + tid, nblocks - 1);
     for (int spin = 0; __builtin_amdgcn_ballot_w64(__hip_atomic_load(marks + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch) != 0; ++spin) {
-      if (spin >= MERGE_SPIN_LIMIT) { grid_ok = false; break; }
+      if (spin >= EPOCH_SPIN_LIMIT) { grid_ok = false; break; }
       __builtin_amdgcn_s_sleep(1);
     }
   }

@@ -129,3 +129,26 @@ def test_rows_of_many_heads_go_longest_first():
     first, alone = layer._ws[(len(lens), n_kv, 2)].pm[:2 * n_kv], layer._ws[(1, n_kv, 2)].pm
     assert torch.equal(first & 0xFFFFFFFF, alone & 0xFFFFFFFF)
     layer.check()
+
+
+def test_the_last_block_waits_for_a_long_launch():
+    """A row of sixteen million tokens next to one of a single token, four blocks in all: the grid's last block is done at once and waits
+    for the others for a good part of a second before it advances the epoch."""
+    dev = require_gpu()
+    from gaac_amd import CompressedKVCache
+    gen = torch.Generator(device=dev).manual_seed(9)
+    b = torch.full((1, 128), 120, dtype=torch.uint8)
+    cache = CompressedKVCache(2, 1, 1 << 24, dict(k3=b, k4=b, v3=b, v4=b), device=dev)
+    part = 1 << 16
+    k, v = (_rows(gen, part, 1, dev).repeat(255, 1, 1) for _ in range(2))
+    cache.prefill(0, k, v)
+    cache.prefill(1, k[:1], v[:1])
+    del k, v
+    q = (torch.randn(2, 1, 128, generator=gen, device=dev) * 0.5).to(torch.bfloat16)
+    slots = torch.arange(2, dtype=torch.int32, device=dev)
+    want = cache.attention(q, slots, SCALE, nsplit=64).float()
+    for rnd in range(2):
+        assert_rows_close(cache.attention(q, slots, SCALE, nsplit=2).float(), want)
+        ws = cache._partials[(2, 1, 2)]
+        assert ws.failure_bits() == 0 and int(ws.epoch[0]) == rnd + 1
+    cache.check_capacity()
