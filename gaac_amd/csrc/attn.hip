@@ -234,11 +234,13 @@ __device__ __forceinline__ void merge_half_head(const AttnArgs& A, long rec, int
   GAAC_MSTAMP(4, wall_clock64());
   wave_lds_sync();      // the wave's LDS region is free for its next item
 }
-// The same for a head of at most WAVE_MERGE_SLOTS splits, by ONE wave: lane = channel, all records of the half head in flight together.
-// With few splits there are few mergers, and a block that works on one half head at a time pays a trip to memory for each (2 splits and
-// 4 query heads: four in a row): here each wave of the merging blocks takes a half head of its own.  Launches over 1000 tokens x 8 kv
-// heads: 18.1 -> 13.2 us with two splits, 15.1 -> 11.3 with three, 12.8 -> 10.6 with four, 11.1 -> 9.0 with six.  With as many
-// splits as half heads the block-wise merge has one trip as well, and spreads its records over more waves.
+// The same for a head of at most WAVE_MERGE_SLOTS splits, and of fewer splits than half heads, by ONE wave: lane = channel, all records of
+// the half head in flight together.  With few splits there are few mergers, and a block that works on one half head at a time pays a trip
+// to memory for each (2 splits and 4 query heads: four in a row): here each wave of the merging blocks takes a half head of its own.
+// Launches over 1000 tokens x 8 kv heads, block-wise -> wave-wise: 18.1 -> 13.2 us with two splits, 15.1 -> 11.3 with three, 12.8 -> 10.6
+// with four, 11.1 -> 9.0 with six; 4000 tokens, 1 kv head with 16 query heads: 20.4 -> 15.9 with nine, 18.2 -> 14.8 with twelve, 15.8 -> 13.8
+// with sixteen, which is as many as a lane keeps records for; 2 kv heads with 8: 15.6 -> 13.5 with nine, 13.0 -> 11.6 with fifteen.
+// With as many splits as half heads each merging block has one half head, a single trip as well, and spreads its records over more waves.
 constexpr int WAVE_MERGE_SLOTS = 16;
 template <int SLOTS>      // how many it reads (those past the last split again: no load under a branch)
 __device__ __forceinline__ void merge_half_head_wave(const AttnArgs& A, long rec, int nslot, long row, int half, u32 epoch, int lane) {

@@ -16,8 +16,9 @@ char* last_error_buffer() { static thread_local char buf[512] = {0}; return buf;
 // every wave reads channels 2l and 2l+1 of a row (one 256-byte row per wave-wide load) and counts in a table of 256 x 64 words that the
 // block's waves share: word (bin, l) holds the counts of the two channels in its 16-bit halves (a chunk has at most 65535 tokens), so a
 // lane only ever touches bank l and the LDS adds of a wave never collide, however alike the exponents are.  A table of one word per
-// (channel, bin) with eight lanes to a row (16-byte loads) sent all rows of a wave to the same few words of a channel: 66 us for
-// the K and the V of 32768 tokens x 8 kv heads (134 MB, two launches), this one 36 us (3.7 TB/s; its loads alone take 27).
+// (channel, bin) with eight lanes to a row (16-byte loads) sent all rows of a wave to the same few words of a channel: 61 to 66 us
+// for the K and the V of 32768 tokens x 8 kv heads (134 MB, two launches); this one 35.5 us where the rows come from HBM (3.8 TB/s), 23.6
+// where the Infinity Cache still holds them (5.7 TB/s).
 // Non-zero counts are added to the global histogram at the end: PACKED = false: 64-bit counts hist[row][256], the layout that
 // gaac_exponent_hist hands out; PACKED = true: scratch[pair][bin][64] with the two 32-bit counts of a lane in one 64-bit word, so that a
 // wave's adds of a bin are one contiguous 512-byte access (prompts of up to 2^32 - 1 tokens).
@@ -61,7 +62,7 @@ __global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArg
 }
 static void launch_hist(HistArgs& A, int kinds, bool packed, hipStream_t stream) {
   // one block per CU, at least 256 tokens each, so that clearing and scanning the 64 KB table stays the smaller part (two blocks per CU,
-  // which the LDS has room for: 32 against 30 us for 2 x 8 heads x 32768 tokens)
+  // which the LDS has room for: 26 against 23.6 us for 2 x 8 heads x 32768 tokens)
   const int pairs = kinds * A.n_kv;
   long nchunk = min((A.n_tok + 255) / 256, (long)max(1, 256 / pairs));
   nchunk = max(nchunk, (A.n_tok + HIST_MAX_CHUNK - 1) / HIST_MAX_CHUNK);
