@@ -73,8 +73,8 @@ def launch_nsplit(B: int, n_kv: int, S: int, ragged: bool) -> int:
         but 12 of 100..1000 13.7 / 15.8, 16 of 1000 14.7 / 16.8, 32 of 100..500 12.0 / 16.6.  From 170 heads to 256 this is a bet on
         rows that differ: where long rows turn out equal, one block per (row, head) was faster (24 of 3000: 40.3 / 45.3, 32 of 3000:
         46.2 / 49.9, 24 of 12000: 138 / 151, 28 of 4000..5000: 63 / 70);
-      * ragged, more heads than CUs: two splits, one / two: 48 rows of 300..8000 x 8 heads 132 / 109, 48 of 100..2000 39.6 / 37.5, 64 of
-        200..4000 82.5 / 79.0; but 64 of 100..2000 42.2 / 49.3, 200 of 300 x 2 heads 15.6 / 17.8.  Equal: 48 of 2000 54.6 / 55.2."""
+      * ragged, more heads than CUs: two splits, one / two: 48 rows of 300..8000 x 8 heads 132 / 108, 48 of 100..2000 39.6 / 38.5, 64 of
+        200..4000 82.5 / 78; but 64 of 100..2000 41.7 / 49.3, 200 of 300 x 2 heads 14.7 / 17.5.  Equal: 48 of 2000 54.6 / 55.7."""
     H = B * n_kv
     if S <= 256: return 1
     if ragged and B > 1 and 64 < H <= 256 and S >= max(1500, 7 * H): n = -(-512 // H)
