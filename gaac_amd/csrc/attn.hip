@@ -656,30 +656,6 @@ __device__ __forceinline__ void load_tile(const Bases& B, int tile, int lane, co
 // ---------------------------------------------------------------------------------------------------- one tile pair
 struct WaveState { f32x4 acc[8]; float m_run, mu_run, l_run; };     // acc[i][r] = O[head a][group 4q+r, element i]; m in raw score units
 
-// unit decode with the escape contribution already expanded to exponent-field words x (see AttnLds::xlut)
-__device__ __forceinline__ void decode_unit_x(u32 slo, u32 shi, u32 g24, const u32x4& x, const u32x4& bw, u32* __restrict__ out) {
-  // low-half codes stay at bits 3p, high-half codes move to bits 16 + 3p; the bits this leaves at 12..15 and 28..31 never reach the
-  // fields the four masks below keep
-  const u32 cw = ((g24 << 4) & 0x0FFF0000u) | (g24 & ~0x0FFF0000u);
-  const u32 c0 = (cw << 7) & 0x03800380u, c1 = (cw << 4) & 0x03800380u, c2 = (cw << 1) & 0x03800380u, c3 = (cw >> 2) & 0x03800380u;
-  // bw: the base words of the unit's tier (3-bit base, or 4-bit base for promoted and raw groups: their x holds hi5 - base4)
-  const u32 e0 = c0 + bw[0] + x[0], e1 = c1 + bw[1] + x[1], e2 = c2 + bw[2] + x[2], e3 = c3 + bw[3] + x[3];
-  out[0] = (e0 & EXP_MASK2) | (__builtin_amdgcn_perm(shi, slo, 0x04040000u) & ~EXP_MASK2);
-  out[1] = (e1 & EXP_MASK2) | (__builtin_amdgcn_perm(shi, slo, 0x05050101u) & ~EXP_MASK2);
-  out[2] = (e2 & EXP_MASK2) | (__builtin_amdgcn_perm(shi, slo, 0x06060202u) & ~EXP_MASK2);
-  out[3] = (e3 & EXP_MASK2) | (__builtin_amdgcn_perm(shi, slo, 0x07070303u) & ~EXP_MASK2);
-}
-// raw group: 8 x 5 high exponent bits (40-bit little endian in lo/hi) as exponent-field words MINUS the 4-bit base words,
-// so that code + base4 + x reproduces code | hi5 << 3 exactly (32-bit arithmetic, the base cancels)
-__device__ __forceinline__ u32x4 raw_x_words(u32 lo, u32 hi, const u32x4& b4w) {
-  u32x4 x;
-  x[0] = (((lo) & 31u) << 10 | ((lo >> 20) & 31u) << 26) - b4w[0];
-  x[1] = (((lo >> 5) & 31u) << 10 | ((lo >> 25) & 31u) << 26) - b4w[1];
-  x[2] = (((lo >> 10) & 31u) << 10 | (__builtin_amdgcn_alignbit(hi, lo, 30) & 31u) << 26) - b4w[2];
-  x[3] = (((lo >> 15) & 31u) << 10 | ((hi >> 3) & 31u) << 26) - b4w[3];
-  return x;
-}
-
 // The x words of the lane's four units.  Common case: 4-bit groups only -> one v_perm + four table reads.  A wave with a raw
 // group somewhere (most tiles, few lanes) patches those units from the prefetched bytes.  A lane with two or more raw groups
 // (its bytes may not fit the 8 prefetched ones) re-reads memory: only the SLOW instantiation contains those loads, so the

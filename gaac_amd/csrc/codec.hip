@@ -362,27 +362,27 @@ __global__ void __launch_bounds__(256) k_row_offsets(const int* __restrict__ fla
 }
 
 // ---------------------------------------------------------------------------------------------------- page decoder
-// One wave per tile and block: short-lived waves at full occupancy overlap the dependent loads of a tile (tag words -> escape
-// bytes) with the arithmetic and the stores of others (four tiles in a row per wave were a third slower).
+// One wave per tile: short-lived waves at full occupancy overlap the dependent loads of a tile (tag words -> escape bytes) with the
+// arithmetic and the stores of others (four tiles in a row per wave were a third slower; four waves a block: 8 x 65536 tokens 40.8 -> 41.6 us).
+// Bound by the copy rate: 229 MB of a 64K-token page of 8 heads in 40.8 us = 5.6 TB/s in + out.  Before (bases read byte by byte from global
+// memory, escape bytes one load after the other, rows stored through the caches) K took 47.6 and V 49.1; 8 x 16384: 13.6 and 15.4 -> 11.6.
+struct DecodeArgs {
+  const uint8_t* sm; const uint8_t* cd; const int* flags; const int* tile_off; const uint8_t* ovf; const int* head_start;
+  const uint8_t* base3; const uint8_t* base4; int n_kv; const int* bidx; int S, S_pad; u16* out; long out_head_stride, out_row_stride;
+};
 template <int KIND>
-__global__ void __launch_bounds__(64) k_decode_tiles(const uint8_t* __restrict__ sm, const uint8_t* __restrict__ cd, const int* __restrict__ flags,
-                                                     const int* __restrict__ tile_off, const uint8_t* __restrict__ ovf,
-                                                     const int* __restrict__ head_start, const uint8_t* __restrict__ base3,
-                                                     const uint8_t* __restrict__ base4, int n_kv, const int* __restrict__ bidx,
-                                                     int S, int S_pad, u16* __restrict__ out, long out_head_stride, long out_row_stride) {
-  const int tile = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  const int brow = bidx ? bidx[h] : h % n_kv;
-  const long row0 = (long)h * S_pad + (long)tile * T;
+__global__ void __launch_bounds__(64) k_decode_tiles(const DecodeArgs A) {
+  __shared__ DecodeLds<KIND> L;
+  const int lane = threadIdx.x, tile = blockIdx.x, h = blockIdx.y;
+  const int brow = A.bidx ? A.bidx[h] : h % A.n_kv, nvalid = min(T, A.S - tile * T);
+  const long row0 = (long)h * A.S_pad + (long)tile * T, boff = (long)brow * D;
   // rows beyond S carry tag 0 (the encoder writes every word of a tile) and are not written
-  __shared__ __align__(16) u16 stage[T * STAGE_ROW];
-  u16* dst = out + (long)h * out_head_stride + (long)tile * T * out_row_stride;
-  const uint8_t* esc = ovf + head_start[h] + tile_off[(long)h * (S_pad / T) + tile];
-  if ((out_row_stride & 7) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0)
-    decode_tile_staged<KIND>(sm + row0 * D, cd + row0 * CB, flags + row0, esc, base3 + (long)brow * D, base4 + (long)brow * D, lane,
-                             min(T, S - tile * T), stage, dst, out_row_stride);
+  u16* dst = A.out + (long)h * A.out_head_stride + (long)tile * T * A.out_row_stride;
+  const uint8_t* esc = A.ovf + A.head_start[h] + A.tile_off[(long)h * (A.S_pad / T) + tile];
+  if ((A.out_row_stride & 7) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0)
+    decode_tile_staged<KIND>(A.sm + row0 * D, A.cd + row0 * CB, A.flags + row0, esc, A.base3 + boff, A.base4 + boff, lane, nvalid, L, dst, A.out_row_stride);
   else      // rows that are not 16-byte aligned: element stores
-    decode_tile_rows<KIND>(sm + row0 * D, cd + row0 * CB, flags + row0, esc, base3 + (long)brow * D, base4 + (long)brow * D, lane,
-                           min(T, S - tile * T), dst, out_row_stride);
+    decode_tile_rows<KIND>(A.sm + row0 * D, A.cd + row0 * CB, A.flags + row0, esc, A.base3 + boff, A.base4 + boff, lane, nvalid, dst, A.out_row_stride);
 }
 
 // ---------------------------------------------------------------------------------------------------- prompt into the slot cache
@@ -500,9 +500,10 @@ int gaac_decode_tiles(int kind, const uint8_t* sm, const uint8_t* codes, const i
   GAAC_REQUIRE(kind == 0 || kind == 1, "gaac_decode_tiles: kind must be 0 (k) or 1 (v)");
   GAAC_REQUIRE(sm && codes && flags && tile_off && ovf && head_start && base3 && base4 && out, "gaac_decode_tiles: null pointer");
   GAAC_REQUIRE(H > 0 && S > 0 && S_pad >= (S + T - 1) / T * T && S_pad % T == 0 && n_kv > 0, "gaac_decode_tiles: bad sizes");
-  dim3 grid((S + T - 1) / T, H);
-  if (kind == 0) hipLaunchKernelGGL(k_decode_tiles<KIND_K>, grid, dim3(64), 0, (hipStream_t)stream, sm, codes, flags, tile_off, ovf, head_start, base3, base4, n_kv, bidx, S, S_pad, (u16*)out, out_head_stride, out_row_stride);
-  else hipLaunchKernelGGL(k_decode_tiles<KIND_V>, grid, dim3(64), 0, (hipStream_t)stream, sm, codes, flags, tile_off, ovf, head_start, base3, base4, n_kv, bidx, S, S_pad, (u16*)out, out_head_stride, out_row_stride);
+  const DecodeArgs A{sm, codes, flags, tile_off, ovf, head_start, base3, base4, n_kv, bidx, S, S_pad, (u16*)out, out_head_stride, out_row_stride};
+  const dim3 grid((S + T - 1) / T, H);
+  if (kind == 0) hipLaunchKernelGGL(k_decode_tiles<KIND_K>, grid, dim3(64), 0, (hipStream_t)stream, A);
+  else hipLaunchKernelGGL(k_decode_tiles<KIND_V>, grid, dim3(64), 0, (hipStream_t)stream, A);
   return launch_status("gaac_decode_tiles");
 }
 
