@@ -44,13 +44,10 @@ __device__ __forceinline__ void append_one(const CacheStore& st, const u16* __re
   uint8_t* sm_tile = st.sm + row0 * D; uint8_t* cd_tile = st.cd + row0 * CB; int* fl_tile = st.flags + row0;
   const int used = st.ovf_used[h];
   uint8_t* dst = st.ovf + (long)h * A.ovf_cap + used;
-  int total; bool fits = true;
-  if (used + TILE_MAX_ESC + 8 <= A.ovf_cap) total = encode_staged_tile<KIND>(L, Bs, T, lane, sm_tile, cd_tile, fl_tile, dst);
-  else {      // less than one worst-case tile of room: count first, write only what fits
-    total = encode_staged_tile<KIND>(L, Bs, T, lane, sm_tile, cd_tile, fl_tile, nullptr);
-    fits = used + total + 8 <= A.ovf_cap;
-    if (fits) encode_staged_tile<KIND>(L, Bs, T, lane, sm_tile, cd_tile, fl_tile, dst);
-  }
+  UnitEscapes E;
+  const int total = encode_staged_tile<KIND, false>(L, Bs, T, lane, sm_tile, cd_tile, fl_tile, E);
+  const bool fits = (long)used + total + 8 <= A.ovf_cap;
+  if (fits) write_tile_escapes(E, dst);
   if (fits) {
     if (lane == 0) { st.tile_off[(long)h * (A.cap / T) + tile] = used; st.ovf_used[h] = used + total; }
   } else {    // keep every later reader in bounds: the tile reads as all tier 0 (wrong values, flagged)

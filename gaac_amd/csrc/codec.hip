@@ -155,6 +155,12 @@ __global__ void __launch_bounds__(256) k_bases_from_hist(const long long* __rest
 // A block of four waves takes 4 * TPW consecutive tiles of one head, wave w the tiles w, w+4, ... of them (one-wave blocks, one per tile,
 // would be limited by the rate at which workgroups can be launched).  The rows of a wave's next tile are fetched into registers while it
 // encodes the current one.  K and V of a prompt share a launch (blockIdx.z): one start-up and one drain for both.
+// Bound by the memory rate: 229 MB of a 64K-token page of 8 heads in 42 us.  What goes past the caches is chosen by what comes next, so that the
+// Infinity Cache keeps the rest:
+//   * the rows of a large launch (TPW > 1) are read for the last time: 64K page 44.6 -> 42.3 us; the 32768-token prompt's call, where the histogram has
+//     just brought them in, 109 -> 101 us;
+//   * a prompt's tiles (PROMPT) are stored past them, or they would push out rows that are still to be read: 119 -> 109 us; a page's are not,
+//     the caller is as likely to read them at once: 64K page and back 107 us past the caches, 101 through them.
 constexpr int CODEC_WAVES = 4;
 struct EncodeKind {      // one of K, V
   const u16* x; long head_stride, row_stride;
@@ -163,13 +169,13 @@ struct EncodeKind {      // one of K, V
   uint8_t* slots; int* tile_bytes;                 // [H][ntiles] worst-case escape slots and the bytes used in each
 };
 struct EncodeArgs { EncodeKind k, v; int kind0, S, S_pad, ntiles, brow0, NB; const int* bidx; };      // blockIdx.z = 0 is kind0
-template <int KIND, int TPW>
+template <int KIND, int TPW, bool PROMPT>
 __device__ __forceinline__ void encode_tiles_body(const EncodeArgs& A, const EncodeKind& J, EncodeLds& L, int h, int tile, int lane) {
   const int S = A.S, ntiles = A.ntiles;
   const int brow = A.bidx ? A.bidx[h] : (A.brow0 + h) % A.NB;
   const u16* xh = J.x + (long)h * J.head_stride;
   RowRegs R, Rn;
-  load_rows(R, xh + (long)tile * T * J.row_stride, J.row_stride, min(T, S - tile * T), lane);
+  load_rows<(TPW > 1)>(R, xh + (long)tile * T * J.row_stride, J.row_stride, min(T, S - tile * T), lane);
   stage_bases(L, J.b3 + (long)brow * D, J.b4 + (long)brow * D, lane);
   wave_lds_sync();
   BaseRegs Bs;                // the base words of the lane's units: the same for every tile of the head
@@ -177,32 +183,34 @@ __device__ __forceinline__ void encode_tiles_body(const EncodeArgs& A, const Enc
   for (int i = 0; i < TPW && tile < ntiles; ++i, tile += CODEC_WAVES) {
     const int nvalid = min(T, S - tile * T), next = tile + CODEC_WAVES;
     store_rows(L, R, lane);
-    if (i + 1 < TPW && next < ntiles) load_rows(Rn, xh + (long)next * T * J.row_stride, J.row_stride, min(T, S - next * T), lane);
+    if (i + 1 < TPW && next < ntiles) load_rows<(TPW > 1)>(Rn, xh + (long)next * T * J.row_stride, J.row_stride, min(T, S - next * T), lane);
     wave_lds_sync();
     const long row0 = (long)h * A.S_pad + (long)tile * T;
-    const int total = encode_staged_tile<KIND>(L, Bs, nvalid, lane, J.sm + row0 * D, J.cd + row0 * CB, J.flags + row0,
-                                               J.slots + ((long)h * ntiles + tile) * TILE_MAX_ESC);
+    UnitEscapes E;
+    const int total = encode_staged_tile<KIND, PROMPT>(L, Bs, nvalid, lane, J.sm + row0 * D, J.cd + row0 * CB, J.flags + row0, E);
+    write_tile_escapes(E, J.slots + ((long)h * ntiles + tile) * TILE_MAX_ESC);
     if (lane == 0) J.tile_bytes[(long)h * ntiles + tile] = total;
-    wave_lds_sync();          // the staged rows and tag words are free again
+    wave_lds_sync();          // the staged rows are free again
     R = Rn;
   }
 }
-template <int TPW>
+template <int TPW, bool PROMPT>
 __global__ void __launch_bounds__(64 * CODEC_WAVES) k_encode_tiles(const EncodeArgs A) {
   __shared__ EncodeLds Ls[CODEC_WAVES];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, tile = blockIdx.x * (CODEC_WAVES * TPW) + wave;
   if (tile >= A.ntiles) return;
-  if (A.kind0 + (int)blockIdx.z == KIND_K) encode_tiles_body<KIND_K, TPW>(A, A.k, Ls[wave], blockIdx.y, tile, lane);
-  else encode_tiles_body<KIND_V, TPW>(A, A.v, Ls[wave], blockIdx.y, tile, lane);
+  if (A.kind0 + (int)blockIdx.z == KIND_K) encode_tiles_body<KIND_K, TPW, PROMPT>(A, A.k, Ls[wave], blockIdx.y, tile, lane);
+  else encode_tiles_body<KIND_V, TPW, PROMPT>(A, A.v, Ls[wave], blockIdx.y, tile, lane);
 }
+template <bool PROMPT>
 static void launch_encode(const EncodeArgs& A, int H, int kinds, hipStream_t stream) {
   // Four tiles in a row per wave hide a tile's row loads behind the previous tile and share the base words; below 8192 tiles (eight
   // waves per SIMD with one tile each) that leaves SIMDs idle, and one tile per wave is faster:
-  // 7.9 against 10.4 us at 2048 tiles, 17.8 against 15.8 us at 8192, 56 against 52 us at 32768
+  // 7.9 against 10.4 us at 2048 tiles, 17.0 against 14.8 us at 8192, 50.6 against 44.8 us at 32768 (K)
   if ((long)A.ntiles * H * kinds >= 8192)
-    hipLaunchKernelGGL(k_encode_tiles<4>, dim3((A.ntiles + 4 * CODEC_WAVES - 1) / (4 * CODEC_WAVES), H, kinds), dim3(64 * CODEC_WAVES), 0, stream, A);
+    hipLaunchKernelGGL((k_encode_tiles<4, PROMPT>), dim3((A.ntiles + 4 * CODEC_WAVES - 1) / (4 * CODEC_WAVES), H, kinds), dim3(64 * CODEC_WAVES), 0, stream, A);
   else
-    hipLaunchKernelGGL(k_encode_tiles<1>, dim3((A.ntiles + CODEC_WAVES - 1) / CODEC_WAVES, H, kinds), dim3(64 * CODEC_WAVES), 0, stream, A);
+    hipLaunchKernelGGL((k_encode_tiles<1, PROMPT>), dim3((A.ntiles + CODEC_WAVES - 1) / CODEC_WAVES, H, kinds), dim3(64 * CODEC_WAVES), 0, stream, A);
 }
 
 // Exclusive prefix sums of one head's tile sizes into off, and their total; called by all threads of a block, of which each SCAN_NT
@@ -453,7 +461,7 @@ int gaac_encode_tiles(int kind, const void* x, long x_head_stride, long x_row_st
   EncodeArgs A{};
   A.kind0 = kind; A.S = S; A.S_pad = S_pad; A.ntiles = (S + T - 1) / T; A.brow0 = 0; A.NB = n_kv; A.bidx = bidx;
   (kind == 0 ? A.k : A.v) = EncodeKind{(const u16*)x, x_head_stride, x_row_stride, base3, base4, sm, codes, flags, esc_slots, tile_bytes};
-  launch_encode(A, H, 1, (hipStream_t)stream);
+  launch_encode<false>(A, H, 1, (hipStream_t)stream);
   return launch_status("gaac_encode_tiles");
 }
 
@@ -540,7 +548,7 @@ int gaac_cache_prefill(
     E.kind0 = KIND_K; E.S = ntiles * T; E.S_pad = cap; E.ntiles = ntiles; E.brow0 = head0; E.NB = NB; E.bidx = nullptr;
     E.k = EncodeKind{(const u16*)k, k_head_stride, k_row_stride, k_base3, k_base4, k_sm + row0 * D, k_codes + row0 * CB, k_flags + row0, esc_slots, tile_bytes};
     E.v = EncodeKind{(const u16*)v, v_head_stride, v_row_stride, v_base3, v_base4, v_sm + row0 * D, v_codes + row0 * CB, v_flags + row0, v_slots, v_bytes};
-    launch_encode(E, n_kv, 2, st);
+    launch_encode<true>(E, n_kv, 2, st);
   }
   const int window = ovf_cap - (TILE_MAX_ESC + 8);      // room for one more worst-case tile and the readers' padding stays free
   PromptScanArgs P{};

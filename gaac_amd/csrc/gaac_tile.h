@@ -11,19 +11,23 @@ namespace gaac {
 constexpr int XROW = D + 8;     // staged row stride in elements: 16 padding bytes spread the sixteen rows of a column over the banks
 struct EncodeLds {
   u16 x[T * XROW];     // the tile's BF16 bit patterns, token-major, natural channel order (rows >= nvalid are zero)
-  uint8_t b3[D], b4[D];
-  u32 tags[T];
-  int rowoff[T + 1];   // exclusive prefix of per-row escape bytes; [16] = tile total
+  __align__(4) uint8_t b3[D], b4[D];
 };
 
-// 16 rows of 128 BF16 (row r at src + r*row_stride elements): lane's four 16-byte pieces; rows >= nvalid read as zero.
+// 16 rows of 128 BF16 (row r at src + r*row_stride elements): lane's four 16-byte pieces; rows >= nvalid read as zero (the last valid row is
+// loaded in their place: a load under a branch would be waited for by itself).  STREAM: a prompt larger than the caches, read once.
 struct RowRegs { u32x4 v[4]; };
+template <bool STREAM>
 __device__ __forceinline__ void load_rows(RowRegs& R, const u16* __restrict__ src, long row_stride, int nvalid, int lane) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int idx = k * 64 + lane, row = idx >> 4, c16 = idx & 15;
-    R.v[k] = u32x4{0u, 0u, 0u, 0u};
-    if (row < nvalid) R.v[k] = *reinterpret_cast<const u32x4*>(src + (long)row * row_stride + c16 * 8);
+    const int row = 4 * k + (lane >> 4);
+    const u32x4* p = reinterpret_cast<const u32x4*>(src + (long)min(row, nvalid - 1) * row_stride + 8 * (lane & 15));
+    R.v[k] = STREAM ? __builtin_nontemporal_load(p) : *p;
+  }
+  if (nvalid < T) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) if (4 * k + (lane >> 4) >= nvalid) R.v[k] = u32x4{0u, 0u, 0u, 0u};
   }
 }
 __device__ __forceinline__ void store_rows(EncodeLds& L, const RowRegs& R, int lane) {
@@ -33,16 +37,9 @@ __device__ __forceinline__ void store_rows(EncodeLds& L, const RowRegs& R, int l
     *reinterpret_cast<u32x4*>(&L.x[row * XROW + c16 * 8]) = R.v[k];
   }
 }
-// Stage 16 rows into lds.x
-__device__ __forceinline__ void stage_rows(EncodeLds& L, const u16* __restrict__ src, long row_stride, int nvalid, int lane) {
-  RowRegs R;
-  load_rows(R, src, row_stride, nvalid, lane);
-  store_rows(L, R, lane);
-}
 __device__ __forceinline__ void stage_bases(EncodeLds& L, const uint8_t* __restrict__ b3row, const uint8_t* __restrict__ b4row, int lane) {
   if (lane < 32) reinterpret_cast<u32*>(L.b3)[lane] = reinterpret_cast<const u32*>(b3row)[lane];
   else reinterpret_cast<u32*>(L.b4)[lane - 32] = reinterpret_cast<const u32*>(b4row)[lane - 32];
-  if (lane < T) L.tags[lane] = 0u;
 }
 
 // Orders the LDS traffic of ONE wave (LDS operations of a wave complete in program order; the fences only stop the compiler from
@@ -56,15 +53,24 @@ __device__ __forceinline__ void wave_lds_sync() {
 struct BaseRegs { u32 b3[4][4], b4[4][4]; };      // [unit][i]: base of element i | base of element i+4 << 16
 template <int KIND>
 __device__ __forceinline__ void load_base_regs(const EncodeLds& L, int a, int q, BaseRegs& B) {
+  const auto load = [&](const uint8_t* b, u32 (&w)[4], int u) {
+    if (KIND == KIND_K) {      // elements (2m, 2m+1) are the adjacent channels 32u + 2q + 8m (+1)
+      const u16* r = reinterpret_cast<const u16*>(b) + 16 * u + q;
+      const u32 r0 = r[0], r1 = r[4], r2 = r[8], r3 = r[12];
+      w[0] = __builtin_amdgcn_perm(r2, r0, 0x0C040C00u); w[1] = __builtin_amdgcn_perm(r2, r0, 0x0C050C01u);
+      w[2] = __builtin_amdgcn_perm(r3, r1, 0x0C040C00u); w[3] = __builtin_amdgcn_perm(r3, r1, 0x0C050C01u);
+    } else {
+      const uint8_t* r = b + 64 * (a & 1) + (a >> 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = (u32)r[8 * i] | ((u32)r[8 * i + 32] << 16);
+    }
+  };
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const int grp = unit_group<KIND>(a, q, u);
+    if (KIND == KIND_V && u > 0) {      // a lane's units are of one group
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c0 = chan_of<KIND>(8 * grp + i), c1 = chan_of<KIND>(8 * grp + i + 4);
-      B.b3[u][i] = (u32)L.b3[c0] | ((u32)L.b3[c1] << 16);
-      B.b4[u][i] = (u32)L.b4[c0] | ((u32)L.b4[c1] << 16);
-    }
+      for (int i = 0; i < 4; ++i) { B.b3[u][i] = B.b3[0][i]; B.b4[u][i] = B.b4[0][i]; }
+    } else { load(L.b3, B.b3[u], u); load(L.b4, B.b4[u], u); }
   }
 }
 // the four data words of unit u of lane (a, q)
@@ -88,75 +94,87 @@ __device__ __forceinline__ u32 pk_sub_u16(u32 x, u32 y) {
   return __builtin_bit_cast(u32, (u16x2_t)(__builtin_bit_cast(u16x2_t, x) - __builtin_bit_cast(u16x2_t, y)));
 }
 
-// Encodes the tile staged in L (after a barrier).  Writes the native sign/mantissa and code bytes, the 16 tag words (one per line) and
-// the escape bytes (at esc_dst + offset-in-tile; nullptr = count only).  Returns the tile's escape byte count (all lanes).
-// Must be called by all 64 lanes of the wave that owns L; it synchronises that wave only.  B: load_base_regs of the same L.
-template <int KIND>
-__device__ __forceinline__ int encode_staged_tile(EncodeLds& L, const BaseRegs& B, int nvalid, int lane, uint8_t* __restrict__ sm_tile,
-                                                  uint8_t* __restrict__ cd_tile, int* __restrict__ flags_tile,
-                                                  uint8_t* __restrict__ esc_dst) {
+// What a lane's four units add to the escape stream: tags, the 4th code bits of a 4-bit group, the exponent words of a raw one, and where the
+// lane's bytes start among the tile's.
+struct UnitEscapes { u32 tag[4], eb[4], ew[4][4]; int pos; };
+// bitwise or across the four 16-lane rows at fixed column
+__device__ __forceinline__ u32 quad_rows_or(u32 x) {
+  auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  x = r[0] | r[1];
+  auto s = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  return s[0] | s[1];
+}
+
+// Encodes the tile staged in L (after a barrier).  Writes the native sign/mantissa and code bytes and the 16 tag words (one per line); the
+// escape bytes stay with the lanes for write_tile_escapes, so that a caller can see their number before it says where they go.
+// Returns the tile's escape byte count (all lanes).  Must be called by all 64 lanes of the wave that owns L.  B: load_base_regs of the same L.
+// STREAM: the bytes go past the caches.
+template <int KIND, bool STREAM>
+__device__ __forceinline__ int encode_staged_tile(const EncodeLds& L, const BaseRegs& B, int nvalid, int lane, uint8_t* __restrict__ sm_tile,
+                                                  uint8_t* __restrict__ cd_tile, int* __restrict__ flags_tile, UnitEscapes& E) {
   const int a = lane & 15, q = lane >> 4;
-  u32 slo[4], shi[4], g24[4], tag[4], eb[4], ew[4][4];
+  u32 slo[4], shi[4], g24[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     u32 W[4], d3[4], d4[4];
     unit_data_words<KIND>(L, a, q, u, W);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      ew[u][i] = (W[i] >> 7) & 0x00FF00FFu;                      // exponents
-      d3[i] = pk_sub_u16(ew[u][i], B.b3[u][i]); d4[i] = pk_sub_u16(ew[u][i], B.b4[u][i]);      // negative differences wrap to >= 0xFF01
+      E.ew[u][i] = (W[i] >> 7) & 0x00FF00FFu;                    // exponents
+      d3[i] = pk_sub_u16(E.ew[u][i], B.b3[u][i]); d4[i] = pk_sub_u16(E.ew[u][i], B.b4[u][i]);      // negative differences wrap to >= 0xFF01
     }
     // tier rule (codec.py:144-150): all eight differences in 0..7, else all in 0..15, else raw
     const bool fit3 = ((d3[0] | d3[1] | d3[2] | d3[3]) & 0xFFF8FFF8u) == 0u, fit4 = ((d4[0] | d4[1] | d4[2] | d4[3]) & 0xFFF0FFF0u) == 0u;
-    const bool valid = unit_token<KIND>(a, q, u) < nvalid;       // padded rows: tier 0, code 0, sign/mantissa 0
     u32 cacc = 0u, xacc = 0u, sb[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const u32 c = fit3 ? d3[i] : (fit4 ? d4[i] : ew[u][i]);
+      const u32 c = fit3 ? d3[i] : (fit4 ? d4[i] : E.ew[u][i]);
       cacc |= (c & 0x00070007u) << (3 * i);                       // code of element i at bits 3i, of element i+4 at 16 + 3i
       xacc |= (d4[i] & 0x00080008u) << i;                         // 4th code bit of element i at bit 3 + i, of i+4 at 19 + i
-      sb[i] = ((W[i] >> 8) & 0x00800080u) | (W[i] & 0x007F007Fu); // sign/mantissa bytes at bits 0..7 and 16..23
+      sb[i] = ((W[i] >> 8) & ~0x007F007Fu) | (W[i] & 0x007F007Fu); // sign/mantissa bytes at bits 0..7 and 16..23 (the other bytes are not taken)
     }
     const u32 p01 = __builtin_amdgcn_perm(sb[1], sb[0], 0x06020400u), p23 = __builtin_amdgcn_perm(sb[3], sb[2], 0x06020400u);
-    const u32 s_lo = __builtin_amdgcn_perm(p23, p01, 0x05040100u), s_hi = __builtin_amdgcn_perm(p23, p01, 0x07060302u);
-    tag[u] = !valid || fit3 ? 0u : (fit4 ? 1u : 3u);
-    g24[u] = valid ? (cacc & 0xFFFu) | ((cacc >> 16) << 12) : 0u;
-    slo[u] = valid ? s_lo : 0u; shi[u] = valid ? s_hi : 0u;
-    eb[u] = ((xacc >> 3) & 0xFu) | ((xacc >> 19) << 4);
+    slo[u] = __builtin_amdgcn_perm(p23, p01, 0x05040100u); shi[u] = __builtin_amdgcn_perm(p23, p01, 0x07060302u);
+    E.tag[u] = fit3 ? 0u : (fit4 ? 1u : 3u);
+    g24[u] = (cacc & 0xFFFu) | ((cacc >> 16) << 12);
+    E.eb[u] = ((xacc >> 3) & 0xFu) | ((xacc >> 19) << 4);
   }
-  // tag word of line a: this lane owns bits 8q..8q+7 (its four units)
-  reinterpret_cast<uint8_t*>(L.tags)[4 * a + q] = (uint8_t)(tag[0] | (tag[1] << 2) | (tag[2] << 4) | (tag[3] << 6));
+  if (nvalid < T) {      // padded rows: tier 0, code 0, sign/mantissa 0
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (unit_token<KIND>(a, q, u) >= nvalid) { E.tag[u] = 0u; g24[u] = 0u; slo[u] = 0u; shi[u] = 0u; }
+  }
   u32x4 s0 = {slo[0], shi[0], slo[1], shi[1]}, s1 = {slo[2], shi[2], slo[3], shi[3]};
-  *reinterpret_cast<u32x4*>(sm_tile + 16 * lane) = s0;
-  *reinterpret_cast<u32x4*>(sm_tile + 1024 + 16 * lane) = s1;
-  *reinterpret_cast<u32*>(cd_tile + 4 * lane) = g24[0] | (g24[1] << 24);
-  *reinterpret_cast<u32*>(cd_tile + 256 + 4 * lane) = (g24[1] >> 8) | (g24[2] << 16);
-  *reinterpret_cast<u32*>(cd_tile + 512 + 4 * lane) = (g24[2] >> 16) | (g24[3] << 8);
-  wave_lds_sync();
-  {
-    const u32 f = L.tags[a];
-    const u32 rb = (u32)esc_bytes(f), incl = row_scan16(rb);
-    if (lane < T) { L.rowoff[lane] = (int)(incl - rb); flags_tile[lane] = (int)f; if (lane == T - 1) L.rowoff[T] = (int)incl; }
-  }
-  wave_lds_sync();
-  if (esc_dst) {
-    uint8_t* p = esc_dst + L.rowoff[a] + esc_prefix(L.tags[a], 8 * q);
+  const u32 c0 = g24[0] | (g24[1] << 24), c1 = (g24[1] >> 8) | (g24[2] << 16), c2 = (g24[2] >> 16) | (g24[3] << 8);
+  u32x4* sm = reinterpret_cast<u32x4*>(sm_tile + 16 * lane); u32* cd = reinterpret_cast<u32*>(cd_tile + 4 * lane);
+  if (STREAM) {
+    __builtin_nontemporal_store(s0, sm); __builtin_nontemporal_store(s1, sm + 64);
+    __builtin_nontemporal_store(c0, cd); __builtin_nontemporal_store(c1, cd + 64); __builtin_nontemporal_store(c2, cd + 128);
+  } else { sm[0] = s0; sm[64] = s1; cd[0] = c0; cd[64] = c1; cd[128] = c2; }
+  // tag word of line a: this lane owns bits 8q..8q+7 (its four units)
+  const u32 f = quad_rows_or((E.tag[0] | (E.tag[1] << 2) | (E.tag[2] << 4) | (E.tag[3] << 6)) << (8 * q));
+  if (lane < T) flags_tile[lane] = (int)f;
+  const u32 rb = (u32)esc_bytes(f), incl = row_scan16(rb);
+  E.pos = (int)(incl - rb) + esc_prefix(f, 8 * q);
+  return __builtin_amdgcn_readlane((int)incl, 15);
+}
+// The escape bytes of an encoded tile, to esc_tile (the tile's first) on
+__device__ __forceinline__ void write_tile_escapes(const UnitEscapes& E, uint8_t* esc_tile) {
+  uint8_t* p = esc_tile + E.pos;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (tag[u] == 1u) { p[0] = (uint8_t)eb[u]; p += 1; }
-      else if (tag[u] == 3u) {
-        // raw group: the upper five exponent bits of the eight elements, 40 bits little-endian (element i at bit 5i)
-        u32 hl = 0u, hh = 0u;
+  for (int u = 0; u < 4; ++u) {
+    if (E.tag[u] == 1u) p[0] = (uint8_t)E.eb[u];
+    else if (E.tag[u] == 3u) {
+      // raw group: the upper five exponent bits of the eight elements, 40 bits little-endian (element i at bit 5i)
+      u32 hl = 0u, hh = 0u;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { hl |= ((ew[u][i] >> 3) & 0x1Fu) << (5 * i); hh |= ((ew[u][i] >> 19) & 0x1Fu) << (5 * i); }
-        const u64 h = (u64)hl | ((u64)hh << 20);
+      for (int i = 0; i < 4; ++i) { hl |= ((E.ew[u][i] >> 3) & 0x1Fu) << (5 * i); hh |= ((E.ew[u][i] >> 19) & 0x1Fu) << (5 * i); }
+      const u64 h = (u64)hl | ((u64)hh << 20);
 #pragma unroll
-        for (int k = 0; k < 5; ++k) p[k] = (uint8_t)(h >> (8 * k));
-        p += 5;
-      }
+      for (int k = 0; k < 5; ++k) p[k] = (uint8_t)(h >> (8 * k));
     }
+    p += tag_size(E.tag[u]);
   }
-  return L.rowoff[T];
 }
 
 // Per-lane metadata of a stored tile: the 2-bit tag of each of the lane's four units and the offset of the unit's escape

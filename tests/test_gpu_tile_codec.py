@@ -1,4 +1,4 @@
-"""The tile decoder at every combination of tiers that a lane can hold (its four groups raw, 4-bit or 3-bit): what it reads of the escape bytes,
+"""The tile encoder at the edges of the room its escape bytes have, and the tile decoder at every combination of tiers that a lane can hold (its four groups raw, 4-bit or 3-bit): what it reads of the escape bytes,
 and where it takes them from, depends on that.  Pages and paged slots, rows of every alignment; the result is the input, bit for bit."""
 import itertools
 import numpy as np
@@ -84,4 +84,52 @@ def test_paged_slots_of_every_combination_of_tiers(ovf_slot, p_raw):
         layer.decode_blocks(pool, pairs, sk, sv)
         for got, want in ((sk, k16), (sv, v16)):
             assert np.array_equal(to_u16(got[:, :n_kv * 128].contiguous()).reshape(L, n_kv, 128), want) and not to_u16(got[:, n_kv * 128:].contiguous()).any()
+    layer.check()
+
+
+@pytest.mark.parametrize("room", [0, -1])
+@pytest.mark.parametrize("raw_groups", [256, 3])
+def test_append_fills_its_window_to_the_last_byte(room, raw_groups):
+    """The tile that a decode step completes needs 5 bytes a raw group: a window of exactly that many takes it, one byte less does not."""
+    dev = require_gpu()
+    from gaac_amd import CompressedKVCache
+    rng = np.random.default_rng(raw_groups)
+    tiers = np.zeros((1, 16, 16), int)
+    tiers.reshape(-1)[rng.permutation(256)[:raw_groups]] = 3
+    k16, v16 = (_tiers_to_rows(tiers, kind, rng).transpose(1, 0, 2) for kind in "kv")
+    k, v = to_bf16(k16, dev), to_bf16(v16, dev)
+    full = lambda b: torch.full((1, 128), b, dtype=torch.uint8)
+    cache = CompressedKVCache(1, 1, 16, dict(k3=full(B3), k4=full(B4), v3=full(B3), v4=full(B4)), ovf_bytes_per_tile=5 * raw_groups + room)
+    slots = torch.zeros(1, dtype=torch.int32, device=dev)
+    for i in range(16): cache.append(slots, k[i:i + 1], v[i:i + 1])
+    assert int(cache.overflow) == (0 if room == 0 else 2)
+    for st, x16 in ((cache.k, k16), (cache.v, v16)):
+        assert int(st.ovf_used[0]) == (5 * raw_groups if room == 0 else 0) and bool((st.flags != 0).any()) == (room == 0)
+    if room == 0:
+        dk, dv = cache.decompress(0)
+        assert np.array_equal(to_u16(dk), k16) and np.array_equal(to_u16(dv), v16)
+
+
+@pytest.mark.parametrize("held", [0, 1, 5, 15])
+@pytest.mark.parametrize("groups", [16, 17])
+def test_paged_store_completes_a_block_from_held_and_new_rows(held, groups):
+    """A block of 16 or 17 four-bit groups against slots with room for 16 escape bytes, completed on top of `held` raw rows."""
+    dev = require_gpu()
+    from gaac_amd.paged import LayerState, build_store_entries
+    rng = np.random.default_rng(held)
+    tiers = np.zeros((2, 16, 16), int)
+    for h in range(2): tiers[h].reshape(-1)[rng.permutation(256)[:groups]] = 1
+    k16, v16 = (np.ascontiguousarray(_tiers_to_rows(tiers, kind, rng).transpose(1, 0, 2)) for kind in "kv")
+    k, v = to_bf16(k16, dev), to_bf16(v16, dev)
+    full = lambda b: torch.full((2, 128), b, dtype=torch.uint8)
+    layer = LayerState(3, 2, 8, dict(k3=full(B3), k4=full(B4), v3=full(B3), v4=full(B4)), ovf_slot=16)
+    pool = torch.full((LayerState.pool_bytes(3, 2, 16),), 255, dtype=torch.uint8, device=dev)
+    entries = lambda c, n: torch.from_numpy(build_store_entries([c], [n], [[1]])).to(dev)
+    if held: layer.store(k[:held], v[:held], pool, entries(0, held))
+    layer.store(k[held:], v[held:], pool, entries(held, 16 - held))
+    fits = groups <= 16
+    assert bool((layer.mt.view(3, 4)[1] >= 0).all()) == fits and int(layer.top) == (8 if fits else 4)
+    sk, sv = torch.zeros(16, 2, 128, dtype=torch.bfloat16, device=dev), torch.zeros(16, 2, 128, dtype=torch.bfloat16, device=dev)
+    layer.decode_blocks(pool, torch.tensor([[1, 0, 16]], dtype=torch.int32, device=dev), sk, sv)
+    assert np.array_equal(to_u16(sk), k16) and np.array_equal(to_u16(sv), v16)
     layer.check()
