@@ -364,135 +364,70 @@ __device__ __forceinline__ void merge_heads(const AttnArgs& A, long qh0, int G, 
 }
 
 // ---------------------------------------------------------------------------------------------------- uncompressed rows
-// Attention of the block's G query heads over up to 16 rows kept as plain BF16 (the raw tail of a cache head, gaac_tail of
-// /root/reference/gaac/kernel.py:220-279), done by the block's first 256 threads in fp32 on the VALU (all threads take part in the barriers).  The result is folded into the running
-// partial (m, l, acc) that the block merge treats as a fifth wave; several calls accumulate (online softmax).
-struct RawScratch {              // lives in the block-merge buffer, which is idle until the waves have finished their tiles
-  float qs[GMAX][D];             // the query heads in fp32, natural channel order
-  float sc[GMAX][T];             // scores, then probabilities
-  float alpha[GMAX];             // rescale factor of the running partial
-  u16 krows[T * D], vrows[T * D];   // a compressed tile decoded next to a raw one (paged mode: only one kind of a tile is raw)
-};
-template <int NT>
-__device__ __forceinline__ void raw_rows_begin(RawScratch& R, const AttnArgs& A, long qh0, int G, int tid) {
-  for (int i = tid; i < G * D; i += NT) R.qs[i >> 7][i & 127] = bf16_bits_to_float(A.q[qh0 * D + i]);
-}
-// krows / vrows: 16 x 128 BF16, row stride D; rows >= nvalid are ignored.  m5/l5/acc5: the running partial [GMAX], [GMAX], [GMAX][D].
-template <int NT>
-__device__ __forceinline__ void raw_rows_attend(RawScratch& R, const u16* __restrict__ krows, const u16* __restrict__ vrows, int nvalid,
-                                                float scale_log2e, int G, int tid, float* __restrict__ m5, float* __restrict__ l5,
-                                                float (*__restrict__ acc5)[D]) {
-  __syncthreads();               // qs is filled / the previous call is done with sc
-  const int t = tid >> 4, c = tid & 15;
-  // all global loads of the call up front (one memory latency): this thread's piece of a K row, and for the output the two
-  // channels 2 (tid & 63), +1 of all 16 V rows
-  u32x4 kv = {0u, 0u, 0u, 0u};
-  if (t < nvalid && t < T) kv = *reinterpret_cast<const u32x4*>(krows + t * D + 8 * c);
-  u32 vv[T];
+// Attention of the block's query heads over up to 16 rows kept as plain BF16: the raw tail of a cache head (gaac_tail of
+// /root/reference/gaac/kernel.py:220-279) or a raw tile of the paged pool.  ONE wave does it, ahead of its tiles, and the block's other
+// waves take the tiles that it does not get to.  All rows and queries are loaded in one batch, so it costs one trip to memory and some
+// 60 matrix products however many query heads there are; weights and sums stay in fp32:
+//   * scores: 4 x v_mfma_f32_16x16x32_bf16 over the rows as they lie (products of BF16 are exact in fp32), lane (head a, quad q) gets tokens 4q + r;
+//   * output: 32 x v_mfma_f32_16x16x4_f32; its B operand is the weight p[r] where the score product left it, A the V row 4q + r in fp32.
+// Before, in vector arithmetic with a trip to memory per query head for its queries: 3 us beyond the tiles of the block with 4 query heads, 10
+// with 16, at the end of which the launch waited; a raw tile of the paged pool was taken by the whole block behind its tiles, through six
+// barriers, one of which every block of the launch paid for.  Launches in a graph, us: slot cache, 4 rows of 790 tokens x 8 kv heads x 4 query
+// heads 11.1 -> 9.8, 1 row x 1 kv head x 16 21.0 -> 13.6; paged, 8 sequences of 200..3000 x 8 kv heads 24.0 -> 21.7, 16 of 32000 276 -> 249,
+// 16 of 4096..65536 297 -> 284, 1 of 900 x 1 kv head x 16 29.0 -> 19.0.
+struct RawState { f32x4 acc[8]; float m, l; };      // acc[i][r] = O[head a][channel 8 (4q + r) + i]; m in the base-2 domain
+// krows / vrows: rows of 128 BF16 back to back, of which the first nvalid (1..16) count; qr[j]: channels 32j + 8q .. + 8 of query head a
+__device__ __forceinline__ void raw_rows_attend(const u16* krows, const u16* vrows, int nvalid, const u32x4 (&qr)[4], float scale_log2e, int a, int q, RawState& st) {
+  u32x4 k[4], v[4];      // no load under a branch: rows past the end read the last valid row
 #pragma unroll
-  for (int tk = 0; tk < T; ++tk) vv[tk] = *reinterpret_cast<const u32*>(vrows + min(tk, max(nvalid - 1, 0)) * D + 2 * (tid & 63));
+  for (int j = 0; j < 4; ++j) k[j] = *reinterpret_cast<const u32x4*>(krows + min(a, nvalid - 1) * D + 32 * j + 8 * q);
 #pragma unroll
-  for (int tk = 0; tk < T; ++tk) vv[tk] = tk < nvalid ? vv[tk] : 0u;      // rows past the end weigh 0: keep an Inf of the clamped row out of 0 * Inf
-  float kr[8];
+  for (int r = 0; r < 4; ++r) v[r] = *reinterpret_cast<const u32x4*>(vrows + min(4 * q + r, nvalid - 1) * D + 8 * a);
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) { kr[2 * i] = bf16_bits_to_float(kv[i] & 0xFFFFu); kr[2 * i + 1] = bf16_bits_to_float(kv[i] >> 16); }
-  for (int g = 0; g < G; ++g) {
-    float d = 0.f;
+  for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k[j]), __builtin_bit_cast(bf16x8, qr[j]), s, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) d += R.qs[g][8 * c + i] * kr[i];
+  for (int r = 0; r < 4; ++r) s[r] = 4 * q + r < nvalid ? s[r] * scale_log2e : -INFINITY;
+  const float m = fmaxf(st.m, quad_rows_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])))), mu = m == -INFINITY ? 0.f : m;
+  const float alpha = st.m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(st.m - mu);
+  float p[4];
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1) d += __shfl_xor(d, o, 16);
-    if (c == 0 && t < T) R.sc[g][t] = t < nvalid ? d * scale_log2e : -INFINITY;
-  }
-  __syncthreads();
-  {   // thread (g = tid >> 4, token = tid & 15): softmax over the 16 lanes of the row, merged into the running partial
-    const int g = tid >> 4, tk = tid & 15;
-    const float s = g < G ? R.sc[g][tk] : -INFINITY;
-    float mt = s;
+  for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(s[r] - mu);      // rows past the end: exp2(-inf) = 0
+  st.m = m; st.l = st.l * alpha + quad_rows_sum((p[0] + p[1]) + (p[2] + p[3]));
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1) mt = fmaxf(mt, __shfl_xor(mt, o, 16));
-    const float m_old = g < G ? m5[g] : -INFINITY, m_new = fmaxf(m_old, mt), mu = m_new == -INFINITY ? 0.f : m_new;
-    const float p = __builtin_amdgcn_exp2f(s - mu);        // rows >= nvalid: exp2(-inf) = 0
-    float lt = p;
+  for (int i = 0; i < 8; ++i) st.acc[i] *= alpha;
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1) lt += __shfl_xor(lt, o, 16);
-    __syncthreads();
-    if (g < G) {
-      R.sc[g][tk] = p;
-      if (tk == 0) {
-        const float al = m_old == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_old - mu);
-        R.alpha[g] = al; m5[g] = m_new; l5[g] = l5[g] * al + lt;
-      }
+  for (int r = 0; r < 4; ++r) {
+    const bool there = 4 * q + r < nvalid;      // rows past the end weigh 0: keep an Inf of the clamped row out of 0 * Inf
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const u32 w = there ? v[r][i] : 0u;
+      st.acc[2 * i] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf16_bits_to_float(w & 0xFFFFu), p[r], st.acc[2 * i], 0, 0, 0);
+      st.acc[2 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(w & 0xFFFF0000u), p[r], st.acc[2 * i + 1], 0, 0, 0);
     }
-  }
-  __syncthreads();
-  const int d2 = 2 * (tid & 63);
-  for (int g = tid >> 6; g < G; g += NT / 64) {
-    const float al = R.alpha[g];
-    float a0 = acc5[g][d2] * al, a1 = acc5[g][d2 + 1] * al;
-#pragma unroll
-    for (int tk = 0; tk < T; ++tk) { const float p = R.sc[g][tk]; a0 += p * bf16_bits_to_float(vv[tk] & 0xFFFFu); a1 += p * bf16_bits_to_float(vv[tk] >> 16); }
-    acc5[g][d2] = a0; acc5[g][d2 + 1] = a1;
   }
 }
-
-// The same for ONE wave and rows in global memory: the raw tail of a cache head is attended by wave 0 of the block that owns the last
-// split, before that wave joins the block's tile hand-out (the other waves pick up the tiles it does not get to).  No block barrier.
-// Lane (t = lane >> 2, c = lane & 3) takes row t, channels 32c .. 32c+31 for the scores; lane owns output dims 2*lane, 2*lane+1.
-__device__ __forceinline__ void wave_rows_attend(float (*__restrict__ sc)[T], const u16* __restrict__ krows, const u16* __restrict__ vrows,
-                                                 int nvalid, const u16* __restrict__ qrows, float scale_log2e, int G, int lane,
-                                                 float* __restrict__ m5, float* __restrict__ l5, float (*__restrict__ acc5)[D]) {
-  const int t = lane >> 2, c = lane & 3;
-  float kr[32];
-  {
-    u32x4 kv[4];
+__device__ __forceinline__ void raw_queries(const u16* qrows, int G, int a, int q, u32x4 (&qr)[4]) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {      // no load under a branch: rows past the end read the last valid row and are zeroed
-      kv[j] = *reinterpret_cast<const u32x4*>(krows + min(t, nvalid - 1) * D + 32 * c + 8 * j);
-      if (t >= nvalid) kv[j] = u32x4{0u, 0u, 0u, 0u};
-    }
+  for (int j = 0; j < 4; ++j) qr[j] = *reinterpret_cast<const u32x4*>(qrows + min(a, G - 1) * D + 32 * j + 8 * q);      // (heads past the last: any valid row)
+}
+// the result as one more partial of the block's merge: m, l [GMAX], acc [GMAX][D]
+__device__ __forceinline__ void raw_rows_store(const RawState& st, int a, int q, float* __restrict__ m, float* __restrict__ l, float (*__restrict__ acc)[D]) {
+  if (q == 0) { m[a] = st.m; l[a] = st.l; }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { kr[8 * j + 2 * i] = bf16_bits_to_float(kv[j][i] & 0xFFFFu); kr[8 * j + 2 * i + 1] = bf16_bits_to_float(kv[j][i] >> 16); }
+  for (int r = 0; r < 4; ++r) {
+    float* o = &acc[a][8 * (4 * q + r)];
+    *reinterpret_cast<f32x4*>(o) = f32x4{st.acc[0][r], st.acc[1][r], st.acc[2][r], st.acc[3][r]};
+    *reinterpret_cast<f32x4*>(o + 4) = f32x4{st.acc[4][r], st.acc[5][r], st.acc[6][r], st.acc[7][r]};
   }
-  for (int g = 0; g < G; ++g) {
-    float d = 0.f;
+}
+// ... and back, for a block that meets further raw rows
+__device__ __forceinline__ void raw_rows_load(RawState& st, int a, int q, const float* __restrict__ m, const float* __restrict__ l, const float (*__restrict__ acc)[D]) {
+  st.m = m[a]; st.l = l[a];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const u32x4 qv = *reinterpret_cast<const u32x4*>(qrows + g * D + 32 * c + 8 * j);
+  for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) d += bf16_bits_to_float(qv[i] & 0xFFFFu) * kr[8 * j + 2 * i] + bf16_bits_to_float(qv[i] >> 16) * kr[8 * j + 2 * i + 1];
-    }
-    d += __shfl_xor(d, 1, 64); d += __shfl_xor(d, 2, 64);
-    if (c == 0) sc[g][t] = t < nvalid ? d * scale_log2e : -INFINITY;
-  }
-  wave_lds_sync();
-  for (int g = lane >> 4; g < G; g += 4) {      // 16 lanes per head: softmax over the row
-    const int tk = lane & 15;
-    const float s = sc[g][tk];
-    float mt = s;
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) mt = fmaxf(mt, __shfl_xor(mt, o, 16));
-    const float p = __builtin_amdgcn_exp2f(s - (mt == -INFINITY ? 0.f : mt));
-    float lt = p;
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) lt += __shfl_xor(lt, o, 16);
-    sc[g][tk] = p;
-    if (tk == 0) { m5[g] = mt; l5[g] = lt; }
-  }
-  wave_lds_sync();
-  u32 vv[T];
-#pragma unroll
-  for (int tk = 0; tk < T; ++tk) vv[tk] = *reinterpret_cast<const u32*>(vrows + min(tk, nvalid - 1) * D + 2 * lane);
-#pragma unroll
-  for (int tk = 0; tk < T; ++tk) vv[tk] = tk < nvalid ? vv[tk] : 0u;      // rows past the end weigh 0: keep an Inf of the clamped row out of 0 * Inf
-  for (int g = 0; g < G; ++g) {
-    float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-    for (int tk = 0; tk < T; ++tk) { const float p = sc[g][tk]; a0 += p * bf16_bits_to_float(vv[tk] & 0xFFFFu); a1 += p * bf16_bits_to_float(vv[tk] >> 16); }
-    acc5[g][2 * lane] = a0; acc5[g][2 * lane + 1] = a1;
-  }
+    for (int r = 0; r < 4; ++r) st.acc[i][r] = st.m == -INFINITY ? 0.f : acc[a][8 * (4 * q + r) + i];      // (none yet: may hold anything)
 }
 
 // ---------------------------------------------------------------------------------------------------- block tables (LDS)
@@ -507,10 +442,10 @@ struct AttnLds {
   u32x4 bwk[2][NG], bwv[2][NG];
   u32x4 qw[GMAX][NG];
 };
-// Block merge: one partial per wave plus one (index NW) for the uncompressed rows.  acc[0..3] double as RawScratch before the waves
-// publish, acc[0..NW-1] as the merge factors afterwards.
+// Block merge: one partial per wave plus one (index NW) for the uncompressed rows.  Before the waves publish, wave 0 keeps the decoded side of a
+// half raw tile in acc[0]; afterwards the mergers' scratch lies in acc.
 template <int NW> struct MergeLds { float m[NW + 1][GMAX], l[NW + 1][GMAX]; float acc[NW + 1][GMAX][D]; };
-static_assert(sizeof(RawScratch) <= 4 * GMAX * D * sizeof(float) && sizeof(MergeScratch<4>) <= 5 * GMAX * D * sizeof(float) &&
+static_assert(T * D * sizeof(u16) <= GMAX * D * sizeof(float) && sizeof(MergeScratch<4>) <= 5 * GMAX * D * sizeof(float) &&
               sizeof(MergeScratch<8>) <= 9 * GMAX * D * sizeof(float), "scratch views must fit the merge buffer");
 struct TableRegs { u32 b0, b1; u32 qlo[4], qhi[4]; };      // one thread's raw inputs of the per-block tables
 // Global loads only, in two parts so that each can be issued as soon as its address is known (the query rows need the batch row, the
@@ -590,7 +525,7 @@ __device__ __forceinline__ void load_tags(const Bases& B, const TileTable& TT, i
   if (PAGED) {
     const int2 e = TT.tt[tile - TT.tlo];
     const int ek = __builtin_amdgcn_readfirstlane(e.x), ev = __builtin_amdgcn_readfirstlane(e.y);
-    Tg.raw = (ek | ev) < 0;                       // a tile with a raw side is skipped here and handled by raw_rows_attend
+    Tg.raw = (ek | ev) < 0;                       // a tile with a raw side is skipped here, see attend_raw_tiles
     Tg.kto = (u32)max(ek, 0); Tg.vto = (u32)max(ev, 0);
     Tg.kfl = reinterpret_cast<const u32*>(B.kov + (size_t)Tg.kto * (size_t)B.TS + SLOT_FL)[a];
     Tg.vfl = reinterpret_cast<const u32*>(B.vov + (size_t)Tg.vto * (size_t)B.TS + SLOT_FL)[a];
@@ -1087,15 +1022,19 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, a = lane & 15, q = lane >> 4;
   Bases B;
   TileTable TT{tile_table, tlo};
+  bool any_raw = false;
   if (PAGED) {
     // logical tile -> block table -> mode table (paged_kernel.py:137-138), resolved once per block into LDS
     B.kov = B.vov = A.pool; B.TS = A.TS;
     B.ksm = B.kcd = B.vsm = B.vcd = nullptr; B.kfl = B.kto = B.vfl = B.vto = nullptr;
+    bool raw = false;
     for (int i = tid; i < thi_fast - tlo; i += NT) {
       const long pc = (long)A.bt[(long)b * A.bt_stride + tlo + i] * (2 * A.n_kv) + 2 * kvh;
-      tile_table[i] = int2{A.mt[pc], A.mt[pc + 1]};
+      const int2 e = {A.mt[pc], A.mt[pc + 1]};
+      tile_table[i] = e;
+      raw |= (e.x | e.y) < 0;
     }
-    __syncthreads();
+    any_raw = __syncthreads_or(raw);
   } else {
     const long rowb = (long)ch * A.S_pad, tileb = (long)ch * (A.S_pad / T);
     // (the escape streams start at head_start[ch], a loaded value: they are set where the first escape bytes are fetched, so that the
@@ -1150,16 +1089,51 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   for (int i = 0; i < 8; ++i) st.acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   st.m_run = -INFINITY; st.mu_run = 0.f; st.l_run = 0.f;
 
-  // ---- the raw tail of the cache head: wave 0 of the last split's block, before it joins the tile hand-out
+  // ---- uncompressed rows, taken by wave 0 before it joins the tile hand-out: the raw tail of the cache head (in the last split's block), or
+  // the raw tiles of the paged pool among the split's tiles
   if (!PAGED && A.kt && split == ns - 1 && wave == 0) {
     const int TL = slot < 0 ? 0 : min(__builtin_amdgcn_readfirstlane(TLh), A.tcap);
     if (TL > 0) {
-      // probabilities go through this wave's own merge slot: the other waves write theirs as soon as they run out of tiles
-      float (*sc)[T] = reinterpret_cast<float (*)[T]>(&M.acc[0][0][0]);
-      wave_rows_attend(sc, A.kt + (long)ch * A.tcap * D, A.vt + (long)ch * A.tcap * D, TL, A.q + qh0 * D, A.scale_log2e, G, lane,
-                       M.m[NW], M.l[NW], M.acc[NW]);
+      u32x4 qr[4];
+      raw_queries(A.q + qh0 * D, G, a, q, qr);
+      RawState rs = {};
+      rs.m = -INFINITY;
+      raw_rows_attend(A.kt + (long)ch * A.tcap * D, A.vt + (long)ch * A.tcap * D, TL, qr, A.scale_log2e, a, q, rs);
+      raw_rows_store(rs, a, q, M.m[NW], M.l[NW], M.acc[NW]);
     }
   }
+  // Paged pool, wave 0: the tiles c0 .. c1 - 1, whose entries the table holds, that have a raw side (the block that is still filling, or
+  // escapes that did not fit the slot).  Raw sides are read in place, the compressed side of a half raw tile is decoded into LDS.
+  const auto attend_raw_tiles = [&](int c0, int c1) {
+    RawState rs;
+    u32x4 qr[4];
+    raw_queries(A.q + qh0 * D, G, a, q, qr);
+    raw_rows_load(rs, a, q, M.m[NW], M.l[NW], M.acc[NW]);
+    u16* decoded = reinterpret_cast<u16*>(&M.acc[0][0][0]);      // (wave 0's own place in the block merge)
+    const long boff = (long)(ch % A.NB) * D;
+    for (int i0 = 0; i0 < c1 - c0; i0 += 64) {
+      const int2 own = tile_table[min(i0 + lane, c1 - c0 - 1)];
+      for (u64 left = __builtin_amdgcn_ballot_w64(i0 + lane < c1 - c0 && (own.x | own.y) < 0); left != 0; left &= left - 1) {
+        const int l = __builtin_ctzll(left), ex = __builtin_amdgcn_readlane(own.x, l), ey = __builtin_amdgcn_readlane(own.y, l);
+        const u16* krows = decoded; const u16* vrows = decoded;
+        wave_lds_sync();
+        if (ex < 0) krows = A.raw + (long)(~ex) * T * D;
+        else {
+          const uint8_t* sl = A.pool + (size_t)ex * (size_t)A.TS;
+          decode_tile_rows<KIND_K>(sl, sl + SLOT_CD, reinterpret_cast<const int*>(sl + SLOT_FL), sl + SLOT_OV, A.k.base3 + boff, A.k.base4 + boff, lane, T, decoded, D);
+        }
+        if (ey < 0) vrows = A.raw + (long)(~ey) * T * D;
+        else {
+          const uint8_t* sl = A.pool + (size_t)ey * (size_t)A.TS;
+          decode_tile_rows<KIND_V>(sl, sl + SLOT_CD, reinterpret_cast<const int*>(sl + SLOT_FL), sl + SLOT_OV, A.v.base3 + boff, A.v.base4 + boff, lane, T, decoded, D);
+        }
+        wave_lds_sync();
+        raw_rows_attend(krows, vrows, min(T, S - (c0 + i0 + l) * T), qr, A.scale_log2e, a, q, rs);
+      }
+    }
+    raw_rows_store(rs, a, q, M.m[NW], M.l[NW], M.acc[NW]);
+  };
+  if (PAGED && any_raw && wave == 0) attend_raw_tiles(tlo, thi_fast);
 
   if (!PAGED) { B.kov = A.k.ovf + __builtin_amdgcn_readfirstlane((int)khs); B.vov = A.v.ovf + __builtin_amdgcn_readfirstlane((int)vhs); }
   if (any_tile) {
@@ -1195,59 +1169,29 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   if (A.dbg && lane == 0) A.dbg[((long)gridDim.x + blockIdx.x) * 8 + wave] = wall_clock64();
 #endif
   // ---- what the pipelined loop left: (1) the partly filled last tile of the sequence; (2) paged pool: a split longer than the LDS tile
-  // table goes on in further rounds of MAX_CHUNK tiles (table refilled); (3) paged pool: tiles whose K or V side is a raw tile (the
-  // block that is still filling, or escapes that did not fit the slot), attended by the whole block round by round, while the table
-  // holds their entries.  Tiles of (1) and (2) are taken by the waves in turn, one at a time without the prefetch pipeline (of the
-  // block's waves some compute while others wait for their tile; both cases are rare), through ONE instantiation of the masking tile
-  // code.
+  // table goes on in further rounds of MAX_CHUNK tiles (table refilled, raw tiles again by wave 0).  Tiles are taken by the waves in turn, one
+  // at a time without the prefetch pipeline (of the block's waves some compute while others wait for their tile; both cases are
+  // rare), through ONE instantiation of the masking tile code.
   if (tlo < thi) {
-    bool raw_started = false;
     for (int c0 = tlo;;) {
       const int c1 = PAGED ? min(c0 + MAX_CHUNK, thi) : thi;
       if (PAGED && c0 != tlo) {
         __syncthreads();      // everybody is done with the previous round's entries
+        bool raw = false;
         for (int i = tid; i < c1 - c0; i += NT) {
           const long pc = (long)A.bt[(long)b * A.bt_stride + c0 + i] * (2 * A.n_kv) + 2 * kvh;
-          tile_table[i] = int2{A.mt[pc], A.mt[pc + 1]};
+          const int2 e = {A.mt[pc], A.mt[pc + 1]};
+          tile_table[i] = e;
+          raw |= (e.x | e.y) < 0;
         }
-        __syncthreads();
+        any_raw = __syncthreads_or(raw);
         TT.tlo = c0;
+        if (any_raw && wave == 0) attend_raw_tiles(c0, c1);
       }
       for (int t = (c0 == tlo ? tlo + n_own : c0) + wave; t < c1; t += NW) {      // first round: only the partial tile is left (wave 0)
         load_tags<PAGED>(B, TT, t, a, Tg);
         load_tile<PAGED>(B, t, lane, Tg, R0);
         if (!PAGED || !Tg.raw) consume<PAGED, true>(R0, st, L, B, Tg.kto, Tg.vto, t, S, A.scale_log2e, a, q, qf);
-      }
-      if (PAGED) {
-        bool mine = false;
-        for (int i = tid; i < c1 - c0; i += NT) mine |= (tile_table[i].x | tile_table[i].y) < 0;
-        if (__syncthreads_or(mine)) {
-          RawScratch& R = *reinterpret_cast<RawScratch*>(&M.acc[0][0][0]);
-          if (!raw_started) {
-            for (int g = tid >> 7; g < G; g += NT / 128) M.acc[NW][g][tid & 127] = 0.f;
-            raw_rows_begin<NT>(R, A, qh0, G, tid);
-            raw_started = true;
-          }
-          const uint8_t* b3k = A.k.base3 + (long)(ch % A.NB) * D; const uint8_t* b4k = A.k.base4 + (long)(ch % A.NB) * D;
-          const uint8_t* b3v = A.v.base3 + (long)(ch % A.NB) * D; const uint8_t* b4v = A.v.base4 + (long)(ch % A.NB) * D;
-          for (int i = 0; i < c1 - c0; ++i) {
-            const int2 e = tile_table[i];
-            if ((e.x | e.y) >= 0) continue;
-            const u16* krows = R.krows; const u16* vrows = R.vrows;
-            if (e.x < 0) krows = A.raw + (long)(~e.x) * T * D;
-            else if (wave == 0) {
-              const uint8_t* sl = A.pool + (size_t)e.x * (size_t)A.TS;
-              decode_tile_rows<KIND_K>(sl, sl + SLOT_CD, reinterpret_cast<const int*>(sl + SLOT_FL), sl + SLOT_OV, b3k, b4k, lane, T, R.krows, D);
-            }
-            if (e.y < 0) vrows = A.raw + (long)(~e.y) * T * D;
-            else if (wave == 1) {
-              const uint8_t* sl = A.pool + (size_t)e.y * (size_t)A.TS;
-              decode_tile_rows<KIND_V>(sl, sl + SLOT_CD, reinterpret_cast<const int*>(sl + SLOT_FL), sl + SLOT_OV, b3v, b4v, lane, T, R.vrows, D);
-            }
-            raw_rows_attend<NT>(R, krows, vrows, min(T, S - (c0 + i) * T), A.scale_log2e, G, tid, M.m[NW], M.l[NW], M.acc[NW]);
-            __syncthreads();      // staging rows are free again
-          }
-        }
       }
       c0 = c1;
       if (c0 >= thi) break;
