@@ -118,7 +118,8 @@ int gaac_attn_combine(const float* pm, const float* pl, const float* pa, void* o
  * they are ordered on one stream.  The fp32 partial buffers of gaac_attn_split / gaac_attn_launch must be other memory than these
  * records (plain values could be taken for records of some epoch).
  * S_all >= 0: every cache head the launch addresses holds exactly S_all compressed tokens (a Page: lengths are known to the host);
- * SL is then not read and may be NULL, which takes one dependent load off the start of every block.  S_all < 0: lengths come from SL. */
+ * SL is then not read and may be NULL, which takes one dependent load off the start of every block, and nsplit is an upper bound: no split
+ * gets fewer than four tiles or none.  S_all < 0: lengths come from SL. */
 int gaac_attn_fused(
     const uint8_t* smk, const uint8_t* ck, const int* fk, const int* tok, const uint8_t* ovk, const int* ohsk, const uint8_t* b3k, const uint8_t* b4k,
     const uint8_t* smv, const uint8_t* cv, const int* fv, const int* tov, const uint8_t* ovv, const int* ohsv, const uint8_t* b3v, const uint8_t* b4v,
