@@ -137,7 +137,8 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // LDS of a merging block: per wave the (m, then weight) and l of every slot.
 template <int NW> struct MergeScratch { float f[NW][MAX_SLOTS], l[NW][MAX_SLOTS]; };
 
-// One merger's work for half a query head (64 output channels), shared by the NW waves of the block.  A wave owns 64 / NW channels
+// One merger's work for half a query head (64 output channels), shared by NW waves (of the block, or half the block's: see merge_heads), of which
+// this is the wave-th; fs, ls: its own part of the scratch.  A wave owns 64 / NW channels
 // and sums them over ALL slots, so the waves exchange nothing and no block barrier lies between the records' arrival and the
 // output: lane (g, c) = (lane / CPW, lane % CPW) reads the accumulator records of channel c of the wave for the slots g, g + SG, ...
 // (SG = 64 / CPW slot groups); the groups' sums meet through DPP.  Every wave reads the m / l records of all slots (lane = slot)
@@ -146,14 +147,13 @@ __device__ __forceinline__ void merge_failed(const AttnArgs& A, u32 bit) {
   __hip_atomic_fetch_or(A.epochs + 1, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <int NW>
-__device__ __forceinline__ void merge_half_head(const AttnArgs& A, long rec, int nslot, long row, int half, u32 epoch, MergeScratch<NW>& X, int wave, int lane) {
+__device__ __forceinline__ void merge_half_head(const AttnArgs& A, long rec, int nslot, long row, int half, u32 epoch, float* fs, float* ls, int wave, int lane) {
   constexpr int CPW = 64 / NW, SG = 64 / CPW;      // channels per wave (8 | 16), slot groups (8 | 4)
   constexpr int CH = 8;                             // accumulator records in flight per lane: one round for up to CH * SG splits
   const int g = lane / CPW, d = 64 * half + CPW * wave + lane % CPW;
   const u64* rm = reinterpret_cast<const u64*>(A.pm) + rec;
   const u64* rl = reinterpret_cast<const u64*>(A.pl) + rec;
   const u64* ra = reinterpret_cast<const u64*>(A.pa) + rec * D + d;
-  float* fs = X.f[wave]; float* ls = X.l[wave];
   bool ok = true;
   // all loads of the first round are issued before the first use, none under a branch (a slot past the end reads the last slot
   // instead and is ignored): the lane's first CH accumulator records ...
@@ -355,10 +355,15 @@ __device__ __forceinline__ void merge_heads(const AttnArgs& A, long qh0, int G, 
         if (nslot <= 8) merge_half_head_wave<8>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, lane);
         else merge_half_head_wave<WAVE_MERGE_SLOTS>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, lane);
       }
+    } else if (NW == 8 && 2 * G > mergers) {
+      // more half heads than mergers (nine query heads and up): the block's halves take one each.  One after the other they were two trips to
+      // memory: 1 kv head of 16 query heads, 2000 tokens in 32 splits 11.7 -> 9.9 us, 6000 in 64 12.2 -> 11.6, slot cache 790 in 25 12.5 -> 10.8
+      const int item = rank + mergers * (wave >> 2);
+      if (item < 2 * G) merge_half_head<4>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, X.f[wave], X.l[wave], wave & 3, lane);
     } else {
       int item = rank;
-      if (item < 2 * G) { merge_half_head<NW>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, X, wave, lane); item += mergers; }
-      for (; item < 2 * G; item += mergers) merge_half_head<NW>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, X, wave, lane);
+      if (item < 2 * G) { merge_half_head<NW>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, X.f[wave], X.l[wave], wave, lane); item += mergers; }
+      for (; item < 2 * G; item += mergers) merge_half_head<NW>(A, rec0 + (long)(item >> 1) * nslot, nslot, qh0 + (item >> 1), item & 1, epoch, X.f[wave], X.l[wave], wave, lane);
     }
   }
   if (last) advance_epoch<NW>(A, epoch, tid, xm, &X.l[0][0], MAX_SLOTS);

@@ -22,3 +22,20 @@ def test_splits_of_a_known_length(S, B, n_kv, G):
     for nsplit in (1, 2, 5, 31, 100, 2):
         got = O.bf16_to_f32(to_u16(attention(to_bf16(q16, dev), kp, vp, SCALE, nsplit=nsplit)))
         assert np.abs(got - ref).max() <= 2e-2 * np.abs(ref).max() + 1e-3, nsplit      # the bound of test_attention_matches_reference
+
+
+@pytest.mark.parametrize("n_kv,G", [(1, 16), (2, 9), (1, 8)])
+@pytest.mark.parametrize("L", [37, 1100])      # with empty splits, without
+def test_more_half_heads_than_mergers(n_kv, G, L):
+    """Nine query heads and up: the halves of an eight-wave block take a half head each, up to 32 splits in one round of records, then in more."""
+    from gaac_amd import CompressedKVCache
+    dev = require_gpu()
+    cache = CompressedKVCache(1, n_kv, 1200, None, device=dev)
+    k, v, q = randn_bf16((L, n_kv, 128), seed=31), randn_bf16((L, n_kv, 128), seed=32), randn_bf16((1, n_kv * G, 128), seed=33)
+    cache.prefill(0, to_bf16(k, dev), to_bf16(v, dev))
+    ref, tol = attention_error_bound(q[0], k, v, SCALE)
+    slots = torch.zeros(1, dtype=torch.int32, device=dev)
+    for nsplit in (15, 16, 17, 31, 32, 33, 63, 64, 65, 128, 300, 17):      # 300: four-wave blocks
+        got = O.bf16_to_f32(to_u16(cache.attention(to_bf16(q, dev), slots, SCALE, nsplit=nsplit)))[0]
+        assert (np.abs(got - ref) <= tol).all(), nsplit
+    cache.check_capacity()
