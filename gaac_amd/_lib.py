@@ -1,16 +1,18 @@
-"""ctypes binding of gaac_amd/libgaac_hip.so (see include/gaac_hip.h).  There is no fallback: if the library is
-missing, or a call is made without a GPU, the call raises."""
+"""gaac_amd/libgaac_hip.so (see include/gaac_hip.h): calls() has its entry points as functions that take tensors (gaac_amd/_binding.so), load()
+is the library for ctypes.  There is no fallback: if one of the two is missing, or a call is made without a GPU, the call raises."""
 from __future__ import annotations
 import ctypes, os
 import torch
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libgaac_hip.so")
 _lib = None
+_calls = None
 
 c_int, c_long, c_float, c_void_p = ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_void_p
 P = c_void_p
 
 _SIGNATURES = {
+    "gaac_wait_host": [P, P],
     "gaac_exponent_hist": [P, c_long, c_int, P, P],
     "gaac_bases_from_hist": [P, c_int, P, P, P],
     "gaac_encode_tiles": [c_int, P, c_long, c_long, c_int, c_int, c_int, P, P, c_int, P, P, P, P, P, P, P],
@@ -62,6 +64,21 @@ def load():
     return _lib
 
 
+def calls():
+    """The entry points as functions, in the order of arguments of include/gaac_hip.h: tensors on the device, addresses or None for pointers,
+    numbers, last the stream (its handle, or the function `stream`).  They raise RuntimeError with the library's message."""
+    global _calls
+    if _calls is None:
+        load()
+        try:
+            from . import _binding
+        except ImportError as e:
+            raise RuntimeError(f"gaac_amd/_binding.so is missing or does not fit the installed torch ({e}): build it with `python -m gaac_amd.build`") from e
+        _binding.bind(lib_path())
+        _calls = _binding
+    return _calls
+
+
 def exported_symbols() -> list[str]:
     return ["gaac_last_error", *_SIGNATURES]
 
@@ -81,7 +98,4 @@ def stream() -> int:
 
 
 def call(name: str, *args):
-    lib = load()
-    rc = getattr(lib, name)(*args)
-    if rc != 0:
-        raise RuntimeError(f"{name} failed ({rc}): {lib.gaac_last_error().decode(errors='replace')}")
+    getattr(_calls or calls(), name)(*args)

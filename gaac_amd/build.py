@@ -1,6 +1,7 @@
-"""Builds gaac_amd/libgaac_hip.so (hand-written HIP kernels for gfx950 + the extern "C" entry points) with hipcc.
+"""Builds gaac_amd/libgaac_hip.so (hand-written HIP kernels for gfx950 + the extern "C" entry points) with hipcc, and gaac_amd/_binding.so (the
+Python calls of these entry points) with g++.
 
-    python -m gaac_amd.build          # or: from gaac_amd.build import build; build()
+    python -m gaac_amd.build          # or: from gaac_amd.build import build, build_binding; build(); build_binding()
 
 The library is built in-tree; nothing is compiled at import time or on the GPU box."""
 from __future__ import annotations
@@ -11,6 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgaac_hip.so")
 LIB_W12 = os.path.join(HERE, "libgaac_hip_w12.so")            # measurement build -DGAAC_WAVES12: twelve-wave blocks, three waves per SIMD (see attn.hip); on demand only
 LIB_TIMING = os.path.join(HERE, "libgaac_hip_timing.so")      # same sources with -DGAAC_PHASE_TIMING (per-block phase time stamps); built on demand only
+BINDING = os.path.join(HERE, "_binding.so")
 SOURCES = ["codec.hip", "attn.hip", "cache.hip", "paged.hip"]
 # bench.py's measurement aids (read probe, plain copy): their own library next to bench.py, not in the product library
 BENCH_SRC = os.path.join(os.path.dirname(HERE), "bench_kernels.hip")
@@ -51,6 +53,22 @@ def build(verbose: bool = True, extra_flags: list[str] | None = None, timing: bo
     return out
 
 
+def build_binding(verbose: bool = True) -> str:
+    """csrc/binding.cpp -> gaac_amd/_binding.so, the Python calls of the library (host code, with the C++ headers of the installed torch)."""
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{d}" for d in [*include_paths(), sysconfig.get_paths()["include"]]), os.path.join(CSRC, "binding.cpp"), "-o", BINDING,
+           "-L" + libs, "-Wl,-rpath," + libs, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-ldl"]
+    if verbose: print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed on binding.cpp:\n" + r.stderr)
+    return BINDING
+
+
 def build_bench_lib(verbose: bool = True) -> str:
     """bench_kernels.hip -> libgaac_bench.so (beside bench.py)."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -62,9 +80,10 @@ def build_bench_lib(verbose: bool = True) -> str:
     return BENCH_LIB
 
 
-if __name__ == "__main__":      # no option: the library and bench.py's kernels; --timing / --waves12: only that measurement build
+if __name__ == "__main__":      # no option: the library, its Python calls and bench.py's kernels; --timing / --waves12: only that measurement build
     if "--timing" in sys.argv: print(build(timing=True))
     if "--waves12" in sys.argv: print(build(waves12=True))
     if "--timing" not in sys.argv and "--waves12" not in sys.argv:
         print(build())
+        print(build_binding())
         print(build_bench_lib())

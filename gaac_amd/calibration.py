@@ -16,7 +16,7 @@ class BaseCollector:
 
     def _add(self, hist: torch.Tensor, x: torch.Tensor, n_kv: int):
         x = x.contiguous()
-        _lib.call("gaac_exponent_hist", _lib.ptr(x), x.numel() // (n_kv * D), n_kv, _lib.ptr(hist), _lib.stream())
+        _lib.call("gaac_exponent_hist", x, x.numel() // (n_kv * D), n_kv, hist, _lib.stream)
 
     def observe(self, layer: int, k: torch.Tensor, v: torch.Tensor):
         """k, v: [N, n_kv, D] bf16 of one prefill step."""

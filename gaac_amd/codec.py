@@ -68,7 +68,7 @@ def exponent_hist(x: torch.Tensor, n_kv: int) -> torch.Tensor:
     """Counts of the 8-bit exponent per (kv head, channel): x bf16 [..., n_kv, D] -> int64 [n_kv*D, 256] (the quantity of codec.py:80-84)."""
     x = x.contiguous()
     hist = torch.zeros(n_kv * D, 256, dtype=torch.int64, device=x.device)
-    _lib.call("gaac_exponent_hist", _lib.ptr(x), x.numel() // (n_kv * D), n_kv, _lib.ptr(hist), _lib.stream())
+    _lib.call("gaac_exponent_hist", x, x.numel() // (n_kv * D), n_kv, hist, _lib.stream)
     return hist
 
 
@@ -78,7 +78,7 @@ def bases_from_hist(hist: torch.Tensor, n_kv: int) -> tuple[torch.Tensor, torch.
     hist = hist.to(torch.int64).contiguous()
     b3 = torch.empty(n_kv, D, dtype=torch.uint8, device=hist.device)
     b4 = torch.empty(n_kv, D, dtype=torch.uint8, device=hist.device)
-    _lib.call("gaac_bases_from_hist", _lib.ptr(hist), n_kv * D, _lib.ptr(b3), _lib.ptr(b4), _lib.stream())
+    _lib.call("gaac_bases_from_hist", hist, n_kv * D, b3, b4, _lib.stream)
     return b3, b4
 
 
@@ -121,7 +121,7 @@ def row_offsets(flags: torch.Tensor, S: int) -> torch.Tensor:
     out = torch.empty(H, S, dtype=torch.int32, device=flags.device)
     if S:
         sums = torch.empty(H * ((S + 2047) // 2048), dtype=torch.int32, device=flags.device)
-        _lib.call("gaac_row_offsets", _lib.ptr(flags), H, S, S_pad, _lib.ptr(sums), _lib.ptr(out), _lib.stream())
+        _lib.call("gaac_row_offsets", flags, H, S, S_pad, sums, out, _lib.stream)
     return out
 
 
@@ -159,19 +159,20 @@ def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Te
     S_pad = (S + T - 1) // T * T
     nt = H * (S_pad // T)
     new = lambda *shape, dtype=torch.uint8: torch.empty(shape, dtype=dtype, device=dev)
-    sm, cd = new(H, S_pad * D), new(H, S_pad * CB)
+    st = _lib.stream
+    # each buffer is made when the next launch needs it, the last ones while the device is at work
+    sm, cd, flags = new(H, S_pad * D), new(H, S_pad * CB), new(H, S_pad, dtype=torch.int32)
     slots = scratch(nt * TILE_MAX_ESC, dev) if scratch else new(nt * TILE_MAX_ESC)
-    flags, ovf_off, tile_off = new(H, S_pad, dtype=torch.int32), new(H, S, dtype=torch.int32), new(H, S_pad // T, dtype=torch.int32)
-    head_start, sizes = new(H + 1, dtype=torch.int32), new(nt + H, dtype=torch.int32)      # sizes: per tile, then per head
-    totals = torch.empty(H, dtype=torch.int32, pin_memory=True)
-    p, st = _lib.ptr, _lib.stream()
-    tile_bytes, head_bytes = p(sizes), p(sizes) + 4 * nt
-    _lib.call("gaac_encode_tiles", 0 if kind == "k" else 1, p(x), hs, rs, H, S, S_pad, p(base3), p(base4), n_kv, None,
-              p(sm), p(cd), p(flags), p(slots), tile_bytes, st)
-    _lib.call("gaac_tile_scan", tile_bytes, H, S_pad // T, p(tile_off), head_bytes, totals.data_ptr(), st)
-    torch.cuda.current_stream(dev).synchronize()
+    sizes = new(nt + H, dtype=torch.int32)      # per tile, then per head
+    head_bytes = sizes.data_ptr() + 4 * nt
+    _lib.call("gaac_encode_tiles", 0 if kind == "k" else 1, x, hs, rs, H, S, S_pad, base3, base4, n_kv, None,
+              sm, cd, flags, slots, sizes, st)
+    totals, tile_off = torch.empty(H, dtype=torch.int32, pin_memory=True), new(H, S_pad // T, dtype=torch.int32)
+    _lib.call("gaac_tile_scan", sizes, H, S_pad // T, tile_off, head_bytes, totals.data_ptr(), st)
+    ovf_off, head_start = new(H, S, dtype=torch.int32), new(H + 1, dtype=torch.int32)
+    _lib.call("gaac_wait_host", totals.data_ptr(), st)
     ovf = new(stream_bytes(totals.tolist()) + 8)
-    _lib.call("gaac_page_pack", p(slots), tile_bytes, p(tile_off), head_bytes, p(flags), H, S, S_pad, p(head_start), p(ovf), p(ovf_off), st)
+    _lib.call("gaac_page_pack", slots, sizes, tile_off, head_bytes, flags, H, S, S_pad, head_start, ovf, ovf_off, st)
     return Page(sm, cd, flags, ovf_off, ovf, head_start, tile_off, base3, base4, H, S, n_kv, kind)
 
 
@@ -205,7 +206,7 @@ class Codec:
         S_pad = page.sm.shape[1] // D
         out = torch.empty(H, S, D, dtype=torch.bfloat16, device=page.sm.device)
         if S:
-            _lib.call("gaac_decode_tiles", 0 if page.kind == "k" else 1, _lib.ptr(page.sm), _lib.ptr(page.codes), _lib.ptr(page.flags),
-                      _lib.ptr(page.tile_off), _lib.ptr(page.ovf), _lib.ptr(page.ovf_head_start), _lib.ptr(page.base3), _lib.ptr(page.base4),
-                      page.n_kv, None, H, S, S_pad, _lib.ptr(out), S * D, D, _lib.stream())
+            _lib.call("gaac_decode_tiles", 0 if page.kind == "k" else 1, page.sm, page.codes, page.flags,
+                      page.tile_off, page.ovf, page.ovf_head_start, page.base3, page.base4,
+                      page.n_kv, None, H, S, S_pad, out, S * D, D, _lib.stream)
         return out

@@ -434,6 +434,12 @@ extern "C" {
 
 const char* gaac_last_error(void) { return last_error_buffer(); }
 
+int gaac_wait_host(const void* host, void* stream) {
+  GAAC_REQUIRE(host, "gaac_wait_host: null pointer");
+  const hipError_t e = hipStreamSynchronize((hipStream_t)stream);
+  return e == hipSuccess ? 0 : gaac::fail("gaac_wait_host: %s", hipGetErrorString(e));
+}
+
 int gaac_exponent_hist(const void* x, long n_tokens, int n_kv, long long* hist, void* stream) {
   GAAC_REQUIRE(x && hist && n_kv > 0 && n_tokens >= 0, "gaac_exponent_hist: bad arguments");
   if (n_tokens == 0) return 0;

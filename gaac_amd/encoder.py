@@ -44,16 +44,16 @@ class TileEncoder:
         x, hs, rs = rows_in_place(x, 0, 1)
         slots = self._scratch(H * ntiles * SLOT, dev)
         tile_bytes = torch.empty(H, ntiles, dtype=torch.int32, device=dev)
-        _lib.call("gaac_encode_tiles", 0 if self.kind == "k" else 1, _lib.ptr(x), hs, rs, H, S, S_pad, _lib.ptr(base3), _lib.ptr(base4),
-                  n_kv, _lib.ptr(bidx), _lib.ptr(sm), _lib.ptr(cd), _lib.ptr(flags), _lib.ptr(slots), _lib.ptr(tile_bytes), _lib.stream())
+        _lib.call("gaac_encode_tiles", 0 if self.kind == "k" else 1, x, hs, rs, H, S, S_pad, base3, base4,
+                  n_kv, bidx, sm, cd, flags, slots, tile_bytes, _lib.stream)
         return tile_bytes
 
     def compact(self, tile_bytes, head_start, ovf) -> torch.Tensor:
         """Pack the scratch slots into ovf at head_start[h] + tile_off[h, t]; returns tile_off int32 [H, ntiles]."""
         H, ntiles = tile_bytes.shape
         tile_off = torch.empty_like(tile_bytes)
-        _lib.call("gaac_compact", _lib.ptr(self._slots), _lib.ptr(tile_bytes), _lib.ptr(tile_off), _lib.ptr(head_start), _lib.ptr(ovf),
-                  H, ntiles, _lib.stream())
+        _lib.call("gaac_compact", self._slots, tile_bytes, tile_off, head_start, ovf,
+                  H, ntiles, _lib.stream)
         return tile_off
 
     def encode(self, codec: Codec, x: torch.Tensor) -> Page:

@@ -34,12 +34,10 @@ class _Ext:
         has_tail = kt.numel() > 0
         out = torch.empty(B * n_q, D, dtype=q.dtype, device=q.device)
         ws = shared_workspace(B * n_q, nsplit, q.dtype, q.device)
-        p = _lib.ptr
-        _lib.call("gaac_attn_fused", p(smk), p(ck), p(fk), p(tok), p(ovk), p(ohsk), p(b3k), p(b4k),
-                  p(smv), p(cv), p(fv), p(tov), p(ovv), p(ohsv), p(b3v), p(b4v),
-                  p(q), p(slot), B, n_q, n_kv, p(SL), int(S_pad), float(scale), int(nsplit), b3k.shape[0],
-                  p(kt) if has_tail else None, p(vt) if has_tail else None, p(TL) if has_tail else None, int(TCAP) if has_tail else 0,
-                  -1, p(ws.pm), p(ws.pl), p(ws.pa), p(ws.epoch), p(out), _lib.stream())
+        _lib.call("gaac_attn_fused", smk, ck, fk, tok, ovk, ohsk, b3k, b4k, smv, cv, fv, tov, ovv, ohsv, b3v, b4v,
+                  q, slot, B, n_q, n_kv, SL, int(S_pad), float(scale), int(nsplit), b3k.shape[0],
+                  kt if has_tail else None, vt if has_tail else None, TL if has_tail else None, int(TCAP) if has_tail else 0,
+                  -1, ws.pm, ws.pl, ws.pa, ws.epoch, out, _lib.stream)
         return out
 
 
@@ -111,10 +109,11 @@ class AttnWorkspace:
         """Host read of the failure word (synchronizes with the device)."""
         return int(self.epoch[1])
 
-    def check(self):
+    def check(self, bits: int | None = None):
         """Raises if a one-kernel launch on this workspace gave up a wait since the last reset() (its output rows are NaN, or the
-        epoch stands still); poll it where the engine polls its other device-side error words."""
-        bits = self.failure_bits()
+        epoch stands still); poll it where the engine polls its other device-side error words.  bits: failure_bits() if the
+        caller fetched them already."""
+        if bits is None: bits = self.failure_bits()
         if bits:
             raise RuntimeError("fused decode attention gave up waiting for" + (" a split's partial (rows written as NaN)" if bits & 1 else "") +
                                (" the other blocks of the launch (epoch not advanced)" if bits & 2 else "") +
@@ -150,14 +149,13 @@ def shared_workspace(rows: int, nslot: int, dtype, dev) -> AttnWorkspace:
 
 
 def _store_args(st):
-    p = _lib.ptr
     hs = st.head_start if hasattr(st, "head_start") else st.ovf_head_start
-    return (p(st.sm), p(st.codes), p(st.flags), p(st.tile_off), p(st.ovf), p(hs), p(st.base3), p(st.base4))
+    return st.sm, st.codes, st.flags, st.tile_off, st.ovf, hs, st.base3, st.base4
 
 
-def attn_launch(K, V, q2d, slots, n_q, n_kv, SL, S_pad, scale, nsplit, kt=None, vt=None, TL=None, TCAP=0, ws=None, phase="fused", S_all=-1):
+def attn_launch(K, V, q2d, slots, n_q, n_kv, SL, S_pad, scale, nsplit, kt=None, vt=None, TL=None, TCAP=0, ws=None, phase="fused", S_all=-1, out=None):
     """K, V: objects with sm, codes, flags, tile_off, ovf, head_start|ovf_head_start, base3, base4 (a Page or a cache store).
-    q2d: [B*n_q, D] bf16 contiguous.  Returns [B*n_q, D] bf16.  phase: "fused" (one kernel, one block of each
+    q2d: [B*n_q, D] or [B, n_q, D] bf16 contiguous.  Returns out, or if none is given [B*n_q, D] bf16.  phase: "fused" (one kernel, one block of each
     kv head merges) | "both" (split kernel then merge kernel) | "split" | "combine" (the halves of "both").
     S_all >= 0: every addressed head holds exactly S_all compressed tokens (SL is not read by the one-kernel launch)."""
     G = n_q // max(1, n_kv)
@@ -165,29 +163,28 @@ def attn_launch(K, V, q2d, slots, n_q, n_kv, SL, S_pad, scale, nsplit, kt=None, 
         raise RuntimeError(f"GQA group size must be 1..{GMAX}")
     if q2d.shape[-1] != D:
         raise RuntimeError("head_dim must be 128")
-    B = slots.shape[0] if slots is not None else q2d.shape[0] // n_q      # slots=None: row b attends over cache heads b*n_kv ..
+    B = slots.shape[0] if slots is not None else q2d.numel() // (n_q * D)      # slots=None: row b attends over cache heads b*n_kv ..
     has_tail = kt is not None and kt.numel() > 0
     nslot = nsplit        # the raw tail is folded into the last split's partial
     if ws is None:
         ws = shared_workspace(B * n_q, nslot, q2d.dtype, q2d.device)
     elif ws.rows != B * n_q or ws.nslot != nslot:
         raise RuntimeError("attention workspace does not match the launch shape")
-    p = _lib.ptr
-    out = ws.out if ws.out is not None else torch.empty(B * n_q, D, dtype=q2d.dtype, device=q2d.device)
+    if out is None: out = ws.out if ws.out is not None else torch.empty(B * n_q, D, dtype=q2d.dtype, device=q2d.device)
     if phase == "combine":
         pm, pl, pa = ws.f32_partials()
-        _lib.call("gaac_attn_combine", p(pm), p(pl), p(pa), p(out), B * n_q, nslot, _lib.stream())
+        _lib.call("gaac_attn_combine", pm, pl, pa, out, B * n_q, nslot, _lib.stream)
         return out
-    args = (*_store_args(K), *_store_args(V), p(q2d), p(slots), B, n_q, n_kv, p(SL), S_pad, float(scale), nsplit, K.base3.shape[0],
-            p(kt) if has_tail else None, p(vt) if has_tail else None, p(TL) if has_tail else None, TCAP if has_tail else 0)
+    args = (*_store_args(K), *_store_args(V), q2d, slots, B, n_q, n_kv, SL, S_pad, float(scale), nsplit, K.base3.shape[0],
+            kt if has_tail else None, vt if has_tail else None, TL if has_tail else None, TCAP if has_tail else 0)
     if phase == "fused":
-        _lib.call("gaac_attn_fused", *args, int(S_all), p(ws.pm), p(ws.pl), p(ws.pa), p(ws.epoch), p(out), _lib.stream())
+        _lib.call("gaac_attn_fused", *args, int(S_all), ws.pm, ws.pl, ws.pa, ws.epoch, out, _lib.stream)
         return out
-    args = (*args, *(p(t) for t in ws.f32_partials()))
+    args = (*args, *ws.f32_partials())
     if phase == "split":
-        _lib.call("gaac_attn_split", *args, _lib.stream())
+        _lib.call("gaac_attn_split", *args, _lib.stream)
     else:
-        _lib.call("gaac_attn_launch", *args, p(out), _lib.stream())
+        _lib.call("gaac_attn_launch", *args, out, _lib.stream)
     return out
 
 
@@ -199,9 +196,9 @@ def attention(q, kp, vp, scale=None, nsplit=None, phase="fused"):
     if nsplit is None: nsplit = launch_nsplit(B, n_kv, kp.S, ragged=False)
     # the one-kernel launch takes the length as an argument; the other phases read one per head
     SL = None if phase == "fused" else torch.full((kp.H,), kp.S, dtype=torch.int32, device=q.device)
-    out = attn_launch(kp, vp, q.reshape(B * n_q, Dq).contiguous(), None, n_q, n_kv, SL, kp.sm.shape[1] // D,
-                      scale if scale is not None else Dq ** -0.5, nsplit, phase=phase, S_all=kp.S)
-    return out.view(B, n_q, Dq)
+    out = torch.empty(B, n_q, Dq, dtype=q.dtype, device=q.device)
+    return attn_launch(kp, vp, q.contiguous(), None, n_q, n_kv, SL, kp.sm.shape[1] // D,
+                       scale if scale is not None else Dq ** -0.5, nsplit, phase=phase, S_all=kp.S, out=out)
 
 
 def bf16_attention(q, k, v, scale=None, nsplit=None, ws=None, seq_lens=None, out=None):
@@ -216,7 +213,6 @@ def bf16_attention(q, k, v, scale=None, nsplit=None, ws=None, seq_lens=None, out
     if ws is None: ws = shared_workspace(B * n_q, nsplit, q.dtype, q.device)
     elif ws.rows != B * n_q or ws.nslot != nsplit: raise RuntimeError("attention workspace does not match the launch shape")
     if out is None: out = ws.out if ws.out is not None else torch.empty(B * n_q, D, dtype=q.dtype, device=q.device)
-    p = _lib.ptr
-    _lib.call("gaac_bf16_attn", p(k), p(v), S, p(seq_lens), k.stride(0) // D, p(q.contiguous()), B, n_q, n_kv,
-              float(scale if scale is not None else Dq ** -0.5), nsplit, p(ws.pm), p(ws.pl), p(ws.pa), p(ws.epoch), p(out), _lib.stream())
+    _lib.call("gaac_bf16_attn", k, v, S, seq_lens, k.stride(0) // D, q.contiguous(), B, n_q, n_kv,
+              float(scale if scale is not None else Dq ** -0.5), nsplit, ws.pm, ws.pl, ws.pa, ws.epoch, out, _lib.stream)
     return out.view(B, n_q, Dq)

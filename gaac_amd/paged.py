@@ -69,14 +69,11 @@ class LayerState:
     def bases(self):
         return (self.b3k, self.b4k, self.b3v, self.b4v)
 
-    def _base_ptrs(self):
-        return tuple(_lib.ptr(t) for t in self.bases)
-
     def _flush_free(self):
         if self._pending_free is not None:
             freeq, n = self._pending_free
             self._pending_free = None
-            _lib.call("gaac_paged_free", _lib.ptr(freeq), n, _lib.ptr(self.stack), _lib.ptr(self.top), _lib.stream())
+            _lib.call("gaac_paged_free", freeq, n, self.stack, self.top, _lib.stream)
 
     def store(self, key: torch.Tensor, value: torch.Tensor, buf: torch.Tensor, ent: torch.Tensor, freeq: torch.Tensor | None = None,
               defer_free: bool = False):
@@ -91,9 +88,8 @@ class LayerState:
             raise RuntimeError("store expects K/V rows of n_kv*128 contiguous elements")
         n = E * 2 * self.n_kv
         if freeq is None: freeq = torch.empty(n, dtype=torch.int32, device=buf.device)
-        p = _lib.ptr
-        _lib.call("gaac_paged_store", p(key), p(value), key.stride(0), value.stride(0), p(ent), E, p(buf), self.TS, p(self.raw), p(self.mt),
-                  p(self.stack), p(self.top), p(self.err), p(freeq), *self._base_ptrs(), self.n_kv, _lib.stream())
+        _lib.call("gaac_paged_store", key, value, key.stride(0), value.stride(0), ent, E, buf, self.TS, self.raw, self.mt,
+                  self.stack, self.top, self.err, freeq, *self.bases, self.n_kv, _lib.stream)
         self._pending_free = (freeq, n)
         if not defer_free: self._flush_free()
 
@@ -103,17 +99,14 @@ class LayerState:
         if P == 0: return
         if sk.stride(0) != sv.stride(0) or sk.stride(0) < self.n_kv * D:
             raise RuntimeError("decode_blocks expects K/V scratch rows of at least n_kv*128 elements and equal strides")
-        p = _lib.ptr
-        _lib.call("gaac_paged_decode", p(buf), self.TS, p(self.raw), p(self.mt), p(pairs), P, p(sk), p(sv), sk.stride(0),
-                  *self._base_ptrs(), self.n_kv, _lib.stream())
+        _lib.call("gaac_paged_decode", buf, self.TS, self.raw, self.mt, pairs, P, sk, sv, sk.stride(0), *self.bases, self.n_kv, _lib.stream)
 
     def release_blocks(self, blocks: torch.Tensor):
         """blocks: int32 [F] block ids whose content is dead."""
         F = blocks.shape[0]
         if F == 0: return
         self._flush_free()
-        p = _lib.ptr
-        _lib.call("gaac_paged_release", p(blocks), F, p(self.mt), p(self.stack), p(self.top), self.n_kv, _lib.stream())
+        _lib.call("gaac_paged_release", blocks, F, self.mt, self.stack, self.top, self.n_kv, _lib.stream)
 
     def check(self):
         """Host poll (every 16 steps in the reference, backend.py:233-236): raises when the raw side pool ran dry."""
@@ -145,10 +138,7 @@ def paged_attention(q, out, buf, raw, mt, bt, seq_lens, bases, TS, n_q, n_kv, ns
     if max_seq_len is None: max_seq_len = bt.shape[1] * BLOCK
     if ws is None: ws = shared_workspace(B * n_q, nsplit, q.dtype, q.device)
     elif ws.rows != B * n_q or ws.nslot != nsplit: raise RuntimeError("attention workspace does not match the launch shape")
-    p = _lib.ptr
-    q = q.contiguous()
-    _lib.call("gaac_paged_attn", p(buf), TS, p(raw), p(mt), p(bt), bt.stride(0), p(seq_lens), int(max_seq_len), p(q), B, n_q, n_kv,
-              float(1.0 / (D ** 0.5)), nsplit, p(bases[0]), p(bases[1]), p(bases[2]), p(bases[3]), bases[0].shape[0],
-              p(ws.pm), p(ws.pl), p(ws.pa), p(ws.epoch), p(out),
-              *((p(free[0]), int(free[1]), p(free[2]), p(free[3])) if free is not None else (None, 0, None, None)), _lib.stream())
+    _lib.call("gaac_paged_attn", buf, TS, raw, mt, bt, bt.stride(0), seq_lens, int(max_seq_len), q.contiguous(), B, n_q, n_kv,
+              float(1.0 / (D ** 0.5)), nsplit, *bases, bases[0].shape[0], ws.pm, ws.pl, ws.pa, ws.epoch, out,
+              *((free[0], int(free[1]), free[2], free[3]) if free is not None else (None, 0, None, None)), _lib.stream)
     return out

@@ -23,6 +23,9 @@ extern "C" {
 
 const char* gaac_last_error(void);
 
+/* Waits until the stream has done what was enqueued on it, and with that written host (memory of the host that a launch fills, such as host_bytes below). */
+int gaac_wait_host(const void* host, void* stream);
+
 /* exponent_hist(x, n_kv), /root/reference/gaac/codec.py:80-84.  x: bf16 [n_tokens, n_kv, 128] token-major;
  * hist: int64 [n_kv*128, 256], ACCUMULATED into (zero it first). */
 int gaac_exponent_hist(const void* x, long n_tokens, int n_kv, long long* hist, void* stream);
