@@ -13,12 +13,14 @@ P = c_void_p
 
 _SIGNATURES = {
     "gaac_wait_host": [P, P],
+    "gaac_wait_words": [P, c_int, P],
     "gaac_exponent_hist": [P, c_long, c_int, P, P],
     "gaac_bases_from_hist": [P, c_int, P, P, P],
     "gaac_encode_tiles": [c_int, P, c_long, c_long, c_int, c_int, c_int, P, P, c_int, P, P, P, P, P, P, P],
     "gaac_compact": [P, P, P, P, P, c_int, c_int, P],
     "gaac_tile_scan": [P, c_int, c_int, P, P, P, P],
     "gaac_page_pack": [P, P, P, P, P, c_int, c_int, c_int, P, P, P, P],
+    "gaac_page_finish": [P, P, P, c_int, c_int, c_int, P, P, P, P, P, c_long, P, P],
     "gaac_row_offsets": [P, c_int, c_int, c_int, P, P, P],
     "gaac_decode_tiles": [c_int, P, P, P, P, P, P, P, P, c_int, P, c_int, c_int, c_int, P, c_long, c_long, P],
     "gaac_cache_prefill": [P, P] + [c_long] * 4 + [c_int] * 7 + [P] * 27,

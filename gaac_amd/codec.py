@@ -148,11 +148,16 @@ def stream_bytes(totals: list[int]) -> int:
     return total
 
 
+STREAM_ROOM = 3      # bytes per row that a page's escape stream is given ahead of its size: measured rows have 1.9, of 182 in all
+
+
 def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Tensor, n_kv: int, scratch=None) -> Page:
-    """Encode x (bf16 [H, S, D], on the GPU) with the given bases.  Three launches: every tile is encoded with its escapes in a worst-case
-    slot; the sizes of the slots are scanned per head; then, with the stream sized by the host (the totals arrive in host memory that
-    the scan writes to), the slots are packed head by head and the row offsets written (the steps of encoder.py:111-123).
-    scratch(n, device): where the slots' n bytes come from, if not from torch's allocator."""
+    """Encode x (bf16 [H, S, D], on the GPU) with the given bases.  Every tile is encoded with its escapes in a worst-case slot; then the
+    sizes of the slots are scanned per head, the slots packed head by head and the row offsets written (the steps of encoder.py:111-123),
+    without the host in between: the stream goes into a buffer with room for STREAM_ROOM bytes a row, which the page keeps a view of, and the
+    heads' totals, which arrive in host memory while the slots are packed, say whether it was enough.  Longer streams (those of more than 15 %
+    four-bit or 2.5 % raw groups, about) are packed again, into a buffer of their size.
+    scratch(n, device): where the n bytes of slots and sizes come from, if not from torch's allocator."""
     H, S, _ = x.shape
     dev = x.device
     x, hs, rs = rows_in_place(x, 0, 1)
@@ -160,19 +165,26 @@ def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Te
     nt = H * (S_pad // T)
     new = lambda *shape, dtype=torch.uint8: torch.empty(shape, dtype=dtype, device=dev)
     st = _lib.stream
-    # each buffer is made when the next launch needs it, the last ones while the device is at work
+    # each buffer is made when the next launch needs it
     sm, cd, flags = new(H, S_pad * D), new(H, S_pad * CB), new(H, S_pad, dtype=torch.int32)
-    slots = scratch(nt * TILE_MAX_ESC, dev) if scratch else new(nt * TILE_MAX_ESC)
-    sizes = new(nt + H, dtype=torch.int32)      # per tile, then per head
-    head_bytes = sizes.data_ptr() + 4 * nt
+    # slots | sizes per tile | per head
+    n_slots = nt * TILE_MAX_ESC
+    slots = scratch(n_slots + 4 * (nt + H), dev) if scratch else new(n_slots + 4 * (nt + H))
+    sizes = slots.data_ptr() + n_slots
+    head_bytes = sizes + 4 * nt
     _lib.call("gaac_encode_tiles", 0 if kind == "k" else 1, x, hs, rs, H, S, S_pad, base3, base4, n_kv, None,
               sm, cd, flags, slots, sizes, st)
     totals, tile_off = torch.empty(H, dtype=torch.int32, pin_memory=True), new(H, S_pad // T, dtype=torch.int32)
-    _lib.call("gaac_tile_scan", sizes, H, S_pad // T, tile_off, head_bytes, totals.data_ptr(), st)
     ovf_off, head_start = new(H, S, dtype=torch.int32), new(H + 1, dtype=torch.int32)
-    _lib.call("gaac_wait_host", totals.data_ptr(), st)
-    ovf = new(stream_bytes(totals.tolist()) + 8)
-    _lib.call("gaac_page_pack", slots, sizes, tile_off, head_bytes, flags, H, S, S_pad, head_start, ovf, ovf_off, st)
+    room = STREAM_ROOM * H * S + 8
+    ovf = new(room)
+    _lib.call("gaac_page_finish", slots, sizes, flags, H, S, S_pad, tile_off, head_bytes, totals.data_ptr(), head_start, ovf, room, ovf_off, st)
+    _lib.call("gaac_wait_words", totals.data_ptr(), H, st)
+    n = stream_bytes(totals.tolist()) + 8
+    if n <= room: ovf = ovf[:n]
+    else:
+        ovf = new(n)
+        _lib.call("gaac_page_pack", slots, sizes, tile_off, head_bytes, flags, H, S, S_pad, head_start, ovf, ovf_off, st)
     return Page(sm, cd, flags, ovf_off, ovf, head_start, tile_off, base3, base4, H, S, n_kv, kind)
 
 

@@ -4,6 +4,7 @@
 //   row_offsets                       /root/reference/gaac/codec.py:221-225
 //   decode_tiles                      /root/reference/gaac/codec.py:186-218
 #include <algorithm>
+#include <chrono>
 #include "gaac_tile.h"
 #include "gaac_capi.h"
 #include "../../include/gaac_hip.h"
@@ -246,6 +247,8 @@ __device__ __forceinline__ int scan_tile_bytes(const int* __restrict__ tb, int* 
   }
   return carry;
 }
+// A word of host memory that the host polls (gaac_wait_words): there before the kernel ends.
+__device__ __forceinline__ void store_to_host(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM); }
 // Tile offsets and escape totals of the heads, one block per head.  host_bytes (or null): the totals once more in host memory that the
 // device can write, for the caller that sizes the stream: it spares a copy and its latency.
 __global__ void __launch_bounds__(SCAN_NT) k_tile_scan(const int* __restrict__ tile_bytes, int* __restrict__ tile_off, int ntiles,
@@ -255,7 +258,7 @@ __global__ void __launch_bounds__(SCAN_NT) k_tile_scan(const int* __restrict__ t
   const int total = scan_tile_bytes(tile_bytes + h * ntiles, tile_off + h * ntiles, ntiles, threadIdx.x, sh);
   if (threadIdx.x == 0) {
     if (head_bytes) head_bytes[h] = total;
-    if (host_bytes) host_bytes[h] = total;
+    if (host_bytes) store_to_host(host_bytes + h, total);
   }
 }
 
@@ -263,7 +266,7 @@ __global__ void __launch_bounds__(SCAN_NT) k_tile_scan(const int* __restrict__ t
 // offsets of its tiles in one load each, then the first 64 bytes of all 16 slots in flight together (a tile has about 30 escape bytes;
 // what is beyond 64 follows in a loop).  A wave that copied its tiles one after the other, each a chain of size -> bytes -> store, took
 // 20.7 us for the 8 x 4096 tiles of a 64K-token page; this one takes 6.6 us and writes the row offsets as well (9.2 us of their own before).
-// HEADS: the streams lie back to back and the block derives its head's start from the totals of the heads before it (a Page; it also
+// HEADS: the streams lie back to back and the block derives its head's start from the totals of the heads (a Page; it also
 // writes head_start, the row offsets and the stream's padding); else head_start is given and a head whose window is too small is left out.
 constexpr int PACK_TPB = 64;
 struct PackKind { const uint8_t* slots; const int* tile_bytes; const int* tile_off; long off_stride; const int* head_start; uint8_t* ovf; };
@@ -271,6 +274,7 @@ struct PackArgs {
   PackKind j[2]; int ntiles;
   const int* head_bytes;                 // [kinds * H] totals (null without HEADS: every window is large enough)
   int window;                            // bytes that a head's stream must fit in (without HEADS)
+  long ovf_cap;                          // bytes there are for all streams and the padding: where they are too few, none is written (HEADS)
   const int* flags; int S, S_pad; int* head_start_out; int* ovf_off;      // HEADS
 };
 template <bool HEADS>
@@ -285,20 +289,22 @@ __global__ void __launch_bounds__(256) k_pack(const PackArgs A) {
 #pragma unroll
   for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, A.ntiles - 1) * TILE_MAX_ESC + lane];
   long start = 0;
+  bool fits = true;
   if (HEADS) {
-    __shared__ int part[4];
-    int before = 0;
-    for (int i = tid; i < h; i += 256) before += A.head_bytes[i];
+    __shared__ long part[2][4];
+    long before = 0, all = 0;
+    for (int i = tid; i < H; i += 256) { const int n = A.head_bytes[i]; all += n; before += i < h ? n : 0; }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
-    if (lane == 0) part[wave] = before;
+    for (int o = 32; o > 0; o >>= 1) { before += __shfl_xor(before, o, 64); all += __shfl_xor(all, o, 64); }
+    if (lane == 0) { part[0][wave] = before; part[1][wave] = all; }
     __syncthreads();
-    start = part[0] + part[1] + part[2] + part[3];
+    start = (part[0][0] + part[0][1]) + (part[0][2] + part[0][3]); all = (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]);
+    fits = all < 0x7FFFFFFF && all + 8 <= A.ovf_cap;      // (a head's total stops at 2^31 - 1)
     if (blockIdx.x == 0 && tid == 0) {
       A.head_start_out[h] = (int)start;
-      if (h == H - 1) A.head_start_out[H] = (int)start + A.head_bytes[h];
+      if (h == H - 1) A.head_start_out[H] = (int)all;
     }
-    if (blockIdx.x == 0 && h == H - 1 && tid < 8) J.ovf[start + A.head_bytes[h] + tid] = 0;      // readers fetch eight bytes at a time
+    if (fits && blockIdx.x == 0 && h == H - 1 && tid < 8) J.ovf[all + tid] = 0;      // readers fetch eight bytes at a time
   } else {
     if (A.head_bytes && A.head_bytes[(long)blockIdx.z * H + h] > A.window) return;
     start = J.head_start[h];
@@ -307,7 +313,7 @@ __global__ void __launch_bounds__(256) k_pack(const PackArgs A) {
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
     const int n = __builtin_amdgcn_readlane(nb, k), o = __builtin_amdgcn_readlane(of, k);
-    if (k >= n_own) break;
+    if (k >= n_own || !fits) break;
     if (lane < n) dst[o + lane] = (uint8_t)v[k];
     for (int i = 64 + lane; i < n; i += 64) dst[o + i] = src[(long)(t0 + k) * TILE_MAX_ESC + i];
   }
@@ -320,6 +326,78 @@ __global__ void __launch_bounds__(256) k_pack(const PackArgs A) {
       const int to = __shfl(of, 4 * k + (lane >> 4), 64);
       if (i < A.S && n_own > 0) A.ovf_off[(long)h * A.S + i] = to + (int)(incl - rb);
     }
+  }
+}
+
+// k_tile_scan and k_pack<HEADS> in one launch, for pages of up to PAGE_PACK_TILES tiles over all heads: a block of 64 tiles adds up the sizes of all
+// tiles, of the heads before its own and of the tiles before its own by itself (PER loads a thread in flight, from the L2).  Latency, like the two.
+// In a graph, us, one launch against two: 2048 tiles 5.4 / 7.9, 8192 6.1 / 8.0, 16384 7.6 / 8.1, 32768 13.7 / 8.7 (every block reads every size).
+// It and the two others are launched without a look at the totals by the host, which sees them while the slots are packed:
+// 8 x 4096 tokens encoded and expanded again 45.2 -> 37.9 us a call, 8 x 65536 100.0 -> 90.4.
+constexpr int PAGE_PACK_TILES = 16384;
+struct PagePackArgs {
+  const uint8_t* slots; const int* tile_bytes; int* tile_off; int* head_bytes; int* host_bytes; int ntiles;
+  const int* flags; int S, S_pad; int* head_start; uint8_t* ovf; long ovf_cap; int* ovf_off;
+};
+__global__ void __launch_bounds__(256) k_page_pack(const PagePackArgs A) {
+  constexpr int PER = 16;
+  __shared__ u32x4 part[4];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = blockIdx.y, H = gridDim.y, ntiles = A.ntiles;
+  const int tile0 = blockIdx.x * PACK_TPB, t0 = tile0 + 16 * wave, n_own = min(16, ntiles - t0);      // (n_own may be <= 0)
+  const int head0 = h * ntiles, own0 = head0 + tile0, all_tiles = H * ntiles;
+  // every load up front, none under a branch
+  const uint8_t* src = A.slots + (long)head0 * TILE_MAX_ESC;
+  int n = A.tile_bytes[head0 + min(tile0 + lane, ntiles - 1)];
+  u32 v[16], fl[4];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, ntiles - 1) * TILE_MAX_ESC + lane];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) fl[k] = (u32)A.flags[(long)h * A.S_pad + min(t0 * T + 64 * k + lane, A.S_pad - 1)];
+  int all = 0, heads = 0, before = 0, mine = 0;      // of all tiles, of the heads before, of the head's tiles before the block's, of the head
+  for (int base = 0; base < all_tiles; base += 256 * PER) {
+    int w[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) w[k] = A.tile_bytes[min(base + 256 * k + tid, all_tiles - 1)];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int i = base + 256 * k + tid, x = i < all_tiles ? w[k] : 0;
+      all += x; heads += i < head0 ? x : 0; before += i >= head0 && i < own0 ? x : 0; mine += i >= head0 && i < head0 + ntiles ? x : 0;
+    }
+  }
+  u64 s0 = (u64)(u32)all | ((u64)(u32)heads << 32), s1 = (u64)(u32)before | ((u64)(u32)mine << 32);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) { s0 += __shfl_xor(s0, o, 64); s1 += __shfl_xor(s1, o, 64); }
+  if (lane == 0) part[wave] = u32x4{(u32)s0, (u32)(s0 >> 32), (u32)s1, (u32)(s1 >> 32)};
+  __syncthreads();
+  const u32x4 sums = (part[0] + part[1]) + (part[2] + part[3]);
+  all = (int)sums[0]; heads = (int)sums[1]; before = (int)sums[2]; mine = (int)sums[3];
+  const bool fits = (long)all + 8 <= A.ovf_cap;
+  if (blockIdx.x == 0 && tid == 0) {
+    if (A.host_bytes) store_to_host(A.host_bytes + h, mine);
+    A.head_bytes[h] = mine; A.head_start[h] = heads;
+    if (h == H - 1) A.head_start[H] = all;
+  }
+  if (fits && blockIdx.x == 0 && h == H - 1 && tid < 8) A.ovf[all + tid] = 0;      // readers fetch eight bytes at a time
+  // lane: a tile of the block
+  n = tile0 + lane < ntiles ? n : 0;
+  const int x = (int)row_scan16((u32)n), r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31), r2 = __builtin_amdgcn_readlane(x, 47);
+  const int of = before + x + (lane >= 16 ? r0 : 0) + (lane >= 32 ? r1 : 0) + (lane >= 48 ? r2 : 0) - n;
+  if (wave == 0 && tile0 + lane < ntiles) A.tile_off[head0 + tile0 + lane] = of;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {      // row offsets: tile offset + the escape bytes of the tile's earlier tag words
+    const int i = t0 * T + 64 * k + lane;
+    const u32 rb = (u32)esc_bytes(fl[k]), incl = row_scan16(rb);
+    const int to = __shfl(of, 16 * wave + 4 * k + (lane >> 4), 64);
+    if (i < A.S && n_own > 0) A.ovf_off[(long)h * A.S + i] = to + (int)(incl - rb);
+  }
+  if (!fits) return;
+  uint8_t* dst = A.ovf + heads;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int nk = __builtin_amdgcn_readlane(n, 16 * wave + k), o = __builtin_amdgcn_readlane(of, 16 * wave + k);
+    if (k >= n_own) break;
+    if (lane < nk) dst[o + lane] = (uint8_t)v[k];
+    for (int i = 64 + lane; i < nk; i += 64) dst[o + i] = src[(long)(t0 + k) * TILE_MAX_ESC + i];
   }
 }
 
@@ -508,6 +586,22 @@ int gaac_wait_host(const void* host, void* stream) {
   return e == hipSuccess ? 0 : gaac::fail("gaac_wait_host: %s", hipGetErrorString(e));
 }
 
+int gaac_wait_words(const int* words, int n, void* stream) {
+  GAAC_REQUIRE(words && n > 0, "gaac_wait_words: bad arguments");
+  const auto there = [&] {
+    for (int i = 0; i < n; ++i) if (__atomic_load_n(words + i, __ATOMIC_ACQUIRE) < 0) return false;
+    return true;
+  };
+  const auto give_up = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+  do {
+    for (int spin = 0; spin < 64; ++spin) if (there()) return 0;
+  } while (std::chrono::steady_clock::now() < give_up);
+  const hipError_t e = hipStreamSynchronize((hipStream_t)stream);      // a busy stream, or one that failed
+  if (e != hipSuccess) return gaac::fail("gaac_wait_words: %s", hipGetErrorString(e));
+  GAAC_REQUIRE(there(), "gaac_wait_words: the stream is done and has not written all words");
+  return 0;
+}
+
 int gaac_exponent_hist(const void* x, long n_tokens, int n_kv, long long* hist, void* stream) {
   GAAC_REQUIRE(x && hist && n_kv > 0 && n_tokens >= 0, "gaac_exponent_hist: bad arguments");
   if (n_tokens == 0) return 0;
@@ -552,9 +646,31 @@ int gaac_page_pack(const uint8_t* esc_slots, const int* tile_bytes, const int* t
   PackArgs A{};
   A.ntiles = (S + T - 1) / T;
   A.j[0] = PackKind{esc_slots, tile_bytes, tile_off, A.ntiles, nullptr, ovf};
-  A.head_bytes = head_bytes; A.flags = flags; A.S = S; A.S_pad = S_pad; A.head_start_out = head_start; A.ovf_off = ovf_off;
+  A.head_bytes = head_bytes; A.flags = flags; A.S = S; A.S_pad = S_pad; A.head_start_out = head_start; A.ovf_off = ovf_off; A.ovf_cap = 0x7FFFFFFFL + 8;
   hipLaunchKernelGGL(k_pack<true>, dim3((A.ntiles + PACK_TPB - 1) / PACK_TPB, H), dim3(256), 0, (hipStream_t)stream, A);
   return launch_status("gaac_page_pack");
+}
+
+int gaac_page_finish(const uint8_t* esc_slots, const int* tile_bytes, const int* flags, int H, int S, int S_pad, int* tile_off, int* head_bytes,
+                     int* host_bytes, int* head_start, uint8_t* ovf, long ovf_cap, int* ovf_off, void* stream) {
+  GAAC_REQUIRE(esc_slots && tile_bytes && tile_off && head_bytes && host_bytes && flags && head_start && ovf && ovf_off, "gaac_page_finish: null pointer");
+  GAAC_REQUIRE(H > 0 && S > 0 && S_pad >= (S + T - 1) / T * T && S_pad % T == 0 && ovf_cap >= 8, "gaac_page_finish: bad sizes H=%d S=%d S_pad=%d ovf_cap=%ld", H, S, S_pad, ovf_cap);
+  hipStream_t st = (hipStream_t)stream;
+  const int ntiles = (S + T - 1) / T;
+  const dim3 grid((ntiles + PACK_TPB - 1) / PACK_TPB, H);
+  for (int h = 0; h < H; ++h) __atomic_store_n(host_bytes + h, -1, __ATOMIC_RELAXED);      // not there yet
+  if ((long)H * ntiles <= PAGE_PACK_TILES) {
+    const PagePackArgs A{esc_slots, tile_bytes, tile_off, head_bytes, host_bytes, ntiles, flags, S, S_pad, head_start, ovf, ovf_cap, ovf_off};
+    hipLaunchKernelGGL(k_page_pack, grid, dim3(256), 0, st, A);
+  } else {
+    hipLaunchKernelGGL(k_tile_scan, dim3(H), dim3(SCAN_NT), 0, st, tile_bytes, tile_off, ntiles, head_bytes, host_bytes);
+    PackArgs A{};
+    A.ntiles = ntiles;
+    A.j[0] = PackKind{esc_slots, tile_bytes, tile_off, ntiles, nullptr, ovf};
+    A.head_bytes = head_bytes; A.flags = flags; A.S = S; A.S_pad = S_pad; A.head_start_out = head_start; A.ovf_off = ovf_off; A.ovf_cap = ovf_cap;
+    hipLaunchKernelGGL(k_pack<true>, grid, dim3(256), 0, st, A);
+  }
+  return launch_status("gaac_page_finish");
 }
 
 int gaac_compact(const uint8_t* esc_slots, const int* tile_bytes, int* tile_off, const int* head_start, uint8_t* ovf,

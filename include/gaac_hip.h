@@ -26,6 +26,10 @@ const char* gaac_last_error(void);
 /* Waits until the stream has done what was enqueued on it, and with that written host (memory of the host that a launch fills, such as host_bytes below). */
 int gaac_wait_host(const void* host, void* stream);
 
+/* Waits until none of the n words is negative: host memory that a launch on the stream fills (gaac_page_finish's host_bytes), possibly ahead of the
+ * stream's later work, which is not waited for. */
+int gaac_wait_words(const int* words, int n, void* stream);
+
 /* exponent_hist(x, n_kv), /root/reference/gaac/codec.py:80-84.  x: bf16 [n_tokens, n_kv, 128] token-major;
  * hist: int64 [n_kv*128, 256], ACCUMULATED into (zero it first). */
 int gaac_exponent_hist(const void* x, long n_tokens, int n_kv, long long* hist, void* stream);
@@ -57,6 +61,11 @@ int gaac_compact(const uint8_t* esc_slots, const int* tile_bytes, int* tile_off,
 int gaac_tile_scan(const int* tile_bytes, int H, int ntiles, int* tile_off, int* head_bytes, int* host_bytes, void* stream);
 int gaac_page_pack(const uint8_t* esc_slots, const int* tile_bytes, const int* tile_off, const int* head_bytes, const int* flags, int H, int S, int S_pad,
                    int* head_start, uint8_t* ovf, int* ovf_off, void* stream);
+/* gaac_page_finish: both steps at once into a stream of ovf_cap bytes, which may turn out too small (sum of head_bytes + 8 > ovf_cap): then everything
+ * but ovf is written, and gaac_page_pack with a larger one completes the page.  host_bytes [H]: host memory that the device can write, set to -1 by the call
+ * and to the totals when the stream has come that far (gaac_wait_words). */
+int gaac_page_finish(const uint8_t* esc_slots, const int* tile_bytes, const int* flags, int H, int S, int S_pad, int* tile_off, int* head_bytes,
+                     int* host_bytes, int* head_start, uint8_t* ovf, long ovf_cap, int* ovf_off, void* stream);
 
 /* row_offsets(flags, S), /root/reference/gaac/codec.py:221-225.  flags: int32 [H, S_pad]; out: int32 [H, S];
  * chunk_sums: scratch, int32 [H * ceil(S / 2048)] (escape bytes per chunk of 2048 rows; written, then read). */
