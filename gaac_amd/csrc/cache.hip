@@ -74,6 +74,28 @@ __global__ void __launch_bounds__(128) k_cache_append(const AppendArgs A) {
   }
 }
 
+// What check_capacity looks at, gathered in host memory by one launch: the failure words of up to CHECK_WORDS attention workspaces, the append's overflow
+// bits and the largest escape count of the heads.  Through torch (two maxima, their maximum, a concatenation, a copy and its wait) it took 36 us, now 10.
+constexpr int CHECK_WORDS = 32;
+struct CheckArgs { const u32* failed[CHECK_WORDS]; int n; const int* overflow; const int* used[2]; int H; int* host; };      // host [n + 2]; used null: host [n + 1]
+__global__ void __launch_bounds__(1024) k_cache_check(const CheckArgs A) {
+  __shared__ int part[16];
+  const int tid = threadIdx.x;
+  if (tid < A.n) store_to_host(A.host + tid, (int)__hip_atomic_load(A.failed[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  if (A.overflow && tid == 0) store_to_host(A.host + A.n, *A.overflow);
+  if (!A.used[0]) return;
+  int most = 0;
+  for (int i = tid; i < A.H; i += 1024) most = max(most, max(A.used[0][i], A.used[1][i]));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
+  if ((tid & 63) == 0) part[tid >> 6] = most;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < 16; ++w) most = max(most, part[w]);
+    store_to_host(A.host + A.n + 1, most);
+  }
+}
+
 }  // namespace gaac
 
 using namespace gaac;
@@ -94,4 +116,21 @@ extern "C" int gaac_cache_append(
   A.cap = cap; A.ovf_cap = ovf_cap; A.n_kv = n_kv; A.NB = NB; A.err = err;
   hipLaunchKernelGGL(k_cache_append, dim3(B * n_kv), dim3(128), 0, (hipStream_t)stream, A);
   return launch_status("gaac_cache_append");
+}
+
+extern "C" int gaac_cache_check(const unsigned long long* epochs, int n_epochs, const int* err, const int* k_ovf_used, const int* v_ovf_used, int H, int* host,
+                                void* stream) {
+  GAAC_REQUIRE((epochs || n_epochs == 0) && n_epochs >= 0 && err && host, "gaac_cache_check: bad arguments");
+  GAAC_REQUIRE(!k_ovf_used == !v_ovf_used && (!k_ovf_used || H > 0), "gaac_cache_check: escape counters of K and V, or none");
+  for (int i = 0; i < n_epochs + 1 + (k_ovf_used ? 1 : 0); ++i) __atomic_store_n(host + i, -1, __ATOMIC_RELAXED);      // not there yet
+  for (int at = 0; at == 0 || at < n_epochs; at += CHECK_WORDS) {
+    CheckArgs A{};
+    const bool last = at + CHECK_WORDS >= n_epochs;      // takes the other words along
+    A.n = last ? n_epochs - at : CHECK_WORDS;
+    for (int i = 0; i < A.n; ++i) A.failed[i] = reinterpret_cast<const u32*>(static_cast<uintptr_t>(epochs[at + i])) + 1;
+    if (last) { A.overflow = err; A.used[0] = k_ovf_used; A.used[1] = v_ovf_used; A.H = H; }
+    A.host = host + at;
+    hipLaunchKernelGGL(k_cache_check, dim3(1), dim3(A.used[0] ? 1024 : 64), 0, (hipStream_t)stream, A);
+  }
+  return launch_status("gaac_cache_check");
 }

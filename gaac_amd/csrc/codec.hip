@@ -247,8 +247,6 @@ __device__ __forceinline__ int scan_tile_bytes(const int* __restrict__ tb, int* 
   }
   return carry;
 }
-// A word of host memory that the host polls (gaac_wait_words): there before the kernel ends.
-__device__ __forceinline__ void store_to_host(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM); }
 // Tile offsets and escape totals of the heads, one block per head.  host_bytes (or null): the totals once more in host memory that the
 // device can write, for the caller that sizes the stream: it spares a copy and its latency.
 __global__ void __launch_bounds__(SCAN_NT) k_tile_scan(const int* __restrict__ tile_bytes, int* __restrict__ tile_off, int ntiles,

@@ -48,6 +48,9 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// A word of host memory that the host polls (gaac_wait_words): there before the kernel ends.
+__device__ __forceinline__ void store_to_host(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM); }
+
 // The encoder works on 32-bit words that hold elements i and i+4 of a unit in their 16-bit halves (the decoder's word order), two
 // elements per VALU operation.
 struct BaseRegs { u32 b3[4][4], b4[4][4]; };      // [unit][i]: base of element i | base of element i+4 << 16

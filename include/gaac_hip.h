@@ -173,6 +173,12 @@ int gaac_cache_append(
     void* v_tail, const uint8_t* v_base3, const uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
     int* err, void* stream);
 
+/* What CompressedKVCache.check_capacity looks at (/root/reference/gaac/kv_cache.py:198-203): host [n_epochs + 2] (host memory that the device can write, set
+ * to -1 by the call; gaac_wait_words) = the failure words of the epoch buffers of gaac_attn_fused whose addresses epochs holds (host memory), *err of
+ * gaac_cache_append, and the largest of the H ovf_used of K and of V (left out, as is its word, where both are NULL). */
+int gaac_cache_check(const unsigned long long* epochs, int n_epochs, const int* err, const int* k_ovf_used, const int* v_ovf_used, int H, int* host,
+                     void* stream);
+
 /* ---- paged slot pool (the layout of /root/reference/gaac/vllm/paged_kernel.py:3-6 and store.py:17-19) -------------------------------
  * pool: tile slots of TS bytes, physical tile p = block*2*n_kv + 2*kvh + kind: [0,2048) sign/mantissa | [2048,2816) codes |
  * [2816,2880) 16 tag words | [2880,TS) escape bytes.  mt int32 [num_blocks*2*n_kv]: p = compressed in its slot, ~r = raw BF16 tile r of
