@@ -12,7 +12,6 @@ c_int, c_long, c_float, c_void_p = ctypes.c_int, ctypes.c_long, ctypes.c_float, 
 P = c_void_p
 
 _SIGNATURES = {
-    "gaac_wait_host": [P, P],
     "gaac_wait_words": [P, c_int, P],
     "gaac_exponent_hist": [P, c_long, c_int, P, P],
     "gaac_bases_from_hist": [P, c_int, P, P, P],

@@ -91,7 +91,7 @@ PyObject* invoke(const char* name, int (*fn)(A...), PyObject* const* args, Py_ss
 }
 
 #define GAAC_ENTRY_POINTS(X)                                                                                                              \
-  X(gaac_wait_host) X(gaac_wait_words) X(gaac_page_finish) X(gaac_cache_check)                                                            \
+  X(gaac_wait_words) X(gaac_page_finish) X(gaac_cache_check)                                                                              \
   X(gaac_exponent_hist) X(gaac_bases_from_hist) X(gaac_encode_tiles) X(gaac_compact) X(gaac_tile_scan) X(gaac_page_pack)                  \
   X(gaac_row_offsets) X(gaac_decode_tiles) X(gaac_cache_prefill) X(gaac_attn_split) X(gaac_attn_combine) X(gaac_cache_append)             \
   X(gaac_paged_store) X(gaac_paged_free) X(gaac_paged_release) X(gaac_paged_decode) X(gaac_paged_attn) X(gaac_bf16_attn)                  \

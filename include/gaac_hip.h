@@ -23,11 +23,8 @@ extern "C" {
 
 const char* gaac_last_error(void);
 
-/* Waits until the stream has done what was enqueued on it, and with that written host (memory of the host that a launch fills, such as host_bytes below). */
-int gaac_wait_host(const void* host, void* stream);
-
-/* Waits until none of the n words is negative: host memory that a launch on the stream fills (gaac_page_finish's host_bytes), possibly ahead of the
- * stream's later work, which is not waited for. */
+/* Waits until none of the n words is negative: host memory that a launch on the stream fills (host_bytes of gaac_page_finish and gaac_cache_prefill).
+ * Later work of the stream is not waited for. */
 int gaac_wait_words(const int* words, int n, void* stream);
 
 /* exponent_hist(x, n_kv), /root/reference/gaac/codec.py:80-84.  x: bf16 [n_tokens, n_kv, 128] token-major;
@@ -84,7 +81,7 @@ int gaac_decode_tiles(int kind, const uint8_t* sm, const uint8_t* codes, const i
  * head_start[head]).  Scratch: hist uint64 [2*n_kv*256*64] (calibrate only), esc_slots [2*n_kv*(L/16)*1280], tile_bytes
  * int32 [2*n_kv*(L/16)], head_bytes int32 [2*n_kv].  head_bytes and host_bytes (or NULL; host memory the device can write) receive the
  * heads' escape totals, K's first: a head whose total + 1288 exceeds ovf_cap is left EMPTY (S = tail_len = 0), and the caller repeats
- * the call with larger windows. */
+ * the call with larger windows.  host_bytes is set to -1 by the call and to the totals when all of the prompt is in place (gaac_wait_words). */
 int gaac_cache_prefill(
     const void* k, const void* v, long k_head_stride, long k_row_stride, long v_head_stride, long v_row_stride, int L, int n_kv, int head0,
     int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
