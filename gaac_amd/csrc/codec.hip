@@ -14,17 +14,19 @@ namespace gaac {
 char* last_error_buffer() { static thread_local char buf[512] = {0}; return buf; }
 
 // ---------------------------------------------------------------------------------------------------- calibration
-// Exponent histogram per (kv head, channel).  A block owns the 128 channels of one kv head of K or of V and a chunk of tokens.  Lane l of
-// every wave reads channels 2l and 2l+1 of a row (one 256-byte row per wave-wide load) and counts in a table of 256 x 64 words that the
-// block's waves share: word (bin, l) holds the counts of the two channels in its 16-bit halves (a chunk has at most 65535 tokens), so a
-// lane only ever touches bank l and the LDS adds of a wave never collide, however alike the exponents are.  A table of one word per
-// (channel, bin) with eight lanes to a row (16-byte loads) sent all rows of a wave to the same few words of a channel: 61 to 66 us
-// for the K and the V of 32768 tokens x 8 kv heads (134 MB, two launches); this one 35.5 us where the rows come from HBM (3.8 TB/s), 23.6
-// where the Infinity Cache still holds them (5.7 TB/s).
+// Exponent histogram per (kv head, channel).  A block owns the 128 channels of one kv head of K or of V and a chunk of tokens.  A lane
+// of every wave counts two adjacent channels of a row in a table of 256 x 64 words that the block's waves share: word (bin, lane) holds the counts of
+// the two in its 16-bit halves (a chunk has at most 65535 tokens), so a lane only ever touches its own bank and the LDS adds of a wave never collide,
+// however alike the exponents are.  (A table of one word per (channel, bin) with eight lanes to a row sent all rows of a wave to the same
+// few words of a channel and took twice as long.)  A load takes four rows, 16 bytes a lane; sixteen lanes of a row each hold four words, and two lane
+// exchanges give every lane one word of all four rows.
+// Bound by the reads (without counting at all: 29 us with the launch).  K and V of 32768 tokens x 8 kv heads, 134 MB: 27.3 us = 4.9 TB/s; eight waves that read
+// 4 bytes a lane, sixteen rows at a time, 28.4 with whole batches and 33 with the rest of a chunk row by row: a prompt of 30011 tokens 90.2 us a call
+// -> 86.6, of 12345 62.7 -> 57.3, of 4000 44.2 -> 40.3, of 32768 91.3 -> 90.4.  More loads in flight are slower: 28.2 with three, 27.9 with eight.
 // Non-zero counts are added to the global histogram at the end: PACKED = false: 64-bit counts hist[row][256], the layout that
 // gaac_exponent_hist hands out; PACKED = true: scratch[pair][bin][64] with the two 32-bit counts of a lane in one 64-bit word, so that a
 // wave's adds of a bin are one contiguous 512-byte access (prompts of up to 2^32 - 1 tokens).
-constexpr int HIST_WAVES = 8, HIST_MAX_CHUNK = 65535, HIST_ROWS = 16;      // HIST_ROWS: rows in flight per wave
+constexpr int HIST_WAVES = 16, HIST_MAX_CHUNK = 65535, HIST_LOADS = 2;      // HIST_LOADS: loads of four rows in flight per wave
 struct HistArgs { const u16* x[2]; long head_stride[2], row_stride[2]; long n_tok; int chunk, n_kv; unsigned long long* hist; };
 template <bool PACKED>
 __global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArgs A) {
@@ -32,31 +34,50 @@ __global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArg
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, head = blockIdx.y, kind = blockIdx.z;
   const long t0 = (long)blockIdx.x * A.chunk, t1 = min(t0 + (long)A.chunk, A.n_tok);
   const long rs = A.row_stride[kind];
-  const u16* xp = A.x[kind] + (long)head * A.head_stride[kind] + 2 * lane;
-  for (int i = tid; i < 256 * 64 / 4; i += 64 * HIST_WAVES) reinterpret_cast<u32x4*>(h)[i] = u32x4{0u, 0u, 0u, 0u};
-  __syncthreads();
+  const u16* xp = A.x[kind] + (long)head * A.head_stride[kind] + 8 * (lane & 15);
   u32* hc = h + lane;
   const auto count = [&](u32 w) {
     atomicAdd(&hc[((w >> 7) & 0xFFu) << 6], 1u);
     atomicAdd(&hc[((w >> 23) & 0xFFu) << 6], 0x10000u);
   };
-  long t = t0 + wave;
-  for (; t + (HIST_ROWS - 1) * HIST_WAVES < t1; t += HIST_ROWS * HIST_WAVES) {
-    u32 w[HIST_ROWS];
+  // Rows of the chunk: a load of the wave takes four, 4 HIST_WAVES further on than the one before; each is repeated for the next round as soon as its
+  // rows are counted.  Rows past the end read the last one (no load under a branch) and are not counted.
+  const int n = (int)(t1 - t0), r0 = 4 * __builtin_amdgcn_readfirstlane(wave);
+  const u16* x0 = xp + t0 * rs;
+  const auto load = [&](int r) { return load_u32x4_unaligned(x0 + (long)min(r + (lane >> 4), n - 1) * rs); };
+  u32x4 w[HIST_LOADS];
 #pragma unroll
-    for (int k = 0; k < HIST_ROWS; ++k) w[k] = *reinterpret_cast<const u32*>(xp + (t + k * HIST_WAVES) * rs);
+  for (int k = 0; k < HIST_LOADS; ++k) w[k] = load(r0 + 4 * HIST_WAVES * k);
+  for (int i = tid; i < 256 * 64 / 4; i += 64 * HIST_WAVES) reinterpret_cast<u32x4*>(h)[i] = u32x4{0u, 0u, 0u, 0u};
+  __syncthreads();
+  for (int r = r0; r < n; r += 4 * HIST_WAVES * HIST_LOADS) {
 #pragma unroll
-    for (int k = 0; k < HIST_ROWS; ++k) count(w[k]);
+    for (int k = 0; k < HIST_LOADS; ++k) {
+      // lane (q, c) = (lane >> 4, lane & 15) has words 4c .. 4c + 3 of row q; after the exchange it has word 4c + q of all four rows
+      u32 x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = (u32)__builtin_amdgcn_mov_dpp((int)w[k][j], 0xE4 /* quad_perm: in place */, 0xF, 0xF, true);      // (a copy: exchanged in place, the loop's end waits for all loads)
+      const auto a = __builtin_amdgcn_permlane32_swap(x[0], x[2], false, false), b = __builtin_amdgcn_permlane32_swap(x[1], x[3], false, false);
+      const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false), hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+      const int row = r + 4 * HIST_WAVES * k;
+      w[k] = load(row + 4 * HIST_WAVES * HIST_LOADS);
+      if (row + 3 < n) { count(lo[0]); count(lo[1]); count(hi[0]); count(hi[1]); }
+      else {
+        if (row < n) count(lo[0]);
+        if (row + 1 < n) count(lo[1]);
+        if (row + 2 < n) count(hi[0]);
+      }
+    }
   }
-  for (; t < t1; t += HIST_WAVES) count(*reinterpret_cast<const u32*>(xp + t * rs));
   __syncthreads();
   const long pair = (long)kind * A.n_kv + head;
   for (int i = tid; i < 256 * 64; i += 64 * HIST_WAVES) {
     const u32 c = h[i];
     if (c == 0u) continue;
-    if (PACKED) atomicAdd(&A.hist[pair * (256 * 64) + i], (unsigned long long)(c & 0xFFFFu) | ((unsigned long long)(c >> 16) << 32));
+    const int word = 4 * (i & 15) + ((i >> 4) & 3);      // of the row, that the lane counted
+    if (PACKED) atomicAdd(&A.hist[pair * (256 * 64) + (i & ~63) + word], (unsigned long long)(c & 0xFFFFu) | ((unsigned long long)(c >> 16) << 32));
     else {
-      unsigned long long* row = A.hist + (pair * D + 2 * (i & 63)) * 256 + (i >> 6);
+      unsigned long long* row = A.hist + (pair * D + 2 * word) * 256 + (i >> 6);
       if (c & 0xFFFFu) atomicAdd(row, (unsigned long long)(c & 0xFFFFu));
       if (c >> 16) atomicAdd(row + 256, (unsigned long long)(c >> 16));
     }
