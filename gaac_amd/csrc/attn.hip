@@ -759,6 +759,11 @@ constexpr int PLAN_ROWS = 256;           // larger batches take nsplit splits pe
 constexpr float ONE_ROUND_LOSS = 48.f;   // tiles of a four-wave block
 // Smaller splits cost more in the merge than they gain: 30 sequences of up to 3000 tokens, one kv head with 16 query heads: 31.4 us
 // with at least 4 tiles, 27.4 with 12, 30.1 with 20; eight sequences of up to 3000 tokens, 8 kv heads: 21.6, 21.8, 24.5.
+// Splits of about this many tiles and up are ordered by size (plan_rows), where rows have few of them: 30 rows of 300 tokens beside one of 6000 x 8 kv heads (19 tiles) 19.1 us ordered by
+// kind, 21.1 by size, 48 of 100..6000 x 2 (24 tiles) 23.5 and 25.0; 32 of 100..2000 x 8 (40 tiles) 29.6 and 27.9; 12 of
+// 300..8000 x 8 (5 splits a row) 35.7 and 36.3, 20 of 100..16000 (3) 55.8 and 54.5.
+constexpr float SORTED_SPLIT_TILES = 28.f;
+constexpr int SORTED_ROW_SPLITS = 4;
 constexpr float MIN_SPLIT_TILES = 12.f;  // of a four-wave block; half as many for an eight-wave block
 struct RowPlan { int b, S, kvh, idx, ns, off, slot; };      // idx: the block's place among the ns blocks of (row, kv head); off: splits of the rows before
 __device__ __forceinline__ int plan_splits(int tiles, float c, float rc) {      // about ceil(tiles / c), the same wherever it is asked; no row (tiles < 0): none
@@ -814,7 +819,7 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
   total = wave_sum(total);
   const int units = min(nsplit * B, A.plan), u = uniform(div_below_2_21(block, A.n_kv));     // a unit is a split for every kv head: n_kv blocks
   const float fu = (float)units;
-  int ns = nsplit, b = 0, off = 0;
+  int ns = nsplit, b = 0, off = 0, w = -1;      // w: the block's place among the ns blocks of each of the row's kv heads, where that is not block - off * n_kv
   if (equal) {
     // batch order, with nsplit splits per row, or as many as make one round where that loses less than several rounds, or where the last
     // of several rounds would be much emptier (24 rows of 12000 tokens x 8 kv heads, 3 splits: 576 blocks 171 us, 2 splits 152)
@@ -852,30 +857,55 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
         lo = fmaxf(c_best - step, c_min); width = step * (1.f / 16.f);
       }
       if (one_round) {
-        // All blocks start together, two to a CU, the later half beside the earlier one: rows of several splits, whose blocks are all
-        // long, come first, then the others, either in batch order (all in batch order: 28 rows of 300..6000 tokens x 8 kv heads 54.6 us
-        // instead of 52.3, but 100 of 100..4000 x 4 70.5 instead of 77; longest first 52.5 and 77.7, and it takes a search).  The counts of
-        // the two kinds run in the halves of one word.
         const float rc = __builtin_amdgcn_rcpf(c_best);
-        u32 n[K], end[K], sum = 0u;
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          n[k] = (u32)plan_splits(tiles[k], c_best, rc);
-          n[k] = n[k] > 1u ? n[k] : n[k] << 16;
-          const u32 x = row_scan16(n[k]), r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31), r2 = __builtin_amdgcn_readlane(x, 47);
-          end[k] = sum + x + (lane >= 16 ? r0 : 0u) + (lane >= 32 ? r1 : 0u) + (lane >= 48 ? r2 : 0u);
-          sum = (u32)__builtin_amdgcn_readlane((int)end[k], 63);
-        }
         b = -1;
+        if (K == 1 && NW == 4 && units < SORTED_ROW_SPLITS * B && __builtin_amdgcn_ballot_w64(c_best >= SORTED_SPLIT_TILES) != 0) {
+          // All blocks start together, two four-wave blocks to a CU, the later half of the launch beside the earlier one: the longest splits first,
+          // and in the later half the shortest first, so that every CU gets about the same.  A lane adds up the splits of the rows ahead of its own.
+          // By kind, as below -> by size, us, 8 kv heads: 32 rows of 300..6000 tokens 61.6 -> 55.5, 48 of 100..8000 79.9 -> 65.1, 28 of 300..6000
+          // 60.2 -> 55.7, 32 of 100..2000 29.6 -> 27.9, 20 of 100..16000 55.8 -> 54.2; with four classes of size 62.3 for the first.
+          const int n = plan_splits(tiles[0], c_best, rc);      // (at most `units`, 512)
+          const int key = tiles[0] < 0 ? -1 : min((int)((float)tiles[0] * __builtin_amdgcn_rcpf((float)n) * rc * 16383.f), 32767) << 16 | (63 - lane) << 10 | n;
+          int before = 0;
+#pragma unroll 1
+          for (int i = 0; i < B; i += 8)
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-          const bool several = n[k] < 65536u;
-          const int mine = several ? (int)n[k] : (int)(n[k] >> 16), to = several ? (int)(end[k] & 65535u) : (int)((end[k] >> 16) + (sum & 65535u));
-          const u64 own = __builtin_amdgcn_ballot_w64(u >= to - mine && u < to);
-          if (own != 0) {
-            const int l = __builtin_ctzll(own);
-            b = 64 * k + l; ns = __builtin_amdgcn_readlane(mine, l); off = __builtin_amdgcn_readlane(to, l) - ns;
-            break;
+            for (int r = 0; r < 8; ++r) {
+              const int other = __builtin_amdgcn_readlane(key, i + r);
+              before += other > key ? other & 1023 : 0;      // (a lane without a row: below all others)
+            }
+          const int used = units * A.n_kv, half = (units >> 1) * A.n_kv;
+          if (block >= used) return false;
+          const int v = block < half ? block : used - 1 - (block - half), uv = uniform(div_below_2_21(v, A.n_kv));      // the block's place in that order
+          const u64 own = __builtin_amdgcn_ballot_w64(uv >= before && uv < before + n);
+          if (own == 0) return false;
+          b = __builtin_ctzll(own); ns = __builtin_amdgcn_readlane(n, b); off = __builtin_amdgcn_readlane(before, b);
+          // a head's splits in the order of the blocks' indexes also where that runs backwards (see merge_heads: a merger waits for blocks that start before it)
+          const int row0 = off * A.n_kv;
+          w = block < half ? v - row0 : max(row0, half) + ns * A.n_kv - 1 - v;
+        } else {
+          // Short splits, and more rows than a wave has lanes: the rows of several splits, whose blocks are all long and are waited for by a merge, come first,
+          // then the others, either in batch order (100 rows of 100..4000 x 4 kv heads 70.5 us, all longest first 77).  The counts of the two
+          // kinds run in the halves of one word.
+          u32 n[K], end[K], sum = 0u;
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            n[k] = (u32)plan_splits(tiles[k], c_best, rc);
+            n[k] = n[k] > 1u ? n[k] : n[k] << 16;
+            const u32 x = row_scan16(n[k]), r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31), r2 = __builtin_amdgcn_readlane(x, 47);
+            end[k] = sum + x + (lane >= 16 ? r0 : 0u) + (lane >= 32 ? r1 : 0u) + (lane >= 48 ? r2 : 0u);
+            sum = (u32)__builtin_amdgcn_readlane((int)end[k], 63);
+          }
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            const bool several = n[k] < 65536u;
+            const int mine = several ? (int)n[k] : (int)(n[k] >> 16), to = several ? (int)(end[k] & 65535u) : (int)((end[k] >> 16) + (sum & 65535u));
+            const u64 own = __builtin_amdgcn_ballot_w64(u >= to - mine && u < to);
+            if (own != 0) {
+              const int l = __builtin_ctzll(own);
+              b = 64 * k + l; ns = __builtin_amdgcn_readlane(mine, l); off = __builtin_amdgcn_readlane(to, l) - ns;
+              break;
+            }
           }
         }
         if (b < 0) return false;
@@ -924,7 +954,7 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
       }
     }
   }
-  const int w = block - off * A.n_kv;
+  if (w < 0) w = block - off * A.n_kv;
   R.b = b; R.ns = ns; R.off = off; R.kvh = uniform(div_below_2_21(w, ns)); R.idx = w - R.kvh * ns;
   R.slot = 0;
   if (!PAGED) {
