@@ -743,11 +743,14 @@ __device__ __forceinline__ int uniform_tile(int v) { return __builtin_amdgcn_rea
 //   * nearly equal rows (within 1/32 of the first one): nsplit splits per row in batch order, as without a plan, or as many as fill one round.
 //   * one round: the launch uses no more blocks than are resident at once (two four-wave blocks or one eight-wave block per CU), rows get
 //     splits of about c tiles, c the smallest size for which sum ceil(tiles / c) fits (found to 1/120 of c).  Blocks beyond have nothing to do.
-//   * several rounds, where half a split per row, which rounding costs, is more than starting and merging blocks again: nsplit splits per
-//     row, longest row first (blocks start in index order, so that the short rows fill the end of the launch).  The splits' sizes differ from
-//     row to row, which keeps the rounds from starting and ending in step.
+//   * several rounds, where half a split per row, which rounding costs, is more than starting and merging blocks again and the rows do not differ
+//     much, or where one round would make splits that the paged kernel's tile table does not hold: nsplit splits per row, longest row first (blocks
+//     start in index order, so that the short rows fill the end of the launch).  The splits' sizes differ from row to row, which keeps the rounds
+//     from starting and ending in step.
 // The line: a four-wave block takes about 0.5 us per tile and a round costs some 20 us of starts and merges.  16 sequences of 1000..16000
-// tokens (rounding costs 17 tiles): 91 us in one round, 102 in four; 4096..65536 tokens (68 tiles): 325 in one round, 277 in four.
+// tokens (rounding costs 17 tiles): 91 us in one round, 102 in four.  Where the longest row has half as much again as the mean, splits of many sizes meet
+// on the CUs and even that out, if they are paired by size (plan_rows): paged, 8 kv heads, several rounds / one, us: 16 rows of 4096..65536 tokens (68
+// tiles) 284 / 272, 32 of 500..20000 182 / 169, 24 of 2000..30000 207 / 193, 20 of 10000..40000 262 / 244.
 // Measured with warm caches, 4 query heads per kv head, against equal split counts in batch order: paged, 8 sequences of 200..3000 tokens x 8
 // kv heads: 27.0 -> 20.6 us, 16 of 500..6000: 71 -> 44; slot cache, 4 rows of 2000..32000: 47.4 -> 37.4, 12 of 300..8000: 53.5 -> 32.2,
 // 32 of 300..6000: 68 -> 61.
@@ -757,14 +760,16 @@ __device__ __forceinline__ int uniform_tile(int v) { return __builtin_amdgcn_rea
 // 500 tokens x 16 kv heads and 64.5 for the 4 rows above.
 constexpr int PLAN_ROWS = 256;           // larger batches take nsplit splits per row in batch order
 constexpr float ONE_ROUND_LOSS = 48.f;   // tiles of a four-wave block
+constexpr float ONE_ROUND_MIXED = 1.5f;  // longest row over the mean
 // Smaller splits cost more in the merge than they gain: 30 sequences of up to 3000 tokens, one kv head with 16 query heads: 31.4 us
 // with at least 4 tiles, 27.4 with 12, 30.1 with 20; eight sequences of up to 3000 tokens, 8 kv heads: 21.6, 21.8, 24.5.
-// Splits of about this many tiles and up are ordered by size (plan_rows), where rows have few of them: 30 rows of 300 tokens beside one of 6000 x 8 kv heads (19 tiles) 19.1 us ordered by
-// kind, 21.1 by size, 48 of 100..6000 x 2 (24 tiles) 23.5 and 25.0; 32 of 100..2000 x 8 (40 tiles) 29.6 and 27.9; 12 of
-// 300..8000 x 8 (5 splits a row) 35.7 and 36.3, 20 of 100..16000 (3) 55.8 and 54.5.
-constexpr float SORTED_SPLIT_TILES = 28.f;
-constexpr int SORTED_ROW_SPLITS = 4;
 constexpr float MIN_SPLIT_TILES = 12.f;  // of a four-wave block; half as many for an eight-wave block
+// Splits of about this many tiles and up are ordered by size (plan_rows), where rows have few of them: 30 rows of 300 tokens beside one of 6000 x 8 kv
+// heads (19 tiles) 19.1 us ordered by kind, 21.1 by size, 48 of 100..6000 x 2 (24 tiles) 23.5 and 25.0; 32 of 100..2000 x 8 (40 tiles) 29.6 and
+// 27.9; 12 of 300..8000 x 8 (5 splits a row) 35.7 and 36.3, 20 of 100..16000 (3) 55.8 and 54.5.
+constexpr int SORTED_SPLIT_TILES = 28;
+constexpr int SORTED_ROW_SPLITS = 4;
+constexpr int LONG_SPLIT_TILES = 128;      // from here on in any case
 struct RowPlan { int b, S, kvh, idx, ns, off, slot; };      // idx: the block's place among the ns blocks of (row, kv head); off: splits of the rows before
 __device__ __forceinline__ int plan_splits(int tiles, float c, float rc) {      // about ceil(tiles / c), the same wherever it is asked; no row (tiles < 0): none
   return tiles < 0 ? 0 : min(max((int)(((float)tiles + (c - 1.f)) * rc), 1), MAX_SLOTS);
@@ -834,6 +839,8 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
   } else {
     // half a split per row goes to rounding: total / units * B / (2 units) tiles on every block
     bool one_round = nsplit > 1 && units >= B && (resident || __builtin_amdgcn_ballot_w64(total * (float)B > ONE_ROUND_LOSS * 2.f * fu * fu) == 0);
+    if (K == 1 && __builtin_expect(!one_round && nsplit > 1 && units >= B, 0))      // very different rows; paged: the splits of one round stay within one fill of the tile table
+      one_round = __builtin_amdgcn_ballot_w64(wave_max(longest) * (float)B > ONE_ROUND_MIXED * total && (!PAGED || total <= 0.75f * MAX_CHUNK * fu)) != 0;
     if (one_round) {
       // sixteen sizes from the mean to three times that, then sixteen between the first that fits and the one before it; lane (j, r) =
       // (lane & 15, lane >> 4) tries size j over the rows r, r + 4, ...
@@ -859,7 +866,7 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
       if (one_round) {
         const float rc = __builtin_amdgcn_rcpf(c_best);
         b = -1;
-        if (K == 1 && NW == 4 && units < SORTED_ROW_SPLITS * B && __builtin_amdgcn_ballot_w64(c_best >= SORTED_SPLIT_TILES) != 0) {
+        if (K == 1 && NW == 4 && __builtin_expect(uniform((int)c_best) >= (units < SORTED_ROW_SPLITS * B ? SORTED_SPLIT_TILES : LONG_SPLIT_TILES), 0)) {
           // All blocks start together, two four-wave blocks to a CU, the later half of the launch beside the earlier one: the longest splits first,
           // and in the later half the shortest first, so that every CU gets about the same.  A lane adds up the splits of the rows ahead of its own.
           // By kind, as below -> by size, us, 8 kv heads: 32 rows of 300..6000 tokens 61.6 -> 55.5, 48 of 100..8000 79.9 -> 65.1, 28 of 300..6000
@@ -1498,6 +1505,14 @@ static int plan_units(int B, int n_kv, int nsplit, long max_tiles) {
   return 8 * max_tiles >= blocks * nsplit ? units : 0;
 }
 
+// Splits of a planned launch: no more than twice the resident blocks' worth.  A plan of one round leaves the other blocks without a part, and they start,
+// look at the rows and are waited for behind the others; of several rounds, two do.  Paged, 8 kv heads, us, the caller's splits / these: 32 rows of
+// 500..20000 tokens, 8 splits 168 / 166, 24 splits 181 / 165; 16 of 9000..11000 92 / 88, 20 of 39000..40000 405 / 389.
+static int planned_splits(int B, int n_kv, int nsplit, int plan, long least) {      // least: for splits that the paged kernel's tile table holds
+  const long heads = (long)B * n_kv;
+  return plan >= B ? (int)std::min<long>(nsplit, std::max((1024 + heads - 1) / heads, least)) : nsplit;
+}
+
 // Splits of a launch whose length the host knows: those of nsplit that get tiles, at least MIN_HOST_TILES each (the caller's count is an upper
 // bound here, as it is in a planned launch; it sizes the workspace).  Empty splits and splits of a tile or two are blocks that only start, publish
 // and are waited for.  us with splits of 2 or 3 / 3 / 4 / 6 tiles: 1000 tokens x 8 kv heads 9.3 / 8.4 / 8.4 / 9.1, 300 x 8 8.3 / 7.6 / 7.5 / 8.0,
@@ -1527,6 +1542,8 @@ static int attn_split_impl(
   GAAC_REQUIRE(nsplit >= 1 && nsplit <= MAX_SLOTS, "gaac_attn: nsplit must be in 1..%d", MAX_SLOTS);
   GAAC_REQUIRE(S_pad > 0 && S_pad <= (1 << 24), "gaac_attn: at most %d tokens per cache head (32-bit byte offsets inside a head)", 1 << 24);
   if (epoch && S_all >= 0) nsplit = host_splits((S_all + T - 1) / T, nsplit);
+  const int plan = epoch && S_all < 0 ? plan_units(B, n_kv, nsplit, S_pad / T) : 0;
+  nsplit = planned_splits(B, n_kv, nsplit, plan, 1);
   const int nslot = nsplit;
   AttnArgs A;
   A.k = StoreView{smk, ck, fk, tok, ovk, ohsk, b3k, b4k};
@@ -1536,7 +1553,7 @@ static int attn_split_impl(
   A.n_kv = n_kv; A.n_q = n_q; A.G = n_q / n_kv; A.NB = NB;
   A.kt = (const u16*)kt; A.vt = (const u16*)vt; A.tl = TL; A.tcap = TCAP;
   A.epochs = epoch; A.out = (u16*)out;
-  A.B = B; A.plan = epoch && S_all < 0 ? plan_units(B, n_kv, nsplit, S_pad / T) : 0;
+  A.B = B; A.plan = plan;
   GAAC_REQUIRE(!epoch || out, "gaac_attn: the fused merge needs an output buffer");
   A.pool = nullptr; A.raw = nullptr; A.mt = nullptr; A.bt = nullptr; A.bt_stride = 0; A.TS = 0;
   A.freeq = nullptr; A.n_free = 0; A.stack = nullptr; A.top = nullptr;
@@ -1716,6 +1733,8 @@ extern "C" int gaac_paged_attn(
   GAAC_REQUIRE(nsplit >= 1 && nsplit <= MAX_SLOTS, "gaac_paged_attn: nsplit must be in 1..%d", MAX_SLOTS);
   const long max_tiles = ((long)max_seq_len + T - 1) / T;
   GAAC_REQUIRE(max_seq_len >= 0 && max_tiles <= (long)bt_stride, "gaac_paged_attn: max_seq_len %d needs %ld blocks per row, the block table has %d", max_seq_len, max_tiles, bt_stride);
+  const int plan = plan_units(B, n_kv, nsplit, max_tiles);
+  nsplit = planned_splits(B, n_kv, nsplit, plan, (max_tiles + MAX_CHUNK - 1) / MAX_CHUNK);
   AttnArgs A;
   A.k = StoreView{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, b3k, b4k};
   A.v = StoreView{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, b3v, b4v};
@@ -1724,7 +1743,7 @@ extern "C" int gaac_paged_attn(
   A.n_kv = n_kv; A.n_q = n_q; A.G = n_q / n_kv; A.NB = NB;
   A.kt = nullptr; A.vt = nullptr; A.tl = nullptr; A.tcap = 0;
   A.epochs = epoch; A.out = (u16*)out;
-  A.B = B; A.plan = plan_units(B, n_kv, nsplit, max_tiles);
+  A.B = B; A.plan = plan;
   A.pool = pool; A.raw = (const u16*)raw; A.mt = mt; A.bt = bt; A.bt_stride = bt_stride; A.TS = TS;
   A.freeq = freeq; A.n_free = freeq ? n_free : 0; A.stack = stack; A.top = top;
 #ifdef GAAC_PHASE_TIMING
