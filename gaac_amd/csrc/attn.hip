@@ -977,6 +977,7 @@ __device__ __forceinline__ bool plan_block(const AttnArgs& A, int lane, RowPlan&
 }
 
 // ---------------------------------------------------------------------------------------------------- main kernel
+constexpr int PRIO_TILES = 28;      // of a split whose block goes first on half the SIMDs (k_attn_split)
 // NW = waves per block: 4 (two blocks per CU) or 8 (one block per CU: half as many partials to merge for the same occupancy)
 // HOST_LEN: the compressed length of every addressed head is the kernel argument S_all (not read from memory)
 template <bool PAGED, int NW, bool HOST_LEN>
@@ -1179,6 +1180,12 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   if (PAGED && any_raw && wave == 0) attend_raw_tiles(tlo, thi_fast);
 
   if (!PAGED) { B.kov = A.k.ovf + __builtin_amdgcn_readfirstlane((int)khs); B.vov = A.v.ovf + __builtin_amdgcn_readfirstlane((int)vhs); }
+  // Two four-wave blocks share a CU, a wave of each on every SIMD, and the arbiter prefers the older one: of 16 paged rows of up to 64K tokens the
+  // blocks of the launch's earlier half were through after 227 us, the later half's after 287, 60 of them with half the CU's waves.  Two of the later block's
+  // waves go first instead, so that each block is ahead on two SIMDs (its waves share its tiles).  us, 8 kv heads: paged, 16 rows of 4096..65536 tokens
+  // 274 -> 262, 16 of 31000..32000 249 -> 236, 20 of 39000..40000 389 -> 368; slot cache, 32 rows of 300..6000 67.8 -> 65.2; 128 paged rows of 200..8000
+  // x 2 heads 92.6 -> 85.  Splits of a dozen tiles gain nothing: 8 rows of 200..3000 18.7 -> 18.8.
+  if (NW == 4 && n_own >= PRIO_TILES && (blockIdx.x & 256u) != 0u && wave < 2) __builtin_amdgcn_s_setprio(1);
   if (any_tile) {
     if (PAGED) m0 = TileMeta{Tg.kto, Tg.vto, Tg.raw};
     load_tile_escapes<PAGED>(B, lane, Tg, R0);
@@ -1205,6 +1212,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     }
   }
 #undef TILE
+  if (NW == 4) __builtin_amdgcn_s_setprio(0);
   // arrival mark of the block for the fused merge (see merge_heads): the wave has no load in flight here
   if (A.epochs != nullptr && A.nslot > 1 && tid == 0) mark_arrival(A, epoch);
   GAAC_STAMP(2);
