@@ -68,9 +68,8 @@ def launch_nsplit(B: int, n_kv: int, S: int, ragged: bool) -> int:
       * ragged rows whose heads alone take more than a quarter of the CUs: two four-wave blocks per CU, to have enough of them to share
         out, once the rows are long enough to pay for more starts and merges.  x 8 heads, one block per CU / two: 12 rows of 300..8000
         tokens 37.2 / 31.5, 24 of 300..6000 67 / 45, 24 of 300..3000 37.3 / 28.3, 32 of 300..6000 68 / 59.5, 32 of 100..2000 27.9 / 26.4;
-        but 12 of 100..1000 13.7 / 15.8, 16 of 1000 14.7 / 16.8, 32 of 100..500 12.0 / 16.6.  From 170 heads to 256 this is a bet on
-        rows that differ: where long rows turn out equal, one block per (row, head) was faster (24 of 3000: 40.3 / 45.3, 32 of 3000:
-        46.2 / 49.9, 24 of 12000: 138 / 151, 28 of 4000..5000: 63 / 70);
+        but 12 of 100..1000 13.7 / 15.8, 16 of 1000 14.7 / 16.8, 32 of 100..500 12.0 / 16.6.  Where long rows turn out equal it
+        costs little (24 of 3000: 42.3 / 43.4, 32 of 3000: 47.7 / 48.4, 24 of 12000: 142 / 145, 28 of 4000..5000: 64.4 / 64.9);
       * ragged, more heads than CUs: two splits, one / two: 48 rows of 300..8000 x 8 heads 132 / 108, 48 of 100..2000 39.6 / 38.5, 64 of
         200..4000 82.5 / 78; but 64 of 100..2000 41.7 / 49.3, 200 of 300 x 2 heads 14.7 / 17.5.  Equal: 48 of 2000 54.6 / 55.7."""
     H = B * n_kv
