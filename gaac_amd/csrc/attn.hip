@@ -450,7 +450,7 @@ struct AttnLds {
 };
 // Block merge: one partial per wave plus one (index NW) for the uncompressed rows.  Before the waves publish, wave 0 keeps the decoded side of a
 // half raw tile in acc[0]; afterwards the mergers' scratch lies in acc.
-template <int NW> struct MergeLds { float m[NW + 1][GMAX], l[NW + 1][GMAX]; float acc[NW + 1][GMAX][MROW]; };
+template <int NW> struct MergeLds { float m[NW + 1][GMAX], l[NW + 1][GMAX]; __align__(16) float acc[NW + 1][GMAX][MROW]; };
 static_assert(T * D * sizeof(u16) <= GMAX * D * sizeof(float) && sizeof(MergeScratch<4>) <= 5 * GMAX * D * sizeof(float) &&
               sizeof(MergeScratch<8>) <= 9 * GMAX * D * sizeof(float), "scratch views must fit the merge buffer");
 struct TableRegs { u32 b0, b1; u32 qlo[4], qhi[4]; };      // one thread's raw inputs of the per-block tables
@@ -985,6 +985,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   constexpr int NT = 64 * NW;
   // one LDS object so that the tables the tile loop reads sit at the lowest addresses (immediate offsets of the LDS loads)
   struct BlockLds { AttnLds L; int next_tile; int2 tile_table[PAGED ? MAX_CHUNK : 1]; MergeLds<NW> M; };
+  static_assert(offsetof(BlockLds, M.acc) % 16 == 0, "the block merge's accumulators are stored and a decoded raw tile is read 16 bytes at a time");
   __shared__ BlockLds lds;
   AttnLds& L = lds.L; MergeLds<NW>& M = lds.M; int2* tile_table = lds.tile_table; int& next_tile = lds.next_tile;
   const int tid = threadIdx.x;

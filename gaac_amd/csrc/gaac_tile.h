@@ -10,7 +10,7 @@ namespace gaac {
 // LDS scratch of one encoding wave
 constexpr int XROW = D + 8;     // staged row stride in elements: 16 padding bytes spread the sixteen rows of a column over the banks
 struct EncodeLds {
-  u16 x[T * XROW];     // the tile's BF16 bit patterns, token-major, natural channel order (rows >= nvalid are zero)
+  __align__(16) u16 x[T * XROW];     // the tile's BF16 bit patterns, token-major, natural channel order (rows >= nvalid are zero)
   __align__(4) uint8_t b3[D], b4[D];
 };
 
