@@ -1,7 +1,8 @@
 """gaac_amd/libgaac_hip.so (see include/gaac_hip.h): calls() has its entry points as functions that take tensors (gaac_amd/_binding.so), load()
-is the library for ctypes.  There is no fallback: if one of the two is missing, or a call is made without a GPU, the call raises."""
+is the library for ctypes, which takes the calls where there is no binding for the installed torch.  There is no other fallback: if the library is
+missing, or a call is made without a GPU, the call raises."""
 from __future__ import annotations
-import ctypes, os
+import ctypes, os, warnings
 import torch
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libgaac_hip.so")
@@ -66,18 +67,39 @@ def load():
     return _lib
 
 
+class _CtypesCalls:
+    """calls() through ctypes, for any torch: 13.4 us for an attention() where the binding takes 7.8."""
+    def __getattr__(self, name):
+        fn, n, error = getattr(load(), name), len(_SIGNATURES[name]), load().gaac_last_error
+        def entry(*args):
+            if len(args) != n: raise TypeError(f"{name} takes {n} arguments ({len(args)} given)")
+            args = [ptr(a) if isinstance(a, torch.Tensor) else a() if callable(a) else a for a in args]
+            try: rc = fn(*args)
+            except ctypes.ArgumentError as e: raise TypeError(f"{name}: {e}") from None
+            if rc != 0: raise RuntimeError(f"{name} failed ({rc}): {error().decode(errors='replace')}")
+        setattr(self, name, entry)
+        return entry
+
+
 def calls():
     """The entry points as functions, in the order of arguments of include/gaac_hip.h: tensors on the device, addresses or None for pointers,
-    numbers, last the stream (its handle, or the function `stream`).  They raise RuntimeError with the library's message."""
+    numbers, last the stream (its handle, or the function `stream`).  They raise RuntimeError with the library's message.  The binding reads
+    tensors by the layout of the torch that it was built with, and is left alone where another one is installed."""
     global _calls
     if _calls is None:
         load()
         try:
             from . import _binding
+            wrong = _binding.torch_version != torch.__version__ and f"is built for torch {_binding.torch_version}"
         except ImportError as e:
-            raise RuntimeError(f"gaac_amd/_binding.so is missing or does not fit the installed torch ({e}): build it with `python -m gaac_amd.build`") from e
-        _binding.bind(lib_path())
-        _calls = _binding
+            wrong = f"cannot be loaded ({e})"
+        if wrong:
+            warnings.warn(f"gaac_amd/_binding.so {wrong}: calls go through ctypes and cost the host about twice the time; build it with `python -m gaac_amd.build`",
+                          RuntimeWarning, stacklevel=2)
+            _calls = _CtypesCalls()
+        else:
+            _binding.bind(lib_path())
+            _calls = _binding
     return _calls
 
 

@@ -60,6 +60,7 @@ def build_binding(verbose: bool = True) -> str:
     from torch.utils.cpp_extension import include_paths
     libs = os.path.join(os.path.dirname(torch.__file__), "lib")
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DGAAC_TORCH_VERSION="{torch.__version__}"',
            *(f"-isystem{d}" for d in [*include_paths(), sysconfig.get_paths()["include"]]), os.path.join(CSRC, "binding.cpp"), "-o", BINDING,
            "-L" + libs, "-Wl,-rpath," + libs, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-ldl"]
     if verbose: print(" ".join(cmd), flush=True)
