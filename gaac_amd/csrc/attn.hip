@@ -770,7 +770,18 @@ constexpr float MIN_SPLIT_TILES = 12.f;  // of a four-wave block; half as many f
 constexpr int SORTED_SPLIT_TILES = 28;
 constexpr int SORTED_ROW_SPLITS = 4;
 constexpr int LONG_SPLIT_TILES = 128;      // from here on in any case
-struct RowPlan { int b, S, kvh, idx, ns, off, slot; };      // idx: the block's place among the ns blocks of (row, kv head); off: splits of the rows before
+// Two four-wave blocks share a CU, a wave of each on every SIMD, and the arbiter prefers the older one: of 16 paged rows of up to 64K tokens the
+// blocks of the launch's earlier half were through after 227 us, the later half's after 287, 60 of them with half the CU's waves.  Two of the later block's
+// waves go first instead, so that each block is ahead on two SIMDs (its waves share its tiles).  us, 8 kv heads: paged, 16 rows of 4096..65536 tokens
+// 277 -> 270, 16 of 31000 240 -> 232; slot cache, 24 of 4000..12000 73.3 -> 69.9, 30 rows of 1000..32000 x 4 heads 62 -> 58.
+//   * Only where the launch is one round (RowPlan::first): of several, bit 8 of a block's index does not tell which of two came first, and a split that
+//     others put back ends later still: 40 rows of 6000 in two rounds 146 us, 179 with priorities, 40 of 5000..7000 149 and 173.
+//   * Not beside a split of more than twice the length, which the CU then waits for: 61 rows of 2000 tokens and one of 16000 116 us, 126 with priorities;
+//     50 of 500 and one of 20000 40.8 and 42.5.  The other block is at most as long as the plan's size of a split.
+//   * Splits of a dozen tiles gain nothing: with a line at 12 tiles all within 1 us of 28; at 60, 32 rows of 300..4000 32.6 -> 35.4.
+constexpr int PRIO_TILES = 28;
+constexpr float PRIO_SHARE = 0.5f;
+struct RowPlan { int b, S, kvh, idx, ns, off, slot; bool first; };      // idx: the block's place among the ns blocks of (row, kv head); off: splits of the rows before; first: see PRIO_TILES
 __device__ __forceinline__ int plan_splits(int tiles, float c, float rc) {      // about ceil(tiles / c), the same wherever it is asked; no row (tiles < 0): none
   return tiles < 0 ? 0 : min(max((int)(((float)tiles + (c - 1.f)) * rc), 1), MAX_SLOTS);
 }
@@ -809,10 +820,11 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
   for (int k = 0; k < K; ++k) differs |= 32 * abs(tiles[k] - t0) > t0;
   const bool equal = __builtin_amdgcn_ballot_w64(differs) == 0, resident = nsplit * B <= A.plan;      // equal: within 1/32 of the first row
   const auto stay = [&]() {      // at the place of equal rows
-    R.b = b_eq; R.kvh = kvh_eq; R.idx = block - bh * nsplit; R.ns = nsplit; R.off = b_eq * nsplit; R.slot = slot_eq; R.S = max(len_eq, 0);
+    R.b = b_eq; R.kvh = kvh_eq; R.idx = block - bh * nsplit; R.ns = nsplit; R.off = b_eq * nsplit; R.slot = slot_eq; R.S = max(len_eq, 0); R.first = resident;
     return true;
   };
   if (equal && resident) return stay();
+  R.first = false;
   float total = 0.f, longest = 0.f, shortest = -INFINITY;      // (shortest: negated)
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -834,7 +846,7 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
       if (10 * nsplit < 9 * rounds * n1 || __builtin_amdgcn_ballot_w64(loss > ONE_ROUND_LOSS) == 0) ns = n1;
     }
     if (ns == nsplit) return stay();
-    b = uniform(div_below_2_21(u, ns)); off = b * ns;
+    b = uniform(div_below_2_21(u, ns)); off = b * ns; R.first = true;
     if (b >= B) return false;
   } else {
     // half a split per row goes to rounding: total / units * B / (2 units) tiles on every block
@@ -865,6 +877,7 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
       }
       if (one_round) {
         const float rc = __builtin_amdgcn_rcpf(c_best);
+        const auto long_split = [&](int row_tiles) { return __builtin_amdgcn_ballot_w64((float)row_tiles >= PRIO_SHARE * c_best * (float)ns) != 0; };
         b = -1;
         if (K == 1 && NW == 4 && __builtin_expect(uniform((int)c_best) >= (units < SORTED_ROW_SPLITS * B ? SORTED_SPLIT_TILES : LONG_SPLIT_TILES), 0)) {
           // All blocks start together, two four-wave blocks to a CU, the later half of the launch beside the earlier one: the longest splits first,
@@ -887,6 +900,7 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
           const u64 own = __builtin_amdgcn_ballot_w64(uv >= before && uv < before + n);
           if (own == 0) return false;
           b = __builtin_ctzll(own); ns = __builtin_amdgcn_readlane(n, b); off = __builtin_amdgcn_readlane(before, b);
+          R.first = long_split(__builtin_amdgcn_readlane(tiles[0], b));
           // a head's splits in the order of the blocks' indexes also where that runs backwards (see merge_heads: a merger waits for blocks that start before it)
           const int row0 = off * A.n_kv;
           w = block < half ? v - row0 : max(row0, half) + ns * A.n_kv - 1 - v;
@@ -911,6 +925,7 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
             if (own != 0) {
               const int l = __builtin_ctzll(own);
               b = 64 * k + l; ns = __builtin_amdgcn_readlane(mine, l); off = __builtin_amdgcn_readlane(to, l) - ns;
+              R.first = long_split(__builtin_amdgcn_readlane(tiles[k], l));
               break;
             }
           }
@@ -977,7 +992,6 @@ __device__ __forceinline__ bool plan_block(const AttnArgs& A, int lane, RowPlan&
 }
 
 // ---------------------------------------------------------------------------------------------------- main kernel
-constexpr int PRIO_TILES = 28;      // of a split whose block goes first on half the SIMDs (k_attn_split)
 // NW = waves per block: 4 (two blocks per CU) or 8 (one block per CU: half as many partials to merge for the same occupancy)
 // HOST_LEN: the compressed length of every addressed head is the kernel argument S_all (not read from memory)
 template <bool PAGED, int NW, bool HOST_LEN>
@@ -1027,7 +1041,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     }
   } else {
     const int bh = __builtin_amdgcn_readfirstlane(small_div(blockIdx.x, A.nsplit));
-    R.b = __builtin_amdgcn_readfirstlane(small_div(bh, A.n_kv)); R.kvh = bh - R.b * A.n_kv; R.idx = (int)blockIdx.x - bh * A.nsplit; R.ns = A.nsplit; R.off = R.b * A.nsplit; R.S = -1;
+    R.b = __builtin_amdgcn_readfirstlane(small_div(bh, A.n_kv)); R.kvh = bh - R.b * A.n_kv; R.idx = (int)blockIdx.x - bh * A.nsplit; R.ns = A.nsplit; R.off = R.b * A.nsplit; R.S = -1; R.first = gridDim.x <= 512u;
     // (no slot map = row b attends over cache heads b*n_kv ..: one level of dependent loads less)
     R.slot = PAGED ? 0 : (A.slot ? A.slot[R.b] : R.b);
     if (!PAGED && !HOST_LEN) R.S = A.sl[max(R.slot, 0) * A.n_kv + R.kvh];
@@ -1181,12 +1195,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   if (PAGED && any_raw && wave == 0) attend_raw_tiles(tlo, thi_fast);
 
   if (!PAGED) { B.kov = A.k.ovf + __builtin_amdgcn_readfirstlane((int)khs); B.vov = A.v.ovf + __builtin_amdgcn_readfirstlane((int)vhs); }
-  // Two four-wave blocks share a CU, a wave of each on every SIMD, and the arbiter prefers the older one: of 16 paged rows of up to 64K tokens the
-  // blocks of the launch's earlier half were through after 227 us, the later half's after 287, 60 of them with half the CU's waves.  Two of the later block's
-  // waves go first instead, so that each block is ahead on two SIMDs (its waves share its tiles).  us, 8 kv heads: paged, 16 rows of 4096..65536 tokens
-  // 274 -> 262, 16 of 31000..32000 249 -> 236, 20 of 39000..40000 389 -> 368; slot cache, 32 rows of 300..6000 67.8 -> 65.2; 128 paged rows of 200..8000
-  // x 2 heads 92.6 -> 85.  Splits of a dozen tiles gain nothing: 8 rows of 200..3000 18.7 -> 18.8.
-  if (NW == 4 && n_own >= PRIO_TILES && (blockIdx.x & 256u) != 0u && wave < 2) __builtin_amdgcn_s_setprio(1);
+  if (NW == 4 && R.first && n_own >= PRIO_TILES && (blockIdx.x & 256u) != 0u && wave < 2) __builtin_amdgcn_s_setprio(1);
   if (any_tile) {
     if (PAGED) m0 = TileMeta{Tg.kto, Tg.vto, Tg.raw};
     load_tile_escapes<PAGED>(B, lane, Tg, R0);
