@@ -744,13 +744,14 @@ __device__ __forceinline__ int uniform_tile(int v) { return __builtin_amdgcn_rea
 //   * one round: the launch uses no more blocks than are resident at once (two four-wave blocks or one eight-wave block per CU), rows get
 //     splits of about c tiles, c the smallest size for which sum ceil(tiles / c) fits (found to 1/120 of c).  Blocks beyond have nothing to do.
 //   * several rounds, where half a split per row, which rounding costs, is more than starting and merging blocks again and the rows do not differ
-//     much, or where one round would make splits that the paged kernel's tile table does not hold: nsplit splits per row, longest row first (blocks
-//     start in index order, so that the short rows fill the end of the launch).  The splits' sizes differ from row to row, which keeps the rounds
-//     from starting and ending in step.
-// The line: a four-wave block takes about 0.5 us per tile and a round costs some 20 us of starts and merges.  16 sequences of 1000..16000
-// tokens (rounding costs 17 tiles): 91 us in one round, 102 in four.  Where the longest row has half as much again as the mean, splits of many sizes meet
+//     much, where one round would leave the longest row in pieces far above the mean, or in splits that the paged kernel's tile table does not hold: nsplit
+//     splits per row, longest row first (blocks start in index order, so that the short rows fill the end of the launch).  The splits' sizes differ
+//     from row to row, which keeps the rounds from starting and ending in step.  Where that would still leave the longest row in pieces far above the mean: splits
+//     of about c tiles, c the smallest size for which they fit the launch's nsplit * B units, the longest first.
+// The lines: a four-wave block takes about 0.5 us per tile and a round costs some 20 us of starts and merges.  16 sequences of 1000..16000
+// tokens (rounding costs 17 tiles): 91 us in one round, 102 in four.  Where the rows differ, splits of many sizes meet
 // on the CUs and even that out, if they are paired by size (plan_rows): paged, 8 kv heads, several rounds / one, us: 16 rows of 4096..65536 tokens (68
-// tiles) 284 / 272, 32 of 500..20000 182 / 169, 24 of 2000..30000 207 / 193, 20 of 10000..40000 262 / 244.
+// tiles) 284 / 270, 32 of 500..20000 182 / 166, 24 of 2000..30000 207 / 190, 20 of 10000..40000 262 / 245.
 // Measured with warm caches, 4 query heads per kv head, against equal split counts in batch order: paged, 8 sequences of 200..3000 tokens x 8
 // kv heads: 27.0 -> 20.6 us, 16 of 500..6000: 71 -> 44; slot cache, 4 rows of 2000..32000: 47.4 -> 37.4, 12 of 300..8000: 53.5 -> 32.2,
 // 32 of 300..6000: 68 -> 61.
@@ -760,16 +761,29 @@ __device__ __forceinline__ int uniform_tile(int v) { return __builtin_amdgcn_rea
 // 500 tokens x 16 kv heads and 64.5 for the 4 rows above.
 constexpr int PLAN_ROWS = 256;           // larger batches take nsplit splits per row in batch order
 constexpr float ONE_ROUND_LOSS = 48.f;   // tiles of a four-wave block
-constexpr float ONE_ROUND_MIXED = 1.5f;  // longest row over the mean
+// Rows whose longest has this much over the mean go into one round also where rounding costs more.  us, slot cache / paged, several rounds -> one: 40 rows
+// of 4500..7500 tokens x 8 kv heads (1.24) 144 -> 139 / 143 -> 147, 40 of 3500..8500 (1.41) 150 -> 135 / 143 -> 143, 20 of 14000..26000 (1.28) 220 -> 200 / 228 -> 204;
+// but 40 of 5000..7000 (1.16) 151 -> 142 / 144 -> 150.
+constexpr float ONE_ROUND_MIXED = 1.2f;
+// ... if the size found is no more than this much over the mean share of a block, or ONE_ROUND_LOSS tiles above it: where there is hardly more than a unit for
+// each row, the short rows take them and leave the long one in pieces that the launch waits for.  Paged, 8 kv heads, one round / several: 61 rows of 2000 tokens and
+// one of 16000 (2.5 of the mean) 126 / 109 us, slot cache 116 / 102, 56 of 500..6000 (2.2) 90 / 80; 48 of 100..8000 (1.7) 111 / 116, 40 of 300..8500 (1.6) 75 / 86;
+// 50 of 500 and one of 20000 (2.0, 44 tiles) 41 / 45.
+constexpr float ONE_ROUND_SIZE = 1.8f;
+// In several rounds the rows get splits of one size instead of nsplit each where a split of the longest would be this much over the mean share of a
+// block.  us, nsplit each / one size, slot cache, two splits a row on average: 63 rows of 2000 tokens and one of 16000 x 8 kv heads (3.6) 162 / 101, 200 of 3000 and one
+// of 30000 x 2 (6.1) 289 / 101, 64 of 200..8000 (1.9) 89 / 86; 56 of 500..6000 (1.5) 78 / 82; paged, 128 of 100..4000 x 4 (1.7) 70 / 75.
+constexpr float SIZED_SPLIT = 1.75f;
 // Smaller splits cost more in the merge than they gain: 30 sequences of up to 3000 tokens, one kv head with 16 query heads: 31.4 us
 // with at least 4 tiles, 27.4 with 12, 30.1 with 20; eight sequences of up to 3000 tokens, 8 kv heads: 21.6, 21.8, 24.5.
 constexpr float MIN_SPLIT_TILES = 12.f;  // of a four-wave block; half as many for an eight-wave block
-// Splits of about this many tiles and up are ordered by size (plan_rows), where rows have few of them: 30 rows of 300 tokens beside one of 6000 x 8 kv
-// heads (19 tiles) 19.1 us ordered by kind, 21.1 by size, 48 of 100..6000 x 2 (24 tiles) 23.5 and 25.0; 32 of 100..2000 x 8 (40 tiles) 29.6 and
-// 27.9; 12 of 300..8000 x 8 (5 splits a row) 35.7 and 36.3, 20 of 100..16000 (3) 55.8 and 54.5.
+// Splits of about this many tiles and up are ordered by size (plan_rows).  us, slot cache, 8 kv heads, by kind / by size; up to two units a row: 30 rows of 300 tokens
+// beside one of 6000 (19 tiles) 19.1 / 21.1, 32 of 300..4000 33.2 / 32.6 (a line at 18 tiles: 34.7), 32 of 200..3000 (61) 37.2 / 35.7.  More units a
+// row: 28 rows of 100..2600 (47) 31.0 / 32.1, 60 of 100..2600 x 4 heads (40) 33.5 / 36.0; from 60 tiles to 120 the two are within 1 us; 16 of
+// 3000..30000 (290) 134.8 / 131, paged 142.6 / 135.6.
 constexpr int SORTED_SPLIT_TILES = 28;
-constexpr int SORTED_ROW_SPLITS = 4;
-constexpr int LONG_SPLIT_TILES = 128;      // from here on in any case
+constexpr int SORTED_ROW_SPLITS = 2;
+constexpr int LONG_SPLIT_TILES = 96;
 // Two four-wave blocks share a CU, a wave of each on every SIMD, and the arbiter prefers the older one: of 16 paged rows of up to 64K tokens the
 // blocks of the launch's earlier half were through after 227 us, the later half's after 287, 60 of them with half the CU's waves.  Two of the later block's
 // waves go first instead, so that each block is ahead on two SIMDs (its waves share its tiles).  us, 8 kv heads: paged, 16 rows of 4096..65536 tokens
@@ -849,17 +863,19 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
     b = uniform(div_below_2_21(u, ns)); off = b * ns; R.first = true;
     if (b >= B) return false;
   } else {
+    const auto holds = [](bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; };      // (of values that are the same in all lanes)
     // half a split per row goes to rounding: total / units * B / (2 units) tiles on every block
-    bool one_round = nsplit > 1 && units >= B && (resident || __builtin_amdgcn_ballot_w64(total * (float)B > ONE_ROUND_LOSS * 2.f * fu * fu) == 0);
-    if (K == 1 && __builtin_expect(!one_round && nsplit > 1 && units >= B, 0))      // very different rows; paged: the splits of one round stay within one fill of the tile table
-      one_round = __builtin_amdgcn_ballot_w64(wave_max(longest) * (float)B > ONE_ROUND_MIXED * total && (!PAGED || total <= 0.75f * MAX_CHUNK * fu)) != 0;
-    if (one_round) {
+    const bool can = nsplit > 1 && units >= B;
+    bool one_round = can && (resident || holds(total * (float)B <= ONE_ROUND_LOSS * 2.f * fu * fu)), mixed = false, sized = false;
+    if (K == 1 && can && !one_round) one_round = mixed = holds(wave_max(longest) * (float)B > ONE_ROUND_MIXED * total);
+    float c_best = 1e9f;
+    const auto find_size = [&](int use) {      // c_best: the smallest size whose splits fit `use` units
       // sixteen sizes from the mean to three times that, then sixteen between the first that fits and the one before it; lane (j, r) =
       // (lane & 15, lane >> 4) tries size j over the rows r, r + 4, ...
-      const float c_min = fmaxf(floorf(total * __builtin_amdgcn_rcpf(fu)) + 1.f, NW == 4 ? MIN_SPLIT_TILES : 0.5f * MIN_SPLIT_TILES), step = c_min * (2.f / 15.f);
-      float lo = c_min, width = step, c_best = 0.f;
+      const float c_min = fmaxf(floorf(total * __builtin_amdgcn_rcpf((float)use)) + 1.f, NW == 4 ? MIN_SPLIT_TILES : 0.5f * MIN_SPLIT_TILES), step = c_min * (2.f / 15.f);
+      float lo = c_min, width = step;
 #pragma unroll 1
-      for (int pass = 0; pass < 2 && one_round; ++pass) {
+      for (int pass = 0; pass < 2; ++pass) {
         const float c = lo + width * (float)(lane & 15), rc = __builtin_amdgcn_rcpf(c);
         float n = 0.f;
 #pragma unroll
@@ -870,111 +886,123 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
             for (int j = 0; j < 16; j += 4) n += (float)plan_splits(__builtin_amdgcn_ds_bpermute(4 * (i + j + (lane >> 4)), tiles[k]), c, rc);
         }
         n = quad_rows_sum(n);
-        const u64 fits = __builtin_amdgcn_ballot_w64(n <= fu) & 0xFFFFull;
+        const u64 fits = __builtin_amdgcn_ballot_w64(n <= (float)use) & 0xFFFFull;
         if (fits) c_best = __uint_as_float((u32)__builtin_amdgcn_readlane((int)__float_as_uint(c), __builtin_ctzll(fits)));
-        else one_round = pass != 0;
+        else if (pass == 0) return false;
         lo = fmaxf(c_best - step, c_min); width = step * (1.f / 16.f);
       }
-      if (one_round) {
-        const float rc = __builtin_amdgcn_rcpf(c_best);
-        const auto long_split = [&](int row_tiles) { return __builtin_amdgcn_ballot_w64((float)row_tiles >= PRIO_SHARE * c_best * (float)ns) != 0; };
-        b = -1;
-        if (K == 1 && NW == 4 && __builtin_expect(uniform((int)c_best) >= (units < SORTED_ROW_SPLITS * B ? SORTED_SPLIT_TILES : LONG_SPLIT_TILES), 0)) {
-          // All blocks start together, two four-wave blocks to a CU, the later half of the launch beside the earlier one: the longest splits first,
-          // and in the later half the shortest first, so that every CU gets about the same.  A lane adds up the splits of the rows ahead of its own.
-          // By kind, as below -> by size, us, 8 kv heads: 32 rows of 300..6000 tokens 61.6 -> 55.5, 48 of 100..8000 79.9 -> 65.1, 28 of 300..6000
-          // 60.2 -> 55.7, 32 of 100..2000 29.6 -> 27.9, 20 of 100..16000 55.8 -> 54.2; with four classes of size 62.3 for the first.
-          const int n = plan_splits(tiles[0], c_best, rc);      // (at most `units`, 512)
-          const int key = tiles[0] < 0 ? -1 : min((int)((float)tiles[0] * __builtin_amdgcn_rcpf((float)n) * rc * 16383.f), 32767) << 16 | (63 - lane) << 10 | n;
-          int before = 0;
-#pragma unroll 1
-          for (int i = 0; i < B; i += 8)
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-              const int other = __builtin_amdgcn_readlane(key, i + r);
-              before += other > key ? other & 1023 : 0;      // (a lane without a row: below all others)
-            }
-          const int used = units * A.n_kv, half = (units >> 1) * A.n_kv;
-          if (block >= used) return false;
-          const int v = block < half ? block : used - 1 - (block - half), uv = uniform(div_below_2_21(v, A.n_kv));      // the block's place in that order
-          const u64 own = __builtin_amdgcn_ballot_w64(uv >= before && uv < before + n);
-          if (own == 0) return false;
-          b = __builtin_ctzll(own); ns = __builtin_amdgcn_readlane(n, b); off = __builtin_amdgcn_readlane(before, b);
-          R.first = long_split(__builtin_amdgcn_readlane(tiles[0], b));
-          // a head's splits in the order of the blocks' indexes also where that runs backwards (see merge_heads: a merger waits for blocks that start before it)
-          const int row0 = off * A.n_kv;
-          w = block < half ? v - row0 : max(row0, half) + ns * A.n_kv - 1 - v;
-        } else {
-          // Short splits, and more rows than a wave has lanes: the rows of several splits, whose blocks are all long and are waited for by a merge, come first,
-          // then the others, either in batch order (100 rows of 100..4000 x 4 kv heads 70.5 us, all longest first 77).  The counts of the two
-          // kinds run in the halves of one word.
-          u32 n[K], end[K], sum = 0u;
-#pragma unroll
-          for (int k = 0; k < K; ++k) {
-            n[k] = (u32)plan_splits(tiles[k], c_best, rc);
-            n[k] = n[k] > 1u ? n[k] : n[k] << 16;
-            const u32 x = row_scan16(n[k]), r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31), r2 = __builtin_amdgcn_readlane(x, 47);
-            end[k] = sum + x + (lane >= 16 ? r0 : 0u) + (lane >= 32 ? r1 : 0u) + (lane >= 48 ? r2 : 0u);
-            sum = (u32)__builtin_amdgcn_readlane((int)end[k], 63);
-          }
-#pragma unroll
-          for (int k = 0; k < K; ++k) {
-            const bool several = n[k] < 65536u;
-            const int mine = several ? (int)n[k] : (int)(n[k] >> 16), to = several ? (int)(end[k] & 65535u) : (int)((end[k] >> 16) + (sum & 65535u));
-            const u64 own = __builtin_amdgcn_ballot_w64(u >= to - mine && u < to);
-            if (own != 0) {
-              const int l = __builtin_ctzll(own);
-              b = 64 * k + l; ns = __builtin_amdgcn_readlane(mine, l); off = __builtin_amdgcn_readlane(to, l) - ns;
-              R.first = long_split(__builtin_amdgcn_readlane(tiles[k], l));
-              break;
-            }
-          }
-        }
-        if (b < 0) return false;
+      return true;
+    };
+    if (one_round) {
+      one_round = find_size(units);
+      if (__builtin_expect(!resident && (mixed || PAGED), 0)) {
+        const float mean = total * __builtin_amdgcn_rcpf(fu);
+        one_round = one_round && (!mixed || holds(c_best <= fmaxf(ONE_ROUND_SIZE * mean, mean + ONE_ROUND_LOSS))) && (!PAGED || holds(c_best <= (float)MAX_CHUNK));
       }
     }
-    if (!one_round) {      // nsplit splits per row, longest first
-      const int place = uniform(div_below_2_21(u, nsplit));
-      off = place * nsplit;
-      if (K == 1) {      // each row counts the rows ahead of it (16 rows: 80 instructions, the bisection below 250)
-        const int key = tiles[0] * 64 + 63 - lane;      // (below zero: not there)
-        int ahead = 0;
-#pragma unroll 1
-        for (int i = 0; i < B; i += 8)
+    if (__builtin_expect(!one_round && can, 0)) sized = holds(wave_max(longest) > SIZED_SPLIT * (float)nsplit * total * __builtin_amdgcn_rcpf(fu)) && find_size(nsplit * B);
+    const float rc = __builtin_amdgcn_rcpf(c_best);
+    const auto long_split = [&](int row_tiles) { return holds((float)row_tiles >= PRIO_SHARE * c_best * (float)ns); };
+    b = -1;
+    const bool by_kind = one_round && (K > 1 || NW != 4 || uniform((int)c_best) < (units <= SORTED_ROW_SPLITS * B ? SORTED_SPLIT_TILES : LONG_SPLIT_TILES));
+    if (by_kind) {
+      // Short splits, and more rows than a wave has lanes: the rows of several splits, whose blocks are all long and are waited for by a merge, come first,
+      // then the others, either in batch order (100 rows of 100..4000 x 4 kv heads 70.5 us, all longest first 77).  The counts of the two
+      // kinds run in the halves of one word.
+      u32 n[K], end[K], sum = 0u;
 #pragma unroll
-          for (int r = 0; r < 8; ++r) ahead += __builtin_amdgcn_readlane(key, i + r) > key ? 1 : 0;
-        b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(ahead == place && key >= 0));
-      } else {
-        int below = uniform((int)-wave_max(shortest)) - 1, own = uniform((int)wave_max(longest)), ahead = 0;
-#pragma unroll 1
-        while (own - below > 1) {
-          const int mid = (own + below) >> 1;
-          int n = 0;
+      for (int k = 0; k < K; ++k) {
+        n[k] = (u32)plan_splits(tiles[k], c_best, rc);
+        n[k] = n[k] > 1u ? n[k] : n[k] << 16;
+        const u32 x = row_scan16(n[k]), r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31), r2 = __builtin_amdgcn_readlane(x, 47);
+        end[k] = sum + x + (lane >= 16 ? r0 : 0u) + (lane >= 32 ? r1 : 0u) + (lane >= 48 ? r2 : 0u);
+        sum = (u32)__builtin_amdgcn_readlane((int)end[k], 63);
+      }
 #pragma unroll
-          for (int k = 0; k < K; ++k) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(tiles[k] > mid));
-          if (n <= place) { own = mid; ahead = n; } else below = mid;
-          if (n == place) break;
-        }
-        if (ahead == place) {      // the next row of up to `own` tiles
-          float t = -1.f;
-#pragma unroll
-          for (int k = 0; k < K; ++k) t = fmaxf(t, tiles[k] <= own ? (float)tiles[k] : -1.f);
-          own = uniform((int)wave_max(t));
-        }
-        int rank = place - ahead;      // the block's row is the rank-th, in batch order, of those of this length
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          const u64 m = __builtin_amdgcn_ballot_w64(tiles[k] == own);
-          const int n = __builtin_popcountll(m);
-          if (rank < n) {
-            const int before = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
-            b = 64 * k + __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles[k] == own && before == rank));
-            break;
-          }
-          rank -= n;
+      for (int k = 0; k < K; ++k) {
+        const bool several = n[k] < 65536u;
+        const int mine = several ? (int)n[k] : (int)(n[k] >> 16), to = several ? (int)(end[k] & 65535u) : (int)((end[k] >> 16) + (sum & 65535u));
+        const u64 own = __builtin_amdgcn_ballot_w64(u >= to - mine && u < to);
+        if (own != 0) {
+          const int l = __builtin_ctzll(own);
+          b = 64 * k + l; ns = __builtin_amdgcn_readlane(mine, l); off = __builtin_amdgcn_readlane(to, l) - ns;
+          R.first = long_split(__builtin_amdgcn_readlane(tiles[k], l));
+          break;
         }
       }
+    } else if (K == 1) {
+      // The longest splits first, or the longest row where each has nsplit.  A lane adds up the splits of the rows ahead of its own.
+      // One round: all blocks start together, two four-wave blocks to a CU, the later half of the launch beside the earlier one, and in the later half the
+      // shortest go first, so that every CU gets about the same.
+      // (With the order turning at the 256th block, where the second ones come, 300 to 400 blocks take the same to 1 us.)
+      // By kind, as above -> by size, us, 8 kv heads: 32 rows of 300..6000 tokens 61.6 -> 55.5, 48 of 100..8000 79.9 -> 65.1, 28 of 300..6000
+      // 60.2 -> 55.7, 32 of 100..2000 29.6 -> 27.9, 20 of 100..16000 55.8 -> 54.2; with four classes of size 62.3 for the first.
+      const bool by_size = one_round || sized;
+      const int n = by_size ? min(plan_splits(tiles[0], c_best, rc), 1023) : tiles[0] < 0 ? 0 : nsplit, mask = by_size ? 1023 : 0, add = by_size ? 0 : nsplit;
+      const int key = by_size && tiles[0] >= 0 ? min((int)((float)tiles[0] * __builtin_amdgcn_rcpf((float)n) * rc * 16383.f), 32767) << 16 | (63 - lane) << 10 | n
+                                               : tiles[0] * 64 + 63 - lane;      // (below zero: not there)
+      int before = 0;
+#pragma unroll 1
+      for (int i = 0; i < B; i += 8)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int other = __builtin_amdgcn_readlane(key, i + r);
+          before += other > key ? (other & mask) + add : 0;
+        }
+      const int used = (one_round ? units : nsplit * B) * A.n_kv, half = one_round ? (units >> 1) * A.n_kv : used;
+      if (block >= used) return false;
+      const int v = block < half ? block : used - 1 - (block - half), uv = uniform(div_below_2_21(v, A.n_kv));      // the block's place in that order
+      const u64 own = __builtin_amdgcn_ballot_w64(uv >= before && uv < before + n);
+      if (own == 0) return false;
+      b = __builtin_ctzll(own); ns = __builtin_amdgcn_readlane(n, b); off = __builtin_amdgcn_readlane(before, b);
+      R.first = one_round && long_split(__builtin_amdgcn_readlane(tiles[0], b));
+      // a head's splits in the order of the blocks' indexes also where that runs backwards (see merge_heads: a merger waits for blocks that start before it)
+      const int row0 = off * A.n_kv;
+      w = block < half ? v - row0 : max(row0, half) + ns * A.n_kv - 1 - v;
+    } else {
+      // Several rounds of more rows than a wave has lanes, longest row first: the splits of the rows longer than m tiles become fewer as m grows, and
+      // the block's row is where they pass its place.
+      const auto splits_above = [&](int m) {
+        int n = 0;
+        if (sized) {
+#pragma unroll
+          for (int k = 0; k < K; ++k) n += tiles[k] > m ? plan_splits(tiles[k], c_best, rc) : 0;
+          return uniform((int)wave_sum((float)n));
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(tiles[k] > m));
+        return n * nsplit;
+      };
+      int below = uniform((int)-wave_max(shortest)) - 1, own = uniform((int)wave_max(longest)), ahead = 0;
+      if (splits_above(below) <= u) return false;
+#pragma unroll 1
+      while (own - below > 1) {
+        const int mid = (own + below) >> 1, n = splits_above(mid);
+        if (n <= u) { own = mid; ahead = n; } else below = mid;
+        if (n == u) break;
+      }
+      if (ahead == u) {      // the next row of up to `own` tiles
+        float t = -1.f;
+#pragma unroll
+        for (int k = 0; k < K; ++k) t = fmaxf(t, tiles[k] <= own ? (float)tiles[k] : -1.f);
+        own = uniform((int)wave_max(t));
+      }
+      if (sized) ns = uniform(plan_splits(own, c_best, rc));
+      int rank = uniform(div_below_2_21(u - ahead, ns));      // the block's row is the rank-th, in batch order, of those of this length
+      off = ahead + rank * ns;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const u64 m = __builtin_amdgcn_ballot_w64(tiles[k] == own);
+        const int n = __builtin_popcountll(m);
+        if (rank < n) {
+          const int before = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
+          b = 64 * k + __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles[k] == own && before == rank));
+          break;
+        }
+        rank -= n;
+      }
     }
+    if (b < 0) return false;
   }
   if (w < 0) w = block - off * A.n_kv;
   R.b = b; R.ns = ns; R.off = off; R.kvh = uniform(div_below_2_21(w, ns)); R.idx = w - R.kvh * ns;
@@ -1524,8 +1552,9 @@ static int plan_units(int B, int n_kv, int nsplit, long max_tiles) {
 }
 
 // Splits of a planned launch: no more than twice the resident blocks' worth.  A plan of one round leaves the other blocks without a part, and they start,
-// look at the rows and are waited for behind the others; of several rounds, two do.  Paged, 8 kv heads, us, the caller's splits / these: 32 rows of
-// 500..20000 tokens, 8 splits 168 / 166, 24 splits 181 / 165; 16 of 9000..11000 92 / 88, 20 of 39000..40000 405 / 389.
+// look at the rows and are waited for behind the others; of several rounds, two do, as a row that needs more splits than the others gets them (SIZED_SPLIT).
+// Paged, 8 kv heads, us, the caller's splits / these: 32 rows of 500..20000 tokens, 8 splits 168 / 166, 24 splits 181 / 165; 16 of 9000..11000 92 / 88, 20 of
+// 39000..40000 405 / 385; 128 of 100..4000 x 4 heads, 4 splits 97 / 70; 64 of 2000, one of them 16000, 4 splits 120 / 111.
 static int planned_splits(int B, int n_kv, int nsplit, int plan, long least) {      // least: for splits that the paged kernel's tile table holds
   const long heads = (long)B * n_kv;
   return plan >= B ? (int)std::min<long>(nsplit, std::max((1024 + heads - 1) / heads, least)) : nsplit;

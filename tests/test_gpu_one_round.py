@@ -21,14 +21,23 @@ def test_rows(path, lens, n_kv, G, nsplit, expect):
     path(lens, n_kv, G, nsplit, expect)
 
 
-def test_splits_stay_within_the_tile_table():
-    """64 heads' worth of rows whose one round would need splits of about 1500 tiles: the paged launch makes more of them, of at most 1024."""
+# 256 heads: sixteen splits a round for eight rows; 512: eight
+@pytest.mark.parametrize("lens,n_kv", [
+    ([60000] * 5 + [200] * 3, 32),        # a mean of more tiles than the table holds
+    ([59200] * 3 + [16] * 5, 32),         # a mean of 694, but one round comes to 1234
+    ([59200] * 2 + [16] * 6, 64),         # two rounds have two splits a row
+])
+def test_splits_stay_within_the_tile_table(lens, n_kv):
+    """Rows whose one round would need splits of more than 1024 tiles: the paged launch makes four of each long row."""
     dev = require_gpu()
     import torch
-    lens, n_kv, ns = [60000] * 2 + [200] * 6, 32, 8      # 256 heads: sixteen splits a round for eight rows
-    gen = torch.Generator(device=dev).manual_seed(3)
+    from test_gpu_long_row import splits_of
+    gen, ns = torch.Generator(device=dev).manual_seed(3), 8
     layer, pool, bt, sl = ragged._paged(lens, n_kv, gen, dev)
     q = torch.randn(len(lens), n_kv, 128, generator=gen, device=dev).to(torch.bfloat16)
+    q[0] = 0
     want = torch.cat([layer.attention(q[i:i + 1], pool, bt[i:i + 1], sl[i:i + 1], 4) for i in range(len(lens))]).float()
-    for _ in range(2): ragged.assert_rows_close(layer.attention(q, pool, bt, sl, ns).float(), want)
+    for _ in range(2):
+        ragged.assert_rows_close(layer.attention(q, pool, bt, sl, ns).float(), want)
+        assert splits_of(layer._ws[(len(lens), n_kv, ns)], n_kv) == 4
     layer.check()
