@@ -103,13 +103,18 @@ class Page:
     @property
     def nbytes(self) -> int:
         """Bytes the page occupies for S tokens per head: token rows (sign/mantissa, codes, tag word), escape bytes and one offset per tile.
-        The base tables are left out (two [n_kv, D] byte tables per kind, shared by every page of a layer)."""
+        The base tables are left out (two [n_kv, D] byte tables per kind, shared by every page of a layer), and what is there besides: the tag words'
+        offsets, the rows up to S_pad and the room behind the escape stream (encode_page), up to STREAM_ROOM bytes a row in all, measured 1.1."""
         esc = int(self.ovf_head_start[-1] - self.ovf_head_start[0])
         return self.H * self.S * (D + CB + 4) + esc + self.H * ((self.S + T - 1) // T) * 4
 
     @property
     def ratio(self) -> float:
         return self.H * self.S * D * 2 / self.nbytes
+
+    def __getstate__(self):
+        """For pickle and torch.save, which write all of a view's storage: the escape stream without the room behind it."""
+        return {**self.__dict__, "ovf": self.ovf.clone() if self.ovf.untyped_storage().nbytes() > self.ovf.numel() else self.ovf}
 
 
 def row_offsets(flags: torch.Tensor, S: int) -> torch.Tensor:
