@@ -866,10 +866,10 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
     const auto holds = [](bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; };      // (of values that are the same in all lanes)
     // half a split per row goes to rounding: total / units * B / (2 units) tiles on every block
     const bool can = nsplit > 1 && units >= B;
-    bool one_round = can && (resident || holds(total * (float)B <= ONE_ROUND_LOSS * 2.f * fu * fu)), mixed = false, sized = false;
-    if (K == 1 && can && !one_round) one_round = mixed = holds(wave_max(longest) * (float)B > ONE_ROUND_MIXED * total);
-    float c_best = 1e9f;
-    const auto find_size = [&](int use) {      // c_best: the smallest size whose splits fit `use` units
+    bool mixed = false, try_one = can && (resident || holds(total * (float)B <= ONE_ROUND_LOSS * 2.f * fu * fu));
+    if (K == 1 && __builtin_expect(can && !try_one, 0)) try_one = mixed = holds(wave_max(longest) * (float)B > ONE_ROUND_MIXED * total);
+    float c_best = 0.f;
+    const auto find_size = [&](int use) {      // c_best: the smallest size whose splits fit `use` units; 0 if there is none
       // sixteen sizes from the mean to three times that, then sixteen between the first that fits and the one before it; lane (j, r) =
       // (lane & 15, lane >> 4) tries size j over the rows r, r + 4, ...
       const float c_min = fmaxf(floorf(total * __builtin_amdgcn_rcpf((float)use)) + 1.f, NW == 4 ? MIN_SPLIT_TILES : 0.5f * MIN_SPLIT_TILES), step = c_min * (2.f / 15.f);
@@ -888,24 +888,23 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
         n = quad_rows_sum(n);
         const u64 fits = __builtin_amdgcn_ballot_w64(n <= (float)use) & 0xFFFFull;
         if (fits) c_best = __uint_as_float((u32)__builtin_amdgcn_readlane((int)__float_as_uint(c), __builtin_ctzll(fits)));
-        else if (pass == 0) return false;
         lo = fmaxf(c_best - step, c_min); width = step * (1.f / 16.f);
       }
-      return true;
     };
-    if (one_round) {
-      one_round = find_size(units);
-      if (__builtin_expect(!resident && (mixed || PAGED), 0)) {
+    if (try_one) {
+      find_size(units);
+      if (PAGED && !resident) c_best = c_best <= (float)MAX_CHUNK ? c_best : 0.f;
+      if (__builtin_expect(mixed, 0)) {
         const float mean = total * __builtin_amdgcn_rcpf(fu);
-        one_round = one_round && (!mixed || holds(c_best <= fmaxf(ONE_ROUND_SIZE * mean, mean + ONE_ROUND_LOSS))) && (!PAGED || holds(c_best <= (float)MAX_CHUNK));
+        c_best = c_best <= fmaxf(ONE_ROUND_SIZE * mean, mean + ONE_ROUND_LOSS) ? c_best : 0.f;
       }
     }
-    if (__builtin_expect(!one_round && can, 0)) sized = holds(wave_max(longest) > SIZED_SPLIT * (float)nsplit * total * __builtin_amdgcn_rcpf(fu)) && find_size(nsplit * B);
-    const float rc = __builtin_amdgcn_rcpf(c_best);
-    const auto long_split = [&](int row_tiles) { return holds((float)row_tiles >= PRIO_SHARE * c_best * (float)ns); };
+    const int c_int = uniform((int)c_best);
+    const bool one_round = c_int != 0;
     b = -1;
-    const bool by_kind = one_round && (K > 1 || NW != 4 || uniform((int)c_best) < (units <= SORTED_ROW_SPLITS * B ? SORTED_SPLIT_TILES : LONG_SPLIT_TILES));
-    if (by_kind) {
+    const auto long_split = [&](int row_tiles) { return holds((float)row_tiles >= PRIO_SHARE * c_best * (float)ns); };
+    if (__builtin_expect(one_round && (K > 1 || NW != 4 || c_int < (units <= SORTED_ROW_SPLITS * B ? SORTED_SPLIT_TILES : LONG_SPLIT_TILES)), 1)) {
+      const float rc = __builtin_amdgcn_rcpf(c_best);
       // Short splits, and more rows than a wave has lanes: the rows of several splits, whose blocks are all long and are waited for by a merge, come first,
       // then the others, either in batch order (100 rows of 100..4000 x 4 kv heads 70.5 us, all longest first 77).  The counts of the two
       // kinds run in the halves of one word.
@@ -930,76 +929,84 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
           break;
         }
       }
-    } else if (K == 1) {
-      // The longest splits first, or the longest row where each has nsplit.  A lane adds up the splits of the rows ahead of its own.
-      // One round: all blocks start together, two four-wave blocks to a CU, the later half of the launch beside the earlier one, and in the later half the
-      // shortest go first, so that every CU gets about the same.
-      // (With the order turning at the 256th block, where the second ones come, 300 to 400 blocks take the same to 1 us.)
-      // By kind, as above -> by size, us, 8 kv heads: 32 rows of 300..6000 tokens 61.6 -> 55.5, 48 of 100..8000 79.9 -> 65.1, 28 of 300..6000
-      // 60.2 -> 55.7, 32 of 100..2000 29.6 -> 27.9, 20 of 100..16000 55.8 -> 54.2; with four classes of size 62.3 for the first.
-      const bool by_size = one_round || sized;
-      const int n = by_size ? min(plan_splits(tiles[0], c_best, rc), 1023) : tiles[0] < 0 ? 0 : nsplit, mask = by_size ? 1023 : 0, add = by_size ? 0 : nsplit;
-      const int key = by_size && tiles[0] >= 0 ? min((int)((float)tiles[0] * __builtin_amdgcn_rcpf((float)n) * rc * 16383.f), 32767) << 16 | (63 - lane) << 10 | n
-                                               : tiles[0] * 64 + 63 - lane;      // (below zero: not there)
-      int before = 0;
-#pragma unroll 1
-      for (int i = 0; i < B; i += 8)
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          const int other = __builtin_amdgcn_readlane(key, i + r);
-          before += other > key ? (other & mask) + add : 0;
-        }
-      const int used = (one_round ? units : nsplit * B) * A.n_kv, half = one_round ? (units >> 1) * A.n_kv : used;
-      if (block >= used) return false;
-      const int v = block < half ? block : used - 1 - (block - half), uv = uniform(div_below_2_21(v, A.n_kv));      // the block's place in that order
-      const u64 own = __builtin_amdgcn_ballot_w64(uv >= before && uv < before + n);
-      if (own == 0) return false;
-      b = __builtin_ctzll(own); ns = __builtin_amdgcn_readlane(n, b); off = __builtin_amdgcn_readlane(before, b);
-      R.first = one_round && long_split(__builtin_amdgcn_readlane(tiles[0], b));
-      // a head's splits in the order of the blocks' indexes also where that runs backwards (see merge_heads: a merger waits for blocks that start before it)
-      const int row0 = off * A.n_kv;
-      w = block < half ? v - row0 : max(row0, half) + ns * A.n_kv - 1 - v;
     } else {
-      // Several rounds of more rows than a wave has lanes, longest row first: the splits of the rows longer than m tiles become fewer as m grows, and
-      // the block's row is where they pass its place.
-      const auto splits_above = [&](int m) {
-        int n = 0;
-        if (sized) {
-#pragma unroll
-          for (int k = 0; k < K; ++k) n += tiles[k] > m ? plan_splits(tiles[k], c_best, rc) : 0;
-          return uniform((int)wave_sum((float)n));
-        }
-#pragma unroll
-        for (int k = 0; k < K; ++k) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(tiles[k] > m));
-        return n * nsplit;
-      };
-      int below = uniform((int)-wave_max(shortest)) - 1, own = uniform((int)wave_max(longest)), ahead = 0;
-      if (splits_above(below) <= u) return false;
+      bool sized = can && !one_round && holds(wave_max(longest) > SIZED_SPLIT * (float)nsplit * total * __builtin_amdgcn_rcpf(fu));
+      if (sized) {      // (with two splits a row and up, three times the mean always fits)
+        find_size(nsplit * B);
+        sized = uniform((int)c_best) != 0;
+      }
+      const float rc = __builtin_amdgcn_rcpf(c_best);
+      if (K == 1) {
+        // The longest splits first, or the longest row where each has nsplit.  A lane adds up the splits of the rows ahead of its own.
+        // One round: all blocks start together, two four-wave blocks to a CU, the later half of the launch beside the earlier one, and in the later half the
+        // shortest go first, so that every CU gets about the same.
+        // (With the order turning at the 256th block, where the second ones come, 300 to 400 blocks take the same to 1 us.)
+        // By kind, as above -> by size, us, 8 kv heads: 32 rows of 300..6000 tokens 61.6 -> 55.5, 48 of 100..8000 79.9 -> 65.1, 28 of 300..6000
+        // 60.2 -> 55.7, 32 of 100..2000 29.6 -> 27.9, 20 of 100..16000 55.8 -> 54.2; with four classes of size 62.3 for the first.
+        const bool by_size = one_round || sized;
+        const int n = by_size ? min(plan_splits(tiles[0], c_best, rc), 1023) : tiles[0] < 0 ? 0 : nsplit, mask = by_size ? 1023 : 0, add = by_size ? 0 : nsplit;
+        const int key = by_size && tiles[0] >= 0 ? min((int)((float)tiles[0] * __builtin_amdgcn_rcpf((float)n) * rc * 16383.f), 32767) << 16 | (63 - lane) << 10 | n
+                                                 : tiles[0] * 64 + 63 - lane;      // (below zero: not there)
+        int before = 0;
 #pragma unroll 1
-      while (own - below > 1) {
-        const int mid = (own + below) >> 1, n = splits_above(mid);
-        if (n <= u) { own = mid; ahead = n; } else below = mid;
-        if (n == u) break;
-      }
-      if (ahead == u) {      // the next row of up to `own` tiles
-        float t = -1.f;
+        for (int i = 0; i < B; i += 8)
 #pragma unroll
-        for (int k = 0; k < K; ++k) t = fmaxf(t, tiles[k] <= own ? (float)tiles[k] : -1.f);
-        own = uniform((int)wave_max(t));
-      }
-      if (sized) ns = uniform(plan_splits(own, c_best, rc));
-      int rank = uniform(div_below_2_21(u - ahead, ns));      // the block's row is the rank-th, in batch order, of those of this length
-      off = ahead + rank * ns;
+          for (int r = 0; r < 8; ++r) {
+            const int other = __builtin_amdgcn_readlane(key, i + r);
+            before += other > key ? (other & mask) + add : 0;
+          }
+        const int used = (one_round ? units : nsplit * B) * A.n_kv, half = one_round ? (units >> 1) * A.n_kv : used;
+        if (block >= used) return false;
+        const int v = block < half ? block : used - 1 - (block - half), uv = uniform(div_below_2_21(v, A.n_kv));      // the block's place in that order
+        const u64 own = __builtin_amdgcn_ballot_w64(uv >= before && uv < before + n);
+        if (own == 0) return false;
+        b = __builtin_ctzll(own); ns = __builtin_amdgcn_readlane(n, b); off = __builtin_amdgcn_readlane(before, b);
+        R.first = one_round && long_split(__builtin_amdgcn_readlane(tiles[0], b));
+        // a head's splits in the order of the blocks' indexes also where that runs backwards (see merge_heads: a merger waits for blocks that start before it)
+        const int row0 = off * A.n_kv;
+        w = block < half ? v - row0 : max(row0, half) + ns * A.n_kv - 1 - v;
+      } else {
+        // Several rounds of more rows than a wave has lanes, longest row first: the splits of the rows longer than m tiles become fewer as m grows, and
+        // the block's row is where they pass its place.
+        const auto splits_above = [&](int m) {
+          int n = 0;
+          if (sized) {
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const u64 m = __builtin_amdgcn_ballot_w64(tiles[k] == own);
-        const int n = __builtin_popcountll(m);
-        if (rank < n) {
-          const int before = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
-          b = 64 * k + __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles[k] == own && before == rank));
-          break;
+            for (int k = 0; k < K; ++k) n += tiles[k] > m ? plan_splits(tiles[k], c_best, rc) : 0;
+            return uniform((int)wave_sum((float)n));
+          }
+#pragma unroll
+          for (int k = 0; k < K; ++k) n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(tiles[k] > m));
+          return n * nsplit;
+        };
+        int below = uniform((int)-wave_max(shortest)) - 1, own = uniform((int)wave_max(longest)), ahead = 0;
+        if (splits_above(below) <= u) return false;
+#pragma unroll 1
+        while (own - below > 1) {
+          const int mid = (own + below) >> 1, n = splits_above(mid);
+          if (n <= u) { own = mid; ahead = n; } else below = mid;
+          if (n == u) break;
         }
-        rank -= n;
+        if (ahead == u) {      // the next row of up to `own` tiles
+          float t = -1.f;
+#pragma unroll
+          for (int k = 0; k < K; ++k) t = fmaxf(t, tiles[k] <= own ? (float)tiles[k] : -1.f);
+          own = uniform((int)wave_max(t));
+        }
+        if (sized) ns = uniform(plan_splits(own, c_best, rc));
+        int rank = uniform(div_below_2_21(u - ahead, ns));      // the block's row is the rank-th, in batch order, of those of this length
+        off = ahead + rank * ns;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const u64 m = __builtin_amdgcn_ballot_w64(tiles[k] == own);
+          const int n = __builtin_popcountll(m);
+          if (rank < n) {
+            const int before = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
+            b = 64 * k + __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles[k] == own && before == rank));
+            break;
+          }
+          rank -= n;
+        }
       }
     }
     if (b < 0) return false;
