@@ -888,6 +888,7 @@ __device__ __forceinline__ bool plan_rows(const AttnArgs& A, int lane, RowPlan& 
         n = quad_rows_sum(n);
         const u64 fits = __builtin_amdgcn_ballot_w64(n <= (float)use) & 0xFFFFull;
         if (fits) c_best = __uint_as_float((u32)__builtin_amdgcn_readlane((int)__float_as_uint(c), __builtin_ctzll(fits)));
+        if (K > 1 && uniform((int)c_best) == 0) break;      // (with K 1 the second look costs less than the branch: it tries what did not fit again)
         lo = fmaxf(c_best - step, c_min); width = step * (1.f / 16.f);
       }
     };
