@@ -103,8 +103,8 @@ class Page:
     @property
     def nbytes(self) -> int:
         """Bytes the page occupies for S tokens per head: token rows (sign/mantissa, codes, tag word), escape bytes and one offset per tile.
-        The base tables are left out (two [n_kv, D] byte tables per kind, shared by every page of a layer), and what is there besides: the tag words'
-        offsets, the rows up to S_pad and the room behind the escape stream (encode_page), up to STREAM_ROOM bytes a row in all, measured 1.1."""
+        The base tables are left out (two [n_kv, D] byte tables per kind, shared by every page of a layer), and so are ovf_off, the rows from S to
+        S_pad and the room behind the escape stream that a page from encode_page holds (less than STREAM_ROOM bytes a row; measured 1.1)."""
         esc = int(self.ovf_head_start[-1] - self.ovf_head_start[0])
         return self.H * self.S * (D + CB + 4) + esc + self.H * ((self.S + T - 1) // T) * 4
 

@@ -1143,7 +1143,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   // a counter in LDS.  Of the two waves that share a SIMD the older one wins the issue arbitration and runs ahead; with a static
   // split it would finish long before the other, which then runs alone and cannot hide its own latencies.  Ping-pong registers
   // R0/R1; tag words are fetched one tile further ahead; indices past the end are clamped for the loads (no load sits under a
-  // branch the consumer has to join) and not consumed.  A partly filled last tile of the sequence is handled at the end by wave 0.
+  // branch the consumer has to join) and not consumed.  A partly filled last tile of the sequence follows at the end, by the first wave without a tile of its own.
   // logical tile index i of this block -> tile tlo + i
   const int full = ntiles - ((S % T) != 0 ? 1 : 0);      // tiles with all 16 rows
   const int n_own = max(min(thi_fast, full) - tlo, 0);

@@ -67,11 +67,11 @@ def launch_nsplit(B: int, n_kv: int, S: int, ragged: bool) -> int:
       * one eight-wave block per CU (256 blocks: a second round of blocks costs more than it evens out);
       * ragged rows whose heads alone take more than a quarter of the CUs: two four-wave blocks per CU, to have enough of them to share
         out, once the rows are long enough to pay for more starts and merges.  x 8 heads, one block per CU / two: 12 rows of 300..8000
-        tokens 37.2 / 31.5, 24 of 300..6000 67 / 45, 24 of 300..3000 37.3 / 28.3, 32 of 300..6000 68 / 59.5, 32 of 100..2000 27.9 / 26.4;
-        but 12 of 100..1000 13.7 / 15.8, 16 of 1000 14.7 / 16.8, 32 of 100..500 12.0 / 16.6.  Where long rows turn out equal it
-        costs little (24 of 3000: 42.3 / 43.4, 32 of 3000: 47.7 / 48.4, 24 of 12000: 142 / 145, 28 of 4000..5000: 64.4 / 64.9);
-      * ragged, more heads than CUs: two splits, one / two: 48 rows of 300..8000 x 8 heads 132 / 108, 48 of 100..2000 39.6 / 38.5, 64 of
-        200..4000 82.5 / 78; but 64 of 100..2000 41.7 / 49.3, 200 of 300 x 2 heads 14.7 / 17.5.  Equal: 48 of 2000 54.6 / 55.7."""
+        tokens 43.6 / 33.3, 24 of 300..6000 81 / 48, 24 of 300..3000 45 / 30, 32 of 300..6000 82.5 / 58, 32 of 100..2000 33.3 / 27.0;
+        but 12 of 100..1000 15.3 / 15.6, 16 of 1000 16.9 / 17.3, 32 of 100..500 14.0 / 17.3.  Where long rows turn out equal it
+        costs little (24 of 3000: 47.6 / 48.7, 32 of 3000: 52.3 / 52.2, 24 of 12000: 159 / 162; 28 of 4000..5000: 73.6 / 68.1);
+      * ragged, more heads than CUs: two splits, one / two: 48 rows of 300..8000 x 8 heads 157 / 117, 48 of 100..2000 47.7 / 38.0, 64 of
+        200..4000 86.2 / 86.4, 64 of 100..2000 50.4 / 48.6; but 200 of 300 x 2 heads 16.5 / 17.1.  Equal: 48 of 2000 59.6 / 59.1."""
     H = B * n_kv
     if S <= 256: return 1
     if ragged and B > 1 and 64 < H <= 256 and S >= max(1500, 7 * H): n = -(-512 // H)
