@@ -68,7 +68,7 @@ def load():
 
 
 class _CtypesCalls:
-    """calls() through ctypes, for any torch: 13.4 us for an attention() where the binding takes 7.8."""
+    """calls() through ctypes, for any torch: 14 us for an attention() where the binding takes 8 to 11."""
     def __getattr__(self, name):
         fn, n, error = getattr(load(), name), len(_SIGNATURES[name]), load().gaac_last_error
         def entry(*args):

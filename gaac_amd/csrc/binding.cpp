@@ -2,8 +2,8 @@
 // library's message where an entry point returns non-zero.  Tensors are handed over as they are; a host tensor raises.  A function in the place of
 // an address (the stream) is called for it once the arguments before it have been looked at: without a GPU, a host tensor is what the error names.
 // What it is for: a launch has up to 47 arguments, half of them tensors.  Through ctypes, with is_cuda and data_ptr() called from Python for each
-// tensor, attention() cost the host 13.4 us, more than the kernel takes over a short context, and a step of append and attention 22; with the
-// arguments converted here 8 to 9.4 and 15.
+// tensor, attention() costs the host 14 us, more than the kernel takes over a short context, and a step of append and attention 24; with the
+// arguments converted here 8 to 11 and 12 to 16.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <dlfcn.h>
