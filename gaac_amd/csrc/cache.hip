@@ -21,7 +21,7 @@ struct AppendArgs {
 };
 
 template <int KIND>
-__device__ __forceinline__ void append_one(const CacheStore& st, const u16* __restrict__ xrow, EncodeLds& L, int h, int pos, int Sh,
+__device__ __forceinline__ void append_one(const CacheStore& st, const u16* __restrict__ xrow, EncodeLds& L, BaseTable& B, int h, int pos, int Sh,
                                            const AppendArgs& A, int lane) {
   u16* tail_h = st.tail + (long)h * T * D;
   if (lane < 16) *reinterpret_cast<u32x4*>(tail_h + pos * D + 8 * lane) = *reinterpret_cast<const u32x4*>(xrow + 8 * lane);
@@ -36,18 +36,16 @@ __device__ __forceinline__ void append_one(const CacheStore& st, const u16* __re
     *reinterpret_cast<u32x4*>(&L.x[row * XROW + c16 * 8]) = *reinterpret_cast<const u32x4*>(src + c16 * 8);
   }
   const int brow = h % A.NB;
-  stage_bases(L, st.base3 + (long)brow * D, st.base4 + (long)brow * D, lane);
+  reinterpret_cast<u32x2*>(&B.w[0][0])[lane] = load_base_pair<KIND>(st.base3 + (long)brow * D, st.base4 + (long)brow * D, lane);
   wave_lds_sync();
-  BaseRegs Bs;
-  load_base_regs<KIND>(L, lane & 15, lane >> 4, Bs);
   const long row0 = (long)h * A.cap + (long)tile * T;
   uint8_t* sm_tile = st.sm + row0 * D; uint8_t* cd_tile = st.cd + row0 * CB; int* fl_tile = st.flags + row0;
   const int used = st.ovf_used[h];
   uint8_t* dst = st.ovf + (long)h * A.ovf_cap + used;
   UnitEscapes E;
-  const int total = encode_staged_tile<KIND, false>(L, Bs, T, lane, sm_tile, cd_tile, fl_tile, E);
+  const int total = encode_staged_tile<KIND, false>(L, B, T, lane, sm_tile, cd_tile, fl_tile, E);
   const bool fits = (long)used + total + 8 <= A.ovf_cap;
-  if (fits) write_tile_escapes(E, dst);
+  if (fits) write_tile_escapes<KIND>(L, E, dst, lane);
   if (fits) {
     if (lane == 0) { st.tile_off[(long)h * (A.cap / T) + tile] = used; st.ovf_used[h] = used + total; }
   } else {    // keep every later reader in bounds: the tile reads as all tier 0 (wrong values, flagged)
@@ -59,13 +57,14 @@ __device__ __forceinline__ void append_one(const CacheStore& st, const u16* __re
 // grid (B*n_kv), 128 threads: wave 0 = K, wave 1 = V of cache head SLOT[b]*n_kv + kvh
 __global__ void __launch_bounds__(128) k_cache_append(const AppendArgs A) {
   __shared__ EncodeLds L[2];
+  __shared__ BaseTable B[2];
   const int i = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int slot = A.slots[i / A.n_kv];
   if (slot < 0) return;
   const int h = slot * A.n_kv + i % A.n_kv;
   const int pos = A.tail_len[h], Sh = A.S[h];
-  if (wave == 0) append_one<KIND_K>(A.k, A.kx + (long)i * D, L[0], h, pos, Sh, A, lane);
-  else append_one<KIND_V>(A.v, A.vx + (long)i * D, L[1], h, pos, Sh, A, lane);
+  if (wave == 0) append_one<KIND_K>(A.k, A.kx + (long)i * D, L[0], B[0], h, pos, Sh, A, lane);
+  else append_one<KIND_V>(A.v, A.vx + (long)i * D, L[1], B[1], h, pos, Sh, A, lane);
   __syncthreads();
   if (tid == 0) {      // _advance (kv_cache.py:86-96)
     const bool full = pos + 1 == T;

@@ -175,12 +175,13 @@ __global__ void __launch_bounds__(256) k_bases_from_hist(const long long* __rest
 }
 
 // ---------------------------------------------------------------------------------------------------- page encoder
-// A block of four waves takes 4 * TPW consecutive tiles of one head, wave w the tiles w, w+4, ... of them (one-wave blocks, one per tile,
-// would be limited by the rate at which workgroups can be launched).  The rows of a wave's next tile are fetched into registers while it
-// encodes the current one.  K and V of a prompt share a launch (blockIdx.z): one start-up and one drain for both.
-// Bound by the memory rate: 229 MB of a 64K-token page of 8 heads in 42 us.  What goes past the caches is chosen by what comes next, so that the
-// Infinity Cache keeps the rest:
-//   * the rows of a large launch (TPW > 1) are read for the last time: 64K page 44.6 -> 42.3 us; the 32768-token prompt's call, where the histogram has
+// A block of four waves takes four consecutive tiles of one head, one each (one-wave blocks would be limited by the rate at which workgroups can be
+// launched), and makes the head's base words for all of them.  K and V of a prompt share a launch (blockIdx.z): one start-up and one drain for both.
+// Bound by the memory rate.  A wave has one tile and 62 registers: eight waves a SIMD hide each other's trips to memory.  Before, a wave took four tiles in
+// a row with the rows of the next one and all base words in registers, 147 of them: three waves a SIMD and a quarter more instructions a tile; 64K page of 8 heads
+// out of memory 47.9 -> 45.0 us (229 MB, 5.1 TB/s), 16K page 15.9 -> 14.6, prompt of 32768 tokens with given bases 49.1 -> 46.6.
+// What goes past the caches is chosen by what comes next, so that the Infinity Cache keeps the rest:
+//   * the rows of a large launch (BIG) are read for the last time: 64K page 44.6 -> 42.3 us; the 32768-token prompt's call, where the histogram has
 //     just brought them in, 109 -> 101 us;
 //   * a prompt's tiles (PROMPT) are stored past them, or they would push out rows that are still to be read: 119 -> 109 us; a page's are not,
 //     the caller is as likely to read them at once: 64K page and back 107 us past the caches, 101 through them.
@@ -192,48 +193,35 @@ struct EncodeKind {      // one of K, V
   uint8_t* slots; int* tile_bytes;                 // [H][ntiles] worst-case escape slots and the bytes used in each
 };
 struct EncodeArgs { EncodeKind k, v; int kind0, S, S_pad, ntiles, brow0, NB; const int* bidx; };      // blockIdx.z = 0 is kind0
-template <int KIND, int TPW, bool PROMPT>
-__device__ __forceinline__ void encode_tiles_body(const EncodeArgs& A, const EncodeKind& J, EncodeLds& L, int h, int tile, int lane) {
-  const int S = A.S, ntiles = A.ntiles;
+struct EncodeBlockLds { BaseTable B; EncodeLds w[CODEC_WAVES]; };
+template <int KIND, bool BIG, bool PROMPT>
+__device__ __forceinline__ void encode_tiles_body(const EncodeArgs& A, const EncodeKind& J, EncodeBlockLds& L, int h, int tile, int wave, int lane) {
+  const int S = A.S, ntiles = A.ntiles, nvalid = min(T, S - tile * T);
   const int brow = A.bidx ? A.bidx[h] : (A.brow0 + h) % A.NB;
-  const u16* xh = J.x + (long)h * J.head_stride;
-  RowRegs R, Rn;
-  load_rows<(TPW > 1)>(R, xh + (long)tile * T * J.row_stride, J.row_stride, min(T, S - tile * T), lane);
-  stage_bases(L, J.b3 + (long)brow * D, J.b4 + (long)brow * D, lane);
-  wave_lds_sync();
-  BaseRegs Bs;                // the base words of the lane's units: the same for every tile of the head
-  load_base_regs<KIND>(L, lane & 15, lane >> 4, Bs);
-  for (int i = 0; i < TPW && tile < ntiles; ++i, tile += CODEC_WAVES) {
-    const int nvalid = min(T, S - tile * T), next = tile + CODEC_WAVES;
-    store_rows(L, R, lane);
-    if (i + 1 < TPW && next < ntiles) load_rows<(TPW > 1)>(Rn, xh + (long)next * T * J.row_stride, J.row_stride, min(T, S - next * T), lane);
-    wave_lds_sync();
-    const long row0 = (long)h * A.S_pad + (long)tile * T;
-    UnitEscapes E;
-    const int total = encode_staged_tile<KIND, PROMPT>(L, Bs, nvalid, lane, J.sm + row0 * D, J.cd + row0 * CB, J.flags + row0, E);
-    write_tile_escapes(E, J.slots + ((long)h * ntiles + tile) * TILE_MAX_ESC);
-    if (lane == 0) J.tile_bytes[(long)h * ntiles + tile] = total;
-    wave_lds_sync();          // the staged rows are free again
-    R = Rn;
-  }
+  RowRegs R;
+  load_rows<BIG>(R, J.x + (long)h * J.head_stride + (long)min(tile, ntiles - 1) * T * J.row_stride, J.row_stride, max(nvalid, 1), lane);
+  if (wave == 0) reinterpret_cast<u32x2*>(&L.B.w[0][0])[lane] = load_base_pair<KIND>(J.b3 + (long)brow * D, J.b4 + (long)brow * D, lane);
+  store_rows(L.w[wave], R, lane);
+  __syncthreads();
+  if (tile >= ntiles) return;
+  const long row0 = (long)h * A.S_pad + (long)tile * T;
+  UnitEscapes E;
+  const int total = encode_staged_tile<KIND, PROMPT>(L.w[wave], L.B, nvalid, lane, J.sm + row0 * D, J.cd + row0 * CB, J.flags + row0, E);
+  write_tile_escapes<KIND>(L.w[wave], E, J.slots + ((long)h * ntiles + tile) * TILE_MAX_ESC, lane);
+  if (lane == 0) J.tile_bytes[(long)h * ntiles + tile] = total;
 }
-template <int TPW, bool PROMPT>
-__global__ void __launch_bounds__(64 * CODEC_WAVES) k_encode_tiles(const EncodeArgs A) {
-  __shared__ EncodeLds Ls[CODEC_WAVES];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, tile = blockIdx.x * (CODEC_WAVES * TPW) + wave;
-  if (tile >= A.ntiles) return;
-  if (A.kind0 + (int)blockIdx.z == KIND_K) encode_tiles_body<KIND_K, TPW, PROMPT>(A, A.k, Ls[wave], blockIdx.y, tile, lane);
-  else encode_tiles_body<KIND_V, TPW, PROMPT>(A, A.v, Ls[wave], blockIdx.y, tile, lane);
+template <bool BIG, bool PROMPT>
+__global__ void __launch_bounds__(64 * CODEC_WAVES, 8) k_encode_tiles(const EncodeArgs A) {
+  __shared__ EncodeBlockLds L;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, tile = blockIdx.x * CODEC_WAVES + wave;
+  if (A.kind0 + (int)blockIdx.z == KIND_K) encode_tiles_body<KIND_K, BIG, PROMPT>(A, A.k, L, blockIdx.y, tile, wave, lane);
+  else encode_tiles_body<KIND_V, BIG, PROMPT>(A, A.v, L, blockIdx.y, tile, wave, lane);
 }
 template <bool PROMPT>
 static void launch_encode(const EncodeArgs& A, int H, int kinds, hipStream_t stream) {
-  // Four tiles in a row per wave hide a tile's row loads behind the previous tile and share the base words; below 8192 tiles (eight
-  // waves per SIMD with one tile each) that leaves SIMDs idle, and one tile per wave is faster:
-  // 7.9 against 10.4 us at 2048 tiles, 17.0 against 14.8 us at 8192, 50.6 against 44.8 us at 32768 (K)
-  if ((long)A.ntiles * H * kinds >= 8192)
-    hipLaunchKernelGGL((k_encode_tiles<4, PROMPT>), dim3((A.ntiles + 4 * CODEC_WAVES - 1) / (4 * CODEC_WAVES), H, kinds), dim3(64 * CODEC_WAVES), 0, stream, A);
-  else
-    hipLaunchKernelGGL((k_encode_tiles<1, PROMPT>), dim3((A.ntiles + CODEC_WAVES - 1) / CODEC_WAVES, H, kinds), dim3(64 * CODEC_WAVES), 0, stream, A);
+  const dim3 grid((A.ntiles + CODEC_WAVES - 1) / CODEC_WAVES, H, kinds);
+  if ((long)A.ntiles * H * kinds >= 8192) hipLaunchKernelGGL((k_encode_tiles<true, PROMPT>), grid, dim3(64 * CODEC_WAVES), 0, stream, A);
+  else hipLaunchKernelGGL((k_encode_tiles<false, PROMPT>), grid, dim3(64 * CODEC_WAVES), 0, stream, A);
 }
 
 // Exclusive prefix sums of one head's tile sizes into off, and their total; called by all threads of a block, of which each SCAN_NT

@@ -9,10 +9,9 @@ namespace gaac {
 
 // LDS scratch of one encoding wave
 constexpr int XROW = D + 8;     // staged row stride in elements: 16 padding bytes spread the sixteen rows of a column over the banks
-struct EncodeLds {
-  __align__(16) u16 x[T * XROW];     // the tile's BF16 bit patterns, token-major, natural channel order (rows >= nvalid are zero)
-  __align__(4) uint8_t b3[D], b4[D];
-};
+struct EncodeLds { __align__(16) u16 x[T * XROW]; };     // the tile's BF16 bit patterns, token-major, natural channel order (rows >= nvalid are zero)
+// Base words of a head, [0] of the 3-bit tier, [1] of the 4-bit tier: one table for all waves that work on the head
+struct BaseTable { u32x4 w[2][NG]; };
 
 // 16 rows of 128 BF16 (row r at src + r*row_stride elements): lane's four 16-byte pieces; rows >= nvalid read as zero (the last valid row is
 // loaded in their place: a load under a branch would be waited for by itself).  STREAM: a prompt larger than the caches, read once.
@@ -37,9 +36,13 @@ __device__ __forceinline__ void store_rows(EncodeLds& L, const RowRegs& R, int l
     *reinterpret_cast<u32x4*>(&L.x[row * XROW + c16 * 8]) = R.v[k];
   }
 }
-__device__ __forceinline__ void stage_bases(EncodeLds& L, const uint8_t* __restrict__ b3row, const uint8_t* __restrict__ b4row, int lane) {
-  if (lane < 32) reinterpret_cast<u32*>(L.b3)[lane] = reinterpret_cast<const u32*>(b3row)[lane];
-  else reinterpret_cast<u32*>(L.b4)[lane - 32] = reinterpret_cast<const u32*>(b4row)[lane - 32];
+// words 2i and 2i + 1 of the table (i < 64)
+template <int KIND>
+__device__ __forceinline__ u32x2 load_base_pair(const uint8_t* __restrict__ b3row, const uint8_t* __restrict__ b4row, int i) {
+  const uint8_t* row = i < 32 ? b3row : b4row;
+  const int g = (i >> 1) & 15, p = 2 * (i & 1);
+  const u32 l0 = row[chan_of<KIND>(8 * g + p)], h0 = row[chan_of<KIND>(8 * g + p + 4)], l1 = row[chan_of<KIND>(8 * g + p + 1)], h1 = row[chan_of<KIND>(8 * g + p + 5)];
+  return u32x2{(l0 << 7) | (h0 << 23), (l1 << 7) | (h1 << 23)};
 }
 
 // Orders the LDS traffic of ONE wave (LDS operations of a wave complete in program order; the fences only stop the compiler from
@@ -51,55 +54,39 @@ __device__ __forceinline__ void wave_lds_sync() {
 // A word of host memory that the host polls (gaac_wait_words): there before the kernel ends.
 __device__ __forceinline__ void store_to_host(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM); }
 
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
 // The encoder works on 32-bit words that hold elements i and i+4 of a unit in their 16-bit halves (the decoder's word order), two
-// elements per VALU operation.
-struct BaseRegs { u32 b3[4][4], b4[4][4]; };      // [unit][i]: base of element i | base of element i+4 << 16
+// elements per VALU operation.  The data words of unit u of lane (a, q), and its sign/mantissa bytes (elements 0..3, 4..7):
 template <int KIND>
-__device__ __forceinline__ void load_base_regs(const EncodeLds& L, int a, int q, BaseRegs& B) {
-  const auto load = [&](const uint8_t* b, u32 (&w)[4], int u) {
-    if (KIND == KIND_K) {      // elements (2m, 2m+1) are the adjacent channels 32u + 2q + 8m (+1)
-      const u16* r = reinterpret_cast<const u16*>(b) + 16 * u + q;
-      const u32 r0 = r[0], r1 = r[4], r2 = r[8], r3 = r[12];
-      w[0] = __builtin_amdgcn_perm(r2, r0, 0x0C040C00u); w[1] = __builtin_amdgcn_perm(r2, r0, 0x0C050C01u);
-      w[2] = __builtin_amdgcn_perm(r3, r1, 0x0C040C00u); w[3] = __builtin_amdgcn_perm(r3, r1, 0x0C050C01u);
-    } else {
-      const uint8_t* r = b + 64 * (a & 1) + (a >> 1);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = (u32)r[8 * i] | ((u32)r[8 * i + 32] << 16);
-    }
-  };
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    if (KIND == KIND_V && u > 0) {      // a lane's units are of one group
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { B.b3[u][i] = B.b3[0][i]; B.b4[u][i] = B.b4[0][i]; }
-    } else { load(L.b3, B.b3[u], u); load(L.b4, B.b4[u], u); }
-  }
-}
-// the four data words of unit u of lane (a, q)
-template <int KIND>
-__device__ __forceinline__ void unit_data_words(const EncodeLds& L, int a, int q, int u, u32* __restrict__ W) {
+__device__ __forceinline__ void unit_words(const EncodeLds& L, int a, int q, int u, u32* __restrict__ W, u32& slo, u32& shi) {
+  u32 l0, h0, l1, h1;      // low and high bytes of elements 0..3 and 4..7
   if (KIND == KIND_K) {
     // elements (2m, 2m+1) are the adjacent channels 32u + 2q + 8m (+1): four aligned words, re-paired to (i, i+4)
     const u32* xr = reinterpret_cast<const u32*>(&L.x[a * XROW + 32 * u + 2 * q]);
     const u32 r0 = xr[0], r1 = xr[4], r2 = xr[8], r3 = xr[12];
     W[0] = __builtin_amdgcn_perm(r2, r0, 0x05040100u); W[1] = __builtin_amdgcn_perm(r2, r0, 0x07060302u);
     W[2] = __builtin_amdgcn_perm(r3, r1, 0x05040100u); W[3] = __builtin_amdgcn_perm(r3, r1, 0x07060302u);
+    l0 = __builtin_amdgcn_perm(r1, r0, 0x06040200u); h0 = __builtin_amdgcn_perm(r1, r0, 0x07050301u);
+    l1 = __builtin_amdgcn_perm(r3, r2, 0x06040200u); h1 = __builtin_amdgcn_perm(r3, r2, 0x07050301u);
   } else {
     // element i is channel 64 (a & 1) + (a >> 1) + 8 i of token 4q + u
     const u16* xr = &L.x[(4 * q + u) * XROW + 64 * (a & 1) + (a >> 1)];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) W[i] = (u32)xr[8 * i] | ((u32)xr[8 * i + 32] << 16);
+    for (int i = 0; i < 4; ++i) W[i] = __builtin_bit_cast(u32, u16x2_t{xr[8 * i], xr[8 * i + 32]});
+    const u32 e0 = __builtin_amdgcn_perm(W[1], W[0], 0x05010400u), e1 = __builtin_amdgcn_perm(W[3], W[2], 0x05010400u);
+    const u32 e2 = __builtin_amdgcn_perm(W[1], W[0], 0x07030602u), e3 = __builtin_amdgcn_perm(W[3], W[2], 0x07030602u);
+    l0 = __builtin_amdgcn_perm(e1, e0, 0x05040100u); h0 = __builtin_amdgcn_perm(e1, e0, 0x07060302u);
+    l1 = __builtin_amdgcn_perm(e3, e2, 0x05040100u); h1 = __builtin_amdgcn_perm(e3, e2, 0x07060302u);
   }
+  slo = (l0 & 0x7F7F7F7Fu) | (h0 & 0x80808080u); shi = (l1 & 0x7F7F7F7Fu) | (h1 & 0x80808080u);
 }
-typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u32 pk_sub_u16(u32 x, u32 y) {
   return __builtin_bit_cast(u32, (u16x2_t)(__builtin_bit_cast(u16x2_t, x) - __builtin_bit_cast(u16x2_t, y)));
 }
 
-// What a lane's four units add to the escape stream: tags, the 4th code bits of a 4-bit group, the exponent words of a raw one, and where the
-// lane's bytes start among the tile's.
-struct UnitEscapes { u32 tag[4], eb[4], ew[4][4]; int pos; };
+// What a lane's four units add to the escape stream: tags (2 bits each), the 4th code bits of a 4-bit group (unit u's at byte u; anything where its tag
+// is not 1), and where the lane's bytes start among the tile's.
+struct UnitEscapes { u32 tag8, eb; int pos; };
 // bitwise or across the four 16-lane rows at fixed column
 __device__ __forceinline__ u32 quad_rows_or(u32 x) {
   auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
@@ -110,42 +97,39 @@ __device__ __forceinline__ u32 quad_rows_or(u32 x) {
 
 // Encodes the tile staged in L (after a barrier).  Writes the native sign/mantissa and code bytes and the 16 tag words (one per line); the
 // escape bytes stay with the lanes for write_tile_escapes, so that a caller can see their number before it says where they go.
-// Returns the tile's escape byte count (all lanes).  Must be called by all 64 lanes of the wave that owns L.  B: load_base_regs of the same L.
+// Returns the tile's escape byte count (all lanes).  Must be called by all 64 lanes of the wave that owns L.  B: the head's base words.
 // STREAM: the bytes go past the caches.
+// A unit is done with before the next one is read, and what a raw group needs is read again where it is written: 64 registers, so that eight waves share a
+// SIMD and hide the trip to memory of a tile's rows (see k_encode_tiles).
 template <int KIND, bool STREAM>
-__device__ __forceinline__ int encode_staged_tile(const EncodeLds& L, const BaseRegs& B, int nvalid, int lane, uint8_t* __restrict__ sm_tile,
+__device__ __forceinline__ int encode_staged_tile(const EncodeLds& L, const BaseTable& B, int nvalid, int lane, uint8_t* __restrict__ sm_tile,
                                                   uint8_t* __restrict__ cd_tile, int* __restrict__ flags_tile, UnitEscapes& E) {
   const int a = lane & 15, q = lane >> 4;
   u32 slo[4], shi[4], g24[4];
+  E.tag8 = 0u; E.eb = 0u;
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     u32 W[4], d3[4], d4[4];
-    unit_data_words<KIND>(L, a, q, u, W);
+    unit_words<KIND>(L, a, q, u, W, slo[u], shi[u]);
+    const u32x4 b3 = B.w[0][unit_group<KIND>(a, q, u)], b4 = B.w[1][unit_group<KIND>(a, q, u)];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      E.ew[u][i] = (W[i] >> 7) & 0x00FF00FFu;                    // exponents
-      d3[i] = pk_sub_u16(E.ew[u][i], B.b3[u][i]); d4[i] = pk_sub_u16(E.ew[u][i], B.b4[u][i]);      // negative differences wrap to >= 0xFF01
+    for (int i = 0; i < 4; ++i) {      // exponents and their differences at bits 7 and up of the halves: nine bits, negative ones wrap to 257 and more
+      W[i] &= EXP_MASK2;
+      d3[i] = pk_sub_u16(W[i], b3[i]); d4[i] = pk_sub_u16(W[i], b4[i]);
     }
     // tier rule (codec.py:144-150): all eight differences in 0..7, else all in 0..15, else raw
-    const bool fit3 = ((d3[0] | d3[1] | d3[2] | d3[3]) & 0xFFF8FFF8u) == 0u, fit4 = ((d4[0] | d4[1] | d4[2] | d4[3]) & 0xFFF0FFF0u) == 0u;
-    u32 cacc = 0u, xacc = 0u, sb[4];
+    const bool fit3 = ((d3[0] | d3[1] | d3[2] | d3[3]) & 0xFC00FC00u) == 0u, fit4 = ((d4[0] | d4[1] | d4[2] | d4[3]) & 0xF800F800u) == 0u;
+    u32 c[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const u32 c = fit3 ? d3[i] : (fit4 ? d4[i] : E.ew[u][i]);
-      cacc |= (c & 0x00070007u) << (3 * i);                       // code of element i at bits 3i, of element i+4 at 16 + 3i
-      xacc |= (d4[i] & 0x00080008u) << i;                         // 4th code bit of element i at bit 3 + i, of i+4 at 19 + i
-      sb[i] = ((W[i] >> 8) & ~0x007F007Fu) | (W[i] & 0x007F007Fu); // sign/mantissa bytes at bits 0..7 and 16..23 (the other bytes are not taken)
-    }
-    const u32 p01 = __builtin_amdgcn_perm(sb[1], sb[0], 0x06020400u), p23 = __builtin_amdgcn_perm(sb[3], sb[2], 0x06020400u);
-    slo[u] = __builtin_amdgcn_perm(p23, p01, 0x05040100u); shi[u] = __builtin_amdgcn_perm(p23, p01, 0x07060302u);
-    E.tag[u] = fit3 ? 0u : (fit4 ? 1u : 3u);
-    g24[u] = (cacc & 0xFFFu) | ((cacc >> 16) << 12);
-    E.eb[u] = ((xacc >> 3) & 0xFu) | ((xacc >> 19) << 4);
-  }
-  if (nvalid < T) {      // padded rows: tier 0, code 0, sign/mantissa 0
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (unit_token<KIND>(a, q, u) >= nvalid) { E.tag[u] = 0u; g24[u] = 0u; slo[u] = 0u; shi[u] = 0u; }
+    for (int i = 0; i < 4; ++i) c[i] = fit3 ? d3[i] : (fit4 ? d4[i] : W[i]);
+    // code of element i to bits 3i, of element i+4 to 16 + 3i; 4th code bits to 7 + i and 23 + i
+    const u32 cacc = ((c[0] >> 7) & 0x00070007u) | ((c[1] >> 4) & 0x00380038u) | ((c[2] >> 1) & 0x01C001C0u) | ((c[3] << 2) & 0x0E000E00u);
+    const u32 xacc = ((d4[0] >> 3) & 0x00800080u) | ((d4[1] >> 2) & 0x01000100u) | ((d4[2] >> 1) & 0x02000200u) | (d4[3] & 0x04000400u);
+    g24[u] = (cacc & 0xFFFu) | ((cacc >> 4) & ~0xFFFu);
+    u32 tag = fit3 ? 0u : (fit4 ? 1u : 3u);
+    if (nvalid < T && unit_token<KIND>(a, q, u) >= nvalid) { tag = 0u; g24[u] = 0u; slo[u] = 0u; shi[u] = 0u; }      // padded rows: tier 0, code 0, sign/mantissa 0
+    E.tag8 |= tag << (2 * u);
+    E.eb |= (((xacc >> 7) & 0xFu) | ((xacc >> 19) & 0xF0u)) << (8 * u);
   }
   u32x4 s0 = {slo[0], shi[0], slo[1], shi[1]}, s1 = {slo[2], shi[2], slo[3], shi[3]};
   const u32 c0 = g24[0] | (g24[1] << 24), c1 = (g24[1] >> 8) | (g24[2] << 16), c2 = (g24[2] >> 16) | (g24[3] << 8);
@@ -155,28 +139,37 @@ __device__ __forceinline__ int encode_staged_tile(const EncodeLds& L, const Base
     __builtin_nontemporal_store(c0, cd); __builtin_nontemporal_store(c1, cd + 64); __builtin_nontemporal_store(c2, cd + 128);
   } else { sm[0] = s0; sm[64] = s1; cd[0] = c0; cd[64] = c1; cd[128] = c2; }
   // tag word of line a: this lane owns bits 8q..8q+7 (its four units)
-  const u32 f = quad_rows_or((E.tag[0] | (E.tag[1] << 2) | (E.tag[2] << 4) | (E.tag[3] << 6)) << (8 * q));
+  const u32 f = quad_rows_or(E.tag8 << (8 * q));
   if (lane < T) flags_tile[lane] = (int)f;
   const u32 rb = (u32)esc_bytes(f), incl = row_scan16(rb);
   E.pos = (int)(incl - rb) + esc_prefix(f, 8 * q);
   return __builtin_amdgcn_readlane((int)incl, 15);
 }
-// The escape bytes of an encoded tile, to esc_tile (the tile's first) on
-__device__ __forceinline__ void write_tile_escapes(const UnitEscapes& E, uint8_t* esc_tile) {
+// The escape bytes of an encoded tile, to esc_tile (the tile's first) on.  L: the tile's rows.
+template <int KIND>
+__device__ __forceinline__ void write_tile_escapes(const EncodeLds& L, const UnitEscapes& E, uint8_t* esc_tile, int lane) {
   uint8_t* p = esc_tile + E.pos;
+  if (__builtin_amdgcn_ballot_w64((E.tag8 & 0xAAu) != 0u) == 0) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if ((E.tag8 >> (2 * u)) & 1u) p[__popc(E.tag8 & ((1u << (2 * u)) - 1u))] = (uint8_t)(E.eb >> (8 * u));
+    return;
+  }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    if (E.tag[u] == 1u) p[0] = (uint8_t)E.eb[u];
-    else if (E.tag[u] == 3u) {
+    const u32 tag = (E.tag8 >> (2 * u)) & 3u;
+    if (tag == 1u) p[0] = (uint8_t)(E.eb >> (8 * u));
+    else if (tag == 3u) {
       // raw group: the upper five exponent bits of the eight elements, 40 bits little-endian (element i at bit 5i)
-      u32 hl = 0u, hh = 0u;
+      u32 W[4], slo, shi, hl = 0u, hh = 0u;
+      unit_words<KIND>(L, lane & 15, lane >> 4, u, W, slo, shi);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) { hl |= ((E.ew[u][i] >> 3) & 0x1Fu) << (5 * i); hh |= ((E.ew[u][i] >> 19) & 0x1Fu) << (5 * i); }
+      for (int i = 0; i < 4; ++i) { hl |= ((W[i] >> 10) & 0x1Fu) << (5 * i); hh |= ((W[i] >> 26) & 0x1Fu) << (5 * i); }
       const u64 h = (u64)hl | ((u64)hh << 20);
 #pragma unroll
       for (int k = 0; k < 5; ++k) p[k] = (uint8_t)(h >> (8 * k));
     }
-    p += tag_size(E.tag[u]);
+    p += tag_size(tag);
   }
 }
 
@@ -291,10 +284,7 @@ __device__ __forceinline__ void decode_tile_staged(const uint8_t* __restrict__ s
                                                    DecodeLds<KIND>& L, u16* __restrict__ out, long row_stride) {
   const int a = lane & 15, q = lane >> 4;
   const u32 f = (u32)flags_tile[a];
-  // base words 2 lane, 2 lane + 1 of the table
-  const uint8_t* row = lane < 32 ? b3row : b4row;
-  const int g = (lane >> 1) & 15, p = 2 * (lane & 1);
-  const u32 l0 = row[chan_of<KIND>(8 * g + p)], h0 = row[chan_of<KIND>(8 * g + p + 4)], l1 = row[chan_of<KIND>(8 * g + p + 1)], h1 = row[chan_of<KIND>(8 * g + p + 5)];
+  const u32x2 base_pair = load_base_pair<KIND>(b3row, b4row, lane);
   Payload P;
   load_payload<false>(sm_tile, cd_tile, lane, P);
   const u32 rb = (u32)esc_bytes(f), tag8 = __builtin_amdgcn_ubfe(f, 8 * q, 8);
@@ -303,7 +293,7 @@ __device__ __forceinline__ void decode_tile_staged(const uint8_t* __restrict__ s
   // (no escapes: any word that is there)
   const uintptr_t e0 = nb ? reinterpret_cast<uintptr_t>(esc) : reinterpret_cast<uintptr_t>(flags_tile), ea = e0 & ~(uintptr_t)3, ez = (e0 + max(nb - 1, 0)) & ~(uintptr_t)3;
   const u32 w0 = *reinterpret_cast<const u32*>(ea), w1 = *reinterpret_cast<const u32*>(min(ea + 4, ez)), w2 = *reinterpret_cast<const u32*>(ez);
-  reinterpret_cast<u32x2*>(&L.bw[0][0])[lane] = u32x2{(l0 << 7) | (h0 << 23), (l1 << 7) | (h1 << 23)};
+  reinterpret_cast<u32x2*>(&L.bw[0][0])[lane] = base_pair;
   wave_lds_sync();
   u32x4 bw[4];
 #pragma unroll

@@ -35,7 +35,7 @@ __device__ __forceinline__ int pop_raw_tile(const PagedStoreArgs& A, int lane) {
 }
 
 template <int KIND>
-__device__ __forceinline__ void store_tile(const PagedStoreArgs& A, EncodeLds& L, int e, int t, int kvh, int lane) {
+__device__ __forceinline__ void store_tile(const PagedStoreArgs& A, EncodeLds& L, BaseTable& B, int e, int t, int kvh, int lane) {
   const int blk = A.ent[4 * e], tok0 = A.ent[4 * e + 1], off0 = A.ent[4 * e + 2], n = A.ent[4 * e + 3];
   const int qi = e * 2 * A.n_kv + t;
   if (blk < 0 || n <= 0 || off0 < 0 || off0 + n > T) { if (lane == 0) A.freeq[qi] = -1; return; }
@@ -65,15 +65,13 @@ __device__ __forceinline__ void store_tile(const PagedStoreArgs& A, EncodeLds& L
         for (int k = 0; k < 4; ++k) if (4 * k + (lane >> 4) < off0) R.v[k] = u32x4{0u, 0u, 0u, 0u};
       }
     }
-    stage_bases(L, (KIND == KIND_K ? A.b3k : A.b3v) + (long)kvh * D, (KIND == KIND_K ? A.b4k : A.b4v) + (long)kvh * D, lane);
+    reinterpret_cast<u32x2*>(&B.w[0][0])[lane] = load_base_pair<KIND>((KIND == KIND_K ? A.b3k : A.b3v) + (long)kvh * D, (KIND == KIND_K ? A.b4k : A.b4v) + (long)kvh * D, lane);
     store_rows(L, R, lane);
     wave_lds_sync();
-    BaseRegs Bs;
-    load_base_regs<KIND>(L, lane & 15, lane >> 4, Bs);
     uint8_t* slot = A.pool + p * A.TS;
     UnitEscapes E;
-    fits = encode_staged_tile<KIND, false>(L, Bs, T, lane, slot, slot + SLOT_CD, reinterpret_cast<int*>(slot + SLOT_FL), E) <= A.ovf_slot;
-    if (fits) write_tile_escapes(E, slot + SLOT_OV);
+    fits = encode_staged_tile<KIND, false>(L, B, T, lane, slot, slot + SLOT_CD, reinterpret_cast<int*>(slot + SLOT_FL), E) <= A.ovf_slot;
+    if (fits) write_tile_escapes<KIND>(L, E, slot + SLOT_OV, lane);
   }
   int r = r_old;
   if (!fits) {      // the rows stay raw: a filling block, or a finished tile whose escapes exceed the slot
@@ -103,9 +101,10 @@ __device__ __forceinline__ void store_tile(const PagedStoreArgs& A, EncodeLds& L
 // loaded one after the other.
 __global__ void __launch_bounds__(64) k_paged_store(const PagedStoreArgs A) {
   __shared__ EncodeLds L;
+  __shared__ BaseTable B;
   const int e = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
-  if (t & 1) store_tile<KIND_V>(A, L, e, t, t >> 1, lane);
-  else store_tile<KIND_K>(A, L, e, t, t >> 1, lane);
+  if (t & 1) store_tile<KIND_V>(A, L, B, e, t, t >> 1, lane);
+  else store_tile<KIND_K>(A, L, B, e, t, t >> 1, lane);
 }
 
 __global__ void __launch_bounds__(256) k_paged_free(const int* __restrict__ freeq, int n_items, int* __restrict__ stack, int* __restrict__ top) {
