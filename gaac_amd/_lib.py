@@ -68,7 +68,9 @@ def load():
 
 
 class _CtypesCalls:
-    """calls() through ctypes, for any torch: 14 us for an attention() where the binding takes 8 to 11."""
+    """calls() through ctypes, for any torch: 14 us for an attention() where the binding takes 8 to 11.  The whole calls (binding.cpp) are left to Python."""
+    def attend(self, *args): return None
+    token_append = prompt_store = page_encode = page_decode = attend
     def __getattr__(self, name):
         fn, n, error = getattr(load(), name), len(_SIGNATURES[name]), load().gaac_last_error
         def entry(*args):
@@ -84,7 +86,8 @@ class _CtypesCalls:
 def calls():
     """The entry points as functions, in the order of arguments of include/gaac_hip.h: tensors on the device, addresses or None for pointers,
     numbers, last the stream (its handle, or the function `stream`).  They raise RuntimeError with the library's message.  The binding reads
-    tensors by the layout of the torch that it was built with, and is left alone where another one is installed."""
+    tensors by the layout of the torch that it was built with, and is left alone where another one is installed.  attend, token_append, prompt_store,
+    page_encode and page_decode make a public call as a whole, or return None and leave it to Python."""
     global _calls
     if _calls is None:
         load()

@@ -165,11 +165,19 @@ def encode_page(x: torch.Tensor, kind: str, base3: torch.Tensor, base4: torch.Te
     scratch(n, device): where the n bytes of slots and sizes come from, if not from torch's allocator."""
     H, S, _ = x.shape
     dev = x.device
+    st = _lib.stream
+    made = None if scratch else (_lib._calls or _lib.calls()).page_encode(x, 0 if kind == "k" else 1, base3, base4, n_kv, STREAM_ROOM, st)
+    if made:
+        sm, cd, flags, ovf_off, ovf, head_start, tile_off, totals, slots = made
+        if ovf is None:
+            ovf = torch.empty(stream_bytes(totals) + 8, dtype=torch.uint8, device=dev)
+            sizes = slots.data_ptr() + H * tile_off.shape[1] * TILE_MAX_ESC
+            _lib.call("gaac_page_pack", slots, sizes, tile_off, sizes + 4 * H * tile_off.shape[1], flags, H, S, flags.shape[1], head_start, ovf, ovf_off, st)
+        return Page(sm, cd, flags, ovf_off, ovf, head_start, tile_off, base3, base4, H, S, n_kv, kind)
     x, hs, rs = rows_in_place(x, 0, 1)
     S_pad = (S + T - 1) // T * T
     nt = H * (S_pad // T)
     new = lambda *shape, dtype=torch.uint8: torch.empty(shape, dtype=dtype, device=dev)
-    st = _lib.stream
     # each buffer is made when the next launch needs it
     sm, cd, flags = new(H, S_pad * D), new(H, S_pad * CB), new(H, S_pad, dtype=torch.int32)
     # slots | sizes per tile | per head
@@ -219,6 +227,8 @@ class Codec:
     @staticmethod
     def decode(page: Page) -> torch.Tensor:
         """The bf16 [H, S, D] tensor the page was made from, bit for bit."""
+        out = (_lib._calls or _lib.calls()).page_decode(page, _lib.stream)
+        if out is not None: return out
         H, S = page.H, page.S
         S_pad = page.sm.shape[1] // D
         out = torch.empty(H, S, D, dtype=torch.bfloat16, device=page.sm.device)
