@@ -9,6 +9,7 @@
 #include <dlfcn.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ops/empty.h>
+#include <algorithm>
 #include <exception>
 #include <tuple>
 #include <type_traits>
@@ -127,7 +128,7 @@ struct Refs {             // objects that are held until the call has been made 
 GAAC_NAMES(X)
 #undef X
 
-constexpr long DIM = 128, TILE = 16, CODE_BYTES = 48, TILE_ESCAPES = 1280, HIST_BYTES = 256 * 64 * 8;
+constexpr long DIM = 128, TILE = 16, CODE_BYTES = 48, TILE_ESCAPES = 1280, HIST_BYTES = 256 * 64 * 4 + 32;
 
 const at::Tensor& tensor(PyObject* o) {
   if (!THPVariable_CheckExact(o)) throw Otherwise{};
@@ -282,8 +283,9 @@ PyObject* prompt_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int *tail_len = address<int>(get(a[0], n_tail_len)), *S = address<int>(get(a[0], n_S)), *head_start = address<int>(get(ko, n_head_start));
     const long ovf_cap = number(get(ko, n_ovf_cap)), nb = tensor(get(ko, n_base3)).size(0);
     void* stream = stream_of(a[4]);
-    // scratch: escape slots | packed histogram | tile sizes | head sizes
-    const long at_hist = nt * TILE_ESCAPES, at_sizes = at_hist + (calibrate ? 2 * n_kv * HIST_BYTES : 0);
+    // scratch: escape slots | exponent counts (hist_bytes in kv_cache.py) | tile sizes | head sizes
+    const long tables = 2 * n_kv * std::max(std::min((L + 255) / 256, std::max(256 / (2 * n_kv), 1l)), (L + 65534) / 65535);
+    const long at_hist = nt * TILE_ESCAPES, at_sizes = at_hist + (calibrate ? tables * HIST_BYTES : 0);
     at::Tensor scratch = bytes(k, {at_sizes + 4 * (nt + 2 * n_kv)}), totals = host_words(2 * n_kv);
     uint8_t* base = static_cast<uint8_t*>(scratch.data_ptr());
     int* words = static_cast<int*>(totals.data_ptr());
@@ -291,7 +293,7 @@ PyObject* prompt_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
     must(at, without_gil([&] {
       return p_gaac_cache_prefill(k.data_ptr(), v.data_ptr(), k_hs, k_rs, v_hs, v_rs, static_cast<int>(L), static_cast<int>(n_kv), static_cast<int>(slot * n_kv), static_cast<int>(cap),
                                   static_cast<int>(ovf_cap), static_cast<int>(nb), calibrate, tail_len, S, head_start, K.tail, K.b3, K.b4, K.sm, K.cd, K.fl, K.ov, K.to, K.used,
-                                  V.tail, V.b3, V.b4, V.sm, V.cd, V.fl, V.ov, V.to, V.used, reinterpret_cast<unsigned long long*>(base + at_hist), base,
+                                  V.tail, V.b3, V.b4, V.sm, V.cd, V.fl, V.ov, V.to, V.used, base + at_hist, at_sizes - at_hist, base,
                                   reinterpret_cast<int*>(base + at_sizes), reinterpret_cast<int*>(base + at_sizes + 4 * nt), words, stream);
     }));
     must("gaac_wait_words", without_gil([&] { return p_gaac_wait_words(words, static_cast<int>(2 * n_kv), stream); }));

@@ -23,12 +23,13 @@ char* last_error_buffer() { static thread_local char buf[512] = {0}; return buf;
 // Bound by the reads (without counting at all: 29 us with the launch).  K and V of 32768 tokens x 8 kv heads, 134 MB: 27.3 us = 4.9 TB/s; eight waves that read
 // 4 bytes a lane, sixteen rows at a time, 28.4 with whole batches and 33 with the rest of a chunk row by row: a prompt of 30011 tokens 90.2 us a call
 // -> 86.6, of 12345 62.7 -> 57.3, of 4000 44.2 -> 40.3, of 32768 91.3 -> 90.4.  More loads in flight are slower: 28.2 with three, 27.9 with eight.
-// Non-zero counts are added to the global histogram at the end: PACKED = false: 64-bit counts hist[row][256], the layout that
-// gaac_exponent_hist hands out; PACKED = true: scratch[pair][bin][64] with the two 32-bit counts of a lane in one 64-bit word, so that a
-// wave's adds of a bin are one contiguous 512-byte access (prompts of up to 2^32 - 1 tokens).
+// PARTS = false: the non-zero counts are added to 64-bit ones at the end, hist[row][256], the layout that gaac_exponent_hist hands out.  PARTS = true: a block leaves
+// its own table, the rows (bins) of it that hold a count, and a bit for each of these; k_prompt_bases adds up the blocks' tables.  Added to one global table,
+// which a launch had to clear first, the counts of a prompt took that launch longer: 32768 tokens x 8 heads 88.1 -> 83.2 us a call, 4000 tokens 26.2 -> 24.5 of
+// kernels.
 constexpr int HIST_WAVES = 16, HIST_MAX_CHUNK = 65535, HIST_LOADS = 2;      // HIST_LOADS: loads of four rows in flight per wave
-struct HistArgs { const u16* x[2]; long head_stride[2], row_stride[2]; long n_tok; int chunk, n_kv; unsigned long long* hist; };
-template <bool PACKED>
+struct HistArgs { const u16* x[2]; long head_stride[2], row_stride[2]; long n_tok; int chunk, n_kv; unsigned long long* hist; u32* rows; u16* bits; };      // rows [pair][chunk][256][64], bits [pair][chunk][16]
+template <bool PARTS>
 __global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArgs A) {
   __shared__ u32 h[256 * 64];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, head = blockIdx.y, kind = blockIdx.z;
@@ -71,50 +72,94 @@ __global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArg
   }
   __syncthreads();
   const long pair = (long)kind * A.n_kv + head;
+  const int word = 4 * (lane & 15) + (lane >> 4);      // of the row, that the lane counted
+  if (PARTS) {
+    constexpr int BINS = 256 / HIST_WAVES;      // a wave's, every sixteenth: the ones in use lie side by side
+    const long at = pair * gridDim.x + blockIdx.x;
+    u32* rows = A.rows + at * (256 * 64);
+    u32 c[BINS], bits = 0u;
+#pragma unroll
+    for (int i = 0; i < BINS; ++i) c[i] = h[64 * (wave + HIST_WAVES * i) + lane];
+#pragma unroll
+    for (int i = 0; i < BINS; ++i)
+      if (__builtin_amdgcn_ballot_w64(c[i] != 0u) != 0) { rows[64 * (wave + HIST_WAVES * i) + word] = c[i]; bits |= 1u << i; }
+    if (lane == 0) A.bits[at * HIST_WAVES + wave] = (u16)bits;
+    return;
+  }
   for (int i = tid; i < 256 * 64; i += 64 * HIST_WAVES) {
     const u32 c = h[i];
     if (c == 0u) continue;
-    const int word = 4 * (i & 15) + ((i >> 4) & 3);      // of the row, that the lane counted
-    if (PACKED) atomicAdd(&A.hist[pair * (256 * 64) + (i & ~63) + word], (unsigned long long)(c & 0xFFFFu) | ((unsigned long long)(c >> 16) << 32));
-    else {
-      unsigned long long* row = A.hist + (pair * D + 2 * word) * 256 + (i >> 6);
-      if (c & 0xFFFFu) atomicAdd(row, (unsigned long long)(c & 0xFFFFu));
-      if (c >> 16) atomicAdd(row + 256, (unsigned long long)(c >> 16));
-    }
+    unsigned long long* row = A.hist + (pair * D + 2 * word) * 256 + (i >> 6);
+    if (c & 0xFFFFu) atomicAdd(row, (unsigned long long)(c & 0xFFFFu));
+    if (c >> 16) atomicAdd(row + 256, (unsigned long long)(c >> 16));
   }
 }
-static void launch_hist(HistArgs& A, int kinds, bool packed, hipStream_t stream) {
+static int hist_chunks(long n_tok, int pairs) {
   // one block per CU, at least 256 tokens each, so that clearing and scanning the 64 KB table stays the smaller part (two blocks per CU,
   // which the LDS has room for: 26 against 23.6 us for 2 x 8 heads x 32768 tokens out of the Infinity Cache, measured with blocks of eight waves)
-  const int pairs = kinds * A.n_kv;
-  long nchunk = min((A.n_tok + 255) / 256, (long)max(1, 256 / pairs));
-  nchunk = max(nchunk, (A.n_tok + HIST_MAX_CHUNK - 1) / HIST_MAX_CHUNK);
+  const long n = min((n_tok + 255) / 256, (long)max(1, 256 / pairs));
+  return (int)max(n, (n_tok + HIST_MAX_CHUNK - 1) / HIST_MAX_CHUNK);
+}
+static int launch_hist(HistArgs& A, int kinds, hipStream_t stream) {      // returns the blocks of a (kind, head), hist_chunks at most
+  const int nchunk = hist_chunks(A.n_tok, kinds * A.n_kv);
   A.chunk = (int)((A.n_tok + nchunk - 1) / nchunk);
   const dim3 grid((unsigned)((A.n_tok + A.chunk - 1) / A.chunk), A.n_kv, kinds);
-  if (packed) hipLaunchKernelGGL(k_exponent_hist<true>, grid, dim3(64 * HIST_WAVES), 0, stream, A);
+  if (A.rows) hipLaunchKernelGGL(k_exponent_hist<true>, grid, dim3(64 * HIST_WAVES), 0, stream, A);
   else hipLaunchKernelGGL(k_exponent_hist<false>, grid, dim3(64 * HIST_WAVES), 0, stream, A);
+  return (int)grid.x;
 }
 
-// The bases of K and V of a prompt from the packed histogram scratch, written to base row row0 + head of the two kinds' tables.  A block
-// takes 32 channels of one (kind, head): their 256 counts in LDS, thread (channel, eighth) slides the two windows over 32 starts.
-struct PromptBasesArgs { const u64* hist; uint8_t* b3[2]; uint8_t* b4[2]; int n_kv, row0; };
-__global__ void __launch_bounds__(256) k_prompt_bases(const PromptBasesArgs A) {
+// The bases of K and V of a prompt from the tables of its k_exponent_hist<true>, written to base row row0 + head of the two kinds' tables.  A block takes 32 channels
+// of one (kind, head): a wave adds up every sixteenth row over the tables, the 256 sums of a channel go to LDS, thread (channel, eighth) slides the two windows over
+// 32 starts.  Latency: two trips to memory, bits and rows.  (A table a wave and LDS atomics for the sums: 6.4 us instead of 4.8.)
+struct PromptBasesArgs { const u32* rows; const u16* bits; int chunks; uint8_t* b3[2]; uint8_t* b4[2]; int n_kv, row0; };
+__global__ void __launch_bounds__(1024) k_prompt_bases(const PromptBasesArgs A) {
   constexpr int STRIDE = 256 + 17;      // odd: the 32 channels of a bin sit in different banks
   __shared__ u32 cnt[32 * STRIDE];
   __shared__ u32 best[2][8][32];
   __shared__ int arg[2][8][32];
   const int tid = threadIdx.x, grp = blockIdx.x, head = blockIdx.y, kind = blockIdx.z;
-  const u64* hp = A.hist + ((long)kind * A.n_kv + head) * (256 * 64) + 16 * grp;
-  u64 w[16];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) { const int i = tid + 256 * k; w[k] = hp[(i >> 4) * 64 + (i & 15)]; }
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const int i = tid + 256 * k, bin = i >> 4, c = 2 * (i & 15);
-    cnt[c * STRIDE + bin] = (u32)w[k]; cnt[(c + 1) * STRIDE + bin] = (u32)(w[k] >> 32);
-  }
-  const int c = tid & 31, part = tid >> 5, st0 = 32 * part;
+  for (int i = tid; i < 32 * STRIDE; i += 1024) cnt[i] = 0u;
   __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const long at0 = ((long)kind * A.n_kv + head) * A.chunks;
+  u32* sums = cnt + 2 * (lane & 15) * STRIDE + wave;
+  for (int c0 = 0; c0 < A.chunks; c0 += 16) {
+    // lane (j, w): word w of the channels' sixteen, of the tables c0 + j, c0 + 4 + j, ...
+    u32 has[4];
+    const u32* rows[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int chunk = c0 + 4 * r + (lane >> 4);
+      const long at = at0 + min(chunk, A.chunks - 1);
+      has[r] = A.bits[at * HIST_WAVES + wave];
+      has[r] = chunk < A.chunks ? has[r] : 0u;
+      rows[r] = A.rows + at * (256 * 64) + 64 * wave + 16 * grp + (lane & 15);
+    }
+    u32 left = __builtin_amdgcn_readfirstlane(quad_rows_or(has[0] | has[1] | has[2] | has[3]));
+    while (left) {      // two rows at a time, four tables a lane
+      const int i0 = __builtin_ctz(left);
+      left &= left - 1;
+      const int i1 = left ? __builtin_ctz(left) : i0;
+      u32 v0[4], v1[4], lo0 = 0u, hi0 = 0u, lo1 = 0u, hi1 = 0u;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) { v0[r] = rows[r][64 * HIST_WAVES * i0]; v1[r] = rows[r][64 * HIST_WAVES * i1]; }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v0[r] = (has[r] >> i0) & 1u ? v0[r] : 0u; v1[r] = (has[r] >> i1) & 1u ? v1[r] : 0u;      // (a row without the bit holds anything)
+        lo0 += v0[r] & 0xFFFFu; hi0 += v0[r] >> 16; lo1 += v1[r] & 0xFFFFu; hi1 += v1[r] >> 16;
+      }
+      lo0 = quad_rows_add(lo0); hi0 = quad_rows_add(hi0); lo1 = quad_rows_add(lo1); hi1 = quad_rows_add(hi1);
+      if (lane < 16) {
+        sums[HIST_WAVES * i0] += lo0; sums[STRIDE + HIST_WAVES * i0] += hi0;
+        if (left) { sums[HIST_WAVES * i1] += lo1; sums[STRIDE + HIST_WAVES * i1] += hi1; }
+      }
+      left &= left - 1;
+    }
+  }
+  __syncthreads();
+  const int c = tid & 31, part = (tid >> 5) & 7, st0 = 32 * part;
+  if (tid < 256) {
   u32 n[32 + 15];      // the counts that the thread's windows cover, read together
 #pragma unroll
   for (int i = 0; i < 32 + 15; ++i) n[i] = cnt[c * STRIDE + min(st0 + i, 255)];
@@ -131,6 +176,7 @@ __global__ void __launch_bounds__(256) k_prompt_bases(const PromptBasesArgs A) {
       if (st0 + i + win <= 256 && sum > b) { b = sum; a = st0 + i; }
     }
     best[pass][part][c] = b; arg[pass][part][c] = a;
+  }
   }
   __syncthreads();
   if (tid < 64) {
@@ -579,10 +625,6 @@ __global__ void __launch_bounds__(256) k_prompt_pack(const PromptPackArgs P) {
 __global__ void __launch_bounds__(64) k_words_to_host(const int* __restrict__ words, int n, int* __restrict__ host) {
   for (int i = threadIdx.x; i < n; i += 64) store_to_host(host + i, words[i]);
 }
-__global__ void __launch_bounds__(256) k_zero16(u32x4* __restrict__ p, long n16) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < n16) p[i] = u32x4{0u, 0u, 0u, 0u};
-}
 
 }  // namespace gaac
 
@@ -612,8 +654,8 @@ int gaac_exponent_hist(const void* x, long n_tokens, int n_kv, long long* hist, 
   GAAC_REQUIRE(x && hist && n_kv > 0 && n_tokens >= 0, "gaac_exponent_hist: bad arguments");
   if (n_tokens == 0) return 0;
   const long row = (long)n_kv * D;
-  HistArgs A{{(const u16*)x, nullptr}, {D, 0}, {row, 0}, n_tokens, 0, n_kv, (unsigned long long*)hist};
-  launch_hist(A, 1, false, (hipStream_t)stream);
+  HistArgs A{{(const u16*)x, nullptr}, {D, 0}, {row, 0}, n_tokens, 0, n_kv, (unsigned long long*)hist, nullptr, nullptr};
+  launch_hist(A, 1, (hipStream_t)stream);
   return launch_status("gaac_exponent_hist");
 }
 
@@ -716,25 +758,28 @@ int gaac_cache_prefill(
     int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
     void* k_tail, uint8_t* k_base3, uint8_t* k_base4, uint8_t* k_sm, uint8_t* k_codes, int* k_flags, uint8_t* k_ovf, int* k_tile_off, int* k_ovf_used,
     void* v_tail, uint8_t* v_base3, uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
-    unsigned long long* hist, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, int* host_bytes, void* stream) {
+    void* hist, long hist_bytes, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, int* host_bytes, void* stream) {
   GAAC_REQUIRE(((k && v) || L == 0) && tail_len && S && head_start && head_bytes, "gaac_cache_prefill: null pointer");
   GAAC_REQUIRE(k_tail && k_base3 && k_base4 && k_sm && k_codes && k_flags && k_ovf && k_tile_off && k_ovf_used, "gaac_cache_prefill: null K store pointer");
   GAAC_REQUIRE(v_tail && v_base3 && v_base4 && v_sm && v_codes && v_flags && v_ovf && v_tile_off && v_ovf_used, "gaac_cache_prefill: null V store pointer");
   GAAC_REQUIRE(L >= 0 && n_kv > 0 && head0 >= 0 && cap > 0 && cap % T == 0 && L <= cap && NB > 0 && ovf_cap >= 8,
                "gaac_cache_prefill: bad sizes L=%d n_kv=%d head0=%d cap=%d ovf_cap=%d NB=%d", L, n_kv, head0, cap, ovf_cap, NB);
   GAAC_REQUIRE(!calibrate || (hist && NB >= head0 + n_kv), "gaac_cache_prefill: calibration needs its scratch and a base row per cache head (NB=%d, heads %d..%d)", NB, head0, head0 + n_kv - 1);
+  const long tables = calibrate ? (long)2 * n_kv * hist_chunks(L, 2 * n_kv) : 0;
+  GAAC_REQUIRE(tables * (256 * 64 * (long)sizeof(u32) + 32) <= hist_bytes || tables == 0, "gaac_cache_prefill: %ld bytes of calibration scratch for %ld tables", hist_bytes, tables);
+  GAAC_REQUIRE((reinterpret_cast<uintptr_t>(hist) & 7) == 0, "gaac_cache_prefill: calibration scratch is not aligned to 8 bytes");
   const int ntiles = L / T;
   GAAC_REQUIRE(ntiles == 0 || (esc_slots && tile_bytes), "gaac_cache_prefill: null scratch");
   GAAC_REQUIRE(L == 0 || (k_row_stride >= D && k_row_stride % 8 == 0 && k_head_stride % 8 == 0 && v_row_stride >= D && v_row_stride % 8 == 0 && v_head_stride % 8 == 0 &&
                           ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0), "gaac_cache_prefill: rows must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
   if (calibrate) {
-    const long n16 = (long)n_kv * 2 * 256 * 64 * (long)sizeof(u64) / 16;
-    hipLaunchKernelGGL(k_zero16, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, reinterpret_cast<u32x4*>(hist), n16);
-    HistArgs H{{(const u16*)k, (const u16*)v}, {k_head_stride, v_head_stride}, {k_row_stride, v_row_stride}, L, 0, n_kv, hist};
-    if (L > 0) launch_hist(H, 2, true, st);
-    const PromptBasesArgs B{reinterpret_cast<const u64*>(hist), {k_base3, v_base3}, {k_base4, v_base4}, n_kv, head0};
-    hipLaunchKernelGGL(k_prompt_bases, dim3(4, n_kv, 2), dim3(256), 0, st, B);
+    u32* rows = (u32*)hist;
+    u16* bits = reinterpret_cast<u16*>(rows + tables * (256 * 64));
+    HistArgs H{{(const u16*)k, (const u16*)v}, {k_head_stride, v_head_stride}, {k_row_stride, v_row_stride}, L, 0, n_kv, nullptr, rows, bits};
+    const int chunks = L > 0 ? launch_hist(H, 2, st) : 0;
+    const PromptBasesArgs B{rows, bits, chunks, {k_base3, v_base3}, {k_base4, v_base4}, n_kv, head0};
+    hipLaunchKernelGGL(k_prompt_bases, dim3(4, n_kv, 2), dim3(1024), 0, st, B);
   }
   const long row0 = (long)head0 * cap, tile0 = (long)head0 * (cap / T), n_all = (long)n_kv * ntiles;
   uint8_t* v_slots = esc_slots ? esc_slots + n_all * TILE_MAX_ESC : nullptr;

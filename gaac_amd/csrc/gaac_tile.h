@@ -95,6 +95,14 @@ __device__ __forceinline__ u32 quad_rows_or(u32 x) {
   return s[0] | s[1];
 }
 
+// ... and their sum
+__device__ __forceinline__ u32 quad_rows_add(u32 x) {
+  auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  x = r[0] + r[1];
+  auto s = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  return s[0] + s[1];
+}
+
 // Encodes the tile staged in L (after a barrier).  Writes the native sign/mantissa and code bytes and the 16 tag words (one per line); the
 // escape bytes stay with the lanes for write_tile_escapes, so that a caller can see their number before it says where they go.
 // Returns the tile's escape byte count (all lanes).  Must be called by all 64 lanes of the wave that owns L.  B: the head's base words.
