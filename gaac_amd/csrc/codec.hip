@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(256) k_bases_from_hist(const long long* __rest
 // launched), and makes the head's base words for all of them.  K and V of a prompt share a launch (blockIdx.z): one start-up and one drain for both.
 // Bound by the memory rate.  A wave has one tile and 62 registers: eight waves a SIMD hide each other's trips to memory.  Before, a wave took four tiles in
 // a row with the rows of the next one and all base words in registers, 147 of them: three waves a SIMD and a quarter more instructions a tile; 64K page of 8 heads
-// out of memory 47.9 -> 45.0 us (229 MB, 5.1 TB/s), 16K page 15.9 -> 14.6, prompt of 32768 tokens with given bases 49.1 -> 46.6.
+// out of memory 47.9 -> 45.0 us (with the slots of write_slot_escapes 41.5: 229 MB, 5.5 TB/s), 16K page 15.9 -> 14.6 (13.4), prompt of 32768 tokens with given bases 49.1 -> 46.6.
 // What goes past the caches is chosen by what comes next, so that the Infinity Cache keeps the rest:
 //   * the rows of a large launch (BIG) are read for the last time: 64K page 44.6 -> 42.3 us; the 32768-token prompt's call, where the histogram has
 //     just brought them in, 109 -> 101 us;
@@ -253,7 +253,7 @@ __device__ __forceinline__ void encode_tiles_body(const EncodeArgs& A, const Enc
   const long row0 = (long)h * A.S_pad + (long)tile * T;
   UnitEscapes E;
   const int total = encode_staged_tile<KIND, PROMPT>(L.w[wave], L.B, nvalid, lane, J.sm + row0 * D, J.cd + row0 * CB, J.flags + row0, E);
-  write_tile_escapes<KIND>(L.w[wave], E, J.slots + ((long)h * ntiles + tile) * TILE_MAX_ESC, lane);
+  write_slot_escapes<KIND>(L.w[wave], E, J.slots + (long)h * ntiles * TILE_MAX_ESC, tile, ntiles, total, lane);
   if (lane == 0) J.tile_bytes[(long)h * ntiles + tile] = total;
 }
 template <bool BIG, bool PROMPT>
@@ -340,7 +340,7 @@ __global__ void __launch_bounds__(256) k_pack(const PackArgs A) {
   const uint8_t* src = J.slots + (long)h * A.ntiles * TILE_MAX_ESC;
   u32 v[16];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, A.ntiles - 1) * TILE_MAX_ESC + lane];
+  for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, A.ntiles - 1) * ESC_HEAD + lane];
   long start = 0;
   bool fits = true;
   if (HEADS) {
@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(256) k_pack(const PackArgs A) {
     const int n = __builtin_amdgcn_readlane(nb, k), o = __builtin_amdgcn_readlane(of, k);
     if (k >= n_own || !fits) break;
     if (lane < n) dst[o + lane] = (uint8_t)v[k];
-    for (int i = 64 + lane; i < n; i += 64) dst[o + i] = src[(long)(t0 + k) * TILE_MAX_ESC + i];
+    for (int i = 64 + lane; i < n; i += 64) dst[o + i] = src[esc_rest(t0 + k, A.ntiles) + i];
   }
   if (HEADS) {      // row offsets: tile offset + the escape bytes of the tile's earlier tag words
     const int* fl = A.flags + (long)h * A.S_pad;
@@ -403,7 +403,7 @@ __global__ void __launch_bounds__(256) k_page_pack(const PagePackArgs A) {
   int n = A.tile_bytes[head0 + min(tile0 + lane, ntiles - 1)];
   u32 v[16], fl[4];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, ntiles - 1) * TILE_MAX_ESC + lane];
+  for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, ntiles - 1) * ESC_HEAD + lane];
 #pragma unroll
   for (int k = 0; k < 4; ++k) fl[k] = (u32)A.flags[(long)h * A.S_pad + min(t0 * T + 64 * k + lane, A.S_pad - 1)];
   int all = 0, heads = 0, before = 0, mine = 0;      // of all tiles, of the heads before, of the head's tiles before the block's, of the head
@@ -450,7 +450,7 @@ __global__ void __launch_bounds__(256) k_page_pack(const PagePackArgs A) {
     const int nk = __builtin_amdgcn_readlane(n, 16 * wave + k), o = __builtin_amdgcn_readlane(of, 16 * wave + k);
     if (k >= n_own) break;
     if (lane < nk) dst[o + lane] = (uint8_t)v[k];
-    for (int i = 64 + lane; i < nk; i += 64) dst[o + i] = src[(long)(t0 + k) * TILE_MAX_ESC + i];
+    for (int i = 64 + lane; i < nk; i += 64) dst[o + i] = src[esc_rest(t0 + k, ntiles) + i];
   }
 }
 
@@ -583,7 +583,7 @@ __global__ void __launch_bounds__(256) k_prompt_pack(const PromptPackArgs P) {
   int n = tb[min(tile0 + lane, ntiles - 1)];
   u32 v[16];
 #pragma unroll
-  for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, ntiles - 1) * TILE_MAX_ESC + lane];
+  for (int k = 0; k < 16; ++k) v[k] = src[(long)min(t0 + k, ntiles - 1) * ESC_HEAD + lane];
   int before = 0, all = 0, all_other = 0;
   for (int base = 0; base < ntiles; base += 256 * 8) {
     int w[8], x[8];
@@ -616,7 +616,7 @@ __global__ void __launch_bounds__(256) k_prompt_pack(const PromptPackArgs P) {
     const int nk = __builtin_amdgcn_readlane(n, 16 * wave + k), o = __builtin_amdgcn_readlane(of, 16 * wave + k);
     if (k >= n_own) break;
     if (lane < nk) dst[o + lane] = (uint8_t)v[k];
-    for (int i = 64 + lane; i < nk; i += 64) dst[o + i] = src[(long)(t0 + k) * TILE_MAX_ESC + i];
+    for (int i = 64 + lane; i < nk; i += 64) dst[o + i] = src[esc_rest(t0 + k, ntiles) + i];
   }
 }
 // The prompt's totals into host memory that the host polls, in a launch of its own: by the time they are there all of the prompt is.  Polling spares

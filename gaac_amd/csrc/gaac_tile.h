@@ -181,6 +181,54 @@ __device__ __forceinline__ void write_tile_escapes(const EncodeLds& L, const Uni
   }
 }
 
+// Collects the escape bytes of an encoded tile in LDS, where its rows were.
+template <int KIND>
+__device__ __forceinline__ const uint8_t* collect_escapes(EncodeLds& L, const UnitEscapes& E, int lane) {
+  uint8_t* out = reinterpret_cast<uint8_t*>(L.x);
+  uint8_t* p = out + E.pos;
+  if (__builtin_amdgcn_ballot_w64((E.tag8 & 0xAAu) != 0u) == 0) {
+    wave_lds_sync();      // (every lane has read its units)
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if ((E.tag8 >> (2 * u)) & 1u) p[__popc(E.tag8 & ((1u << (2 * u)) - 1u))] = (uint8_t)(E.eb >> (8 * u));
+  } else {
+    // raw group: the upper five exponent bits of the eight elements, 40 bits little-endian (element i at bit 5i)
+    u32 lo[4], hi[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      u32 W[4], slo, shi, hl = 0u, hh = 0u;
+      unit_words<KIND>(L, lane & 15, lane >> 4, u, W, slo, shi);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) { hl |= ((W[i] >> 10) & 0x1Fu) << (5 * i); hh |= ((W[i] >> 26) & 0x1Fu) << (5 * i); }
+      lo[u] = hl | (hh << 20); hi[u] = hh >> 12;
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const u32 tag = (E.tag8 >> (2 * u)) & 3u;
+      if (tag == 1u) p[0] = (uint8_t)(E.eb >> (8 * u));
+      else if (tag == 3u) {
+        p[0] = (uint8_t)lo[u]; p[1] = (uint8_t)(lo[u] >> 8); p[2] = (uint8_t)(lo[u] >> 16); p[3] = (uint8_t)(lo[u] >> 24); p[4] = (uint8_t)hi[u];
+      }
+      p += tag_size(tag);
+    }
+  }
+  wave_lds_sync();
+  return out;
+}
+// Into the worst-case slot of tile `tile` of a head with ntiles, whose 1280 bytes a tile start at slots: the first ESC_HEAD bytes of all tiles lie side by
+// side, behind them the rest of each (which a tile in a thousand has), and all of ESC_HEAD is written, whatever of it is used.  Bound by memory: a few bytes
+// at the start of every 1280, a partly written line each, were 7 us of a 64K page's 45 without being 1 % of its bytes; now 41.5, and the packing reads
+// whole lines.  (Where the bytes go at once, to a stream or a paged slot, write_tile_escapes is as fast without the way through LDS.)
+constexpr int ESC_HEAD = 64, ESC_REST = TILE_MAX_ESC - ESC_HEAD;
+__device__ __forceinline__ long esc_rest(int tile, int ntiles) { return (long)ntiles * ESC_HEAD + (long)tile * ESC_REST - ESC_HEAD; }      // where byte 0 of the tile would lie
+template <int KIND>
+__device__ __forceinline__ void write_slot_escapes(EncodeLds& L, const UnitEscapes& E, uint8_t* slots, int tile, int ntiles, int total, int lane) {
+  const uint8_t* from = collect_escapes<KIND>(L, E, lane);
+  if (lane < ESC_HEAD / 4) reinterpret_cast<u32*>(slots + (long)tile * ESC_HEAD)[lane] = reinterpret_cast<const u32*>(from)[lane];
+  for (int i = ESC_HEAD + lane; i < total; i += 64) slots[esc_rest(tile, ntiles) + i] = from[i];
+}
+
 // Per-lane metadata of a stored tile: the 2-bit tag of each of the lane's four units and the offset of the unit's escape
 // bytes from the start of the tile's escape bytes.  tag_word = the tag word of the lane's line, flags_tile[lane & 15].
 struct UnitMeta { u32 tag[4]; int pos[4]; };

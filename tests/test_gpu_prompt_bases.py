@@ -27,3 +27,5 @@ def test_bases(L, n_kv, data):
     for x, st in ((k, cache.k), (v, cache.v)):
         b3, b4 = bases_from_hist(exponent_hist(x, n_kv), n_kv)
         assert torch.equal(st.base3[n_kv:], b3) and torch.equal(st.base4[n_kv:], b4)
+    if L < 10 ** 4:      # (of "bits", tiles of over a thousand escape bytes)
+        for got, x in zip(cache.decompress(1), (k, v)): assert torch.equal(got.view(torch.int16), x.view(torch.int16))
