@@ -123,7 +123,7 @@ struct Refs {             // objects that are held until the call has been made 
 };
 #define GAAC_NAMES(X)                                                                                                                        \
   X(k) X(v) X(sm) X(codes) X(flags) X(tile_off) X(ovf) X(head_start) X(ovf_head_start) X(base3) X(base4) X(tail) X(ovf_used) X(ovf_cap)     \
-  X(n_kv) X(cap) X(S) X(H) X(kind) X(tail_len) X(overflow) X(n_slots) X(per_sequence_bases) X(pm) X(pl) X(pa) X(epoch) X(rows) X(nslot)
+  X(n_kv) X(cap) X(S) X(H) X(kind) X(tail_len) X(overflow) X(n_slots) X(per_sequence_bases) X(_scan) X(pm) X(pl) X(pa) X(epoch) X(rows) X(nslot)
 #define X(name) PyObject* n_##name = nullptr;
 GAAC_NAMES(X)
 #undef X
@@ -282,6 +282,8 @@ PyObject* prompt_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const CacheStore K = cache_store(get, ko), V = cache_store(get, vo);
     int *tail_len = address<int>(get(a[0], n_tail_len)), *S = address<int>(get(a[0], n_S)), *head_start = address<int>(get(ko, n_head_start));
     const long ovf_cap = number(get(ko, n_ovf_cap)), nb = tensor(get(ko, n_base3)).size(0);
+    const at::Tensor& scan = tensor(get(a[0], n__scan));
+    const long scan_row = scan.stride(1);
     void* stream = stream_of(a[4]);
     // scratch: escape slots | exponent counts (hist_bytes in kv_cache.py) | tile sizes | head sizes
     const long tables = 2 * n_kv * std::max(std::min((L + 255) / 256, std::max(256 / (2 * n_kv), 1l)), (L + 65534) / 65535);
@@ -294,7 +296,8 @@ PyObject* prompt_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return p_gaac_cache_prefill(k.data_ptr(), v.data_ptr(), k_hs, k_rs, v_hs, v_rs, static_cast<int>(L), static_cast<int>(n_kv), static_cast<int>(slot * n_kv), static_cast<int>(cap),
                                   static_cast<int>(ovf_cap), static_cast<int>(nb), calibrate, tail_len, S, head_start, K.tail, K.b3, K.b4, K.sm, K.cd, K.fl, K.ov, K.to, K.used,
                                   V.tail, V.b3, V.b4, V.sm, V.cd, V.fl, V.ov, V.to, V.used, base + at_hist, at_sizes - at_hist, base,
-                                  reinterpret_cast<int*>(base + at_sizes), reinterpret_cast<int*>(base + at_sizes + 4 * nt), words, stream);
+                                  reinterpret_cast<int*>(base + at_sizes), reinterpret_cast<int*>(base + at_sizes + 4 * nt),
+                                  static_cast<unsigned long long*>(scan.data_ptr()) + slot * n_kv * scan_row, scan.stride(0), words, stream);
     }));
     must("gaac_wait_words", without_gil([&] { return p_gaac_wait_words(words, static_cast<int>(2 * n_kv), stream); }));
     return numbers(totals);

@@ -619,6 +619,92 @@ __global__ void __launch_bounds__(256) k_prompt_pack(const PromptPackArgs P) {
     for (int i = 64 + lane; i < nk; i += 64) dst[o + i] = src[esc_rest(t0 + k, ntiles) + i];
   }
 }
+// Short prompts (SCAN_PROMPT_TILES, SCAN_PROMPT_ALL_TILES): encoding, tile offsets and the escapes' way into the stream in one launch.  A block of four tiles says how many bytes it has
+// in a 64-bit word that carries the launch's epoch, waits for the words of the head's earlier blocks and puts its escapes, which are in LDS until then, behind theirs.
+// scan: [1 + SCAN_PROMPT_BLOCKS] words for K or V of a cache head, zeroed once: [0] the epoch of the last launch, which every block reads at its start and the
+// head's last block, when it has seen the words of all, advances.  Launches on one cache head are ordered on a stream, as its contents demand.  A block waits for
+// blocks with a smaller index, which start before it and wait only for smaller ones; the wait is bounded all the same, and a head that gave up reports a
+// negative total, which leaves the host's word unwritten (gaac_wait_words raises).
+// Latency: a launch less (5 us), against waiting for the slowest block ahead (2 to 3).  us a call, encoding and packing in two launches / in one: 300 tokens x 8 heads 18.5 /
+// 15.9, 777 18.9 / 16.4, 777 x 16 19.6 / 17.4, 1500 x 8 (1488 tiles) 19.5 / 17.4, 2500 x 8 (2496) 20.1 / 19.1, 4095 x 2 (1020) 18.8 / 17.4; but 4095 x 8 (4080) 21.6 / 22.0: a
+// chip full of blocks that wait.  (A block of sixteen waves for all tiles of a head, which has nobody to wait for: 777 tokens the same as two launches, 2047 30 us
+// against 16.)
+constexpr int SCAN_PROMPT_TILES = 256, SCAN_PROMPT_BLOCKS = SCAN_PROMPT_TILES / CODEC_WAVES, SCAN_PROMPT_ALL_TILES = 3072, SCAN_SPIN_LIMIT = 1 << 20;      // of a head | of all heads, K and V
+struct PromptFusedArgs { EncodeArgs e; PromptScanArgs s; const int* head_start; uint8_t* ovf[2]; u64* scan; long scan_v; };      // scan: of K of head 0 of the call, scan_v words further on V
+template <int KIND>
+__device__ __forceinline__ void prompt_fused_body(const PromptFusedArgs& P, EncodeBlockLds& L, int (&sizes)[CODEC_WAVES], int& ahead, int h, int wave, int lane) {
+  const EncodeArgs& A = P.e;
+  const EncodeKind& J = KIND == KIND_K ? A.k : A.v;
+  const PromptKind& K = P.s.j[KIND];
+  const int ntiles = A.ntiles, block = blockIdx.x, tile = block * CODEC_WAVES + wave, brow = (A.brow0 + h) % A.NB;
+  u64* scan = P.scan + (KIND == KIND_V ? P.scan_v : 0) + (long)h * (1 + SCAN_PROMPT_BLOCKS);
+  const u16* xh = J.x + (long)h * J.head_stride;
+  RowRegs R;
+  load_rows<false>(R, xh + (long)min(tile, ntiles - 1) * T * J.row_stride, J.row_stride, T, lane);
+  if (wave == 0) reinterpret_cast<u32x2*>(&L.B.w[0][0])[lane] = load_base_pair<KIND>(J.b3 + (long)brow * D, J.b4 + (long)brow * D, lane);
+  const u32 last = (u32)__hip_atomic_load(scan, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), epoch = last + (last == 0xFFFFFFFFu ? 2u : 1u);      // (0 is what the words start with)
+  const int head_start = P.head_start[h];
+  store_rows(L.w[wave], R, lane);
+  __syncthreads();
+  int total = 0;
+  const uint8_t* escapes = nullptr;
+  if (tile < ntiles) {
+    const long row0 = (long)h * A.S_pad + (long)tile * T;
+    UnitEscapes E;
+    total = encode_staged_tile<KIND, true>(L.w[wave], L.B, T, lane, J.sm + row0 * D, J.cd + row0 * CB, J.flags + row0, E);
+    escapes = collect_escapes<KIND>(L.w[wave], E, lane);
+  }
+  if (lane == 0) sizes[wave] = total;
+  __syncthreads();
+  const int own = sizes[0] + sizes[1] + sizes[2] + sizes[3];
+  if (wave == 0) {
+    if (lane == 0) __hip_atomic_store(scan + 1 + block, (u64)(u32)own | ((u64)epoch << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // lane: an earlier block (SCAN_PROMPT_BLOCKS of them at most; the others read the block's own word)
+    const u64* w = scan + 1 + min(lane, block);
+    u64 v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    bool ok = true;
+    for (int spin = 0; __builtin_amdgcn_ballot_w64(lane < block && (u32)(v >> 32) != epoch) != 0; ++spin) {
+      if (spin >= SCAN_SPIN_LIMIT) { ok = false; break; }
+      __builtin_amdgcn_s_sleep(1);
+      if ((u32)(v >> 32) != epoch) v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const int x = (int)row_scan16(lane < block ? (u32)v : 0u);
+    const int before = __builtin_amdgcn_readlane(x, 15) + __builtin_amdgcn_readlane(x, 31) + __builtin_amdgcn_readlane(x, 47) + __builtin_amdgcn_readlane(x, 63);
+    if (lane == 0) {
+      ahead = ok ? before : -1;
+      if (block == (int)gridDim.x - 1) {
+        P.s.head_bytes[KIND * P.s.n_kv + h] = ok ? before + own : -1;
+        __hip_atomic_store(scan, (u64)epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  }
+  if (block == 0) copy_prompt_tail(P.s, K, h, 64 * wave + lane);
+  __syncthreads();
+  int at = ahead;
+  if (at < 0 || tile >= ntiles) return;
+#pragma unroll
+  for (int w = 0; w < CODEC_WAVES; ++w) at += w < wave ? sizes[w] : 0;
+  if (lane == 0) K.tile_off[(long)h * P.s.off_stride + tile] = at;
+  if (at + total > P.s.window) return;      // (the head does not fit and is left empty)
+  uint8_t* dst = P.ovf[KIND] + head_start + at;
+  for (int i = lane; i < total; i += 64) dst[i] = escapes[i];
+}
+__global__ void __launch_bounds__(64 * CODEC_WAVES) k_prompt_fused(const PromptFusedArgs P) {
+  __shared__ EncodeBlockLds L;
+  __shared__ int sizes[CODEC_WAVES], ahead;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (blockIdx.z == KIND_K) prompt_fused_body<KIND_K>(P, L, sizes, ahead, blockIdx.y, wave, lane);
+  else prompt_fused_body<KIND_V>(P, L, sizes, ahead, blockIdx.y, wave, lane);
+}
+// ... and the counters of the heads, with the totals in host memory as k_words_to_host puts them there.
+__global__ void __launch_bounds__(64) k_prompt_finish(const PromptScanArgs A, int* __restrict__ host) {
+  for (int h = threadIdx.x; h < A.n_kv; h += 64) {
+    const int k = A.head_bytes[h], v = A.head_bytes[A.n_kv + h], failed = (k | v) < 0 ? 0x7FFFFFFF : 0;      // (a total that fits no window)
+    set_prompt_counters(A, KIND_K, h, max(k, failed), max(v, failed));
+    set_prompt_counters(A, KIND_V, h, max(v, failed), max(k, failed));
+    if (host) { store_to_host(host + h, k); store_to_host(host + A.n_kv + h, v); }
+  }
+}
 // The prompt's totals into host memory that the host polls, in a launch of its own: by the time they are there all of the prompt is.  Polling spares
 // the host the 5 us that a stream's synchronisation takes from the end of its last kernel, for 2 of this launch: a prompt of 777 tokens 26 -> 21.5 us a call,
 // of 32768 95.8 -> 91.4, the case of four short requests 363 -> 308.
@@ -758,7 +844,7 @@ int gaac_cache_prefill(
     int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
     void* k_tail, uint8_t* k_base3, uint8_t* k_base4, uint8_t* k_sm, uint8_t* k_codes, int* k_flags, uint8_t* k_ovf, int* k_tile_off, int* k_ovf_used,
     void* v_tail, uint8_t* v_base3, uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
-    void* hist, long hist_bytes, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, int* host_bytes, void* stream) {
+    void* hist, long hist_bytes, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, unsigned long long* scan, long scan_v, int* host_bytes, void* stream) {
   GAAC_REQUIRE(((k && v) || L == 0) && tail_len && S && head_start && head_bytes, "gaac_cache_prefill: null pointer");
   GAAC_REQUIRE(k_tail && k_base3 && k_base4 && k_sm && k_codes && k_flags && k_ovf && k_tile_off && k_ovf_used, "gaac_cache_prefill: null K store pointer");
   GAAC_REQUIRE(v_tail && v_base3 && v_base4 && v_sm && v_codes && v_flags && v_ovf && v_tile_off && v_ovf_used, "gaac_cache_prefill: null V store pointer");
@@ -784,12 +870,13 @@ int gaac_cache_prefill(
   const long row0 = (long)head0 * cap, tile0 = (long)head0 * (cap / T), n_all = (long)n_kv * ntiles;
   uint8_t* v_slots = esc_slots ? esc_slots + n_all * TILE_MAX_ESC : nullptr;
   int* v_bytes = tile_bytes ? tile_bytes + n_all : nullptr;
+  const bool fused = scan && ntiles > 0 && ntiles <= SCAN_PROMPT_TILES && 2 * n_all <= SCAN_PROMPT_ALL_TILES;
+  EncodeArgs E{};
   if (ntiles > 0) {
-    EncodeArgs E{};
     E.kind0 = KIND_K; E.S = ntiles * T; E.S_pad = cap; E.ntiles = ntiles; E.brow0 = head0; E.NB = NB; E.bidx = nullptr;
     E.k = EncodeKind{(const u16*)k, k_head_stride, k_row_stride, k_base3, k_base4, k_sm + row0 * D, k_codes + row0 * CB, k_flags + row0, esc_slots, tile_bytes};
     E.v = EncodeKind{(const u16*)v, v_head_stride, v_row_stride, v_base3, v_base4, v_sm + row0 * D, v_codes + row0 * CB, v_flags + row0, v_slots, v_bytes};
-    launch_encode<true>(E, n_kv, 2, st);
+    if (!fused) launch_encode<true>(E, n_kv, 2, st);
   }
   const int window = ovf_cap - (TILE_MAX_ESC + 8);      // room for one more worst-case tile and the readers' padding stays free
   PromptScanArgs P{};
@@ -797,6 +884,13 @@ int gaac_cache_prefill(
   P.j[1] = PromptKind{(const u16*)v, v_head_stride, v_row_stride, v_bytes, v_tile_off + tile0, (u16*)v_tail + (long)head0 * T * D, v_ovf_used + head0};
   P.n_kv = n_kv; P.L = L; P.ntiles = ntiles; P.off_stride = cap / T; P.window = window;
   P.S = S + head0; P.tail_len = tail_len + head0; P.head_bytes = head_bytes;
+  if (host_bytes) for (int i = 0; i < 2 * n_kv; ++i) __atomic_store_n(host_bytes + i, -1, __ATOMIC_RELAXED);      // not there yet
+  if (fused) {
+    const PromptFusedArgs A{E, P, head_start + head0, {k_ovf, v_ovf}, reinterpret_cast<u64*>(scan), scan_v};
+    hipLaunchKernelGGL(k_prompt_fused, dim3((ntiles + CODEC_WAVES - 1) / CODEC_WAVES, n_kv, 2), dim3(64 * CODEC_WAVES), 0, st, A);
+    hipLaunchKernelGGL(k_prompt_finish, dim3(1), dim3(64), 0, st, P, host_bytes);
+    return launch_status("gaac_cache_prefill");
+  }
   if (ntiles <= PROMPT_PACK_TILES) {
     const PromptPackArgs A{P, {esc_slots, v_slots}, head_start + head0, {k_ovf, v_ovf}};
     hipLaunchKernelGGL(k_prompt_pack, dim3(std::max((ntiles + PACK_TPB - 1) / PACK_TPB, 1), n_kv, 2), dim3(256), 0, st, A);
@@ -808,10 +902,7 @@ int gaac_cache_prefill(
     A.j[1] = PackKind{v_slots, v_bytes, v_tile_off + tile0, cap / T, head_start + head0, v_ovf};
     hipLaunchKernelGGL(k_pack<false>, dim3((ntiles + PACK_TPB - 1) / PACK_TPB, n_kv, 2), dim3(256), 0, st, A);
   }
-  if (host_bytes) {
-    for (int i = 0; i < 2 * n_kv; ++i) __atomic_store_n(host_bytes + i, -1, __ATOMIC_RELAXED);      // not there yet
-    hipLaunchKernelGGL(k_words_to_host, dim3(1), dim3(64), 0, st, head_bytes, 2 * n_kv, host_bytes);
-  }
+  if (host_bytes) hipLaunchKernelGGL(k_words_to_host, dim3(1), dim3(64), 0, st, head_bytes, 2 * n_kv, host_bytes);
   return launch_status("gaac_cache_prefill");
 }
 

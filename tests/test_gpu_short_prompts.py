@@ -1,0 +1,86 @@
+"""Prompts whose blocks place their escapes among themselves, at the edges of the blocks (four tiles, 64 blocks) and on both sides of the lines to the two
+launches (256 tiles a head, 3072 of all): every field of the slot against a page of the same rows, slots put in again and again, windows that are too small, the
+epoch's wrap-around, prompts into two slots on two streams."""
+import pytest
+import torch
+
+from gpu_util import require_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(L, n_kv, seed, outliers):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(L, n_kv, 128, generator=g, device="cuda")
+    return torch.where(torch.rand(L, n_kv, 128, generator=g, device="cuda") < outliers, x * 1e4, x).to(torch.bfloat16)      # 0.3: a thousand escape bytes a tile
+
+
+def _check(cache, slot, k, v):
+    """The slot's tiles, offsets, escapes, tail and counters are those of pages of the same rows."""
+    from gaac_amd import Codec
+    n_kv, full = cache.n_kv, k.shape[0] // 16 * 16
+    h = slice(slot * n_kv, (slot + 1) * n_kv)
+    assert cache.S[h].tolist() == [full] * n_kv and cache.tail_len[h].tolist() == [k.shape[0] - full] * n_kv
+    for st, x in ((cache.k, k), (cache.v, v)):
+        b = h if cache.per_sequence_bases else slice(0, n_kv)
+        assert torch.equal(st.tail[h, :x.shape[0] - full], x[full:].transpose(0, 1))
+        if not full: continue
+        page = Codec(n_kv).set_bases(st.base3[b], st.base4[b]).encode(x[:full].transpose(0, 1).contiguous(), st.kind)
+        assert torch.equal(st.sm[h, :full * 128], page.sm) and torch.equal(st.codes[h, :full * 48], page.codes)
+        assert torch.equal(st.flags[h, :full], page.flags) and torch.equal(st.tile_off[h, :full // 16], page.tile_off)
+        start = page.ovf_head_start.tolist()
+        assert st.ovf_used[h].tolist() == [b - a for a, b in zip(start, start[1:])]
+        for i in range(n_kv):
+            at = int(st.head_start[slot * n_kv + i])
+            assert torch.equal(st.ovf[at:at + start[i + 1] - start[i]], page.ovf[start[i]:start[i + 1]])
+
+
+@pytest.mark.parametrize("L,n_kv", [(16, 1), (31, 3), (63, 2), (64, 2), (65, 2), (80, 1), (1029, 2), (4096, 1), (4111, 2), (4112, 1), (1536, 16), (1552, 16), (100, 48)])
+@pytest.mark.parametrize("outliers", [1e-3, 0.3])
+def test_slots(L, n_kv, outliers):
+    require_gpu()
+    from gaac_amd import CompressedKVCache
+    cache = CompressedKVCache(3, n_kv, L + 16, None if n_kv != 2 else dict.fromkeys(("k3", "v3"), torch.full((2, 128), 122)) | dict.fromkeys(("k4", "v4"), torch.full((2, 128), 118)),
+                              ovf_bytes_per_tile=1280 if outliers > 0.1 else 160)
+    last = {}
+    for i, slot in enumerate((2, 0, 2, 2, 1)):      # (the third and fourth with fewer blocks than the launch before, and more)
+        n = max(L // 2, 16) if i == 2 else L
+        k, v = _rows(n, n_kv, 10 * i + L, outliers), _rows(n, n_kv, 10 * i + L + 1, outliers)
+        cache.prefill(slot, k, v)
+        last[slot] = k, v
+    for slot, (k, v) in last.items(): _check(cache, slot, k, v)
+    cache._scan[:, :, 0] = 0xFFFFFFFE      # the next epochs: 2^32 - 1, 1, 2
+    for i in range(3):
+        k, v = _rows(L, n_kv, 99 + i, outliers), _rows(L, n_kv, 199 + i, outliers)
+        cache.prefill(0, k, v)
+        _check(cache, 0, k, v)
+    assert cache._scan[:, :n_kv, 0].unique().numel() == 1
+
+
+@pytest.mark.parametrize("many", ["k", "v", "both"])
+def test_windows_that_have_to_grow(many):
+    require_gpu()
+    from gaac_amd import CompressedKVCache
+    cache = CompressedKVCache(2, 2, 640, ovf_bytes_per_tile=40)
+    k0, v0 = _rows(333, 2, 1, 1e-3), _rows(333, 2, 2, 1e-3)
+    cache.prefill(1, k0, v0)
+    cap = cache.k.ovf_cap
+    k, v = _rows(600, 2, 3, 0.3 if many != "v" else 1e-3), _rows(600, 2, 4, 0.3 if many != "k" else 1e-3)
+    cache.prefill(0, k, v)
+    assert cache.k.ovf_cap == cache.v.ovf_cap > cap
+    _check(cache, 0, k, v)
+    _check(cache, 1, k0, v0)
+
+
+def test_two_streams():
+    require_gpu()
+    from gaac_amd import CompressedKVCache
+    cache = CompressedKVCache(2, 8, 800)
+    rows = [[_rows(777, 8, 10 * i + j, 1e-3) for j in range(2)] for i in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for slot, s in enumerate(streams):
+            with torch.cuda.stream(s): cache.prefill(slot, *rows[slot])
+    torch.cuda.synchronize()
+    for slot in range(2): _check(cache, slot, *rows[slot])
