@@ -169,19 +169,18 @@ template <typename F> PyObject* whole_call(Py_ssize_t given, Py_ssize_t n, F bod
   } catch (const Failed& f) {
     PyErr_Format(PyExc_RuntimeError, "%s failed (%d): %s", f.name, f.rc, g_last_error());
     return nullptr;
-  } catch (const std::exception& e) {      // no memory, a tensor without any, ...
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  } catch (const std::exception&) {      // no memory, a tensor without any: Python meets the same and raises its own type (nothing is stored until a call's last launch)
   }
   PyErr_Clear();
   Py_RETURN_NONE;
 }
+struct NoGil {      // (taken back also where an exception leaves: a tensor without an address of its own, as in vmap)
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
 template <typename F> int without_gil(F f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
-  return rc;
+  const NoGil released;
+  return f();
 }
 PyObject* numbers(const at::Tensor& words) {
   const long n = words.numel();

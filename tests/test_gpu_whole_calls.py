@@ -104,3 +104,27 @@ def test_cache(both, form, L, calibrate):
         return run
     i = dict(dtype=torch.int32, device="cuda")
     for slots in (torch.tensor([2, 0], **i), torch.tensor([[2], [-1]], **i), torch.tensor([2, 9, 0, 9], **i)[::2].contiguous(), torch.tensor([2], **i)): _same(*both(f(slots)))
+
+
+def test_tensors_without_an_address_and_a_lack_of_memory_raise_as_through_python(both):
+    require_gpu()
+    from gaac_amd import Codec, CompressedKVCache, attention
+    x = _rows((2, 200000, 128), 1)
+    torch.cuda.empty_cache()      # (no large segment that is only partly in use)
+    codec = Codec(2).calibrate(x)
+    K, V = codec.encode(x, "k"), codec.encode(x, "v")
+    cache, slots = CompressedKVCache(2, 2, 64, dict(k3=codec.base3, k4=codec.base4, v3=codec.base3, v4=codec.base4)), torch.tensor([1], dtype=torch.int32, device="cuda")
+    q, new = _rows((3, 1, 8, 128), 2), _rows((3, 1, 2, 128), 3)
+    def refused(f):
+        try: f()
+        except Exception as e: return type(e)
+    def vmaps():
+        return [refused(lambda: torch.vmap(lambda t: attention(t, K, V))(q)), refused(lambda: torch.vmap(lambda t: cache.append(slots, t, t))(new)), cache.S.tolist(), cache.tail_len.tolist()]
+    a, b = both(vmaps)
+    assert a == b and a[0] is not None and a[1] is not None
+    def no_room():
+        torch.cuda.empty_cache()
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 4096) / torch.cuda.get_device_properties(0).total_memory)
+        try: return refused(lambda: Codec.decode(K)), refused(lambda: codec.encode(x, "k"))
+        finally: torch.cuda.set_per_process_memory_fraction(1.0)
+    assert both(no_room) == [(torch.OutOfMemoryError,) * 2] * 2
