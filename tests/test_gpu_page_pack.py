@@ -1,4 +1,4 @@
-"""Encoder and escape packing at the sizes where their launches change shape: one tile per wave against four (8192 tiles), the packing's
+"""Encoder and escape packing at the sizes where their launches change shape: rows through the caches or past them (8192 tiles), the packing's
 blocks of 64 tiles and waves of 16, the scan's rounds of 4096 tiles, tiles with more than 64 escape bytes, ragged last tiles."""
 import numpy as np
 import pytest
