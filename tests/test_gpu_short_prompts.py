@@ -1,6 +1,6 @@
 """Prompts whose blocks place their escapes among themselves, at the edges of the blocks (four tiles, 64 blocks) and on both sides of the lines to the two
 launches (256 tiles a head, 3072 of all): every field of the slot against a page of the same rows, slots put in again and again, windows that are too small, the
-epoch's wrap-around, prompts into two slots on two streams."""
+epoch's wrap-around, prompts into two slots on two streams, a wait that failed."""
 import pytest
 import torch
 
@@ -84,3 +84,30 @@ def test_two_streams():
             with torch.cuda.stream(s): cache.prefill(slot, *rows[slot])
     torch.cuda.synchronize()
     for slot in range(2): _check(cache, slot, *rows[slot])
+
+
+@pytest.mark.parametrize("through", ["binding", "python"])
+def test_a_failed_wait_leaves_the_slot_armed(through, monkeypatch):
+    require_gpu()
+    from gaac_amd import CompressedKVCache, _lib
+    cache = CompressedKVCache(3, 2, 320)
+    k, v = _rows(300, 2, 1, 1e-3), _rows(300, 2, 2, 1e-3)
+    for slot in range(3): cache.prefill(slot, k, v)
+    armed = cache._scan.clone()
+    binding, call = _lib.calls(), _lib.call
+    class Calls:
+        def __getattr__(self, name): return getattr(binding, name)
+        def prompt_store(self, *a):
+            if through == "python": return None
+            binding.prompt_store(*a)
+            raise RuntimeError("gaac_wait_words failed")
+    def fail(name, *a):
+        call(name, *a)
+        if name == "gaac_wait_words": raise RuntimeError("gaac_wait_words failed")
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "_calls", Calls())
+        m.setattr(_lib, "call", fail)
+        with pytest.raises(RuntimeError, match="gaac_wait_words"): cache.prefill(1, k, v)
+    assert not cache._scan[:, 2:4].any() and torch.equal(cache._scan[:, :2], armed[:, :2]) and torch.equal(cache._scan[:, 4:], armed[:, 4:])
+    cache.prefill(1, v, k)
+    _check(cache, 1, v, k)
