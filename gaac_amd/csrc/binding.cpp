@@ -285,7 +285,7 @@ PyObject* prompt_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const long scan_row = scan.stride(1);
     void* stream = stream_of(a[4]);
     // scratch: escape slots | exponent counts (hist_bytes in kv_cache.py) | tile sizes | head sizes
-    const long tables = 2 * n_kv * std::max(std::min((L + 255) / 256, std::max(256 / (2 * n_kv), 1l)), (L + 65534) / 65535);
+    const long tables = 2 * n_kv * std::max(std::min((L + 255) / 256, std::max(std::min(256 / (2 * n_kv), 64l), 1l)), (L + 65534) / 65535);
     const long at_hist = nt * TILE_ESCAPES, at_sizes = at_hist + (calibrate ? tables * HIST_BYTES : 0);
     at::Tensor scratch = bytes(k, {at_sizes + 4 * (nt + 2 * n_kv)}), totals = host_words(2 * n_kv);
     uint8_t* base = static_cast<uint8_t*>(scratch.data_ptr());

@@ -27,7 +27,7 @@ char* last_error_buffer() { static thread_local char buf[512] = {0}; return buf;
 // its own table, the rows (bins) of it that hold a count, and a bit for each of these; k_prompt_bases adds up the blocks' tables.  Added to one global table,
 // which a launch had to clear first, the counts of a prompt took that launch longer: 32768 tokens x 8 heads 88.1 -> 83.2 us a call, 4000 tokens 26.2 -> 24.5 of
 // kernels.
-constexpr int HIST_WAVES = 16, HIST_MAX_CHUNK = 65535, HIST_LOADS = 2;      // HIST_LOADS: loads of four rows in flight per wave
+constexpr int HIST_WAVES = 16, HIST_MAX_CHUNK = 65535, HIST_LOADS = 2, HIST_TABLES = 64;      // HIST_LOADS: loads of four rows in flight per wave
 struct HistArgs { const u16* x[2]; long head_stride[2], row_stride[2]; long n_tok; int chunk, n_kv; unsigned long long* hist; u32* rows; u16* bits; };      // rows [pair][chunk][256][64], bits [pair][chunk][16]
 template <bool PARTS>
 __global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArgs A) {
@@ -94,14 +94,16 @@ __global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArg
     if (c >> 16) atomicAdd(row + 256, (unsigned long long)(c >> 16));
   }
 }
-static int hist_chunks(long n_tok, int pairs) {
+static int hist_chunks(long n_tok, int pairs, bool parts) {
   // one block per CU, at least 256 tokens each, so that clearing and scanning the 64 KB table stays the smaller part (two blocks per CU,
   // which the LDS has room for: 26 against 23.6 us for 2 x 8 heads x 32768 tokens out of the Infinity Cache, measured with blocks of eight waves)
-  const long n = min((n_tok + 255) / 256, (long)max(1, 256 / pairs));
+  // (tables that another launch adds up: no more than HIST_TABLES of a (kind, head).  32768 tokens x 1 head, 128 / 64 tables: histogram 5.7 / 6.3 us, bases 12.4 / 8.0,
+  // the call 39.1 / 36.4)
+  const long n = min((n_tok + 255) / 256, (long)min(max(1, 256 / pairs), parts ? HIST_TABLES : 256));
   return (int)max(n, (n_tok + HIST_MAX_CHUNK - 1) / HIST_MAX_CHUNK);
 }
 static int launch_hist(HistArgs& A, int kinds, hipStream_t stream) {      // returns the blocks of a (kind, head), hist_chunks at most
-  const int nchunk = hist_chunks(A.n_tok, kinds * A.n_kv);
+  const int nchunk = hist_chunks(A.n_tok, kinds * A.n_kv, A.rows != nullptr);
   A.chunk = (int)((A.n_tok + nchunk - 1) / nchunk);
   const dim3 grid((unsigned)((A.n_tok + A.chunk - 1) / A.chunk), A.n_kv, kinds);
   if (A.rows) hipLaunchKernelGGL(k_exponent_hist<true>, grid, dim3(64 * HIST_WAVES), 0, stream, A);
@@ -111,41 +113,50 @@ static int launch_hist(HistArgs& A, int kinds, hipStream_t stream) {      // ret
 
 // The bases of K and V of a prompt from the tables of its k_exponent_hist<true>, written to base row row0 + head of the two kinds' tables.  A block takes 32 channels
 // of one (kind, head): a wave adds up every sixteenth row over the tables, the 256 sums of a channel go to LDS, thread (channel, eighth) slides the two windows over
-// 32 starts.  Latency: two trips to memory, bits and rows.  (A table a wave and LDS atomics for the sums: 6.4 us instead of 4.8.)
+// 32 starts.  Latency: two trips to memory, bits and rows, if a lane has R loads of a row in flight for up to 4 R tables: with four for any number of them, sixteen
+// tables a trip, 32768 tokens x 1 head (128 tables) took 14.2 us, x 2 (64) 8.6, x 4 (32) 5.8; now, with 64 at most, 8.0, 7.4 and 5.1 (x 8, 16 tables, 4.7).  (A table a
+// wave and LDS atomics for the sums: 6.4 us instead of 4.8.)
 struct PromptBasesArgs { const u32* rows; const u16* bits; int chunks; uint8_t* b3[2]; uint8_t* b4[2]; int n_kv, row0; };
+template <int R>
 __global__ void __launch_bounds__(1024) k_prompt_bases(const PromptBasesArgs A) {
   constexpr int STRIDE = 256 + 17;      // odd: the 32 channels of a bin sit in different banks
   __shared__ u32 cnt[32 * STRIDE];
   __shared__ u32 best[2][8][32];
   __shared__ int arg[2][8][32];
   const int tid = threadIdx.x, grp = blockIdx.x, head = blockIdx.y, kind = blockIdx.z;
-  for (int i = tid; i < 32 * STRIDE; i += 1024) cnt[i] = 0u;
-  __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const long at0 = ((long)kind * A.n_kv + head) * A.chunks;
+  const u16* bits = A.bits + at0 * HIST_WAVES + wave;
+  const u32* words = A.rows + at0 * (256 * 64) + 64 * wave + 16 * grp;
   u32* sums = cnt + 2 * (lane & 15) * STRIDE + wave;
-  for (int c0 = 0; c0 < A.chunks; c0 += 16) {
-    // lane (j, w): word w of the channels' sixteen, of the tables c0 + j, c0 + 4 + j, ...
-    u32 has[4];
-    const u32* rows[4];
+  // lane (j, w): word w of the channels' sixteen, of the tables c0 + j, c0 + 4 + j, ...; the next tables' bits are on their way meanwhile
+  const auto table = [&](int c0, int r) { return c0 + 4 * r + (lane >> 4); };
+  u32 next[R];
+  if (A.chunks > 0)      // (an empty prompt has no tables)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int chunk = c0 + 4 * r + (lane >> 4);
-      const long at = at0 + min(chunk, A.chunks - 1);
-      has[r] = A.bits[at * HIST_WAVES + wave];
-      has[r] = chunk < A.chunks ? has[r] : 0u;
-      rows[r] = A.rows + at * (256 * 64) + 64 * wave + 16 * grp + (lane & 15);
+    for (int r = 0; r < R; ++r) next[r] = bits[(u32)min(table(0, r), A.chunks - 1) * HIST_WAVES];
+  for (int i = tid; i < 32 * STRIDE; i += 1024) cnt[i] = 0u;
+  __syncthreads();
+  for (int c0 = 0; c0 < A.chunks; c0 += 4 * R) {
+    u32 has[R], at[R], any = 0u;
+#pragma unroll
+    for (int r = 0; r < R; ++r) { has[r] = table(c0, r) < A.chunks ? next[r] : 0u; any |= has[r]; }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      at[r] = (u32)min(table(c0, r), A.chunks - 1) * (256 * 64) + (u32)(lane & 15);
+      next[r] = bits[(u32)min(table(c0 + 4 * R, r), A.chunks - 1) * HIST_WAVES];
     }
-    u32 left = __builtin_amdgcn_readfirstlane(quad_rows_or(has[0] | has[1] | has[2] | has[3]));
-    while (left) {      // two rows at a time, four tables a lane
+    u32 left = __builtin_amdgcn_readfirstlane(quad_rows_or(any));
+    while (left) {      // two rows at a time, R tables a lane
       const int i0 = __builtin_ctz(left);
       left &= left - 1;
       const int i1 = left ? __builtin_ctz(left) : i0;
-      u32 v0[4], v1[4], lo0 = 0u, hi0 = 0u, lo1 = 0u, hi1 = 0u;
+      const u32 *w0 = words + 64 * HIST_WAVES * i0, *w1 = words + 64 * HIST_WAVES * i1;
+      u32 v0[R], v1[R], lo0 = 0u, hi0 = 0u, lo1 = 0u, hi1 = 0u;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) { v0[r] = rows[r][64 * HIST_WAVES * i0]; v1[r] = rows[r][64 * HIST_WAVES * i1]; }
+      for (int r = 0; r < R; ++r) { v0[r] = w0[at[r]]; v1[r] = w1[at[r]]; }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
+      for (int r = 0; r < R; ++r) {
         v0[r] = (has[r] >> i0) & 1u ? v0[r] : 0u; v1[r] = (has[r] >> i1) & 1u ? v1[r] : 0u;      // (a row without the bit holds anything)
         lo0 += v0[r] & 0xFFFFu; hi0 += v0[r] >> 16; lo1 += v1[r] & 0xFFFFu; hi1 += v1[r] >> 16;
       }
@@ -851,7 +862,7 @@ int gaac_cache_prefill(
   GAAC_REQUIRE(L >= 0 && n_kv > 0 && head0 >= 0 && cap > 0 && cap % T == 0 && L <= cap && NB > 0 && ovf_cap >= 8,
                "gaac_cache_prefill: bad sizes L=%d n_kv=%d head0=%d cap=%d ovf_cap=%d NB=%d", L, n_kv, head0, cap, ovf_cap, NB);
   GAAC_REQUIRE(!calibrate || (hist && NB >= head0 + n_kv), "gaac_cache_prefill: calibration needs its scratch and a base row per cache head (NB=%d, heads %d..%d)", NB, head0, head0 + n_kv - 1);
-  const long tables = calibrate ? (long)2 * n_kv * hist_chunks(L, 2 * n_kv) : 0;
+  const long tables = calibrate ? (long)2 * n_kv * hist_chunks(L, 2 * n_kv, true) : 0;
   GAAC_REQUIRE(tables * (256 * 64 * (long)sizeof(u32) + 32) <= hist_bytes || tables == 0, "gaac_cache_prefill: %ld bytes of calibration scratch for %ld tables", hist_bytes, tables);
   GAAC_REQUIRE((reinterpret_cast<uintptr_t>(hist) & 7) == 0, "gaac_cache_prefill: calibration scratch is not aligned to 8 bytes");
   const int ntiles = L / T;
@@ -865,7 +876,10 @@ int gaac_cache_prefill(
     HistArgs H{{(const u16*)k, (const u16*)v}, {k_head_stride, v_head_stride}, {k_row_stride, v_row_stride}, L, 0, n_kv, nullptr, rows, bits};
     const int chunks = L > 0 ? launch_hist(H, 2, st) : 0;
     const PromptBasesArgs B{rows, bits, chunks, {k_base3, v_base3}, {k_base4, v_base4}, n_kv, head0};
-    hipLaunchKernelGGL(k_prompt_bases, dim3(4, n_kv, 2), dim3(1024), 0, st, B);
+    // (as many loads in flight as there are tables for: a lane past the last table reads that one again)
+    if (chunks <= 16) hipLaunchKernelGGL(k_prompt_bases<4>, dim3(4, n_kv, 2), dim3(1024), 0, st, B);
+    else if (chunks <= 32) hipLaunchKernelGGL(k_prompt_bases<8>, dim3(4, n_kv, 2), dim3(1024), 0, st, B);
+    else hipLaunchKernelGGL(k_prompt_bases<16>, dim3(4, n_kv, 2), dim3(1024), 0, st, B);
   }
   const long row0 = (long)head0 * cap, tile0 = (long)head0 * (cap / T), n_all = (long)n_kv * ntiles;
   uint8_t* v_slots = esc_slots ? esc_slots + n_all * TILE_MAX_ESC : nullptr;

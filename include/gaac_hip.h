@@ -79,7 +79,7 @@ int gaac_decode_tiles(int kind, const uint8_t* sm, const uint8_t* codes, const i
  * element (token t, head h, channel c) at x[t*row_stride + h*head_stride + c], rows 16-byte aligned, L <= cap tokens.  The first
  * L - L % 16 tokens become tiles, the rest goes to the raw tail; S, tail_len, ovf_used and, with calibrate, the heads' base rows are
  * set.  Store pointers are those of gaac_cache_append (whole cache: token stride cap, escape windows of ovf_cap bytes that start at
- * head_start[head]).  Scratch: hist (calibrate only), 8-byte aligned, hist_bytes >= 65568 * 2*n_kv * max(min(ceil(L/256), max(256/(2*n_kv), 1)), ceil(L/65535)), esc_slots [2*n_kv*(L/16)*1280], tile_bytes
+ * head_start[head]).  Scratch: hist (calibrate only), 8-byte aligned, hist_bytes >= 65568 * 2*n_kv * max(min(ceil(L/256), 64, max(256/(2*n_kv), 1)), ceil(L/65535)), esc_slots [2*n_kv*(L/16)*1280], tile_bytes
  * int32 [2*n_kv*(L/16)], head_bytes int32 [2*n_kv].  scan (or NULL): uint64 [n_kv][65] for K of the call's heads and scan_v words behind
  * it the same for V, zeroed once and kept with the cache heads: short prompts then take a launch less; calls on one
  * cache head must be ordered on one stream.  head_bytes and host_bytes (or NULL; host memory the device can write) receive the

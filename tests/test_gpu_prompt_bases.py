@@ -1,5 +1,5 @@
-"""Bases that a prompt calibrates for itself, from the tables of several blocks per head: one block and many (more than the sixteen that are added up at a time), ends
-of chunks, chunks at the longest length that 16-bit counts hold, every exponent there is and only one, against the histogram over all rows."""
+"""Bases that a prompt calibrates for itself, from the tables of several blocks per head: one block and many (up to sixteen, 32, 64 and more, which are added up in
+turn), none, ends of chunks, chunks at the longest length that 16-bit counts hold, every exponent there is and only one, against the histogram over all rows."""
 import pytest
 import torch
 
@@ -8,7 +8,8 @@ from gpu_util import require_gpu
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("L,n_kv", [(1, 1), (15, 2), (17, 3), (256, 1), (257, 1), (4099, 8), (33000, 1), (5000, 2), (700, 130), (65600, 130)])
+@pytest.mark.parametrize("L,n_kv", [(1, 1), (15, 2), (17, 3), (256, 1), (257, 1), (4099, 8), (33000, 1), (5000, 2), (700, 130), (65600, 130), (0, 1), (4096, 1), (4097, 1), (8192, 2),
+                                    (8193, 1), (16383, 1), (64 * 65535 + 1, 1)])
 @pytest.mark.parametrize("data", ["bits", "normal", "ones"])
 def test_bases(L, n_kv, data):
     dev = require_gpu()
@@ -25,7 +26,7 @@ def test_bases(L, n_kv, data):
     cache = CompressedKVCache(2, n_kv, L + 16, ovf_bytes_per_tile=1280 if data == "bits" else 128)
     for _ in range(2): cache.prefill(1, k, v)      # the second on scratch that another prompt may have left something in
     for x, st in ((k, cache.k), (v, cache.v)):
-        b3, b4 = bases_from_hist(exponent_hist(x, n_kv), n_kv)
+        b3, b4 = bases_from_hist(exponent_hist(x, n_kv) if L else torch.zeros(n_kv, 128, 256, dtype=torch.int64, device=dev), n_kv)
         assert torch.equal(st.base3[n_kv:], b3) and torch.equal(st.base4[n_kv:], b4)
     if L < 10 ** 4:      # (of "bits", tiles of over a thousand escape bytes)
         for got, x in zip(cache.decompress(1), (k, v)): assert torch.equal(got.view(torch.int16), x.view(torch.int16))
