@@ -1590,8 +1590,12 @@ static int plan_units(int B, int n_kv, int nsplit, long max_tiles) {
 // look at the rows and are waited for behind the others; of several rounds, two do, as a row that needs more splits than the others gets them (SIZED_SPLIT).
 // Paged, 8 kv heads, us, the caller's splits / these: 32 rows of 500..20000 tokens, 8 splits 168 / 166, 24 splits 181 / 165; 16 of 9000..11000 92 / 88, 20 of
 // 39000..40000 405 / 385; 128 of 100..4000 x 4 heads, 4 splits 97 / 70; 64 of 2000, one of them 16000, 4 splits 120 / 111.
+// A single row has nothing to share out: its splits are of one length, and where they are more than eight-wave blocks fit the chip, the second round, or half of one, comes
+// on top.  Paged, one row of 65536 tokens, us, splits as of choose_nsplit / these / twice as many: 8 kv heads of 4 query heads 73 (256 splits) / 37.6 (32) / 37.9, 4 of
+// 6 46.6 / 24.6 / 27.6, 2 of 8 27.6 / 19.4 / 27.6, 16 of 2 98 (128) / 65.8 / 65.1; of 16000 tokens 19.2 (62) / 17.2, 13.9 (62, as asked), 13.2 (as asked), 34.5 (62) / 23.5 / 22.8.
 static int planned_splits(int B, int n_kv, int nsplit, int plan, long least) {      // least: for splits that the paged kernel's tile table holds
   const long heads = (long)B * n_kv;
+  if (B == 1) return (int)std::min<long>(nsplit, std::max<long>({256 / n_kv, least, 1}));
   return plan >= B ? (int)std::min<long>(nsplit, std::max((1024 + heads - 1) / heads, least)) : nsplit;
 }
 
@@ -1625,7 +1629,7 @@ static int attn_split_impl(
   GAAC_REQUIRE(S_pad > 0 && S_pad <= (1 << 24), "gaac_attn: at most %d tokens per cache head (32-bit byte offsets inside a head)", 1 << 24);
   if (epoch && S_all >= 0) nsplit = host_splits((S_all + T - 1) / T, nsplit);
   const int plan = epoch && S_all < 0 ? plan_units(B, n_kv, nsplit, S_pad / T) : 0;
-  nsplit = planned_splits(B, n_kv, nsplit, plan, 1);
+  if (epoch && S_all < 0) nsplit = planned_splits(B, n_kv, nsplit, plan, 1);
   const int nslot = nsplit;
   AttnArgs A;
   A.k = StoreView{smk, ck, fk, tok, ovk, ohsk, b3k, b4k};
