@@ -458,9 +458,10 @@ struct AttnLds {
   u32x4 bwk[2][NG], bwv[2][NG];
   u32x4 qw[GMAX][NG];
 };
-// Block merge: one partial per wave plus one (index NW) for the uncompressed rows.  Before the waves publish, wave 0 keeps the decoded side of a
-// half raw tile in acc[0]; afterwards the mergers' scratch lies in acc.
-template <int NW> struct MergeLds { float m[NW + 1][GMAX], l[NW + 1][GMAX]; __align__(16) float acc[NW + 1][GMAX][MROW]; };
+// Block merge: one partial per wave plus one or two (index NW) for the uncompressed rows.  Before the waves publish, a wave w that takes these keeps the
+// decoded side of a half raw tile in acc[w]; afterwards the mergers' scratch lies in acc.
+// RAWS: waves that take uncompressed rows, a partial each.
+template <int NW, int RAWS> struct MergeLds { float m[NW + RAWS][GMAX], l[NW + RAWS][GMAX]; __align__(16) float acc[NW + RAWS][GMAX][MROW]; };
 static_assert(T * D * sizeof(u16) <= GMAX * D * sizeof(float) && sizeof(MergeScratch<4>) <= 5 * GMAX * D * sizeof(float) &&
               sizeof(MergeScratch<8>) <= 9 * GMAX * D * sizeof(float), "scratch views must fit the merge buffer");
 struct TableRegs { u32 b0, b1; u32 qlo[4], qhi[4]; };      // one thread's raw inputs of the per-block tables
@@ -1043,11 +1044,14 @@ __device__ __forceinline__ bool plan_block(const AttnArgs& A, int lane, RowPlan&
 template <bool PAGED, int NW, bool HOST_LEN>
 __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const AttnArgs A) {
   constexpr int NT = 64 * NW;
+  // Raw tiles of the paged pool: a wave for every four of the block, so that a CU has two in either launch form.  Pools of raw tiles only, 8 kv heads, one / two
+  // in an eight-wave block, us: 8 rows of 200..3000 tokens 48 / 33, 4 of 1000..9000 65 / 43, one of 30000 88 / 55.
+  constexpr int RAWS = PAGED && NW == 8 ? 2 : 1;
   // one LDS object so that the tables the tile loop reads sit at the lowest addresses (immediate offsets of the LDS loads)
-  struct BlockLds { AttnLds L; int next_tile; int2 tile_table[PAGED ? MAX_CHUNK : 1]; MergeLds<NW> M; };
+  struct BlockLds { AttnLds L; int next_tile; int2 tile_table[PAGED ? MAX_CHUNK : 1]; MergeLds<NW, RAWS> M; };
   static_assert(offsetof(BlockLds, M.acc) % 16 == 0, "the block merge's accumulators are stored and a decoded raw tile is read 16 bytes at a time");
   __shared__ BlockLds lds;
-  AttnLds& L = lds.L; MergeLds<NW>& M = lds.M; int2* tile_table = lds.tile_table; int& next_tile = lds.next_tile;
+  AttnLds& L = lds.L; MergeLds<NW, RAWS>& M = lds.M; int2* tile_table = lds.tile_table; int& next_tile = lds.next_tile;
   const int tid = threadIdx.x;
   GAAC_STAMP(0);
   // One-dimensional grid, numbered split-fastest: the splits of one kv head go round the eight XCDs (workgroups are dealt to XCDs in
@@ -1180,7 +1184,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   GAAC_STAMP(6);
   if (tid < 256) tables_store(L, Tr, tid, G);
   GAAC_STAMP(7);
-  if (tid < GMAX) { M.m[NW][tid] = -INFINITY; M.l[NW][tid] = 0.f; }
+  if (tid < RAWS * GMAX) { M.m[NW + tid / GMAX][tid % GMAX] = -INFINITY; M.l[NW + tid / GMAX][tid % GMAX] = 0.f; }
   lds_barrier();        // block tables are ready (a barrier that does not wait for the tile loads in flight)
   GAAC_STAMP(1);
   // Q as the B operand of the score product: lane (head a, quad q), product u covers group 4q+u in word order (e, e+4);
@@ -1207,18 +1211,20 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
       raw_rows_store(rs, a, q, M.m[NW], M.l[NW], M.acc[NW]);
     }
   }
-  // Paged pool, wave 0: the tiles c0 .. c1 - 1, whose entries the table holds, that have a raw side (the block that is still filling, or
+  // Paged pool, wave 0, or waves 0 and 1 in turn (RAWS): the tiles c0 .. c1 - 1, whose entries the table holds, that have a raw side (the block that is still filling, or
   // escapes that did not fit the slot).  Raw sides are read in place, the compressed side of a half raw tile is decoded into LDS.
   const auto attend_raw_tiles = [&](int c0, int c1) {
     RawState rs;
     u32x4 qr[4];
     raw_queries(A.q + qh0 * D, G, a, q, qr);
-    raw_rows_load(rs, a, q, M.m[NW], M.l[NW], M.acc[NW]);
-    u16* decoded = reinterpret_cast<u16*>(&M.acc[0][0][0]);      // (wave 0's own place in the block merge)
+    raw_rows_load(rs, a, q, M.m[NW + wave], M.l[NW + wave], M.acc[NW + wave]);
+    u16* decoded = reinterpret_cast<u16*>(&M.acc[wave][0][0]);      // (the wave's own place in the block merge)
+    int other = wave;
     const long boff = (long)(ch % A.NB) * D;
     for (int i0 = 0; i0 < c1 - c0; i0 += 64) {
       const int2 own = tile_table[min(i0 + lane, c1 - c0 - 1)];
       for (u64 left = __builtin_amdgcn_ballot_w64(i0 + lane < c1 - c0 && (own.x | own.y) < 0); left != 0; left &= left - 1) {
+        if (RAWS > 1 && (other++ & 1) != 0) continue;      // (the other wave's)
         const int l = __builtin_ctzll(left), ex = __builtin_amdgcn_readlane(own.x, l), ey = __builtin_amdgcn_readlane(own.y, l);
         const u16* krows = decoded; const u16* vrows = decoded;
         wave_lds_sync();
@@ -1236,9 +1242,9 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
         raw_rows_attend(krows, vrows, min(T, S - (c0 + i0 + l) * T), qr, A.scale_log2e, a, q, rs);
       }
     }
-    raw_rows_store(rs, a, q, M.m[NW], M.l[NW], M.acc[NW]);
+    raw_rows_store(rs, a, q, M.m[NW + wave], M.l[NW + wave], M.acc[NW + wave]);
   };
-  if (PAGED && any_raw && wave == 0) attend_raw_tiles(tlo, thi_fast);
+  if (PAGED && any_raw && wave < RAWS) attend_raw_tiles(tlo, thi_fast);
 
   if (!PAGED) { B.kov = A.k.ovf + __builtin_amdgcn_readfirstlane((int)khs); B.vov = A.v.ovf + __builtin_amdgcn_readfirstlane((int)vhs); }
   if (NW == 4 && R.first && n_own >= PRIO_TILES && (blockIdx.x & 256u) != 0u && wave < 2) __builtin_amdgcn_s_setprio(1);
@@ -1276,7 +1282,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   if (A.dbg && lane == 0) A.dbg[((long)gridDim.x + blockIdx.x) * 8 + wave] = wall_clock64();
 #endif
   // ---- what the pipelined loop left: (1) the partly filled last tile of the sequence; (2) paged pool: a split longer than the LDS tile
-  // table goes on in further rounds of MAX_CHUNK tiles (table refilled, raw tiles again by wave 0).  Tiles are taken by the waves in turn, one
+  // table goes on in further rounds of MAX_CHUNK tiles (table refilled, raw tiles again by the same waves).  Tiles are taken by the waves in turn, one
   // at a time without the prefetch pipeline (of the block's waves some compute while others wait for their tile; both cases are
   // rare), through ONE instantiation of the masking tile code.
   if (tlo < thi) {
@@ -1293,7 +1299,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
         }
         any_raw = __syncthreads_or(raw);
         TT.tlo = c0;
-        if (any_raw && wave == 0) attend_raw_tiles(c0, c1);
+        if (any_raw && wave < RAWS) attend_raw_tiles(c0, c1);
       }
       // first round: only the partial tile is left, for the first wave that has no tile of its own, if there is one (it waits for tag words,
       // then for escape bytes: behind wave 0's own tiles 1000 tokens x 8 kv heads in 16 splits took 9.6 us instead of 8.6)
@@ -1336,19 +1342,19 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   const auto merge_block = [&](auto channels, int g, int c0) {
     constexpr int C = decltype(channels)::value;
     // every LDS read up front and none under a branch: nine dependent round trips otherwise
-    float mv[NW + 1], lv[NW + 1], av[NW + 1][C];
+    float mv[NW + RAWS], lv[NW + RAWS], av[NW + RAWS][C];
 #pragma unroll
-    for (int w = 0; w < NW + 1; ++w) {
+    for (int w = 0; w < NW + RAWS; ++w) {
       mv[w] = M.m[w][g]; lv[w] = M.l[w][g];
 #pragma unroll
       for (int c = 0; c < C; ++c) av[w][c] = M.acc[w][g][c0 + 64 * c + lane];
     }
     float Mx = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < NW + 1; ++w) Mx = fmaxf(Mx, mv[w]);
+    for (int w = 0; w < NW + RAWS; ++w) Mx = fmaxf(Mx, mv[w]);
     float Lc = 0.f, Ac[C] = {};
 #pragma unroll
-    for (int w = 0; w < NW + 1; ++w) {
+    for (int w = 0; w < NW + RAWS; ++w) {
       const bool live = mv[w] != -INFINITY;          // an empty partial's accumulator may hold anything
       const float f = live ? __builtin_amdgcn_exp2f(mv[w] - Mx) : 0.f;
       Lc += lv[w] * f;
@@ -1599,6 +1605,17 @@ static int planned_splits(int B, int n_kv, int nsplit, int plan, long least) {  
   return plan >= B ? (int)std::min<long>(nsplit, std::max((1024 + heads - 1) / heads, least)) : nsplit;
 }
 
+// Paged rows of few heads in all: splits for one round of eight-wave blocks, one per CU, where these fill it, instead of four-wave blocks, two per CU: half the
+// starts, partials and records to wait for, and a wave has as many tiles.  us with the splits of choose_nsplit / these: 8 rows of 200..3000 tokens x 8 kv heads
+// 18.1 / 16.4, 3 of 2900..3000 x 8 17.5 / 13.9, 9 of 39000..40000 x 4 93 / 88, 2 of 4000..60000 x 1 of 16 query heads 33.7 / 19.1, 39 of 1000 and one of 60000 x 1
+// 32 / 20; 4 of 20000..60000 x 8 81.0 / 80.4.  The lines: with fewer CUs in use the gain is lost (52 heads on 208 CUs: 5000..40000 tokens 80.8 / 86.5, 96 on
+// 192: 142 / 187), and four splits of long rows leave too little to even out: 64 heads, 4 rows of 20000..60000 147 / 158, of up to 10000 all 3 to 12 % faster.
+static int wide_splits(int B, int n_kv, int nsplit, long max_tiles, long least) {
+  const long heads = (long)B * n_kv, n = 256 / std::max(heads, 1l);
+  const bool wide = heads <= 40 ? n * heads >= 240 : heads <= 64 && n * heads >= 248 && max_tiles <= 640;
+  return B > 1 && wide && n >= least ? (int)std::min<long>(nsplit, n) : nsplit;
+}
+
 // Splits of a launch whose length the host knows: those of nsplit that get tiles, at least MIN_HOST_TILES each (the caller's count is an upper
 // bound here, as it is in a planned launch; it sizes the workspace).  Empty splits and splits of a tile or two are blocks that only start, publish
 // and are waited for.  us with splits of 2 or 3 / 3 / 4 / 6 tiles: 1000 tokens x 8 kv heads 9.3 / 8.4 / 8.4 / 9.1, 300 x 8 8.3 / 7.6 / 7.5 / 8.0,
@@ -1819,8 +1836,10 @@ extern "C" int gaac_paged_attn(
   GAAC_REQUIRE(nsplit >= 1 && nsplit <= MAX_SLOTS, "gaac_paged_attn: nsplit must be in 1..%d", MAX_SLOTS);
   const long max_tiles = ((long)max_seq_len + T - 1) / T;
   GAAC_REQUIRE(max_seq_len >= 0 && max_tiles <= (long)bt_stride, "gaac_paged_attn: max_seq_len %d needs %ld blocks per row, the block table has %d", max_seq_len, max_tiles, bt_stride);
+  const long least = (max_tiles + MAX_CHUNK - 1) / MAX_CHUNK;
+  nsplit = wide_splits(B, n_kv, nsplit, max_tiles, least);
   const int plan = plan_units(B, n_kv, nsplit, max_tiles);
-  nsplit = planned_splits(B, n_kv, nsplit, plan, (max_tiles + MAX_CHUNK - 1) / MAX_CHUNK);
+  nsplit = planned_splits(B, n_kv, nsplit, plan, least);
   AttnArgs A;
   A.k = StoreView{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, b3k, b4k};
   A.v = StoreView{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, b3v, b4v};

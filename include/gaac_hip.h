@@ -203,8 +203,8 @@ int gaac_paged_decode(const uint8_t* pool, int TS, const void* raw, const int* m
 /* paged_attention -> gaac_vpaged_launch, paged_kernel.py:42-277: decode attention of B rows over the pool through the block table
  * bt int32 [B][bt_stride] and the mode table; seq_lens int32 [B] (tokens incl. the filling block; no separate tail); max_seq_len =
  * an upper bound of seq_lens known to the host (checked against the block table's width).  Any nsplit >= 1 works for any length (a
- * block resolves 1024 tiles of its split at a time); two rows or more may share up to B * nsplit splits out by their lengths, a single row gets 256 / n_kv at
- * most (one at least, and none of more than 1024 tiles of max_seq_len).  Partial records pm, pl [B*n_q*nsplit], pa [B*n_q*nsplit*128] and the epoch
+ * block resolves 1024 tiles of its split at a time); two rows or more may share up to B * nsplit splits out by their lengths; a single row, or rows of up to
+ * 64 heads in all, may be given as few as 256 / (B * n_kv) splits (one at least, and none of more than 1024 tiles of max_seq_len).  Partial records pm, pl [B*n_q*nsplit], pa [B*n_q*nsplit*128] and the epoch
  * buffer [2 + B*n_kv*nsplit] as in gaac_attn_fused; out bf16 [B*n_q][128].
  * freeq != NULL: the launch also does the work of gaac_paged_free(freeq, n_free, stack, top) for the queue the preceding
  * gaac_paged_store filled (the attention pops nothing, so pushes cannot race a pop here): a decode step is then two launches
