@@ -1583,11 +1583,16 @@ using namespace gaac;
 //     order can save is a split of the longest row at the end of the launch, the cost comes with every round.  One split per row, us
 //     without and with the plan: 256 rows of up to 1000 tokens x 16 kv heads (4096 blocks, 67 tiles): 150 and 168, 256 of up to 2000 x
 //     8 (2048, 129): 144 and 144, 128 of up to 4000 x 8 (1024, 254): 159 and 137.
-static int plan_units(int B, int n_kv, int nsplit, long max_tiles) {
+// wide: the caller asked for more splits than the one round of eight-wave blocks that wide_splits left, so that an even share is what a long row loses by.
+// Planned from two tiles a wave on (16 tiles a split) instead of five; us without and with the plan, with the store: 3 rows of 1400..6200 tokens x 8 kv heads
+// 20.7 / 18.6, 5 of 400..2700 x 8 18.0 / 16.8, 8 of 190..1300 x 8 16.4 / 16.3, 2 of 3600..10500 x 4 17.6 / 16.7, 20 of 270..2900 x 2 18.6 / 17.4; alike rows pay the
+// plan's start, 2 of 13000..14000 x 4 18.6 / 19.3, 8 of 1400..1500 x 8 17.3 / 18.0 (22.9 and 21.9 in four-wave blocks, planned).  From one tile a wave on nothing changes further.
+constexpr long WIDE_PLAN = 16;
+static int plan_units(int B, int n_kv, int nsplit, long max_tiles, bool wide = false) {
   const long blocks = (long)B * n_kv * nsplit;
   const int units = std::max((blocks > 256 ? 512 : 256) / n_kv, 1);
   if (B <= 1 || B > PLAN_ROWS || blocks >= SMALL_DIV) return 0;
-  if (blocks <= 256) return nsplit > 1 && max_tiles > 40l * nsplit ? units : 0;
+  if (blocks <= 256) return nsplit > 1 && max_tiles > (wide ? WIDE_PLAN : 40l) * nsplit ? units : 0;
   if (nsplit > 1 && units >= B) return units;
   return 8 * max_tiles >= blocks * nsplit ? units : 0;
 }
@@ -1837,8 +1842,9 @@ extern "C" int gaac_paged_attn(
   const long max_tiles = ((long)max_seq_len + T - 1) / T;
   GAAC_REQUIRE(max_seq_len >= 0 && max_tiles <= (long)bt_stride, "gaac_paged_attn: max_seq_len %d needs %ld blocks per row, the block table has %d", max_seq_len, max_tiles, bt_stride);
   const long least = (max_tiles + MAX_CHUNK - 1) / MAX_CHUNK;
-  nsplit = wide_splits(B, n_kv, nsplit, max_tiles, least);
-  const int plan = plan_units(B, n_kv, nsplit, max_tiles);
+  const int cut = wide_splits(B, n_kv, nsplit, max_tiles, least);
+  const int plan = plan_units(B, n_kv, cut, max_tiles, cut < nsplit);
+  nsplit = cut;
   nsplit = planned_splits(B, n_kv, nsplit, plan, least);
   AttnArgs A;
   A.k = StoreView{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, b3k, b4k};

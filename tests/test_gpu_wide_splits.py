@@ -21,6 +21,7 @@ CASES = [
     ([2600] * 8, 8, 32, 4), (_even(8, 200, 3000), 8, 32, None),     # 64 heads
     ([10240, 100], 32, 32, None), ([10241, 100], 32, 32, None),     # 640 tiles, 641
     (_even(5, 1, 700), 13, 32, None),                               # 65 heads
+    ([100, 2560, 900], 8, 32, None), ([100, 2561, 900], 8, 32, None), ([2561] * 3, 8, 32, 10), ([0, 1, 2600], 8, 11, None),     # ten splits: 160 tiles, 161 and more are planned
     ([500] * 5 + [20000], 4, 85, None), ([0, 5000, 3], 4, 64, None), ([16] * 2, 1, 200, 128),
 ]
 
