@@ -632,10 +632,11 @@ __global__ void __launch_bounds__(256) k_prompt_pack(const PromptPackArgs P) {
 }
 // Short prompts (SCAN_PROMPT_TILES, SCAN_PROMPT_ALL_TILES): encoding, tile offsets and the escapes' way into the stream in one launch.  A block of four tiles says how many bytes it has
 // in a 64-bit word that carries the launch's epoch, waits for the words of the head's earlier blocks and puts its escapes, which are in LDS until then, behind theirs.
-// scan: [1 + SCAN_PROMPT_BLOCKS] words for K or V of a cache head, zeroed once: [0] the epoch of the last launch, which every block reads at its start and the
-// head's last block, when it has seen the words of all, advances.  Launches on one cache head are ordered on a stream, as its contents demand.  A block waits for
-// blocks with a smaller index, which start before it and wait only for smaller ones; the wait is bounded all the same, and a head that gave up reports a
-// negative total, which leaves the host's word unwritten (gaac_wait_words raises).
+// scan: [1 + SCAN_PROMPT_BLOCKS] words for K or V of a cache head, zeroed once: the low half of [0] is the epoch of the last launch, which every block reads at its
+// start and the head's last block, when it has seen the words of all, advances.  Launches on one cache head are ordered on a stream, as its contents demand.  A block
+// waits for blocks with a smaller index, which start before it and wait only for smaller ones; the wait is bounded all the same.  A block that gives up, any of the
+// head's, says so in the high half of [0] (its own size is out by then, so that the last block may see the words of all): k_prompt_finish, behind all blocks, then
+// reports a negative total, which leaves the host's word unwritten (gaac_wait_words raises), and zeroes the words, some of which late blocks may have written.
 // Latency: a launch less (5 us), against waiting for the slowest block ahead (2 to 3).  us a call, encoding and packing in two launches / in one: 300 tokens x 8 heads 18.5 /
 // 15.9, 777 18.9 / 16.4, 777 x 16 19.6 / 17.4, 1500 x 8 (1488 tiles) 19.5 / 17.4, 2500 x 8 (2496) 20.1 / 19.1, 4095 x 2 (1020) 18.8 / 17.4; but 4095 x 8 (4080) 21.6 / 22.0: a
 // chip full of blocks that wait.  (A block of sixteen waves for all tiles of a head, which has nobody to wait for: 777 tokens the same as two launches, 2047 30 us
@@ -653,7 +654,8 @@ __device__ __forceinline__ void prompt_fused_body(const PromptFusedArgs& P, Enco
   RowRegs R;
   load_rows<false>(R, xh + (long)min(tile, ntiles - 1) * T * J.row_stride, J.row_stride, T, lane);
   if (wave == 0) reinterpret_cast<u32x2*>(&L.B.w[0][0])[lane] = load_base_pair<KIND>(J.b3 + (long)brow * D, J.b4 + (long)brow * D, lane);
-  const u32 last = (u32)__hip_atomic_load(scan, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), epoch = last + (last == 0xFFFFFFFFu ? 2u : 1u);      // (0 is what the words start with)
+  u32* state = reinterpret_cast<u32*>(scan);      // epoch | whether a block gave up
+  const u32 last = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), epoch = last + (last == 0xFFFFFFFFu ? 2u : 1u);      // (0 is what the words start with)
   const int head_start = P.head_start[h];
   store_rows(L.w[wave], R, lane);
   __syncthreads();
@@ -683,9 +685,10 @@ __device__ __forceinline__ void prompt_fused_body(const PromptFusedArgs& P, Enco
     const int before = __builtin_amdgcn_readlane(x, 15) + __builtin_amdgcn_readlane(x, 31) + __builtin_amdgcn_readlane(x, 47) + __builtin_amdgcn_readlane(x, 63);
     if (lane == 0) {
       ahead = ok ? before : -1;
-      if (block == (int)gridDim.x - 1) {
-        P.s.head_bytes[KIND * P.s.n_kv + h] = ok ? before + own : -1;
-        __hip_atomic_store(scan, (u64)epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (!ok) __hip_atomic_store(state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else if (block == (int)gridDim.x - 1) {
+        P.s.head_bytes[KIND * P.s.n_kv + h] = before + own;
+        __hip_atomic_store(state, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
   }
@@ -707,12 +710,21 @@ __global__ void __launch_bounds__(64 * CODEC_WAVES) k_prompt_fused(const PromptF
   if (blockIdx.z == KIND_K) prompt_fused_body<KIND_K>(P, L, sizes, ahead, blockIdx.y, wave, lane);
   else prompt_fused_body<KIND_V>(P, L, sizes, ahead, blockIdx.y, wave, lane);
 }
+// The total of one kind of a head, -1 where a block gave up (the words are then zeroed for the next launch: all blocks are through).
+__device__ __forceinline__ int fused_total(int head_bytes, u64* scan) {
+  if (reinterpret_cast<const u32*>(scan)[1] == 0u) return head_bytes;
+  for (int i = 0; i < 1 + SCAN_PROMPT_BLOCKS; ++i) scan[i] = 0ull;
+  return -1;
+}
 // ... and the counters of the heads, with the totals in host memory as k_words_to_host puts them there.
-__global__ void __launch_bounds__(64) k_prompt_finish(const PromptScanArgs A, int* __restrict__ host) {
+__global__ void __launch_bounds__(64) k_prompt_finish(const PromptScanArgs A, u64* scan, long scan_v, int* __restrict__ host) {
   for (int h = threadIdx.x; h < A.n_kv; h += 64) {
-    const int k = A.head_bytes[h], v = A.head_bytes[A.n_kv + h], failed = (k | v) < 0 ? 0x7FFFFFFF : 0;      // (a total that fits no window)
+    u64* words = scan + (long)h * (1 + SCAN_PROMPT_BLOCKS);
+    const int k = fused_total(A.head_bytes[h], words), v = fused_total(A.head_bytes[A.n_kv + h], words + scan_v);
+    const int failed = (k | v) < 0 ? 0x7FFFFFFF : 0;      // (a total that fits no window)
     set_prompt_counters(A, KIND_K, h, max(k, failed), max(v, failed));
     set_prompt_counters(A, KIND_V, h, max(v, failed), max(k, failed));
+    A.head_bytes[h] = k; A.head_bytes[A.n_kv + h] = v;
     if (host) { store_to_host(host + h, k); store_to_host(host + A.n_kv + h, v); }
   }
 }
@@ -902,7 +914,7 @@ int gaac_cache_prefill(
   if (fused) {
     const PromptFusedArgs A{E, P, head_start + head0, {k_ovf, v_ovf}, reinterpret_cast<u64*>(scan), scan_v};
     hipLaunchKernelGGL(k_prompt_fused, dim3((ntiles + CODEC_WAVES - 1) / CODEC_WAVES, n_kv, 2), dim3(64 * CODEC_WAVES), 0, st, A);
-    hipLaunchKernelGGL(k_prompt_finish, dim3(1), dim3(64), 0, st, P, host_bytes);
+    hipLaunchKernelGGL(k_prompt_finish, dim3(1), dim3(64), 0, st, P, A.scan, scan_v, host_bytes);
     return launch_status("gaac_cache_prefill");
   }
   if (ntiles <= PROMPT_PACK_TILES) {

@@ -84,7 +84,8 @@ int gaac_decode_tiles(int kind, const uint8_t* sm, const uint8_t* codes, const i
  * it the same for V, zeroed once and kept with the cache heads: short prompts then take a launch less; calls on one
  * cache head must be ordered on one stream.  head_bytes and host_bytes (or NULL; host memory the device can write) receive the
  * heads' escape totals, K's first: a head whose total + 1288 exceeds ovf_cap is left EMPTY (S = tail_len = 0), and the caller repeats
- * the call with larger windows.  host_bytes is set to -1 by the call and to the totals when all of the prompt is in place (gaac_wait_words). */
+ * the call with larger windows.  With scan, blocks wait for each other for a bounded time: a head where one gave up (a chip that other streams keep busy for
+ * most of a second) is left EMPTY as well, its total is -1 and its words are zero again.  host_bytes is set to -1 by the call and to the totals when all of the prompt is in place (gaac_wait_words). */
 int gaac_cache_prefill(
     const void* k, const void* v, long k_head_stride, long k_row_stride, long v_head_stride, long v_row_stride, int L, int n_kv, int head0,
     int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,

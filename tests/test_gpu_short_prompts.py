@@ -1,6 +1,6 @@
 """Prompts whose blocks place their escapes among themselves, at the edges of the blocks (four tiles, 64 blocks) and on both sides of the lines to the two
 launches (256 tiles a head, 3072 of all): every field of the slot against a page of the same rows, slots put in again and again, windows that are too small, the
-epoch's wrap-around, prompts into two slots on two streams, a wait that failed."""
+epoch's wrap-around, prompts into two slots on two streams, a wait that failed, a block that gave up."""
 import pytest
 import torch
 
@@ -111,3 +111,26 @@ def test_a_failed_wait_leaves_the_slot_armed(through, monkeypatch):
     assert not cache._scan[:, 2:4].any() and torch.equal(cache._scan[:, :2], armed[:, :2]) and torch.equal(cache._scan[:, 4:], armed[:, 4:])
     cache.prefill(1, v, k)
     _check(cache, 1, v, k)
+
+
+@pytest.mark.parametrize("through", ["binding", "python"])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_a_block_that_gave_up_fails_the_prompt_wherever_it_stands(kind, through, monkeypatch):
+    """The mark of a block that gave up, left by the host: the launch itself finds all words, as the last block does if it looks late enough."""
+    require_gpu()
+    from gaac_amd import CompressedKVCache, _lib
+    cache = CompressedKVCache(2, 3, 600)
+    k, v = _rows(577, 3, 1, 1e-3), _rows(577, 3, 2, 1e-3)      # nine blocks a head and a tail
+    for slot in range(2): cache.prefill(slot, k, v)
+    cache._scan[kind, 4, 0] += 1 << 32      # slot 1, head 1
+    other = cache._scan[:, :3].clone()
+    with monkeypatch.context() as m:
+        if through == "python": m.setattr(_lib, "_calls", _lib._CtypesCalls())
+        m.setattr(cache, "_rearm", lambda slot: None)      # the device has it done
+        with pytest.raises(RuntimeError, match="gaac_wait_words"): cache.prefill(1, v, k)
+    assert cache.S.tolist() == [576] * 4 + [0, 576] and cache.tail_len.tolist() == [1] * 4 + [0, 1]
+    assert not cache._scan[kind, 4].any() and torch.equal(cache._scan[:, :3], other) and cache._scan[1 - kind, 4].any()
+    for n in (577, 100, 577):
+        cache.prefill(1, v[:n], k[:n])
+        _check(cache, 1, v[:n], k[:n])
+    _check(cache, 0, k, v)
