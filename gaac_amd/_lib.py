@@ -23,7 +23,8 @@ _SIGNATURES = {
     "gaac_page_finish": [P, P, P, c_int, c_int, c_int, P, P, P, P, P, c_long, P, P],
     "gaac_row_offsets": [P, c_int, c_int, c_int, P, P, P],
     "gaac_decode_tiles": [c_int, P, P, P, P, P, P, P, P, c_int, P, c_int, c_int, c_int, P, c_long, c_long, P],
-    "gaac_cache_prefill": [P, P] + [c_long] * 4 + [c_int] * 7 + [P] * 22 + [c_long] + [P] * 4 + [c_long] + [P] * 2,
+    "gaac_prompt_store": [P, P] + [c_long] * 4 + [c_int] * 7 + [P] * 22 + [c_long] + [P] * 4 + [c_long, c_int, c_int, P, P],
+    "gaac_cache_prefill": [P, P] + [c_long] * 4 + [c_int] * 7 + [P] * 27,
     "gaac_attn_split": [P] * 16 + [P, P, c_int, c_int, c_int, P, c_int, c_float, c_int, c_int, P, P, P, c_int, P, P, P, P],
     "gaac_attn_combine": [P, P, P, P, c_int, c_int, P],
     "gaac_cache_append": [P, c_int, c_int, P, P, P, P, c_int, c_int, c_int] + [P] * 18 + [P, P],

@@ -95,7 +95,8 @@ PyObject* invoke(const char* name, int (*fn)(A...), PyObject* const* args, Py_ss
 #define GAAC_ENTRY_POINTS(X)                                                                                                              \
   X(gaac_wait_words) X(gaac_page_finish) X(gaac_cache_check)                                                                              \
   X(gaac_exponent_hist) X(gaac_bases_from_hist) X(gaac_encode_tiles) X(gaac_compact) X(gaac_tile_scan) X(gaac_page_pack)                  \
-  X(gaac_row_offsets) X(gaac_decode_tiles) X(gaac_cache_prefill) X(gaac_attn_split) X(gaac_attn_combine) X(gaac_cache_append)             \
+  X(gaac_row_offsets) X(gaac_decode_tiles) X(gaac_prompt_store) X(gaac_cache_prefill) X(gaac_attn_split) X(gaac_attn_combine)             \
+  X(gaac_cache_append)                                                                                                                    \
   X(gaac_paged_store) X(gaac_paged_free) X(gaac_paged_release) X(gaac_paged_decode) X(gaac_paged_attn) X(gaac_bf16_attn)                  \
   X(gaac_attn_fused) X(gaac_attn_fused_static) X(gaac_static_init) X(gaac_static_reset) X(gaac_static_flags) X(gaac_attn_launch)
 #define X(name)                                            \
@@ -282,7 +283,7 @@ PyObject* prompt_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int *tail_len = address<int>(get(a[0], n_tail_len)), *S = address<int>(get(a[0], n_S)), *head_start = address<int>(get(ko, n_head_start));
     const long ovf_cap = number(get(ko, n_ovf_cap)), nb = tensor(get(ko, n_base3)).size(0);
     const at::Tensor& scan = tensor(get(a[0], n__scan));
-    const long scan_row = scan.stride(1);
+    const long scan_row = scan.size(2);
     void* stream = stream_of(a[4]);
     // scratch: escape slots | exponent counts (hist_bytes in kv_cache.py) | tile sizes | head sizes
     const long tables = 2 * n_kv * std::max(std::min((L + 255) / 256, std::max(std::min(256 / (2 * n_kv), 64l), 1l)), (L + 65534) / 65535);
@@ -290,13 +291,12 @@ PyObject* prompt_store(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at::Tensor scratch = bytes(k, {at_sizes + 4 * (nt + 2 * n_kv)}), totals = host_words(2 * n_kv);
     uint8_t* base = static_cast<uint8_t*>(scratch.data_ptr());
     int* words = static_cast<int*>(totals.data_ptr());
-    const char* at = "gaac_cache_prefill";
-    must(at, without_gil([&] {
-      return p_gaac_cache_prefill(k.data_ptr(), v.data_ptr(), k_hs, k_rs, v_hs, v_rs, static_cast<int>(L), static_cast<int>(n_kv), static_cast<int>(slot * n_kv), static_cast<int>(cap),
-                                  static_cast<int>(ovf_cap), static_cast<int>(nb), calibrate, tail_len, S, head_start, K.tail, K.b3, K.b4, K.sm, K.cd, K.fl, K.ov, K.to, K.used,
-                                  V.tail, V.b3, V.b4, V.sm, V.cd, V.fl, V.ov, V.to, V.used, base + at_hist, at_sizes - at_hist, base,
-                                  reinterpret_cast<int*>(base + at_sizes), reinterpret_cast<int*>(base + at_sizes + 4 * nt),
-                                  static_cast<unsigned long long*>(scan.data_ptr()) + slot * n_kv * scan_row, scan.stride(0), words, stream);
+    must("gaac_prompt_store", without_gil([&] {
+      return p_gaac_prompt_store(k.data_ptr(), v.data_ptr(), k_hs, k_rs, v_hs, v_rs, static_cast<int>(L), static_cast<int>(n_kv), static_cast<int>(slot * n_kv), static_cast<int>(cap),
+                                 static_cast<int>(ovf_cap), static_cast<int>(nb), calibrate, tail_len, S, head_start, K.tail, K.b3, K.b4, K.sm, K.cd, K.fl, K.ov, K.to, K.used,
+                                 V.tail, V.b3, V.b4, V.sm, V.cd, V.fl, V.ov, V.to, V.used, base + at_hist, at_sizes - at_hist, base,
+                                 reinterpret_cast<int*>(base + at_sizes), reinterpret_cast<int*>(base + at_sizes + 4 * nt),
+                                 static_cast<unsigned long long*>(scan.data_ptr()) + slot * n_kv * scan_row, scan.stride(0), static_cast<int>(scan_row), 0, words, stream);
     }));
     must("gaac_wait_words", without_gil([&] { return p_gaac_wait_words(words, static_cast<int>(2 * n_kv), stream); }));
     return numbers(totals);

@@ -28,6 +28,7 @@ char* last_error_buffer() { static thread_local char buf[512] = {0}; return buf;
 // which a launch had to clear first, the counts of a prompt took that launch longer: 32768 tokens x 8 heads 88.1 -> 83.2 us a call, 4000 tokens 26.2 -> 24.5 of
 // kernels.
 constexpr int HIST_WAVES = 16, HIST_MAX_CHUNK = 65535, HIST_LOADS = 2, HIST_TABLES = 64;      // HIST_LOADS: loads of four rows in flight per wave
+constexpr long HIST_TABLE = 256 * 64 * sizeof(u32) + HIST_WAVES * sizeof(u16);      // bytes
 struct HistArgs { const u16* x[2]; long head_stride[2], row_stride[2]; long n_tok; int chunk, n_kv; unsigned long long* hist; u32* rows; u16* bits; };      // rows [pair][chunk][256][64], bits [pair][chunk][16]
 template <bool PARTS>
 __global__ void __launch_bounds__(64 * HIST_WAVES) k_exponent_hist(const HistArgs A) {
@@ -102,8 +103,7 @@ static int hist_chunks(long n_tok, int pairs, bool parts) {
   const long n = min((n_tok + 255) / 256, (long)min(max(1, 256 / pairs), parts ? HIST_TABLES : 256));
   return (int)max(n, (n_tok + HIST_MAX_CHUNK - 1) / HIST_MAX_CHUNK);
 }
-static int launch_hist(HistArgs& A, int kinds, hipStream_t stream) {      // returns the blocks of a (kind, head), hist_chunks at most
-  const int nchunk = hist_chunks(A.n_tok, kinds * A.n_kv, A.rows != nullptr);
+static int launch_hist(HistArgs& A, int kinds, int nchunk, hipStream_t stream) {      // returns the blocks of a (kind, head), nchunk at most
   A.chunk = (int)((A.n_tok + nchunk - 1) / nchunk);
   const dim3 grid((unsigned)((A.n_tok + A.chunk - 1) / A.chunk), A.n_kv, kinds);
   if (A.rows) hipLaunchKernelGGL(k_exponent_hist<true>, grid, dim3(64 * HIST_WAVES), 0, stream, A);
@@ -632,7 +632,7 @@ __global__ void __launch_bounds__(256) k_prompt_pack(const PromptPackArgs P) {
 }
 // Short prompts (SCAN_PROMPT_TILES, SCAN_PROMPT_ALL_TILES): encoding, tile offsets and the escapes' way into the stream in one launch.  A block of four tiles says how many bytes it has
 // in a 64-bit word that carries the launch's epoch, waits for the words of the head's earlier blocks and puts its escapes, which are in LDS until then, behind theirs.
-// scan: [1 + SCAN_PROMPT_BLOCKS] words for K or V of a cache head, zeroed once: the low half of [0] is the epoch of the last launch, which every block reads at its
+// scan: words for K or V of a cache head, one and one for each of its blocks, zeroed once: the low half of [0] is the epoch of the last launch, which every block reads at its
 // start and the head's last block, when it has seen the words of all, advances.  Launches on one cache head are ordered on a stream, as its contents demand.  A block
 // waits for blocks with a smaller index, which start before it and wait only for smaller ones; the wait is bounded all the same.  A block that gives up, any of the
 // head's, says so in the high half of [0] (its own size is out by then, so that the last block may see the words of all): k_prompt_finish, behind all blocks, then
@@ -641,15 +641,16 @@ __global__ void __launch_bounds__(256) k_prompt_pack(const PromptPackArgs P) {
 // 15.9, 777 18.9 / 16.4, 777 x 16 19.6 / 17.4, 1500 x 8 (1488 tiles) 19.5 / 17.4, 2500 x 8 (2496) 20.1 / 19.1, 4095 x 2 (1020) 18.8 / 17.4; but 4095 x 8 (4080) 21.6 / 22.0: a
 // chip full of blocks that wait.  (A block of sixteen waves for all tiles of a head, which has nobody to wait for: 777 tokens the same as two launches, 2047 30 us
 // against 16.)
-constexpr int SCAN_PROMPT_TILES = 256, SCAN_PROMPT_BLOCKS = SCAN_PROMPT_TILES / CODEC_WAVES, SCAN_PROMPT_ALL_TILES = 3072, SCAN_SPIN_LIMIT = 1 << 20;      // of a head | of all heads, K and V
-struct PromptFusedArgs { EncodeArgs e; PromptScanArgs s; const int* head_start; uint8_t* ovf[2]; u64* scan; long scan_v; };      // scan: of K of head 0 of the call, scan_v words further on V
+constexpr int SCAN_PROMPT_TILES = 256, SCAN_PROMPT_ALL_TILES = 3072, SCAN_SPIN_LIMIT = 1 << 20;      // of a head | of all heads, K and V
+struct ScanWords { u64* k; long v; int row, spins; };      // K's of the call's first head, V's v words further on, row words a head (1 + blocks, or more); re-reads before a block gives up
+struct PromptFusedArgs { EncodeArgs e; PromptScanArgs s; const int* head_start; uint8_t* ovf[2]; ScanWords scan; };
 template <int KIND>
 __device__ __forceinline__ void prompt_fused_body(const PromptFusedArgs& P, EncodeBlockLds& L, int (&sizes)[CODEC_WAVES], int& ahead, int h, int wave, int lane) {
   const EncodeArgs& A = P.e;
   const EncodeKind& J = KIND == KIND_K ? A.k : A.v;
   const PromptKind& K = P.s.j[KIND];
   const int ntiles = A.ntiles, block = blockIdx.x, tile = block * CODEC_WAVES + wave, brow = (A.brow0 + h) % A.NB;
-  u64* scan = P.scan + (KIND == KIND_V ? P.scan_v : 0) + (long)h * (1 + SCAN_PROMPT_BLOCKS);
+  u64* scan = P.scan.k + (KIND == KIND_V ? P.scan.v : 0) + (long)h * P.scan.row;
   const u16* xh = J.x + (long)h * J.head_stride;
   RowRegs R;
   load_rows<false>(R, xh + (long)min(tile, ntiles - 1) * T * J.row_stride, J.row_stride, T, lane);
@@ -672,12 +673,12 @@ __device__ __forceinline__ void prompt_fused_body(const PromptFusedArgs& P, Enco
   const int own = sizes[0] + sizes[1] + sizes[2] + sizes[3];
   if (wave == 0) {
     if (lane == 0) __hip_atomic_store(scan + 1 + block, (u64)(u32)own | ((u64)epoch << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // lane: an earlier block (SCAN_PROMPT_BLOCKS of them at most; the others read the block's own word)
+    // lane: an earlier block (64 blocks at most; the others read the block's own word)
     const u64* w = scan + 1 + min(lane, block);
     u64 v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     bool ok = true;
     for (int spin = 0; __builtin_amdgcn_ballot_w64(lane < block && (u32)(v >> 32) != epoch) != 0; ++spin) {
-      if (spin >= SCAN_SPIN_LIMIT) { ok = false; break; }
+      if (spin >= P.scan.spins) { ok = false; break; }
       __builtin_amdgcn_s_sleep(1);
       if ((u32)(v >> 32) != epoch) v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -711,16 +712,16 @@ __global__ void __launch_bounds__(64 * CODEC_WAVES) k_prompt_fused(const PromptF
   else prompt_fused_body<KIND_V>(P, L, sizes, ahead, blockIdx.y, wave, lane);
 }
 // The total of one kind of a head, -1 where a block gave up (the words are then zeroed for the next launch: all blocks are through).
-__device__ __forceinline__ int fused_total(int head_bytes, u64* scan) {
+__device__ __forceinline__ int fused_total(int head_bytes, u64* scan, int row) {
   if (reinterpret_cast<const u32*>(scan)[1] == 0u) return head_bytes;
-  for (int i = 0; i < 1 + SCAN_PROMPT_BLOCKS; ++i) scan[i] = 0ull;
+  for (int i = 0; i < row; ++i) scan[i] = 0ull;      // (all of them: the epoch starts again from 1, which older launches may have left)
   return -1;
 }
 // ... and the counters of the heads, with the totals in host memory as k_words_to_host puts them there.
-__global__ void __launch_bounds__(64) k_prompt_finish(const PromptScanArgs A, u64* scan, long scan_v, int* __restrict__ host) {
+__global__ void __launch_bounds__(64) k_prompt_finish(const PromptScanArgs A, const ScanWords W, int* __restrict__ host) {
   for (int h = threadIdx.x; h < A.n_kv; h += 64) {
-    u64* words = scan + (long)h * (1 + SCAN_PROMPT_BLOCKS);
-    const int k = fused_total(A.head_bytes[h], words), v = fused_total(A.head_bytes[A.n_kv + h], words + scan_v);
+    u64* words = W.k + (long)h * W.row;
+    const int k = fused_total(A.head_bytes[h], words, W.row), v = fused_total(A.head_bytes[A.n_kv + h], words + W.v, W.row);
     const int failed = (k | v) < 0 ? 0x7FFFFFFF : 0;      // (a total that fits no window)
     set_prompt_counters(A, KIND_K, h, max(k, failed), max(v, failed));
     set_prompt_counters(A, KIND_V, h, max(v, failed), max(k, failed));
@@ -764,7 +765,7 @@ int gaac_exponent_hist(const void* x, long n_tokens, int n_kv, long long* hist, 
   if (n_tokens == 0) return 0;
   const long row = (long)n_kv * D;
   HistArgs A{{(const u16*)x, nullptr}, {D, 0}, {row, 0}, n_tokens, 0, n_kv, (unsigned long long*)hist, nullptr, nullptr};
-  launch_hist(A, 1, (hipStream_t)stream);
+  launch_hist(A, 1, hist_chunks(n_tokens, n_kv, false), (hipStream_t)stream);
   return launch_status("gaac_exponent_hist");
 }
 
@@ -862,31 +863,38 @@ int gaac_decode_tiles(int kind, const uint8_t* sm, const uint8_t* codes, const i
   return launch_status("gaac_decode_tiles");
 }
 
-int gaac_cache_prefill(
+// hist_bytes < 0: hist as gaac_cache_prefill takes it, 2^17 bytes for K and for V of each head, which are a table; prompts that want more tables, or need
+// them, have them where their escapes will be (1280 bytes a tile against a table for 256 tokens or more).
+static int prompt_store(
+    const char* name,
     const void* k, const void* v, long k_head_stride, long k_row_stride, long v_head_stride, long v_row_stride, int L, int n_kv, int head0,
     int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
     void* k_tail, uint8_t* k_base3, uint8_t* k_base4, uint8_t* k_sm, uint8_t* k_codes, int* k_flags, uint8_t* k_ovf, int* k_tile_off, int* k_ovf_used,
     void* v_tail, uint8_t* v_base3, uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
-    void* hist, long hist_bytes, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, unsigned long long* scan, long scan_v, int* host_bytes, void* stream) {
-  GAAC_REQUIRE(((k && v) || L == 0) && tail_len && S && head_start && head_bytes, "gaac_cache_prefill: null pointer");
-  GAAC_REQUIRE(k_tail && k_base3 && k_base4 && k_sm && k_codes && k_flags && k_ovf && k_tile_off && k_ovf_used, "gaac_cache_prefill: null K store pointer");
-  GAAC_REQUIRE(v_tail && v_base3 && v_base4 && v_sm && v_codes && v_flags && v_ovf && v_tile_off && v_ovf_used, "gaac_cache_prefill: null V store pointer");
+    void* hist, long hist_bytes, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, const ScanWords& scan, int* host_bytes, void* stream) {
+  GAAC_REQUIRE(((k && v) || L == 0) && tail_len && S && head_start && head_bytes, "%s: null pointer", name);
+  GAAC_REQUIRE(k_tail && k_base3 && k_base4 && k_sm && k_codes && k_flags && k_ovf && k_tile_off && k_ovf_used, "%s: null K store pointer", name);
+  GAAC_REQUIRE(v_tail && v_base3 && v_base4 && v_sm && v_codes && v_flags && v_ovf && v_tile_off && v_ovf_used, "%s: null V store pointer", name);
   GAAC_REQUIRE(L >= 0 && n_kv > 0 && head0 >= 0 && cap > 0 && cap % T == 0 && L <= cap && NB > 0 && ovf_cap >= 8,
-               "gaac_cache_prefill: bad sizes L=%d n_kv=%d head0=%d cap=%d ovf_cap=%d NB=%d", L, n_kv, head0, cap, ovf_cap, NB);
-  GAAC_REQUIRE(!calibrate || (hist && NB >= head0 + n_kv), "gaac_cache_prefill: calibration needs its scratch and a base row per cache head (NB=%d, heads %d..%d)", NB, head0, head0 + n_kv - 1);
-  const long tables = calibrate ? (long)2 * n_kv * hist_chunks(L, 2 * n_kv, true) : 0;
-  GAAC_REQUIRE(tables * (256 * 64 * (long)sizeof(u32) + 32) <= hist_bytes || tables == 0, "gaac_cache_prefill: %ld bytes of calibration scratch for %ld tables", hist_bytes, tables);
-  GAAC_REQUIRE((reinterpret_cast<uintptr_t>(hist) & 7) == 0, "gaac_cache_prefill: calibration scratch is not aligned to 8 bytes");
+               "%s: bad sizes L=%d n_kv=%d head0=%d cap=%d ovf_cap=%d NB=%d", name, L, n_kv, head0, cap, ovf_cap, NB);
+  GAAC_REQUIRE(!calibrate || (hist && NB >= head0 + n_kv), "%s: calibration needs its scratch and a base row per cache head (NB=%d, heads %d..%d)", name, NB, head0, head0 + n_kv - 1);
   const int ntiles = L / T;
-  GAAC_REQUIRE(ntiles == 0 || (esc_slots && tile_bytes), "gaac_cache_prefill: null scratch");
+  GAAC_REQUIRE(ntiles == 0 || (esc_slots && tile_bytes), "%s: null scratch", name);
   GAAC_REQUIRE(L == 0 || (k_row_stride >= D && k_row_stride % 8 == 0 && k_head_stride % 8 == 0 && v_row_stride >= D && v_row_stride % 8 == 0 && v_head_stride % 8 == 0 &&
-                          ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0), "gaac_cache_prefill: rows must be 16-byte aligned");
+                          ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0), "%s: rows must be 16-byte aligned", name);
+  int tables = calibrate ? hist_chunks(L, 2 * n_kv, true) : 0;      // of a (kind, head)
+  if (calibrate && hist_bytes < 0) {
+    const long room = (2l * n_kv * ntiles * TILE_MAX_ESC - 8) / (2 * n_kv * HIST_TABLE);
+    if (room >= 2 && tables >= 2) { hist = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(esc_slots) + 7) & ~(uintptr_t)7); tables = (int)std::min<long>(tables, room); }
+    else tables = 1;
+  } else if (calibrate) GAAC_REQUIRE(2l * n_kv * tables * HIST_TABLE <= hist_bytes, "%s: %ld bytes of calibration scratch for %ld tables", name, hist_bytes, 2l * n_kv * tables);
+  GAAC_REQUIRE(!calibrate || (reinterpret_cast<uintptr_t>(hist) & 7) == 0, "%s: calibration scratch is not aligned to 8 bytes", name);
   hipStream_t st = (hipStream_t)stream;
   if (calibrate) {
     u32* rows = (u32*)hist;
-    u16* bits = reinterpret_cast<u16*>(rows + tables * (256 * 64));
+    u16* bits = reinterpret_cast<u16*>(rows + 2l * n_kv * tables * (256 * 64));
     HistArgs H{{(const u16*)k, (const u16*)v}, {k_head_stride, v_head_stride}, {k_row_stride, v_row_stride}, L, 0, n_kv, nullptr, rows, bits};
-    const int chunks = L > 0 ? launch_hist(H, 2, st) : 0;
+    const int chunks = L > 0 ? launch_hist(H, 2, tables, st) : 0;
     const PromptBasesArgs B{rows, bits, chunks, {k_base3, v_base3}, {k_base4, v_base4}, n_kv, head0};
     // (as many loads in flight as there are tables for: a lane past the last table reads that one again)
     if (chunks <= 16) hipLaunchKernelGGL(k_prompt_bases<4>, dim3(4, n_kv, 2), dim3(1024), 0, st, B);
@@ -896,7 +904,8 @@ int gaac_cache_prefill(
   const long row0 = (long)head0 * cap, tile0 = (long)head0 * (cap / T), n_all = (long)n_kv * ntiles;
   uint8_t* v_slots = esc_slots ? esc_slots + n_all * TILE_MAX_ESC : nullptr;
   int* v_bytes = tile_bytes ? tile_bytes + n_all : nullptr;
-  const bool fused = scan && ntiles > 0 && ntiles <= SCAN_PROMPT_TILES && 2 * n_all <= SCAN_PROMPT_ALL_TILES;
+  const int nblocks = (ntiles + CODEC_WAVES - 1) / CODEC_WAVES;
+  const bool fused = scan.k && ntiles > 0 && ntiles <= SCAN_PROMPT_TILES && 2 * n_all <= SCAN_PROMPT_ALL_TILES && nblocks < scan.row;
   EncodeArgs E{};
   if (ntiles > 0) {
     E.kind0 = KIND_K; E.S = ntiles * T; E.S_pad = cap; E.ntiles = ntiles; E.brow0 = head0; E.NB = NB; E.bidx = nullptr;
@@ -912,10 +921,10 @@ int gaac_cache_prefill(
   P.S = S + head0; P.tail_len = tail_len + head0; P.head_bytes = head_bytes;
   if (host_bytes) for (int i = 0; i < 2 * n_kv; ++i) __atomic_store_n(host_bytes + i, -1, __ATOMIC_RELAXED);      // not there yet
   if (fused) {
-    const PromptFusedArgs A{E, P, head_start + head0, {k_ovf, v_ovf}, reinterpret_cast<u64*>(scan), scan_v};
-    hipLaunchKernelGGL(k_prompt_fused, dim3((ntiles + CODEC_WAVES - 1) / CODEC_WAVES, n_kv, 2), dim3(64 * CODEC_WAVES), 0, st, A);
-    hipLaunchKernelGGL(k_prompt_finish, dim3(1), dim3(64), 0, st, P, A.scan, scan_v, host_bytes);
-    return launch_status("gaac_cache_prefill");
+    const PromptFusedArgs A{E, P, head_start + head0, {k_ovf, v_ovf}, scan};
+    hipLaunchKernelGGL(k_prompt_fused, dim3(nblocks, n_kv, 2), dim3(64 * CODEC_WAVES), 0, st, A);
+    hipLaunchKernelGGL(k_prompt_finish, dim3(1), dim3(64), 0, st, P, scan, host_bytes);
+    return launch_status(name);
   }
   if (ntiles <= PROMPT_PACK_TILES) {
     const PromptPackArgs A{P, {esc_slots, v_slots}, head_start + head0, {k_ovf, v_ovf}};
@@ -929,7 +938,31 @@ int gaac_cache_prefill(
     hipLaunchKernelGGL(k_pack<false>, dim3((ntiles + PACK_TPB - 1) / PACK_TPB, n_kv, 2), dim3(256), 0, st, A);
   }
   if (host_bytes) hipLaunchKernelGGL(k_words_to_host, dim3(1), dim3(64), 0, st, head_bytes, 2 * n_kv, host_bytes);
-  return launch_status("gaac_cache_prefill");
+  return launch_status(name);
+}
+
+int gaac_prompt_store(
+    const void* k, const void* v, long k_head_stride, long k_row_stride, long v_head_stride, long v_row_stride, int L, int n_kv, int head0,
+    int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
+    void* k_tail, uint8_t* k_base3, uint8_t* k_base4, uint8_t* k_sm, uint8_t* k_codes, int* k_flags, uint8_t* k_ovf, int* k_tile_off, int* k_ovf_used,
+    void* v_tail, uint8_t* v_base3, uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
+    void* hist, long hist_bytes, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, unsigned long long* scan, long scan_v, int scan_row, int scan_spins,
+    int* host_bytes, void* stream) {
+  GAAC_REQUIRE(hist_bytes >= 0 && scan_spins >= 0 && (!scan || scan_row > 0), "gaac_prompt_store: bad sizes hist_bytes=%ld scan_row=%d scan_spins=%d", hist_bytes, scan_row, scan_spins);
+  return prompt_store("gaac_prompt_store", k, v, k_head_stride, k_row_stride, v_head_stride, v_row_stride, L, n_kv, head0, cap, ovf_cap, NB, calibrate, tail_len, S, head_start,
+                      k_tail, k_base3, k_base4, k_sm, k_codes, k_flags, k_ovf, k_tile_off, k_ovf_used, v_tail, v_base3, v_base4, v_sm, v_codes, v_flags, v_ovf, v_tile_off, v_ovf_used,
+                      hist, hist_bytes, esc_slots, tile_bytes, head_bytes, ScanWords{reinterpret_cast<u64*>(scan), scan_v, scan_row, scan_spins ? scan_spins : SCAN_SPIN_LIMIT}, host_bytes, stream);
+}
+
+int gaac_cache_prefill(
+    const void* k, const void* v, long k_head_stride, long k_row_stride, long v_head_stride, long v_row_stride, int L, int n_kv, int head0,
+    int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
+    void* k_tail, uint8_t* k_base3, uint8_t* k_base4, uint8_t* k_sm, uint8_t* k_codes, int* k_flags, uint8_t* k_ovf, int* k_tile_off, int* k_ovf_used,
+    void* v_tail, uint8_t* v_base3, uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
+    unsigned long long* hist, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, int* host_bytes, void* stream) {
+  return prompt_store("gaac_cache_prefill", k, v, k_head_stride, k_row_stride, v_head_stride, v_row_stride, L, n_kv, head0, cap, ovf_cap, NB, calibrate, tail_len, S, head_start,
+                      k_tail, k_base3, k_base4, k_sm, k_codes, k_flags, k_ovf, k_tile_off, k_ovf_used, v_tail, v_base3, v_base4, v_sm, v_codes, v_flags, v_ovf, v_tile_off, v_ovf_used,
+                      hist, -1, esc_slots, tile_bytes, head_bytes, ScanWords{}, host_bytes, stream);
 }
 
 }  // extern "C"

@@ -23,7 +23,7 @@ extern "C" {
 
 const char* gaac_last_error(void);
 
-/* Waits until none of the n words is negative: host memory that a launch on the stream fills (host_bytes of gaac_page_finish and gaac_cache_prefill).
+/* Waits until none of the n words is negative: host memory that a launch on the stream fills (host_bytes of gaac_page_finish, gaac_prompt_store and gaac_cache_prefill).
  * Later work of the stream is not waited for. */
 int gaac_wait_words(const int* words, int n, void* stream);
 
@@ -45,7 +45,7 @@ int gaac_encode_tiles(int kind, const void* x, long x_head_stride, long x_row_st
                       int* tile_bytes, void* stream);
 
 /* TileEncoder.compact, /root/reference/gaac/encoder.py:69-76, 104-109: writes tile_off[h, t] = sum of tile_bytes[h, 0..t) (int32
- * [H, ntiles], output) and copies tile (h, t)'s tile_bytes[h, t] escape bytes from its 1280-byte slot to
+ * [H, ntiles], output) and copies tile (h, t)'s tile_bytes[h, t] escape bytes from where gaac_encode_tiles left them to
  * ovf + head_start[h] + tile_off[h, t]. */
 int gaac_compact(const uint8_t* esc_slots, const int* tile_bytes, int* tile_off, const int* head_start, uint8_t* ovf,
                  int H, int ntiles, void* stream);
@@ -80,18 +80,28 @@ int gaac_decode_tiles(int kind, const uint8_t* sm, const uint8_t* codes, const i
  * L - L % 16 tokens become tiles, the rest goes to the raw tail; S, tail_len, ovf_used and, with calibrate, the heads' base rows are
  * set.  Store pointers are those of gaac_cache_append (whole cache: token stride cap, escape windows of ovf_cap bytes that start at
  * head_start[head]).  Scratch: hist (calibrate only), 8-byte aligned, hist_bytes >= 65568 * 2*n_kv * max(min(ceil(L/256), 64, max(256/(2*n_kv), 1)), ceil(L/65535)), esc_slots [2*n_kv*(L/16)*1280], tile_bytes
- * int32 [2*n_kv*(L/16)], head_bytes int32 [2*n_kv].  scan (or NULL): uint64 [n_kv][65] for K of the call's heads and scan_v words behind
- * it the same for V, zeroed once and kept with the cache heads: short prompts then take a launch less; calls on one
- * cache head must be ordered on one stream.  head_bytes and host_bytes (or NULL; host memory the device can write) receive the
+ * int32 [2*n_kv*(L/16)], head_bytes int32 [2*n_kv].  head_bytes and host_bytes (or NULL; host memory the device can write) receive the
  * heads' escape totals, K's first: a head whose total + 1288 exceeds ovf_cap is left EMPTY (S = tail_len = 0), and the caller repeats
- * the call with larger windows.  With scan, blocks wait for each other for a bounded time: a head where one gave up (a chip that other streams keep busy for
- * most of a second) is left EMPTY as well, its total is -1 and its words are zero again.  host_bytes is set to -1 by the call and to the totals when all of the prompt is in place (gaac_wait_words). */
+ * the call with larger windows.  host_bytes is set to -1 by the call and to the totals when all of the prompt is in place (gaac_wait_words).
+ * scan (or NULL): uint64 [n_kv][scan_row] for K of the call's heads and scan_v words behind it the same for V, zeroed once and kept with the cache heads: prompts
+ * of up to 256 tiles a head, 3072 in all and 64*(scan_row - 1) tokens then take a launch less; calls on one cache head must be ordered on one stream.  Their
+ * blocks wait for each other, for a bounded number of re-reads (scan_spins, or 0: 2^20, most of a second): a head where one gave up is left EMPTY
+ * as well, its total is -1 and its words are zero again. */
+int gaac_prompt_store(
+    const void* k, const void* v, long k_head_stride, long k_row_stride, long v_head_stride, long v_row_stride, int L, int n_kv, int head0,
+    int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
+    void* k_tail, uint8_t* k_base3, uint8_t* k_base4, uint8_t* k_sm, uint8_t* k_codes, int* k_flags, uint8_t* k_ovf, int* k_tile_off, int* k_ovf_used,
+    void* v_tail, uint8_t* v_base3, uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
+    void* hist, long hist_bytes, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, unsigned long long* scan, long scan_v, int scan_row, int scan_spins, int* host_bytes,
+    void* stream);
+
+/* gaac_prompt_store without scan, and with hist (calibrate only) uint64 [2*n_kv*256*64]. */
 int gaac_cache_prefill(
     const void* k, const void* v, long k_head_stride, long k_row_stride, long v_head_stride, long v_row_stride, int L, int n_kv, int head0,
     int cap, int ovf_cap, int NB, int calibrate, int* tail_len, int* S, const int* head_start,
     void* k_tail, uint8_t* k_base3, uint8_t* k_base4, uint8_t* k_sm, uint8_t* k_codes, int* k_flags, uint8_t* k_ovf, int* k_tile_off, int* k_ovf_used,
     void* v_tail, uint8_t* v_base3, uint8_t* v_base4, uint8_t* v_sm, uint8_t* v_codes, int* v_flags, uint8_t* v_ovf, int* v_tile_off, int* v_ovf_used,
-    void* hist, long hist_bytes, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, unsigned long long* scan, long scan_v, int* host_bytes, void* stream);
+    unsigned long long* hist, uint8_t* esc_slots, int* tile_bytes, int* head_bytes, int* host_bytes, void* stream);
 
 /* gaac_attn_launch, /root/reference/gaac/kernel.py:296-326 (kernels :48-294).  Same 16 store tensors, q [B*n_q, 128] bf16,
  * slot map [B] (slot < 0 = padded row, output 0; NULL = the identity, row b attends over cache heads b*n_kv ..), SL [cache heads] compressed tokens per head, S_pad = token stride of a
