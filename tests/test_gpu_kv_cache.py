@@ -219,11 +219,12 @@ def test_bytes_per_slot_is_what_the_cache_allocates(per_sequence_bases):
     per-head tensor of both stores (tile rows, tag words, tile offsets, escape streams, stream starts, counters, raw tails, and for
     per-sequence calibration the base rows) plus the two length vectors add up to n_slots * bytes_per_slot, except for the one closing
     entry of each store's stream-start vector (2 x 4 bytes per cache); per-model base tables (not per slot) are left out, as in the
-    reference's formula.  The oracle's restatement of the formula gives the same number."""
+    reference's formula, and so are the words of short prompts, a four-hundredth of the smallest slot at most.  The oracle's restatement of the formula gives the
+    same number."""
     dev = require_gpu()
     from gaac_amd import CompressedKVCache
     from gaac_amd.codec import exponent_hist, bases_from_hist
-    for (n_slots, n_kv, cap, ovf) in [(1, 1, 16, 128), (3, 2, 1000, 128), (5, 8, 4096, 512), (2, 4, 65536, 64)]:
+    for (n_slots, n_kv, cap, ovf) in [(1, 1, 16, 128), (3, 2, 1000, 128), (5, 8, 4096, 512), (2, 4, 65536, 64), (7, 2, 64, 16), (1, 3, 80, 128)]:
         bases = None
         if not per_sequence_bases:
             x = to_bf16(np.ascontiguousarray(kv_like16(n_kv, 256, seed=1).transpose(1, 0, 2)), dev)
@@ -238,3 +239,4 @@ def test_bytes_per_slot_is_what_the_cache_allocates(per_sequence_bases):
         want = CompressedKVCache.bytes_per_slot(n_kv, cap, ovf, per_sequence_bases)
         assert total - 2 * 4 == n_slots * want, (n_slots, n_kv, cap, ovf)
         assert want == O.bytes_per_slot(n_kv, cap, ovf, per_sequence_bases)
+        assert c._scan.dim() == 3 and 400 * nbytes(c._scan) <= n_slots * want

@@ -10,6 +10,12 @@ pytestmark = pytest.mark.gpu
 GUARD = 64
 
 
+@pytest.fixture(autouse=True)
+def large_blocks_go_back():
+    yield
+    torch.cuda.empty_cache()      # (a workspace that outlives a later test would hold on to one)
+
+
 def _words(cache, slot, k, v):
     """The arguments that both take, up to the stores'."""
     L, n_kv = k.shape[0], cache.n_kv
