@@ -240,3 +240,30 @@ def test_bytes_per_slot_is_what_the_cache_allocates(per_sequence_bases):
         assert total - 2 * 4 == n_slots * want, (n_slots, n_kv, cap, ovf)
         assert want == O.bytes_per_slot(n_kv, cap, ovf, per_sequence_bases)
         assert c._scan.dim() == 3 and 400 * nbytes(c._scan) <= n_slots * want
+
+
+@pytest.mark.parametrize("words", [True, False])
+def test_a_saved_cache_goes_on(words):
+    """Through torch.save and back, also from a file of a cache that had no words for short prompts yet: what it held, then prompts, steps and attention."""
+    import io
+    dev = require_gpu()
+    from gaac_amd import CompressedKVCache
+    g = torch.Generator(device=dev).manual_seed(5)
+    rows = lambda n: torch.randn(n, 2, 128, generator=g, device=dev).to(torch.bfloat16)
+    k, v, new, q, slots = rows(333), rows(333), rows(2), rows(2).repeat(1, 4, 1), torch.tensor([1, 0], dtype=torch.int32, device=dev)
+    a = CompressedKVCache(2, 2, 400)
+    a.prefill(0, k, v)
+    a.attention(q, slots, 128 ** -0.5)
+    if not words: del a._scan
+    f = io.BytesIO()
+    torch.save(a, f)
+    f.seek(0)
+    b = torch.load(f, weights_only=False)
+    if not words: a._arm()
+    for c in (a, b):
+        for n in (333, 100): c.prefill(1, v[:n], k[:n])
+        for _ in range(3): c.append(slots, new, new)
+    assert torch.allclose(a.attention(q, slots, 128 ** -0.5).float(), b.attention(q, slots, 128 ** -0.5).float(), rtol=2e-2, atol=2e-2)      # (waves share tiles out: sums in another order)
+    for slot in range(2):
+        for x, y in zip(a.decompress(slot), b.decompress(slot)): assert torch.equal(x, y)
+    b.check_capacity()
