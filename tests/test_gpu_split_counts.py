@@ -39,3 +39,20 @@ def test_more_half_heads_than_mergers(n_kv, G, L):
         got = O.bf16_to_f32(to_u16(cache.attention(to_bf16(q, dev), slots, SCALE, nsplit=nsplit)))[0]
         assert (np.abs(got - ref) <= tol).all(), nsplit
     cache.check_capacity()
+
+
+def test_max_len_of_any_kind_of_number():
+    """launch_nsplit keeps its results: a zero-dimensional array or tensor, which changes in place or has no hash, is looked at in each call."""
+    dev = require_gpu()
+    from gaac_amd import CompressedKVCache
+    from gaac_amd.kernel import launch_nsplit
+    cache = CompressedKVCache(2, 8, 4096)
+    slots, q = torch.arange(2, dtype=torch.int32, device=dev), torch.zeros(2, 8, 128, dtype=torch.bfloat16, device=dev)
+    m, t = np.array(4000), torch.tensor(4000, device=dev)
+    for n in (4000, 200, 1000):
+        m[()] = n
+        t.fill_(n)
+        for given in (m, t, np.int64(n), n):
+            cache._partials.clear()
+            cache.attention(q, slots, 1.0, max_len=given)
+            assert list(cache._partials) == [(2, 8, launch_nsplit(2, 8, n, True))]
