@@ -1605,16 +1605,29 @@ static int plan_units(int B, int n_kv, int nsplit, long max_tiles, bool wide = f
   return 8 * max_tiles >= blocks * nsplit ? units : 0;
 }
 
+// A single row has nothing to share out: its splits are of one length, and where they are more than eight-wave blocks fit the chip, the second round, or half of one, comes
+// on top.  Paged, one row of 65536 tokens, us, splits as of choose_nsplit / these / twice as many: 8 kv heads of 4 query heads 73 (256 splits) / 37.6 (32) / 37.9, 4 of
+// 6 46.6 / 24.6 / 27.6, 2 of 8 27.6 / 19.4 / 27.6, 16 of 2 98 (128) / 65.8 / 65.1; of 16000 tokens 19.2 (62) / 17.2, 13.9 (62, as asked), 13.2 (as asked), 34.5 (62) / 23.5 / 22.8.
+// That holds with CUs left over as well (wide_splits is for rows that are shared out, which gain from more blocks): as asked / these, of 2000, 8000 and 32000 tokens, 52 heads
+// of 2 query heads (208 CUs) 17.6 / 16.3, 52 / 35, 126 / 110; 72 (216) 18.0 / 18.3, 63 / 43, 160 / 146; 96 (192) 27 / 22, 75 / 59, 205 / 203; 110 (220) 32 / 22, 80 / 60, 231 / 218.
+// From 129 heads on that would be one split a head, and the blocks of long rows are better the smaller ones, two to a CU, in one round if that is
+// nearly full or the row is short; as asked / one split / these, of 700, 2000, 8000 and 24000 tokens: 129 heads 19 / 17 / 17, 34 / 33 / 27, 89 / 104 / 74, 204 / 337 / 204; 160
+// 19 / 17 / 17, 41 / 34 / 27, 102 / 110 / 81, 249 / 341 / 228; 200 19 / 17 / 17, 49 / 35 / 35, 119 / 107 / 106, 302 / 353 / 302; 256 20 / 18 / 18, 62 / 38 / 38, 144 / 123 / 122, 377 / 388 /
+// 354; 320 29 / 25 / 25, 70 / 57 / 57, 175 / 199 / 175, 476 / 680 / 476; 512 37 / 28 / 28, 89 / 66 / 66, 259 / 238 / 238, 718 / 783 / 718.
+static long single_row_splits(int n_kv, int nsplit, long max_tiles) {
+  if (n_kv <= 128) return 256 / n_kv;
+  const long n = 512 / n_kv;                                              // splits of four-wave blocks that fit the chip: 3, 2, 1, 0
+  if (max_tiles <= 128) return n == 3 && nsplit >= 3 ? 3 : 1;             // (two splits of 129 heads are four-wave blocks too, but hardly more than CUs)
+  const bool one_round = max_tiles <= 640 ? n >= 2 || (n == 1 && n_kv >= 384) : n >= 2 && n * n_kv >= 448;
+  return one_round ? n : nsplit;
+}
 // Splits of a planned launch: no more than twice the resident blocks' worth.  A plan of one round leaves the other blocks without a part, and they start,
 // look at the rows and are waited for behind the others; of several rounds, two do, as a row that needs more splits than the others gets them (SIZED_SPLIT).
 // Paged, 8 kv heads, us, the caller's splits / these: 32 rows of 500..20000 tokens, 8 splits 168 / 166, 24 splits 181 / 165; 16 of 9000..11000 92 / 88, 20 of
 // 39000..40000 405 / 385; 128 of 100..4000 x 4 heads, 4 splits 97 / 70; 64 of 2000, one of them 16000, 4 splits 120 / 111.
-// A single row has nothing to share out: its splits are of one length, and where they are more than eight-wave blocks fit the chip, the second round, or half of one, comes
-// on top.  Paged, one row of 65536 tokens, us, splits as of choose_nsplit / these / twice as many: 8 kv heads of 4 query heads 73 (256 splits) / 37.6 (32) / 37.9, 4 of
-// 6 46.6 / 24.6 / 27.6, 2 of 8 27.6 / 19.4 / 27.6, 16 of 2 98 (128) / 65.8 / 65.1; of 16000 tokens 19.2 (62) / 17.2, 13.9 (62, as asked), 13.2 (as asked), 34.5 (62) / 23.5 / 22.8.
-static int planned_splits(int B, int n_kv, int nsplit, int plan, long least) {      // least: for splits that the paged kernel's tile table holds
+static int planned_splits(int B, int n_kv, int nsplit, int plan, long max_tiles, long least) {      // least: for splits that the paged kernel's tile table holds
   const long heads = (long)B * n_kv;
-  if (B == 1) return (int)std::min<long>(nsplit, std::max<long>({256 / n_kv, least, 1}));
+  if (B == 1) return (int)std::min<long>(nsplit, std::max(single_row_splits(n_kv, nsplit, max_tiles), least));
   return plan >= B ? (int)std::min<long>(nsplit, std::max((1024 + heads - 1) / heads, least)) : nsplit;
 }
 
@@ -1659,7 +1672,7 @@ static int attn_split_impl(
   GAAC_REQUIRE(S_pad > 0 && S_pad <= (1 << 24), "gaac_attn: at most %d tokens per cache head (32-bit byte offsets inside a head)", 1 << 24);
   if (epoch && S_all >= 0) nsplit = host_splits((S_all + T - 1) / T, nsplit);
   const int plan = epoch && S_all < 0 ? plan_units(B, n_kv, nsplit, S_pad / T) : 0;
-  if (epoch && S_all < 0) nsplit = planned_splits(B, n_kv, nsplit, plan, 1);
+  if (epoch && S_all < 0) nsplit = planned_splits(B, n_kv, nsplit, plan, S_pad / T, 1);
   const int nslot = nsplit;
   AttnArgs A;
   A.k = StoreView{smk, ck, fk, tok, ovk, ohsk, b3k, b4k};
@@ -1853,7 +1866,7 @@ extern "C" int gaac_paged_attn(
   const int cut = wide_splits(B, n_kv, nsplit, max_tiles, least);
   const int plan = plan_units(B, n_kv, cut, max_tiles, cut < nsplit);
   nsplit = cut;
-  nsplit = planned_splits(B, n_kv, nsplit, plan, least);
+  nsplit = planned_splits(B, n_kv, nsplit, plan, max_tiles, least);
   AttnArgs A;
   A.k = StoreView{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, b3k, b4k};
   A.v = StoreView{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, b3v, b4v};

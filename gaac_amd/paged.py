@@ -19,7 +19,7 @@ SM_OFF, CD_OFF, FL_OFF, OVF_OFF = 0, 2048, 2816, 2880   # byte layout of a tile 
 def choose_nsplit(B: int, n_kv: int, S: int, target_ctas: int = 2048, min_tok: int = 256, cap: int = 256) -> int:
     """Splits per (row, kv head) for the longest sequence S of the batch, at least min_tok tokens each.  An upper bound: sequences of a
     serving batch differ in length, and a launch over two rows or more shares 512 resident blocks, or 1024 in two rounds, out by the lengths it
-    finds on the device; rows of few heads in all, or a single row, get as many as fill 256 blocks.  (Any split count works; a split of more than 1024 tiles leaves the prefetch pipeline after its first 1024
+    finds on the device; rows of few heads in all, or a single row, get as many as fill one round of blocks.  (Any split count works; a split of more than 1024 tiles leaves the prefetch pipeline after its first 1024
     and is slower from there on.)"""
     return max(min(max(1, target_ctas // (B * n_kv)), max(1, S // min_tok), cap), 1)
 

@@ -143,7 +143,7 @@ int gaac_attn_combine(const float* pm, const float* pl, const float* pa, void* o
  * S_all >= 0: every cache head the launch addresses holds exactly S_all compressed tokens (a Page: lengths are known to the host);
  * SL is then not read and may be NULL, which takes one dependent load off the start of every block, and nsplit is an upper bound: no split
  * but the last gets fewer than four tiles.  S_all < 0: lengths come from SL, and a launch of two rows or more may share up to B * nsplit splits
- * out by the rows' lengths, one of a single row makes no more than 256 / n_kv (one at least). */
+ * out by the rows' lengths, one of a single row may make fewer. */
 int gaac_attn_fused(
     const uint8_t* smk, const uint8_t* ck, const int* fk, const int* tok, const uint8_t* ovk, const int* ohsk, const uint8_t* b3k, const uint8_t* b4k,
     const uint8_t* smv, const uint8_t* cv, const int* fv, const int* tov, const uint8_t* ovv, const int* ohsv, const uint8_t* b3v, const uint8_t* b4v,
@@ -215,7 +215,7 @@ int gaac_paged_decode(const uint8_t* pool, int TS, const void* raw, const int* m
  * bt int32 [B][bt_stride] and the mode table; seq_lens int32 [B] (tokens incl. the filling block; no separate tail); max_seq_len =
  * an upper bound of seq_lens known to the host (checked against the block table's width).  Any nsplit >= 1 works for any length (a
  * block resolves 1024 tiles of its split at a time); two rows or more may share up to B * nsplit splits out by their lengths; a single row, or rows of up to
- * 64 heads in all, may be given as few as 256 / (B * n_kv) splits (one at least, and none of more than 1024 tiles of max_seq_len).  Partial records pm, pl [B*n_q*nsplit], pa [B*n_q*nsplit*128] and the epoch
+ * 64 heads in all, may be given fewer (one at least, and none of more than 1024 tiles of max_seq_len).  Partial records pm, pl [B*n_q*nsplit], pa [B*n_q*nsplit*128] and the epoch
  * buffer [2 + B*n_kv*nsplit] as in gaac_attn_fused; out bf16 [B*n_q][128].
  * freeq != NULL: the launch also does the work of gaac_paged_free(freeq, n_free, stack, top) for the queue the preceding
  * gaac_paged_store filled (the attention pops nothing, so pushes cannot race a pop here): a decode step is then two launches
