@@ -1131,7 +1131,14 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, a = lane & 15, q = lane >> 4;
   Bases B;
   TileTable TT{tile_table, tlo};
-  bool any_raw = false;
+  // Waves that the split's raw tiles are shared out to, in turn.  Most splits have none or one, the filling block's: then wave 0 at most, and no further partial to merge.
+  // (A second wave that looked for itself, and its partial in every merge: one row of 300 tokens x 8 kv heads 10.3 -> 11.1 us, of 900 12.0 -> 12.4, 12 of 130..460 x 4 13.0 -> 13.2.)
+  int raws = 0;
+  bool two_raws = false;      // ... in any of the split's rounds
+  const auto count_raws = [&](bool raw) {      // (threads with a raw tile: one that has two, 512 apart, leaves both to wave 0)
+    raws = RAWS > 1 ? min(__syncthreads_count(raw), RAWS) : (int)__syncthreads_or(raw);
+    two_raws |= raws > 1;
+  };
   if (PAGED) {
     // logical tile -> block table -> mode table (paged_kernel.py:137-138), resolved once per block into LDS
     B.kov = B.vov = A.pool; B.TS = A.TS;
@@ -1143,7 +1150,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
       tile_table[i] = e;
       raw |= (e.x | e.y) < 0;
     }
-    any_raw = __syncthreads_or(raw);
+    count_raws(raw);
   } else {
     const long rowb = (long)ch * A.S_pad, tileb = (long)ch * (A.S_pad / T);
     // (the escape streams start at head_start[ch], a loaded value: they are set where the first escape bytes are fetched, so that the
@@ -1211,17 +1218,9 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
       raw_rows_store(rs, a, q, M.m[NW], M.l[NW], M.acc[NW]);
     }
   }
-  // Paged pool, wave 0, or waves 0 and 1 in turn (RAWS): the tiles c0 .. c1 - 1, whose entries the table holds, that have a raw side (the block that is still filling, or
+  // Paged pool, wave 0, or waves 0 and 1 in turn (raws): the tiles c0 .. c1 - 1, whose entries the table holds, that have a raw side (the block that is still filling, or
   // escapes that did not fit the slot).  Raw sides are read in place, the compressed side of a half raw tile is decoded into LDS.
   const auto attend_raw_tiles = [&](int c0, int c1) {
-    if (RAWS > 1 && wave != 0) {      // most splits have the filling block's tile at most: no query loads and no partial for none (9 rows of 150..400 x 8 kv heads with the store 15.8 -> 15.0 us)
-      int n = 0;
-      for (int i0 = 0; i0 < c1 - c0; i0 += 64) {
-        const int2 e = tile_table[min(i0 + lane, c1 - c0 - 1)];
-        n += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i0 + lane < c1 - c0 && (e.x | e.y) < 0));
-      }
-      if (n < 2) return;
-    }
     RawState rs;
     u32x4 qr[4];
     raw_queries(A.q + qh0 * D, G, a, q, qr);
@@ -1232,7 +1231,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     for (int i0 = 0; i0 < c1 - c0; i0 += 64) {
       const int2 own = tile_table[min(i0 + lane, c1 - c0 - 1)];
       for (u64 left = __builtin_amdgcn_ballot_w64(i0 + lane < c1 - c0 && (own.x | own.y) < 0); left != 0; left &= left - 1) {
-        if (RAWS > 1 && (other++ & 1) != 0) continue;      // (the other wave's)
+        if (RAWS > 1 && raws > 1 && (other++ & 1) != 0) continue;      // (the other wave's)
         const int l = __builtin_ctzll(left), ex = __builtin_amdgcn_readlane(own.x, l), ey = __builtin_amdgcn_readlane(own.y, l);
         const u16* krows = decoded; const u16* vrows = decoded;
         wave_lds_sync();
@@ -1252,7 +1251,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     }
     raw_rows_store(rs, a, q, M.m[NW + wave], M.l[NW + wave], M.acc[NW + wave]);
   };
-  if (PAGED && any_raw && wave < RAWS) attend_raw_tiles(tlo, thi_fast);
+  if (PAGED && wave < raws) attend_raw_tiles(tlo, thi_fast);
 
   if (!PAGED) { B.kov = A.k.ovf + __builtin_amdgcn_readfirstlane((int)khs); B.vov = A.v.ovf + __builtin_amdgcn_readfirstlane((int)vhs); }
   if (NW == 4 && R.first && n_own >= PRIO_TILES && (blockIdx.x & 256u) != 0u && wave < 2) __builtin_amdgcn_s_setprio(1);
@@ -1305,9 +1304,9 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
           tile_table[i] = e;
           raw |= (e.x | e.y) < 0;
         }
-        any_raw = __syncthreads_or(raw);
+        count_raws(raw);
         TT.tlo = c0;
-        if (any_raw && wave < RAWS) attend_raw_tiles(c0, c1);
+        if (wave < raws) attend_raw_tiles(c0, c1);
       }
       // first round: only the partial tile is left, for the first wave that has no tile of its own, if there is one (it waits for tag words,
       // then for escape bytes: behind wave 0's own tiles 1000 tokens x 8 kv heads in 16 splits took 9.6 us instead of 8.6)
@@ -1347,22 +1346,22 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   // the lines).  Latency: reads, exponentials, stores; one pass where it was two for more query heads than half the waves.  Paged, 8 sequences of 200..3000
   // tokens x 8 kv heads 23.6 -> 23.1 us with the store, 4000 tokens x 1 kv head of 16 10.1 -> 9.6.  (Without the barrier between this and the split
   // merge, which then needs LDS of its own: 64K x 4 of 6 22.3 -> 22.8.)
-  const auto merge_block = [&](auto channels, int g, int c0) {
-    constexpr int C = decltype(channels)::value;
+  const auto merge_block = [&](auto channels, auto partials, int g, int c0) {
+    constexpr int C = decltype(channels)::value, P = decltype(partials)::value;
     // every LDS read up front and none under a branch: nine dependent round trips otherwise
-    float mv[NW + RAWS], lv[NW + RAWS], av[NW + RAWS][C];
+    float mv[P], lv[P], av[P][C];
 #pragma unroll
-    for (int w = 0; w < NW + RAWS; ++w) {
+    for (int w = 0; w < P; ++w) {
       mv[w] = M.m[w][g]; lv[w] = M.l[w][g];
 #pragma unroll
       for (int c = 0; c < C; ++c) av[w][c] = M.acc[w][g][c0 + 64 * c + lane];
     }
     float Mx = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < NW + RAWS; ++w) Mx = fmaxf(Mx, mv[w]);
+    for (int w = 0; w < P; ++w) Mx = fmaxf(Mx, mv[w]);
     float Lc = 0.f, Ac[C] = {};
 #pragma unroll
-    for (int w = 0; w < NW + RAWS; ++w) {
+    for (int w = 0; w < P; ++w) {
       const bool live = mv[w] != -INFINITY;          // an empty partial's accumulator may hold anything
       const float f = live ? __builtin_amdgcn_exp2f(mv[w] - Mx) : 0.f;
       Lc += lv[w] * f;
@@ -1385,8 +1384,12 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     }
   };
   // two waves to a head while that is one pass, else one
-  if (2 * G <= NW) { if (wave < 2 * G) merge_block(std::integral_constant<int, 1>{}, wave >> 1, 64 * (wave & 1)); }
-  else for (int g = wave; g < G; g += NW) merge_block(std::integral_constant<int, 2>{}, g, 0);
+  const auto merge_partials = [&](auto partials) {
+    if (2 * G <= NW) { if (wave < 2 * G) merge_block(std::integral_constant<int, 1>{}, partials, wave >> 1, 64 * (wave & 1)); }
+    else for (int g = wave; g < G; g += NW) merge_block(std::integral_constant<int, 2>{}, partials, g, 0);
+  };
+  if (RAWS > 1 && two_raws) merge_partials(std::integral_constant<int, NW + RAWS>{});
+  else merge_partials(std::integral_constant<int, NW + 1>{});
   GAAC_STAMP(4);
   if (fused && A.nslot > 1 && ((rank >= 0 && ns > 1) || blockIdx.x == gridDim.x - 1)) {
     lds_barrier();      // every thread is done with the block-merge buffer, which becomes the mergers' scratch

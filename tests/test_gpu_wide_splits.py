@@ -66,3 +66,28 @@ def test_raw_tiles(lens, n_kv, G, kinds):
         outs.append([layer.attention(q, pool, torch.from_numpy(bt).to(dev), sl, n).float() for n in (1, 3, 64)])
         layer.check()
     for got in outs[0] + outs[1]: assert_rows_close(got, outs[0][0])
+
+
+# raw tiles among 1200 of a split: none, one, two of one thread of the block (512 apart) and of two, in the first 1024 tiles and in those behind them
+@pytest.mark.parametrize("raw", [(), (5,), (5, 517), (5, 6), (5, 6, 7), (1030,), (1030, 1031), (5, 1100), (5, 1100, 1101), (5, 6, 1100), (0, 1023, 1024, 1198)])
+@pytest.mark.parametrize("G", [2, 6])
+def test_counts_of_raw_tiles(raw, G):
+    dev = require_gpu()
+    from gaac_amd.codec import bases_from_hist, exponent_hist
+    from gaac_amd.paged import LayerState, build_store_entries
+    gen = torch.Generator(device=dev).manual_seed(G + sum(raw))
+    n, L = 1200, 1200 * 16
+    k, v = (torch.randn(L, 1, 128, generator=gen, device=dev) for _ in range(2))
+    for t in raw:      # exponents all over: escapes beyond a slot's room
+        for x in (k, v): x[16 * t:16 * t + 16] *= torch.exp2(torch.randint(-24, 5, (16, 1, 128), generator=gen, device=dev).float())
+    k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+    b3, b4 = bases_from_hist(exponent_hist(k, 1), 1)
+    layer = LayerState(n, 1, 2 * n, dict(k3=b3, k4=b4, v3=b3, v4=b4), device=dev)
+    pool, bt = torch.zeros(LayerState.pool_bytes(n, 1), dtype=torch.uint8, device=dev), np.arange(n, dtype=np.int32).reshape(1, n)
+    layer.store(k, v, pool, torch.from_numpy(build_store_entries([0], [L], bt)).to(dev))
+    assert (layer.mt < 0).nonzero().flatten().tolist() == [2 * t + j for t in raw for j in range(2)]
+    q = (torch.randn(1, G, 128, generator=gen, device=dev) * 0.5).to(torch.bfloat16)
+    p = torch.softmax(q[0].double() @ k[:, 0].double().T * 128 ** -0.5, -1)
+    want = (p @ v[:, 0].double()).float()[None]
+    for nsplit in (1, 2): assert_rows_close(layer.attention(q, pool, torch.from_numpy(bt).to(dev), torch.tensor([L], dtype=torch.int32, device=dev), nsplit).float().view(1, G, 128), want)
+    layer.check()
