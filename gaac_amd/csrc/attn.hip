@@ -1136,7 +1136,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   int raws = 0;
   bool two_raws = false;      // ... in any of the split's rounds
   const auto count_raws = [&](bool raw) {      // (threads with a raw tile: one that has two, 512 apart, leaves both to wave 0)
-    raws = RAWS > 1 ? min(__syncthreads_count(raw), RAWS) : (int)__syncthreads_or(raw);
+    raws = __builtin_amdgcn_readfirstlane(RAWS > 1 ? min(__syncthreads_count(raw), RAWS) : (int)(__syncthreads_or(raw) != 0));
     two_raws |= raws > 1;
   };
   if (PAGED) {

@@ -650,15 +650,20 @@ __device__ __forceinline__ void prompt_fused_body(const PromptFusedArgs& P, Enco
   const EncodeKind& J = KIND == KIND_K ? A.k : A.v;
   const PromptKind& K = P.s.j[KIND];
   const int ntiles = A.ntiles, block = blockIdx.x, tile = block * CODEC_WAVES + wave, brow = (A.brow0 + h) % A.NB;
+  const int spins = P.scan.spins;
+  asm volatile("" ::"s"(spins));      // with the other arguments: fetched where it is first used, behind the encoder, it made the launch 0.45 us longer
   u64* scan = P.scan.k + (KIND == KIND_V ? P.scan.v : 0) + (long)h * P.scan.row;
   const u16* xh = J.x + (long)h * J.head_stride;
   RowRegs R;
   load_rows<false>(R, xh + (long)min(tile, ntiles - 1) * T * J.row_stride, J.row_stride, T, lane);
   if (wave == 0) reinterpret_cast<u32x2*>(&L.B.w[0][0])[lane] = load_base_pair<KIND>(J.b3 + (long)brow * D, J.b4 + (long)brow * D, lane);
   u32* state = reinterpret_cast<u32*>(scan);      // epoch | whether a block gave up
-  const u32 last = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), epoch = last + (last == 0xFFFFFFFFu ? 2u : 1u);      // (0 is what the words start with)
-  const int head_start = P.head_start[h];
+  const u32 loaded_epoch = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int loaded_start = P.head_start[h];
   store_rows(L.w[wave], R, lane);
+  // (waited for with the rows: where they are used the wait would be for the encoder's stores as well)
+  const u32 last = (u32)__builtin_amdgcn_readfirstlane((int)loaded_epoch), epoch = last + (last == 0xFFFFFFFFu ? 2u : 1u);      // (0 is what the words start with)
+  const int head_start = __builtin_amdgcn_readfirstlane(loaded_start);
   __syncthreads();
   int total = 0;
   const uint8_t* escapes = nullptr;
@@ -678,7 +683,7 @@ __device__ __forceinline__ void prompt_fused_body(const PromptFusedArgs& P, Enco
     u64 v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     bool ok = true;
     for (int spin = 0; __builtin_amdgcn_ballot_w64(lane < block && (u32)(v >> 32) != epoch) != 0; ++spin) {
-      if (spin >= P.scan.spins) { ok = false; break; }
+      if (spin >= spins) { ok = false; break; }
       __builtin_amdgcn_s_sleep(1);
       if ((u32)(v >> 32) != epoch) v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -687,7 +692,7 @@ __device__ __forceinline__ void prompt_fused_body(const PromptFusedArgs& P, Enco
     if (lane == 0) {
       ahead = ok ? before : -1;
       if (!ok) __hip_atomic_store(state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      else if (block == (int)gridDim.x - 1) {
+      else if (block == (ntiles - 1) / CODEC_WAVES) {
         P.s.head_bytes[KIND * P.s.n_kv + h] = before + own;
         __hip_atomic_store(state, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
@@ -711,21 +716,22 @@ __global__ void __launch_bounds__(64 * CODEC_WAVES) k_prompt_fused(const PromptF
   if (blockIdx.z == KIND_K) prompt_fused_body<KIND_K>(P, L, sizes, ahead, blockIdx.y, wave, lane);
   else prompt_fused_body<KIND_V>(P, L, sizes, ahead, blockIdx.y, wave, lane);
 }
-// The total of one kind of a head, -1 where a block gave up (the words are then zeroed for the next launch: all blocks are through).
-__device__ __forceinline__ int fused_total(int head_bytes, u64* scan, int row) {
-  if (reinterpret_cast<const u32*>(scan)[1] == 0u) return head_bytes;
-  for (int i = 0; i < row; ++i) scan[i] = 0ull;      // (all of them: the epoch starts again from 1, which older launches may have left)
-  return -1;
-}
 // ... and the counters of the heads, with the totals in host memory as k_words_to_host puts them there.
 __global__ void __launch_bounds__(64) k_prompt_finish(const PromptScanArgs A, const ScanWords W, int* __restrict__ host) {
   for (int h = threadIdx.x; h < A.n_kv; h += 64) {
-    u64* words = W.k + (long)h * W.row;
-    const int k = fused_total(A.head_bytes[h], words, W.row), v = fused_total(A.head_bytes[A.n_kv + h], words + W.v, W.row);
-    const int failed = (k | v) < 0 ? 0x7FFFFFFF : 0;      // (a total that fits no window)
-    set_prompt_counters(A, KIND_K, h, max(k, failed), max(v, failed));
-    set_prompt_counters(A, KIND_V, h, max(v, failed), max(k, failed));
-    A.head_bytes[h] = k; A.head_bytes[A.n_kv + h] = v;
+    u64 *kw = W.k + (long)h * W.row, *vw = kw + W.v;
+    // (one trip to memory for all four; the rest is as if none had given up, where none has)
+    const u32 k_gave_up = reinterpret_cast<const u32*>(kw)[1], v_gave_up = reinterpret_cast<const u32*>(vw)[1];
+    int k = A.head_bytes[h], v = A.head_bytes[A.n_kv + h];
+    const bool failed = (k_gave_up | v_gave_up) != 0u;
+    k = k_gave_up ? -1 : k; v = v_gave_up ? -1 : v;
+    const int least = failed ? 0x7FFFFFFF : 0;      // (a total that fits no window)
+    set_prompt_counters(A, KIND_K, h, max(k, least), max(v, least));
+    set_prompt_counters(A, KIND_V, h, max(v, least), max(k, least));
+    if (failed) {      // all blocks are through: the words start anew (all of them: the epoch is 1 next, which an old launch may have left)
+      A.head_bytes[h] = k; A.head_bytes[A.n_kv + h] = v;
+      for (int i = 0; i < W.row; ++i) { if (k_gave_up) kw[i] = 0ull; if (v_gave_up) vw[i] = 0ull; }
+    }
     if (host) { store_to_host(host + h, k); store_to_host(host + A.n_kv + h, v); }
   }
 }
