@@ -1048,7 +1048,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   // in an eight-wave block, us: 8 rows of 200..3000 tokens 48 / 33, 4 of 1000..9000 65 / 43, one of 30000 88 / 55.
   constexpr int RAWS = PAGED && NW == 8 ? 2 : 1;
   // one LDS object so that the tables the tile loop reads sit at the lowest addresses (immediate offsets of the LDS loads)
-  struct BlockLds { AttnLds L; int next_tile; int2 tile_table[PAGED ? MAX_CHUNK : 1]; MergeLds<NW, RAWS> M; };
+  struct BlockLds { AttnLds L; int next_tile, two_raws; int2 tile_table[PAGED ? MAX_CHUNK : 1]; MergeLds<NW, RAWS> M; };
   static_assert(offsetof(BlockLds, M.acc) % 16 == 0, "the block merge's accumulators are stored and a decoded raw tile is read 16 bytes at a time");
   __shared__ BlockLds lds;
   AttnLds& L = lds.L; MergeLds<NW, RAWS>& M = lds.M; int2* tile_table = lds.tile_table; int& next_tile = lds.next_tile;
@@ -1132,12 +1132,12 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
   Bases B;
   TileTable TT{tile_table, tlo};
   // Waves that the split's raw tiles are shared out to, in turn.  Most splits have none or one, the filling block's: then wave 0 at most, and no further partial to merge.
-  // (A second wave that looked for itself, and its partial in every merge: one row of 300 tokens x 8 kv heads 10.3 -> 11.1 us, of 900 12.0 -> 12.4, 12 of 130..460 x 4 13.0 -> 13.2.)
+  // (A second wave that looked for itself, and its partial in every merge: one row of 300 tokens x 8 kv heads 10.4 -> 11.2 us, of 900 11.9 -> 12.4, 12 of 130..460 x 4 13.1 -> 13.2.)
   int raws = 0;
-  bool two_raws = false;      // ... in any of the split's rounds
-  const auto count_raws = [&](bool raw) {      // (threads with a raw tile: one that has two, 512 apart, leaves both to wave 0)
-    raws = __builtin_amdgcn_readfirstlane(RAWS > 1 ? min(__syncthreads_count(raw), RAWS) : (int)(__syncthreads_or(raw) != 0));
-    two_raws |= raws > 1;
+  const auto count_raws = [&](bool raw, bool first) {      // (threads with a raw tile: one that has two, 512 apart, leaves both to wave 0)
+    raws = RAWS > 1 ? min(__syncthreads_count(raw), RAWS) : (int)__syncthreads_or(raw);
+    // whether any round of the split has two, for the merge: in LDS, as a register for it costs the tile loop (20 rows of 100..500 x 8 14.2 -> 14.05)
+    if (RAWS > 1 && tid == 0 && (first || raws > 1)) lds.two_raws = raws > 1;
   };
   if (PAGED) {
     // logical tile -> block table -> mode table (paged_kernel.py:137-138), resolved once per block into LDS
@@ -1150,7 +1150,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
       tile_table[i] = e;
       raw |= (e.x | e.y) < 0;
     }
-    count_raws(raw);
+    count_raws(raw, true);
   } else {
     const long rowb = (long)ch * A.S_pad, tileb = (long)ch * (A.S_pad / T);
     // (the escape streams start at head_start[ch], a loaded value: they are set where the first escape bytes are fetched, so that the
@@ -1226,12 +1226,19 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     raw_queries(A.q + qh0 * D, G, a, q, qr);
     raw_rows_load(rs, a, q, M.m[NW + wave], M.l[NW + wave], M.acc[NW + wave]);
     u16* decoded = reinterpret_cast<u16*>(&M.acc[wave][0][0]);      // (the wave's own place in the block merge)
-    int other = wave;
+    int turn = wave;      // even: the next raw tile is this wave's
     const long boff = (long)(ch % A.NB) * D;
     for (int i0 = 0; i0 < c1 - c0; i0 += 64) {
       const int2 own = tile_table[min(i0 + lane, c1 - c0 - 1)];
-      for (u64 left = __builtin_amdgcn_ballot_w64(i0 + lane < c1 - c0 && (own.x | own.y) < 0); left != 0; left &= left - 1) {
-        if (RAWS > 1 && raws > 1 && (other++ & 1) != 0) continue;      // (the other wave's)
+      const bool raw = i0 + lane < c1 - c0 && (own.x | own.y) < 0;
+      u64 left = __builtin_amdgcn_ballot_w64(raw);
+      if (RAWS > 1 && raws > 1) {      // every other one
+        const int ahead = __builtin_amdgcn_mbcnt_hi((u32)(left >> 32), __builtin_amdgcn_mbcnt_lo((u32)left, 0));
+        const int next = turn + __builtin_popcountll(left);
+        left = __builtin_amdgcn_ballot_w64(raw && ((turn + ahead) & 1) == 0);
+        turn = next;
+      }
+      for (; left != 0; left &= left - 1) {
         const int l = __builtin_ctzll(left), ex = __builtin_amdgcn_readlane(own.x, l), ey = __builtin_amdgcn_readlane(own.y, l);
         const u16* krows = decoded; const u16* vrows = decoded;
         wave_lds_sync();
@@ -1304,7 +1311,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
           tile_table[i] = e;
           raw |= (e.x | e.y) < 0;
         }
-        count_raws(raw);
+        count_raws(raw, false);
         TT.tlo = c0;
         if (wave < raws) attend_raw_tiles(c0, c1);
       }
@@ -1388,7 +1395,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const A
     if (2 * G <= NW) { if (wave < 2 * G) merge_block(std::integral_constant<int, 1>{}, partials, wave >> 1, 64 * (wave & 1)); }
     else for (int g = wave; g < G; g += NW) merge_block(std::integral_constant<int, 2>{}, partials, g, 0);
   };
-  if (RAWS > 1 && two_raws) merge_partials(std::integral_constant<int, NW + RAWS>{});
+  if (RAWS > 1 && __builtin_amdgcn_readfirstlane(lds.two_raws)) merge_partials(std::integral_constant<int, NW + RAWS>{});
   else merge_partials(std::integral_constant<int, NW + 1>{});
   GAAC_STAMP(4);
   if (fused && A.nslot > 1 && ((rank >= 0 && ns > 1) || blockIdx.x == gridDim.x - 1)) {
