@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from gpu_util import require_gpu
-from test_gpu_short_prompts import _check, _rows
+from test_gpu_short_prompts import _check, _rows, _words
 
 pytestmark = pytest.mark.gpu
 GUARD = 64
@@ -14,13 +14,6 @@ GUARD = 64
 def large_blocks_go_back():
     yield
     torch.cuda.empty_cache()      # (a workspace that outlives a later test would hold on to one)
-
-
-def _words(cache, slot, k, v):
-    """The arguments that both take, up to the stores'."""
-    L, n_kv = k.shape[0], cache.n_kv
-    return [k, v, 128, n_kv * 128, 128, n_kv * 128, L, n_kv, slot * n_kv, cache.cap, cache.k.ovf_cap, cache.k.base3.shape[0], int(cache.per_sequence_bases), cache.tail_len, cache.S,
-            cache.k.head_start, *cache.k.kernel_args(), *cache.v.kernel_args()]
 
 
 # at 102 tiles a head's escapes have room for one table, at 103 for two, at 65536 tokens one table no longer counts them

@@ -1,6 +1,6 @@
 """Prompts whose blocks place their escapes among themselves, at the edges of the blocks (four tiles, 64 blocks) and on both sides of the lines to the two
 launches (256 tiles a head, 3072 of all): every field of the slot against a page of the same rows, slots put in again and again, windows that are too small, the
-epoch's wrap-around, prompts into two slots on two streams, a wait that failed, a block that gave up."""
+epoch's wrap-around, prompts into two slots on two streams at once, replays of a graph, a wait that failed, a block that gave up."""
 import pytest
 import torch
 
@@ -72,18 +72,64 @@ def test_windows_that_have_to_grow(many):
     _check(cache, 1, k0, v0)
 
 
+def _words(cache, slot, k, v):
+    """The arguments that gaac_prompt_store and gaac_cache_prefill both take, up to the stores'."""
+    L, n_kv = k.shape[0], cache.n_kv
+    return [k, v, 128, n_kv * 128, 128, n_kv * 128, L, n_kv, slot * n_kv, cache.cap, cache.k.ovf_cap, cache.k.base3.shape[0], int(cache.per_sequence_bases), cache.tail_len, cache.S,
+            cache.k.head_start, *cache.k.kernel_args(), *cache.v.kernel_args()]
+
+
+def _bases(n_kv): return dict.fromkeys(("k3", "v3"), torch.full((n_kv, 128), 122)) | dict.fromkeys(("k4", "v4"), torch.full((n_kv, 128), 118))
+
+
+def _scratch(L, n_kv):
+    """Slots, bytes of the tiles, bytes of the heads."""
+    nt = 2 * n_kv * (L // 16)
+    return [torch.empty(n, dtype=torch.uint8, device="cuda") for n in (nt * 1280, nt * 4, 8 * n_kv)]
+
+
 def test_two_streams():
+    """Launches of two slots in flight together: both streams wait for a third before each pair, and the host waits for neither until both have theirs."""
     require_gpu()
-    from gaac_amd import CompressedKVCache
-    cache = CompressedKVCache(2, 8, 800)
-    rows = [[_rows(777, 8, 10 * i + j, 1e-3) for j in range(2)] for i in range(2)]
-    streams = [torch.cuda.Stream() for _ in range(2)]
+    from gaac_amd import CompressedKVCache, _lib
+    cache = CompressedKVCache(2, 8, 800, _bases(8))
+    rows = [[[_rows(777, 8, 10 * i + j, 1e-3) for j in range(2)] for i in range(2)] for _ in range(3)]
+    streams, first = [torch.cuda.Stream() for _ in range(2)], torch.cuda.Stream()
+    scratch, host = [_scratch(777, 8) for _ in range(2)], [torch.empty(16, dtype=torch.int32, pin_memory=True) for _ in range(2)]
     torch.cuda.synchronize()
-    for _ in range(20):
-        for slot, s in enumerate(streams):
-            with torch.cuda.stream(s): cache.prefill(slot, *rows[slot])
-    torch.cuda.synchronize()
-    for slot in range(2): _check(cache, slot, *rows[slot])
+    for n in range(30):
+        with torch.cuda.stream(first): torch.cuda._sleep(5000000)
+        for s in streams: s.wait_stream(first)
+        for slot in ((0, 1), (1, 0))[n % 2]:
+            _lib.call("gaac_prompt_store", *_words(cache, slot, *rows[n % 3][slot]), None, 0, *scratch[slot], cache._scan[0, 8 * slot:], cache._scan.stride(0), cache._scan.shape[2], 0,
+                      host[slot].data_ptr(), streams[slot].cuda_stream)
+        assert n == 0 or all((h < 0).any() for h in host)      # (neither is through; the first pair sets the streams up)
+        for slot in range(2): _lib.call("gaac_wait_words", host[slot].data_ptr(), 16, streams[slot].cuda_stream)
+        for slot in range(2): _check(cache, slot, *rows[n % 3][slot])
+
+
+def test_replays_of_a_graph():
+    """The launches of a prompt in a graph (without words on the host, which nothing in it could wait for), replayed over new rows, with prompts outside it between the replays."""
+    require_gpu()
+    from gaac_amd import CompressedKVCache, _lib
+    cache = CompressedKVCache(2, 3, 800, _bases(3))
+    k, v, scratch = _rows(777, 3, 1, 1e-3), _rows(777, 3, 2, 1e-3), _scratch(777, 3)
+    def store(stream):
+        _lib.call("gaac_prompt_store", *_words(cache, 1, k, v), None, 0, *scratch, cache._scan[0, 3:], cache._scan.stride(0), cache._scan.shape[2], 0, None, stream)
+    store(_lib.stream)
+    _check(cache, 1, k, v)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph): store(_lib.stream)
+    for n in range(5):
+        other = _rows(100 + 150 * n, 3, 50 + n, 1e-3), _rows(100 + 150 * n, 3, 60 + n, 1e-3)
+        cache.prefill(n % 2, *other)      # into the graph's slot, into the other
+        if n % 2 == 0: _check(cache, 0, *other)
+        k.copy_(_rows(777, 3, 10 + n, 1e-3))
+        v.copy_(_rows(777, 3, 20 + n, 1e-3))
+        graph.replay()
+        if n == 3: graph.replay()
+        torch.cuda.synchronize()
+        _check(cache, 1, k, v)
 
 
 @pytest.mark.parametrize("through", ["binding", "python"])

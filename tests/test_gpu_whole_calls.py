@@ -1,5 +1,5 @@
 """Calls that the binding makes as a whole against the same calls through Python (ctypes), over the forms that either takes: contiguous tensors, strided and
-misaligned ones, other shapes of the slot map, escape streams beyond the room, and what is refused."""
+misaligned ones, other shapes of the slot map, escape streams beyond the room, and what is refused.  Which calls the binding makes, and which it gives back, is checked as well."""
 import warnings
 
 import pytest
@@ -11,14 +11,24 @@ from gpu_util import require_gpu
 pytestmark = pytest.mark.gpu
 
 
+WHOLE = ("attend", "token_append", "prompt_store", "page_encode", "page_decode")
+
+
 @pytest.fixture
 def both(monkeypatch):
-    """both(f): f's results with the binding and with Python's calls."""
+    """both(f): f's results with the binding and with Python's calls; both.made: for each whole call that f came to, whether the binding made it."""
     binding = _lib.calls()
     assert hasattr(binding, "bind")
+    class Watched:
+        def __getattr__(self, name):
+            def call(*a):
+                out = getattr(binding, name)(*a)
+                if name in WHOLE: run.made.setdefault(name, []).append(out is not None)
+                return out
+            return call
     def run(f):
-        out = []
-        for calls in (binding, _lib._CtypesCalls()):
+        out, run.made = [], {}
+        for calls in (Watched(), _lib._CtypesCalls()):
             monkeypatch.setattr(_lib, "_calls", calls)
             try: out.append(f())
             except (RuntimeError, AssertionError, TypeError) as e: out.append((type(e), str(e)))
@@ -49,6 +59,8 @@ FORMS = {      # of rows [n, heads, 128]
     "reversed channels": lambda n, h, seed: _rows((n, 128, h), seed).transpose(1, 2),
     "float": lambda n, h, seed: _rows((n, h, 128), seed).float(),
 }
+IN_PLACE = ("plain", "token stride", "head-major")      # what the encoder reads where it lies
+CONTIGUOUS = ("plain", "misaligned")
 
 
 @pytest.mark.parametrize("form", FORMS)
@@ -65,7 +77,10 @@ def test_pages(both, form, kind):
         w = TileEncoder("v" if kind == "k" else "k").encode(codec, other)
         out = attention(q, *((p, w) if kind == "k" else (w, p)))
         return [getattr(p, n) for n in ("sm", "codes", "flags", "ovf_off", "ovf", "ovf_head_start", "tile_off", "H", "S", "n_kv", "kind")], Codec.decode(p), out
-    _same(*both(f))
+    a, b = both(f)
+    _same(a, b)
+    if form == "float": assert a[0] is RuntimeError and both.made == dict(page_encode=[False])
+    else: assert both.made == dict(page_encode=[form in IN_PLACE, True], attend=[form in CONTIGUOUS or form == "token stride"], page_decode=[True])      # (the query is a single row)
 
 
 def test_a_stream_beyond_its_room(both):
@@ -79,7 +94,7 @@ def test_a_stream_beyond_its_room(both):
         return p.ovf[:-8], p.tile_off, Codec.decode(p).view(torch.int16)
     a, b = both(f)
     _same(a, b)
-    assert torch.equal(a[2], x.view(torch.int16))
+    assert torch.equal(a[2], x.view(torch.int16)) and both.made == dict(page_encode=[True], page_decode=[True])
 
 
 @pytest.mark.parametrize("form", FORMS)
@@ -103,7 +118,19 @@ def test_cache(both, form, L, calibrate):
             return [out, cache.k.ovf_cap, cache.S, cache.tail_len, *cache.decompress(0), *cache.decompress(2)]
         return run
     i = dict(dtype=torch.int32, device="cuda")
-    for slots in (torch.tensor([2, 0], **i), torch.tensor([[2], [-1]], **i), torch.tensor([2, 9, 0, 9], **i)[::2].contiguous(), torch.tensor([2], **i)): _same(*both(f(slots)))
+    for slots in (torch.tensor([2, 0], **i), torch.tensor([[2], [-1]], **i), torch.tensor([2, 9, 0, 9], **i)[::2].contiguous(), torch.tensor([2], **i)):
+        a, b = both(f(slots))
+        _same(a, b)
+        made = both.made
+        if form == "float" and L >= 16:
+            assert a[0] is RuntimeError and not made      # refused ahead of the call
+            continue
+        assert made["prompt_store"] == [L >= 16 and form in IN_PLACE] * 2
+        if slots.numel() == 1 or form == "float":
+            assert a[0] is RuntimeError and made["token_append"] == [False] and len(made) == 2
+            continue
+        assert made["token_append"] == [form in CONTIGUOUS] * 3 and made["attend"] == [form in CONTIGUOUS and slots.dim() == 1]
+        assert all(made.get("page_decode", [True])) and (L < 16 or len(made["page_decode"]) == 4)
 
 
 def test_tensors_without_an_address_and_a_lack_of_memory_raise_as_through_python(both):
