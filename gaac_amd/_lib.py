@@ -69,7 +69,7 @@ def load():
 
 
 class _CtypesCalls:
-    """calls() through ctypes, for any torch: 14 us for an attention() where the binding takes 8 to 11.  The whole calls (binding.cpp) are left to Python."""
+    """calls() through ctypes, for any torch: 14 us for an attention() where the binding takes 9.0, or 7.2 as a whole call (binding.cpp).  These are left to Python."""
     def attend(self, *args): return None
     token_append = prompt_store = page_encode = page_decode = attend
     def __getattr__(self, name):

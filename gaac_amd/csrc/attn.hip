@@ -154,7 +154,7 @@ __device__ __forceinline__ void merge_half_head(const AttnArgs& A, long rec, int
   const int g = lane / CPW, d0 = 64 * half + CPW * wave, d = d0 + lane % CPW;
   const u64* rm = reinterpret_cast<const u64*>(A.pm) + rec;
   const u64* rl = reinterpret_cast<const u64*>(A.pl) + rec;
-  // (a uniform base and a 32-bit offset per lane, at most (MAX_SLOTS - 1) * D + 7 records: the addresses of the first round's loads are
+  // (a uniform base and a 32-bit offset per lane, at most (MAX_SLOTS - 1) * D + 15 records: the addresses of the first round's loads are
   // on the way of every launch.  With 64-bit addresses per lane a launch took 0.05-0.2 us more: 2 rows x 4096 tokens 11.64 against 11.45)
   const u64* ra0 = reinterpret_cast<const u64*>(A.pa) + rec * D + d0;
   const u64* ra = ra0 + lane % CPW;
@@ -1045,7 +1045,7 @@ template <bool PAGED, int NW, bool HOST_LEN>
 __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_split(const AttnArgs A) {
   constexpr int NT = 64 * NW;
   // Raw tiles of the paged pool: a wave for every four of the block, so that a CU has two in either launch form.  Pools of raw tiles only, 8 kv heads, one / two
-  // in an eight-wave block, us: 8 rows of 200..3000 tokens 48 / 33, 4 of 1000..9000 65 / 43, one of 30000 88 / 55.
+  // in an eight-wave block, us: 8 rows of 200..3000 tokens 48 / 31.5, 4 of 1000..9000 65 / 42, one of 30000 88 / 54.4.
   constexpr int RAWS = PAGED && NW == 8 ? 2 : 1;
   // one LDS object so that the tables the tile loop reads sit at the lowest addresses (immediate offsets of the LDS loads)
   struct BlockLds { AttnLds L; int next_tile, two_raws; int2 tile_table[PAGED ? MAX_CHUNK : 1]; MergeLds<NW, RAWS> M; };

@@ -3,7 +3,7 @@
 // an address (the stream) is called for it once the arguments before it have been looked at: without a GPU, a host tensor is what the error names.
 // What it is for: a launch has up to 47 arguments, half of them tensors.  Through ctypes, with is_cuda and data_ptr() called from Python for each
 // tensor, attention() costs the host 14 us, more than the kernel takes over a short context, and a step of append and attention 24; with the
-// arguments converted here 8 to 11 and 12 to 16.
+// arguments converted here 9 and 15, made here as a whole (below) 7 and 12.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <dlfcn.h>
