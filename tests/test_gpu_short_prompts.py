@@ -89,6 +89,20 @@ def _scratch(L, n_kv):
 
 
 def test_two_streams():
+    require_gpu()
+    from gaac_amd import CompressedKVCache
+    cache = CompressedKVCache(2, 8, 800)
+    rows = [[_rows(777, 8, 10 * i + j, 1e-3) for j in range(2)] for i in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for slot, s in enumerate(streams):
+            with torch.cuda.stream(s): cache.prefill(slot, *rows[slot])
+    torch.cuda.synchronize()
+    for slot in range(2): _check(cache, slot, *rows[slot])
+
+
+def test_two_streams_at_once():
     """Launches of two slots in flight together: both streams wait for a third before each pair, and the host waits for neither until both have theirs."""
     require_gpu()
     from gaac_amd import CompressedKVCache, _lib
